@@ -176,15 +176,20 @@ __device__ double wg_sum(double v, double *sh) {
 // then out = R^{-1} (full p x p, zero below the diagonal).  The matrix is held in LDS padded to
 // N = 16 * ceil(p / 16) (row stride N + 1, so that row and column walks of 16 lanes hit distinct
 // banks; the padding is zero and factors as dependent columns) and processed in 16 x 16 tiles:
-//   - one wavefront factors each diagonal tile in registers (lane c holds column c, broadcasts by
-//     lane reads) and inverts it (Dinv_J, kept beside the matrix);
-//   - the panel right of it is X = Dinv_J^T A[J, >J] and the trailing update A[I, T] -= X_I^T X_T,
-//     one FP64 16x16x4 MFMA tile per wavefront;
-//   - R^{-1} fills block columns left to right: X[<J, J] = -(X[<J, <J] R[<J, J]) Dinv_J, the product
-//     staged in the (unused) lower block triangle.
+//   - the 16 rows of tile J are factored in registers, one column per lane: lanes 0..15 of every
+//     wavefront hold the diagonal tile, the others 48 columns of the panel right of it, so the panel's
+//     forward substitution is the same instructions as the tile's factorisation and needs neither the
+//     tile's inverse nor a barrier;
+//   - the trailing update A[I, T] -= X_I^T X_T is one FP64 16x16x4 MFMA tile per wavefront;
+//   - R^{-1}: the diagonal tiles are inverted side by side, one wavefront each, then pairs of
+//     inverted blocks of s = 16, 32, 64 columns are merged: X12 = -X11 (R12 X22).
 // A pivot at or below 1e-14 of the largest diagonal entry (or NaN) marks its column as dependent:
 // its row of R and its row and column of R^{-1} are zero, so that a rank-deficient basis gives
 // zero columns instead of overflowing ones.
+// One workgroup per block, so a launch over few blocks is latency: the 16 p / 16 pivots one after
+// another, each a lane read, a reciprocal square root by Newton-Raphson (a square root and a division
+// were four times as long) and up to 15 multiply-adds.  MI355X, 4 blocks, p = 128: 47.5 us, 10.3 us of
+// it independent of p (99.8 us with a barrier and a tile inverse per pivot block).
 constexpr int kNB = 16;  // tile width of the blocked Cholesky / triangular inverse
 
 typedef double d4 __attribute__((ext_vector_type(4)));
@@ -197,104 +202,87 @@ __device__ __forceinline__ double lane_read(double v, int l) {
     return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
 }
 
-// Factor the 16 x 16 diagonal tile at T (row stride ld) in place (upper triangle R_JJ, zero below)
-// and write its inverse to D (16 x 16, row stride 16, zero below).  Called by a whole wavefront;
-// lanes 16..63 compute alongside and store nothing.
-__device__ __forceinline__ void chol_tile(double *T, int ld, double *D, double tol, int lane) {
-    const int c = lane;
+// 1 / sqrt(d) for 1e-280 < d < 1e280: the hardware estimate and two Newton-Raphson steps
+// y <- y + y (1 - d y^2) / 2 (callers scale their matrices to entries of order one)
+__device__ __forceinline__ double rsqrt_nr(double d) {
+    double y = __builtin_amdgcn_rsq(d);
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const double e = fma(-d * y, y, 1.0);
+        y = fma(0.5 * y, e, y);
+    }
+    return y;
+}
+__device__ __forceinline__ double rcp_nr(double d) {  // 1 / d by two Newton-Raphson steps
+    double y = __builtin_amdgcn_rcp(d);
+#pragma unroll
+    for (int i = 0; i < 2; ++i) y = fma(y, fma(-d, y, 1.0), y);
+    return y;
+}
+
+// Factor the 16 rows of the tile at T (row stride ld; the diagonal tile and the `cols` columns right
+// of it).  Called by a whole wavefront: lanes 0..15 hold the diagonal tile, whose factor goes to D
+// (16 x 16, zero below the diagonal; D null: not stored) because other wavefronts still read T's;
+// lanes 16..63 the columns pc0 .. pc0 + 47 of the panel (those below `cols`), factored in place.  One pivot costs a lane read, a reciprocal square root and 15 - k
+// multiply-adds per lane; the pivots are a serial chain, which is what bounds the kernel.
+__device__ __forceinline__ void chol_rows(double *T, int ld, int pc0, int cols, double tol, int lane, double *D) {
+    const int c = lane < 16 ? lane : 16 + pc0 + lane - 16;
+    const bool in = lane < 16 || pc0 + lane - 16 < cols;
     double col[16];
 #pragma unroll
-    for (int r = 0; r < 16; ++r) col[r] = (c < 16 && r <= c) ? T[r * ld + c] : 0.0;
+    for (int r = 0; r < 16; ++r) col[r] = (in && r <= c) ? T[r * ld + c] : 0.0;
 #pragma unroll
     for (int k = 0; k < 16; ++k) {
         const double d = lane_read(col[k], k);
-        const bool live = d > tol;  // false for NaN as well
-        const double rkk = live ? sqrt(d) : 0.0, inv = live ? 1.0 / rkk : 0.0;
-        if (c == k)
-            col[k] = rkk;
-        else if (c > k)
-            col[k] *= inv;
+        const double y = rsqrt_nr(d), inv = d > tol ? y : 0.0;  // 0 for NaN as well
+        // below the diagonal lanes k' < k of the tile hold leftovers that nothing reads
+        col[k] *= inv;
 #pragma unroll
-        for (int i = k + 1; i < 16; ++i) {
-            const double aki = lane_read(col[k], i);
-            if (c >= i) col[i] -= aki * col[k];
-        }
+        for (int i = k + 1; i < 16; ++i) col[i] = fma(-lane_read(col[k], i), col[k], col[i]);
     }
-    double inv[16];
+    if (lane >= 16) {
+        if (in) {
 #pragma unroll
-    for (int r = 0; r < 16; ++r) inv[r] = 0.0;
-#pragma unroll
-    for (int i = 15; i >= 0; --i) {
-        double v = (i == c) ? 1.0 : 0.0;
-#pragma unroll
-        for (int q = i + 1; q < 16; ++q) v -= lane_read(col[i], q) * inv[q];
-        const double rii = lane_read(col[i], i);
-        inv[i] = (i <= c && rii > 0.0) ? v / rii : 0.0;
-    }
-    if (c < 16) {
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            T[r * ld + c] = (r <= c) ? col[r] : 0.0;
-            D[r * 16 + c] = inv[r];
+            for (int r = 0; r < 16; ++r) T[r * ld + c] = col[r];
         }
+    } else if (D) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) D[r * 16 + c] = (r <= c) ? col[r] : 0.0;
     }
 }
 
-__global__ void __launch_bounds__(1024) k_chol_inv(SmallBatch B) {
-    HIP_DYNAMIC_SHARED(double, sm)
-    __shared__ double red[16];
-    const SmallPtrs P = small_ptrs(B);
-    const int p = P.p;
-    const int N = (p + kNB - 1) / kNB * kNB, nb = N / kNB, LD = N + 1;
-    const double *W = P.in;
-    double *Rinv = P.out;
-    double *A = sm;            // N x N at stride LD: R (upper), then R^{-1} in place
-    double *Dv = sm + N * LD;  // nb inverted diagonal tiles
-    const int tid = threadIdx.x, nt = blockDim.x;
+// Inverse of the 16 x 16 upper triangular tile D (row stride 16) into T (row stride ld); a zero
+// diagonal entry gives a zero row and column.  Called by a whole wavefront, lane c < 16 owning column c.
+__device__ __forceinline__ void tri_inv_tile(const double *D, double *T, int ld, int lane) {
+    const int c = lane & 15;
+    double row[16], inv[16];
+#pragma unroll
+    for (int r = 0; r < 16; ++r) row[r] = D[r * 16 + c];
+#pragma unroll
+    for (int i = 15; i >= 0; --i) {
+        const double rii = lane_read(row[i], i);
+        double v = (i == c) ? 1.0 : 0.0;
+#pragma unroll
+        for (int q = i + 1; q < 16; ++q) v = fma(-lane_read(row[i], q), inv[q], v);
+        inv[i] = (i <= c && rii > 0.0) ? v * rcp_nr(rii) : 0.0;
+    }
+    if (lane < 16) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) T[r * ld + c] = inv[r];
+    }
+}
+
+// Right-looking blocked Cholesky W = R^T R of the matrix of nb x nb tiles at A (row stride LD, upper
+// triangle) by the whole workgroup: R above the diagonal tiles in A, the diagonal tiles in Dv.
+__device__ __forceinline__ void chol_factor(double *A, int LD, double *Dv, int nb, double dead_tol, int tid, int nt) {
     const int lane = tid & 63, wave = tid >> 6, nw = nt >> 6;
     const int li = lane & 15, lq = lane >> 4;  // MFMA operand coordinates of this lane
-    double tr = 0, dm = 0;
-    for (int e = tid; e < N * N; e += nt) {
-        const int i = e / N, j = e - i * N;
-        double w = 0.0;
-        if (i < p && j < p && j >= i) w = W[i * p + j];
-        A[i * LD + j] = w;
-        if (i == j && i < p) {
-            tr += w;
-            dm = fmax(dm, w);
-        }
-    }
-    tr = wg_sum(tr, red);
-    for (int o = 32; o > 0; o >>= 1) dm = fmax(dm, __shfl_down(dm, o, 64));
-    if (lane == 0) red[wave] = dm;
-    __syncthreads();
-    dm = 0;
-    for (int i = 0; i < nw; ++i) dm = fmax(dm, red[i]);
-    __syncthreads();
-    const double shift = B.shift_rel * tr / p;
-    const double dead_tol = 1e-14 * (dm + shift);
-    for (int i = tid; i < p; i += nt) A[i * LD + i] += shift;
-    __syncthreads();
-    // ---- right-looking blocked Cholesky W = R^T R
     for (int J = 0; J < nb; ++J) {
-        const int j0 = J * kNB;
-        if (wave == 0) chol_tile(A + j0 * LD + j0, LD, Dv + 256 * J, dead_tol, lane);
-        __syncthreads();
-        // panel rows of block J: X_T = Dinv_J^T A[J, T]
-        for (int T = J + 1 + wave; T < nb; T += nw) {
-            d4 acc = {0, 0, 0, 0};
-#pragma unroll
-            for (int t = 0; t < 4; ++t) {
-                const int k = lq + 4 * t;
-                acc = __builtin_amdgcn_mfma_f64_16x16x4f64(Dv[256 * J + k * 16 + li], A[(j0 + k) * LD + 16 * T + li], acc,
-                                                           0, 0, 0);
-            }
-#pragma unroll
-            for (int v = 0; v < 4; ++v) A[(j0 + lq + 4 * v) * LD + 16 * T + li] = acc[v];
-        }
+        const int j0 = J * kNB, m = nb - 1 - J;
+        if (wave == 0 || 48 * wave < 16 * m)
+            chol_rows(A + j0 * LD + j0, LD, 48 * wave, 16 * m, dead_tol, lane, wave == 0 ? Dv + 256 * J : nullptr);
         __syncthreads();
         // trailing update of the tiles (I, T), J < I <= T: A[I, T] -= X_I^T X_T
-        const int m = nb - 1 - J;
         for (int idx = wave; idx < m * (m + 1) / 2; idx += nw) {
             int I = 0, rem = idx;
             while (rem >= m - I) {
@@ -316,17 +304,55 @@ __global__ void __launch_bounds__(1024) k_chol_inv(SmallBatch B) {
         }
         __syncthreads();
     }
-    // ---- R^{-1} in place: the inverted diagonal tiles, then block columns left to right
-    for (int e = tid; e < nb * 256; e += nt) {
-        const int K = e >> 8, r = (e >> 4) & 15, c = e & 15;
-        A[(16 * K + r) * LD + 16 * K + c] = Dv[e];
+}
+
+__global__ void __launch_bounds__(1024) k_chol_inv(SmallBatch B) {
+    HIP_DYNAMIC_SHARED(double, sm)
+    const SmallPtrs P = small_ptrs(B);
+    const int p = P.p;
+    const int N = (p + kNB - 1) / kNB * kNB, nb = N / kNB, LD = N + 1;
+    const double *W = P.in;
+    double *Rinv = P.out;
+    double *A = sm;            // N x N at stride LD: R (above the diagonal tiles), then R^{-1} in place
+    double *Dv = sm + N * LD;  // nb diagonal tiles of R
+    const int tid = threadIdx.x, nt = blockDim.x;
+    const int lane = tid & 63, wave = tid >> 6, nw = nt >> 6;
+    const int li = lane & 15, lq = lane >> 4;  // MFMA operand coordinates of this lane
+    // trace and largest diagonal entry, the same in every wavefront
+    double tr = 0, dm = 0;
+    for (int i = lane; i < p; i += 64) {
+        const double w = W[i * p + i];
+        tr += w;
+        dm = fmax(dm, w);
     }
+    for (int o = 32; o > 0; o >>= 1) {
+        tr += __shfl_xor(tr, o, 64);
+        dm = fmax(dm, __shfl_xor(dm, o, 64));
+    }
+    // scaled by a power of four (R^{-1} by its root) to pivots between 1e-14 and 4
+    const int e2 = (dm > 0.0 && dm < INFINITY) ? -(ilogb(dm) >> 1) : 0;
+    const double shift = B.shift_rel * tr / p;
+    for (int i = wave; i < N; i += nw)
+        for (int j = lane; j < N; j += 64) {
+            double w = 0.0;
+            if (i < p && j < p && j >= i) w = ldexp(W[i * p + j] + (i == j ? shift : 0.0), 2 * e2);
+            A[i * LD + j] = w;
+        }
+    const double dead_tol = ldexp(1e-14 * (dm + shift), 2 * e2);
     __syncthreads();
-    for (int J = 1; J < nb; ++J) {
-        // S_I = X[I, I..J-1] R[I..J-1, J], staged in block (J, I) of the lower triangle
-        for (int I = wave; I < J; I += nw) {
+    chol_factor(A, LD, Dv, nb, dead_tol, tid, nt);
+    // ---- R^{-1} in place: the diagonal tiles, then pairs of neighbouring inverted blocks merged
+    for (int K = wave; K < nb; K += nw) tri_inv_tile(Dv + 256 * K, A + 16 * K * LD + 16 * K, LD, lane);
+    __syncthreads();
+    for (int s = 1; s < nb; s *= 2) {
+        const int npair = (nb + s - 1) / (2 * s);  // pair q: block rows [2 q s, 2 q s + s) and those after, below nb
+        // S = R12 X22, staged in the lower block triangle (block (J, I) for tile (I, J))
+        for (int idx = wave; idx < npair * s * s; idx += nw) {
+            const int q = idx / (s * s), e = idx - q * s * s;
+            const int I = 2 * q * s + e / s, J = 2 * q * s + s + e % s;
+            if (J >= nb) continue;
             d4 acc = {0, 0, 0, 0};
-            for (int K = I; K < J; ++K) {
+            for (int K = 2 * q * s + s; K <= J; ++K) {
 #pragma unroll
                 for (int t = 0; t < 4; ++t) {
                     const int k = lq + 4 * t;
@@ -338,24 +364,27 @@ __global__ void __launch_bounds__(1024) k_chol_inv(SmallBatch B) {
             for (int v = 0; v < 4; ++v) A[(16 * J + lq + 4 * v) * LD + 16 * I + li] = acc[v];
         }
         __syncthreads();
-        // X[I, J] = -S_I Dinv_J
-        for (int I = wave; I < J; I += nw) {
+        // X12 = -X11 S
+        for (int idx = wave; idx < npair * s * s; idx += nw) {
+            const int q = idx / (s * s), e = idx - q * s * s;
+            const int I = 2 * q * s + e / s, J = 2 * q * s + s + e % s;
+            if (J >= nb) continue;
             d4 acc = {0, 0, 0, 0};
+            for (int K = I; K < 2 * q * s + s; ++K) {
 #pragma unroll
-            for (int t = 0; t < 4; ++t) {
-                const int k = lq + 4 * t;
-                acc = __builtin_amdgcn_mfma_f64_16x16x4f64(-A[(16 * J + li) * LD + 16 * I + k], Dv[256 * J + k * 16 + li],
-                                                           acc, 0, 0, 0);
+                for (int t = 0; t < 4; ++t) {
+                    const int k = lq + 4 * t;
+                    acc = __builtin_amdgcn_mfma_f64_16x16x4f64(-A[(16 * I + li) * LD + 16 * K + k],
+                                                               A[(16 * J + k) * LD + 16 * K + li], acc, 0, 0, 0);
+                }
             }
 #pragma unroll
             for (int v = 0; v < 4; ++v) A[(16 * I + lq + 4 * v) * LD + 16 * J + li] = acc[v];
         }
         __syncthreads();
     }
-    for (int e = tid; e < p * p; e += nt) {
-        const int i = e / p, j = e - i * p;
-        Rinv[e] = (j >= i) ? A[i * LD + j] : 0.0;
-    }
+    for (int i = wave; i < p; i += nw)
+        for (int j = lane; j < p; j += 64) Rinv[i * p + j] = (j >= i) ? ldexp(A[i * LD + j], e2) : 0.0;
 }
 
 // round-robin pairing of round `round` (p even): pair t is (a, b) with a != b, every index once

@@ -116,6 +116,67 @@ inline int __builtin_amdgcn_readlane(int v, int l) {
 // value of v in the wavefront's first lane (every lane is active in the emulation)
 inline int __builtin_amdgcn_readfirstlane(int v) { return __builtin_amdgcn_readlane(v, 0); }
 
+// value of v in lane `src` of the wavefront
+inline int __shfl_any(int v, int src) {
+    int *buf = (int *)emu::wave_buf(0);
+    int l = emu::lane();
+    emu::sync_wave();
+    buf[l] = v;
+    emu::sync_wave();
+    int r = buf[src];
+    emu::sync_wave();
+    return r;
+}
+
+// true in every lane when pred holds in any lane of the wavefront
+inline int __any(int pred) {
+    int *buf = (int *)emu::wave_buf(0);
+    int me = emu::lane(), r = 0;
+    emu::sync_wave();
+    buf[me] = pred;
+    emu::sync_wave();
+    for (int l = 0; l < 64; ++l) r |= buf[l] != 0;
+    emu::sync_wave();
+    return r;
+}
+
+// DPP moves used by the kernels (all rows and banks enabled): quad_perm, row_ror:n, row_half_mirror
+inline int __builtin_amdgcn_update_dpp(int, int src, int ctrl, int, int, bool) {
+    const int l = emu::lane();
+    int from = l;
+    if (ctrl < 0x100)
+        from = (l & ~3) | ((ctrl >> (2 * (l & 3))) & 3);
+    else if (ctrl > 0x120 && ctrl < 0x130)
+        from = (l & ~15) | ((l - (ctrl & 15)) & 15);
+    else if (ctrl == 0x141)
+        from = (l & ~7) | (7 - (l & 7));
+    else
+        abort();
+    return __shfl_any(src, from);
+}
+// v_permlane32_swap / v_permlane16_swap: the upper half (odd rows of 16 lanes) of the first operand
+// trades places with the lower half (even rows) of the second
+typedef unsigned emu_u2 __attribute__((ext_vector_type(2)));
+inline emu_u2 emu_permlane_swap(unsigned a, unsigned b, int w) {
+    unsigned *buf = (unsigned *)emu::wave_buf(0);
+    const int l = emu::lane();
+    emu::sync_wave();
+    buf[l] = a;
+    buf[64 + l] = b;
+    emu::sync_wave();
+    emu_u2 r;
+    r[0] = (l & w) ? buf[64 + (l ^ w)] : a;
+    r[1] = (l & w) ? b : buf[l ^ w];
+    emu::sync_wave();
+    return r;
+}
+inline emu_u2 __builtin_amdgcn_permlane32_swap(unsigned a, unsigned b, bool, bool) { return emu_permlane_swap(a, b, 32); }
+inline emu_u2 __builtin_amdgcn_permlane16_swap(unsigned a, unsigned b, bool, bool) { return emu_permlane_swap(a, b, 16); }
+
+// hardware estimates of 1 / sqrt(x) and 1 / x (the kernels refine them by Newton-Raphson steps)
+inline double __builtin_amdgcn_rsq(double x) { return (double)(float)(1.0 / std::sqrt(x)); }
+inline double __builtin_amdgcn_rcp(double x) { return (double)(float)(1.0 / x); }
+
 // raw buffer resource (stride 0): loads at byte offset voffset + soffset from the base; an offset
 // at or beyond num_records reads zero, as the hardware's range check does
 struct emu_buffer_rsrc {
