@@ -400,6 +400,304 @@ __device__ __forceinline__ void rr_pair(int t, int round, int p, int &i, int &j)
     j = a < b ? b : a;
 }
 
+// ---------------------------------------------------------------------------------------------
+// One-sided Jacobi: the left singular vectors of a set of at most 128 vectors of at most 128
+// components, by rotating pairs of vectors until all are orthogonal.  Two uses, both in svd mode:
+//   - the Rayleigh-Ritz matrix G = Bm Bm^T (p x p): its vectors are the columns of the Cholesky
+//     factor L (G = L L^T), factored here; normalised, the rotated columns are G's eigenvectors.  The
+//     basis comes out of an orthogonal iteration, so G is close to diagonal and L to converged.
+//   - a small block with both sides at most 128: its own columns (m <= n) or rows (m > n); no Gram
+//     matrix squares its condition.
+// One workgroup of W = ceil(nvec / 16) wavefronts per problem.  The vectors live in LDS (vector j at
+// stride N + 1) in 2 W groups of eight; in each of the 2 W - 1 turns of a sweep a wavefront takes two
+// groups into registers (two components of sixteen vectors per lane), does the 64 rotations between
+// them (and, in a sweep's first turn, those within each group) with no barrier, and puts them back.
+// Eight rotations go at a time: their eight dot products are reduced together, so that lanes
+// 8 q .. 8 q + 7 end with the q-th and compute its angle, eight angles per instruction.
+// Against the two-sided kernel below (a barrier pair per 64 rotations, 24 LDS accesses per 2 x 2
+// block and the eigenvectors replayed from a log afterwards) the matrix is touched in LDS once per
+// eight rounds and there is no replay.  It is bound by instruction issue: about 240 instructions of
+// 4 cycles (a lane swap 12) per eight rotations, 8 wavefronts on 4 SIMDs.  MI355X, four 128 x 128
+// problems: blocks of a leg-dim-16 step 3.5 ms -> 1.7 ms, Rayleigh-Ritz matrices of a leg-dim-64 step
+// 1.8 ms -> 0.6 ms.
+// A pair is left alone when |x.y| <= 1e-15 |x| |y| or one of the two is below 1e-15 of the largest
+// vector (the rank rule drops values at 1e-14).  A sweep whose rotations all have |x.y| <= 1e-9 |x| |y|
+// and angles of at most 1e-8 is the last: what they undo in other pairs is their product.  The vectors
+// are taken by decreasing norm, which saves sweeps.
+// ---------------------------------------------------------------------------------------------
+constexpr int kOsMax = 128;    // vectors, and components per vector
+constexpr int kOsEntries = 8;  // geometries per launch
+struct OsEntry {
+    const double *in;
+    double *out;           // (len x p) row-major: column c = the unit vector of the c-th largest norm
+    int64_t din, dout;     // per-problem strides
+    int64_t sv, sc;        // direct: component r of vector j at in[j * sv + r * sc]
+    int32_t nvec, len, p;
+    int32_t direct;        // 0: in is G (p x p), its Cholesky columns are the vectors
+};
+struct OsArgs {
+    int32_t n;
+    int32_t start[kOsEntries + 1];
+    OsEntry e[kOsEntries];
+};
+
+typedef unsigned u2v __attribute__((ext_vector_type(2)));
+template <int CTRL>
+__device__ __forceinline__ double dpp_of(double v) {
+    const u2v u = __builtin_bit_cast(u2v, v);
+    u2v r;
+    r.x = (unsigned)__builtin_amdgcn_update_dpp(0, (int)u.x, CTRL, 0xf, 0xf, true);
+    r.y = (unsigned)__builtin_amdgcn_update_dpp(0, (int)u.y, CTRL, 0xf, 0xf, true);
+    return __builtin_bit_cast(double, r);
+}
+// a summed over lane pairs 32 apart in lanes 0..31, b in lanes 32..63
+__device__ __forceinline__ double fold32(double a, double b) {
+    const u2v x = __builtin_bit_cast(u2v, a), y = __builtin_bit_cast(u2v, b);
+    const auto lo = __builtin_amdgcn_permlane32_swap(x.x, y.x, false, false);
+    const auto hi = __builtin_amdgcn_permlane32_swap(x.y, y.y, false, false);
+    return __builtin_bit_cast(double, u2v{lo[0], hi[0]}) + __builtin_bit_cast(double, u2v{lo[1], hi[1]});
+}
+// a summed over lane pairs 16 apart in the even rows of 16 lanes, b in the odd ones
+__device__ __forceinline__ double fold16(double a, double b) {
+    const u2v x = __builtin_bit_cast(u2v, a), y = __builtin_bit_cast(u2v, b);
+    const auto lo = __builtin_amdgcn_permlane16_swap(x.x, y.x, false, false);
+    const auto hi = __builtin_amdgcn_permlane16_swap(x.y, y.y, false, false);
+    return __builtin_bit_cast(double, u2v{lo[0], hi[0]}) + __builtin_bit_cast(double, u2v{lo[1], hi[1]});
+}
+// sum over the wavefront of v[q] in the lanes 8 q .. 8 q + 7
+__device__ __forceinline__ double reduce8(const double (&v)[8], int lane) {
+    const double u0 = fold32(v[0], v[4]), u1 = fold32(v[1], v[5]), u2 = fold32(v[2], v[6]), u3 = fold32(v[3], v[7]);
+    const double w0 = fold16(u0, u2), w1 = fold16(u1, u3);
+    const bool odd = lane & 8;
+    double x = (odd ? w1 : w0) + dpp_of<0x128>(odd ? w0 : w1);  // row_ror:8
+    x += dpp_of<0x141>(x);                                      // row_half_mirror
+    x += dpp_of<0xB1>(x);                                       // quad_perm [1, 0, 3, 2]
+    x += dpp_of<0x4E>(x);                                       // quad_perm [2, 3, 0, 1]
+    return x;
+}
+
+// Sine s, half-angle tangent h and tangent t of the rotation that makes two vectors with squared norms
+// al, be and dot product g orthogonal: all 0 when they count as orthogonal.  coarse: the rotation may
+// leave other pairs further from orthogonal than the next sweep's threshold.
+__device__ __forceinline__ void os_angle(double al, double be, double g, double zero, double &s, double &h, double &t,
+                                         bool &coarse) {
+    const double gg = g * g, ab = al * be;
+    const bool rot = gg > 1e-30 * ab && al > zero && be > zero;
+    const double d = be - al, g2 = rot ? 2.0 * g : 1.0;
+    const double h2 = fma(d, d, g2 * g2);
+    const double tt = (d >= 0.0 ? g2 : -g2) * rcp_nr(fma(h2, rsqrt_nr(h2), fabs(d)));
+    const double c = rsqrt_nr(fma(tt, tt, 1.0));
+    t = rot ? tt : 0.0;
+    s = rot ? c * tt : 0.0;
+    h = s * rcp_nr(1.0 + c);
+    coarse = coarse || (rot && (gg > 1e-18 * ab || fabs(tt) > 1e-8));
+}
+// (x, y) <- (c x - s y, s x + c y) as three shears, h = s / (1 + c): in place, three multiply-adds
+__device__ __forceinline__ void os_rotate(double (&x)[2], double (&y)[2], double s, double h) {
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+        x[e] = fma(-h, y[e], x[e]);
+        y[e] = fma(s, x[e], y[e]);
+        x[e] = fma(-h, y[e], x[e]);
+    }
+}
+
+__global__ void __launch_bounds__(512) k_jacobi_onesided(OsArgs A) {
+    HIP_DYNAMIC_SHARED(double, sm)
+    __shared__ double red[16];
+    __shared__ int order[kOsMax];
+    __shared__ int active;
+    int gi = 0;
+    while (gi + 1 < A.n && (int)blockIdx.x >= A.start[gi + 1]) ++gi;
+    const OsEntry &E = A.e[gi];
+    const int64_t bi = (int)blockIdx.x - A.start[gi];
+    const double *in = E.in + bi * E.din;
+    double *out = E.out + bi * E.dout;
+    const int nvec = E.nvec, len = E.len, p = E.p;
+    const int W = (nvec + 15) / 16, N = 16 * W, LD = N + 1;  // len <= N
+    double *X = sm;              // vector j at X + j * LD
+    double *nrm = sm + N * LD;   // squared norms (the Cholesky's diagonal tiles before)
+    const int tid = threadIdx.x, nt = blockDim.x, lane = tid & 63, wave = tid >> 6, nw = nt >> 6;
+    // ---- the vectors, scaled by a power of two to entries of order one
+    double mx = 0.0, bad = 0.0;
+    if (E.direct) {
+        // consecutive lanes read consecutive addresses, whichever side the vectors are
+        for (int hi = wave; hi < N; hi += nw)
+            for (int lo = lane; lo < N; lo += 64) {
+                const int j = E.sc == 1 ? hi : lo, r = E.sc == 1 ? lo : hi;
+                const double v = (j < nvec && r < len) ? in[j * E.sv + r * E.sc] : 0.0;
+                X[j * LD + r] = v;
+                mx = fmax(mx, fabs(v));
+                bad += v - v;  // NaN for every inf or NaN
+            }
+    } else {
+        for (int i = wave; i < N; i += nw)
+            for (int j = lane; j < N; j += 64) {
+                const double v = (i < p && j < p && j >= i) ? in[i * p + j] : 0.0;
+                X[i * LD + j] = v;
+                if (i == j) mx = fmax(mx, v);
+                bad += v - v;
+            }
+    }
+    bad = wg_sum(bad, red);
+    for (int o = 32; o > 0; o >>= 1) mx = fmax(mx, __shfl_xor(mx, o, 64));
+    if (lane == 0) red[wave] = mx;
+    if (tid == 0) active = 0;
+    __syncthreads();
+    mx = 0.0;
+    for (int i = 0; i < nw; ++i) mx = fmax(mx, red[i]);
+    if (bad != 0.0 || !(mx > 0.0)) {  // uniform: non-finite input is passed on, zero input has zero vectors
+        for (int e = tid; e < len * p; e += nt) out[e] = bad;
+        return;
+    }
+    const int ex = -ilogb(mx);
+    const double scale = ldexp(1.0, ex > 1000 ? 1000 : ex);
+    for (int e = tid; e < N * LD; e += nt) X[e] *= scale;  // (the pad column is never read)
+    __syncthreads();
+    if (!E.direct) {
+        chol_factor(X, LD, nrm, W, 1e-200, tid, nt);
+        for (int e = tid; e < W * 256; e += nt) {  // the diagonal tiles, and zeros left of them
+            const int K = e >> 8, r = (e >> 4) & 15, c = e & 15;
+            X[(16 * K + r) * LD + 16 * K + c] = nrm[e];
+        }
+        for (int i = 16 + wave; i < N; i += nw)
+            for (int j = lane; j < i / 16 * 16; j += 64) X[i * LD + j] = 0.0;
+        __syncthreads();
+    }
+    // squared norms into nrm, the vectors by decreasing norm (ties by index) into order
+    const bool two = len > 64;
+    auto rank_vectors = [&]() {
+        for (int j = wave; j < N; j += nw) {
+            double a = lane < N ? X[j * LD + lane] : 0.0, b = two && lane + 64 < N ? X[j * LD + lane + 64] : 0.0;
+            a = fma(a, a, b * b);
+            for (int o = 32; o > 0; o >>= 1) a += __shfl_xor(a, o, 64);
+            if (lane == 0) nrm[j] = a;
+        }
+        __syncthreads();
+        for (int e = tid; e < N; e += nt) {
+            const double ke = nrm[e];
+            int rank = 0;
+            for (int f = 0; f < N; ++f) {
+                const double kf = nrm[f];
+                if (kf > ke || (kf == ke && f < e)) ++rank;
+            }
+            order[rank] = e;
+        }
+        __syncthreads();
+    };
+    rank_vectors();
+    double zero = 1e-30 * nrm[order[0]];
+    // ---- sweeps
+    const int nblk = 2 * W, g = lane >> 3;
+    for (int sweep = 0; sweep < kMaxSweeps; ++sweep) {
+        for (int turn = 0; turn < nblk - 1; ++turn) {
+            if (wave < W) {
+                int bi0, bj0;
+                rr_pair(wave, turn, nblk, bi0, bj0);
+                double xa[8][2], xb[8][2];
+                int ra[8], rb[8];
+#pragma unroll
+                for (int q = 0; q < 8; ++q) {
+                    ra[q] = __builtin_amdgcn_readfirstlane(order[8 * bi0 + q]) * LD + lane;
+                    rb[q] = __builtin_amdgcn_readfirstlane(order[8 * bj0 + q]) * LD + lane;
+                    xa[q][0] = lane < N ? X[ra[q]] : 0.0;
+                    xb[q][0] = lane < N ? X[rb[q]] : 0.0;
+                    xa[q][1] = two && lane + 64 < N ? X[ra[q] + 64] : 0.0;
+                    xb[q][1] = two && lane + 64 < N ? X[rb[q] + 64] : 0.0;
+                }
+                bool any = false, coarse = false;
+                auto dots = [&](const double (&x)[8][2], const double (&y)[8][2], double (&v)[8], int shift) {
+#pragma unroll
+                    for (int q = 0; q < 8; ++q)
+                        v[q] = fma(x[q][0], y[(q + shift) & 7][0], x[q][1] * y[(q + shift) & 7][1]);
+                };
+                double v[8], na, nb;
+                dots(xa, xa, v, 0);
+                na = reduce8(v, lane);
+                dots(xb, xb, v, 0);
+                nb = reduce8(v, lane);
+                if (turn == 0) {
+                    // rotations within the two groups: round r pairs (i, j) of 0..7, four in each group
+#pragma unroll
+                    for (int r = 0; r < 7; ++r) {
+                        double w[8], y[8];
+#pragma unroll
+                        for (int q = 0; q < 4; ++q) {
+                            int i, j;
+                            rr_pair(q, r, 8, i, j);
+                            v[q] = fma(xa[i][0], xa[j][0], xa[i][1] * xa[j][1]);
+                            w[q] = fma(xa[i][0], xa[i][0], xa[i][1] * xa[i][1]);
+                            y[q] = fma(xa[j][0], xa[j][0], xa[j][1] * xa[j][1]);
+                            v[q + 4] = fma(xb[i][0], xb[j][0], xb[i][1] * xb[j][1]);
+                            w[q + 4] = fma(xb[i][0], xb[i][0], xb[i][1] * xb[i][1]);
+                            y[q + 4] = fma(xb[j][0], xb[j][0], xb[j][1] * xb[j][1]);
+                        }
+                        double s, h, t;
+                        os_angle(reduce8(w, lane), reduce8(y, lane), reduce8(v, lane), zero, s, h, t, coarse);
+                        if (!__any(s != 0.0)) continue;
+                        any = true;
+#pragma unroll
+                        for (int q = 0; q < 4; ++q) {
+                            int i, j;
+                            rr_pair(q, r, 8, i, j);
+                            os_rotate(xa[i], xa[j], lane_read(s, 8 * q), lane_read(h, 8 * q));
+                            os_rotate(xb[i], xb[j], lane_read(s, 8 * q + 32), lane_read(h, 8 * q + 32));
+                        }
+                    }
+                    dots(xa, xa, v, 0);
+                    na = reduce8(v, lane);
+                    dots(xb, xb, v, 0);
+                    nb = reduce8(v, lane);
+                }
+                // rotations between the groups: round r pairs vector q of the first with (q + r) % 8 of
+                // the second; na, nb are the squared norms of this lane group's pair
+#pragma unroll
+                for (int r = 0; r < 8; ++r) {
+                    dots(xa, xb, v, r);
+                    const double gam = reduce8(v, lane);
+                    double s, h, t;
+                    os_angle(na, nb, gam, zero, s, h, t, coarse);
+                    na = fma(-t, gam, na);
+                    nb = fma(t, gam, nb);
+                    nb = __shfl(nb, (lane + 8) & 63, 64);  // the next round's partner sits one lane group on
+                    if (!__any(s != 0.0)) continue;
+                    any = true;
+#pragma unroll
+                    for (int q = 0; q < 8; ++q) os_rotate(xa[q], xb[(q + r) & 7], lane_read(s, 8 * q), lane_read(h, 8 * q));
+                }
+                if (any) {
+#pragma unroll
+                    for (int q = 0; q < 8; ++q) {
+                        if (lane < N) {
+                            X[ra[q]] = xa[q][0];
+                            X[rb[q]] = xb[q][0];
+                        }
+                        if (two && lane + 64 < N) {
+                            X[ra[q] + 64] = xa[q][1];
+                            X[rb[q] + 64] = xb[q][1];
+                        }
+                    }
+                    if (__any(coarse) && lane == 0) active = 1;  // every writer stores the same value
+                }
+            }
+            __syncthreads();
+        }
+        const int go = active;
+        rank_vectors();  // (its barriers come before the next write of `active`)
+        zero = 1e-30 * nrm[order[0]];
+        if (tid == 0) active = 0;
+        __syncthreads();
+        if (!go) break;
+    }
+    // ---- the vectors by decreasing norm, normalised
+    for (int c = lane; c < p; c += 64) {
+        const int j = order[c];
+        // vectors that no rotation made orthogonal (below the zero rule) are not directions
+        const double f = nrm[j] > 1e-29 * nrm[order[0]] ? 1.0 / sqrt(nrm[j]) : 0.0;
+        for (int r = wave; r < len; r += nw) out[r * p + c] = X[j * LD + r] * f;
+    }
+}
+
 // Cyclic Jacobi on a symmetric p x p matrix (p even) in LDS.  Round-robin pairing gives p/2
 // disjoint rotations per round and every pair once per sweep.  Each round computes its rotations,
 // then applies both sides at once on the upper block triangle: a thread owns the 2 x 2 block of rows
@@ -1464,6 +1762,53 @@ static int jacobi(std::vector<Run> &runs, int by_abs, hipStream_t s) {
     return GTN_OK;
 }
 
+// small blocks that k_jacobi_onesided takes as they are
+static bool onesided_direct(const Blk &b) { return b.small && b.b.m <= kOsMax && b.b.n <= kOsMax; }
+
+// Eigenvectors of the Rayleigh-Ritz matrices of large blocks, singular vectors of small ones with
+// both sides at most 128: Vs of every block, one launch per kOsEntries runs.
+static int jacobi_onesided(std::vector<Run> &runs, hipStream_t s) {
+    for (size_t base = 0; base < runs.size(); base += kOsEntries) {
+        OsArgs a;
+        memset(&a, 0, sizeof(a));
+        int wmax = 1;
+        for (size_t i = base; i < runs.size() && i < base + kOsEntries; ++i) {
+            Run &r = runs[i];
+            Blk &f = *r.f;
+            const gtn_svd_block &B = f.b;
+            OsEntry &e = a.e[a.n];
+            e.p = (int)f.p;
+            e.out = f.Vs;
+            e.dout = r.dws;
+            e.direct = f.small;
+            if (f.small) {
+                const bool left = f.left;  // vectors: columns of M (left) or rows
+                e.in = B.M, e.din = r.dM;
+                e.nvec = (int)(left ? B.n : B.m), e.len = (int)(left ? B.m : B.n);
+                e.sv = left ? 1 : B.lda, e.sc = left ? B.lda : 1;
+                R8N(B.M, ext(B.m, B.n, B.lda), r.dM, r.n, "small block");
+            } else {
+                e.in = f.G, e.din = r.dws;
+                e.nvec = e.len = (int)f.p;
+                e.sv = f.p, e.sc = 1;
+                R8N(f.G, f.p * f.p, r.dws, r.n, "ritz matrix");
+            }
+            GTN_REQUIRE(e.nvec <= kOsMax && e.len <= e.nvec && f.p <= (e.nvec + 15) / 16 * 16,
+                        "gtn_svd_blocks: block beyond the one-sided Jacobi's size");
+            R8N(f.Vs, (int64_t)e.len * f.p, r.dws, r.n, "eigenvectors");
+            a.start[a.n + 1] = a.start[a.n] + r.n;
+            ++a.n;
+            if ((e.nvec + 15) / 16 > wmax) wmax = (e.nvec + 15) / 16;
+        }
+        const int N = 16 * wmax;
+        const size_t shm = sizeof(double) * (size_t)N * (N + 17);  // vectors at stride N + 1, Cholesky diagonal tiles
+        if (dry_run()) continue;
+        GTN_CHECK_HIP(hipFuncSetAttribute((const void *)k_jacobi_onesided, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shm));
+        LAUNCH(k_jacobi_onesided, dim3(a.start[a.n]), dim3(64 * wmax), shm, s, a);
+    }
+    return GTN_OK;
+}
+
 // split-BF16 planes of every block's M and M^T (once per call)
 static int rf_planes_of_blocks(std::vector<Run> &rl, hipStream_t s) {
     for (Run &r : rl) {
@@ -1623,6 +1968,12 @@ static int run_blocks(std::vector<Blk> &blocks, const gtn_svd_opts &o, hipStream
     }
     if (all.empty()) return GTN_OK;
     std::vector<Run> rs = make_runs(small, ismall), rl = make_runs(large, ilarge), ra = make_runs(all, iall);
+    // the p x p problems: one-sided Jacobi wherever its vectors fit (large blocks' Rayleigh-Ritz
+    // matrices, small blocks of at most 128 x 128); the two-sided kernel for eig, whose matrices are
+    // indefinite, and for small blocks with a long side, whose Gram matrix it takes without a
+    // Cholesky factor (that would drop values below ~1e-8 of the largest)
+    std::vector<Run> one, two;
+    for (Run &r : ra) (!eig && (!r.f->small || onesided_direct(*r.f)) ? one : two).push_back(r);
     int rc;
     // ---- small blocks: G = Gram of the short side (svd) or the block itself (eig)
     if (!rs.empty()) {
@@ -1630,6 +1981,7 @@ static int run_blocks(std::vector<Blk> &blocks, const gtn_svd_opts &o, hipStream
         for (Run &r : rs) {
             Blk &f = *r.f;
             const gtn_svd_block &B = f.b;
+            if (!eig && onesided_direct(f)) continue;
             R8N(f.G, f.p * f.p, r.dws, r.n, "small gram");
             LAUNCH(k_fill, grid2(f.p * f.p, r.n), dim3(256), 0, s, f.G, f.p, f.p, f.p, 0.0, r.dws);
             if (eig) {
@@ -1791,7 +2143,9 @@ static int run_blocks(std::vector<Blk> &blocks, const gtn_svd_opts &o, hipStream
         }
     }
     // ---- p x p eigenproblems of every block at once
-    rc = jacobi(ra, eig, s);
+    rc = jacobi(two, eig, s);
+    if (rc) return rc;
+    rc = jacobi_onesided(one, s);
     if (rc) return rc;
     for (Run &r : ra) {
         Blk &f = *r.f;

@@ -1,5 +1,7 @@
-"""GPU tests of gtn_svd_blocks at the sizes where its kernels' tiles end: the block width of the range
-finder (CholeskyQR in 16 x 16 tiles) around multiples of 16.
+"""GPU tests of gtn_svd_blocks at the sizes where its kernels' tiles and vector groups end: small
+blocks (both sides at most 128: one-sided Jacobi on the block, 16 vectors per wavefront in groups of
+eight, one or two components per lane), and the block width of the range finder (CholeskyQR in 16 x 16
+tiles, Rayleigh-Ritz matrix) around multiples of 16.
 
 Tolerances: a backward stable FP64 SVD moves a singular value by at most c eps sigma_0, c of the order
 of the size: 1e-13 sigma_0 for 128, and the vectors' orthogonality and the reconstruction likewise.
@@ -35,6 +37,57 @@ def _check(M, k, out, count, rank=None, tol=1e-13):
     np.testing.assert_allclose(M @ v.T if right else (u.T @ M).T, (u * s) if right else (s[:, None] * v).T, rtol=0,
                                atol=tol * s0)
     assert np.all(np.diff(s) <= tol * s0)
+
+
+@pytest.mark.parametrize("m,n", [(1, 1), (1, 5), (2, 2), (7, 5), (15, 16), (16, 16), (17, 15), (16, 33), (63, 64), (65, 64),
+                                 (64, 128), (113, 112), (127, 128), (128, 127), (128, 128), (128, 129), (40, 300)])
+def test_small_blocks(m, n):
+    """Full decompositions of blocks with a side of at most 128, singular values over three decades."""
+    rng = np.random.default_rng(1000 * m + n)
+    M = rng.standard_normal((m, n)) * 10.0 ** (-1.5 * np.arange(m) / m)[:, None] * 10.0 ** (-1.5 * np.arange(n) / n)
+    k = min(m, n)
+    outs, counts = _run([(M, k)])
+    _check(M, k, outs[0], counts[0])
+
+
+@pytest.mark.parametrize("m,n,r", [(16, 16, 3), (32, 20, 20), (128, 128, 37), (100, 128, 16), (128, 128, 0)])
+def test_small_blocks_of_low_rank(m, n, r):
+    """Rank r (0: the zero block): the rank rule keeps r values, the rest is exactly zero."""
+    rng = np.random.default_rng(m + n + r)
+    M = rng.standard_normal((m, r)) @ rng.standard_normal((r, n)) / max(1, r)
+    outs, counts = _run([(M, min(m, n))])
+    _check(M, min(m, n), outs[0], counts[0], rank=r)
+    assert np.all(outs[0][1].numpy()[r:] == 0.0)
+
+
+def test_small_blocks_scaled_and_repeated():
+    """Entries far from one in magnitude, and values that coincide (a scaled orthogonal block)."""
+    rng = np.random.default_rng(5)
+    Q, _ = np.linalg.qr(rng.standard_normal((48, 48)))
+    for M in (1e-120 * rng.standard_normal((48, 48)), 1e120 * rng.standard_normal((30, 48)), 3.0 * Q):
+        outs, counts = _run([(M, 20)])
+        s = outs[0][1].numpy()
+        ref = np.linalg.svd(M, compute_uv=False)
+        if ref[0] < 1e-28:  # the rank rule, sigma / (sigma_0 + 1e-14) > 1e-14, keeps nothing
+            assert counts[0] == 0 and np.all(s == 0.0)
+            continue
+        np.testing.assert_allclose(s[:20], ref[:20], rtol=0, atol=1e-13 * ref[0])
+        u = outs[0][0].numpy()[:, :20]
+        np.testing.assert_allclose(u.T @ u, np.eye(20), rtol=0, atol=1e-13)
+
+
+def test_mixed_batch_of_small_and_large_blocks():
+    """One call over blocks of several shapes: more runs than one launch of the Jacobi kernel takes,
+    the small ones of them in groups of equal shape."""
+    rng = np.random.default_rng(8)
+    blocks = []
+    for i, (m, n, k) in enumerate([(8, 8, 4), (8, 8, 4), (20, 12, 6), (33, 33, 9), (5, 40, 5), (128, 100, 30), (140, 150, 10),
+                                   (64, 64, 64), (3, 2, 1), (17, 17, 17), (140, 150, 10), (31, 47, 11), (96, 96, 2)]):
+        w = 10.0 ** (-2.0 * np.arange(n) / n)
+        blocks.append((rng.standard_normal((m, n)) * w, k))
+    outs, counts = _run(blocks)
+    for (M, k), o, c in zip(blocks, outs, counts):
+        _check(M, k, o, c, tol=2e-13)
 
 
 @pytest.mark.parametrize("oversample", [3, 8, 9, 24, 25, 57, 89, 96])
