@@ -46,6 +46,23 @@ int check_range(const void *p, int64_t bytes, const char *what);
         if (rc_) return rc_;                              \
     } while (0)
 
+// Operands and epilogue of a grouped FP64 GEMM whose batch entries keep them on the device (the range
+// finder of gtn_svd_blocks, whose blocks stop and trade buffers one by one).  Per batch entry, `stride`
+// 8-byte slots apart: the operand pointers (a null table: the descriptor's pointer and batch stride) and
+// coef = {x, y, z, skip}: C = x A B + y D + z C, D of C's shape and strides; nothing happens when
+// skip is nonzero.
+struct GemmIndirect {
+    const double *const *a, *const *b, *const *d;
+    double *const *c;
+    const double *coef;
+    int64_t stride;
+};
+// gtn_gemm_grouped over such groups (alpha and beta of the descriptors are not used); the launch
+// configuration is the one tuned for the plain signature, tried out with `tune_c` (same shape, free to
+// be overwritten) as output; tune_c null: nothing is tried out
+int gemm_grouped_indirect(const gtn_gemm_desc *groups, const GemmIndirect *ind, int n_groups, void *const *tune_c,
+                          void *stream);
+
 inline hipStream_t as_stream(void *s) { return reinterpret_cast<hipStream_t>(s); }
 
 // graph bookkeeping of the runtime (gtn_runtime.hip): instantiated graphs that may still be

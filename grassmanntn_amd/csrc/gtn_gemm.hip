@@ -39,6 +39,7 @@ struct GemmGroup {
     int32_t splits, kchunk;
     int64_t sam, sak, sbk, sbn, scm, scn, sab, sbb, scb, scs;
     double alpha, beta;
+    GemmIndirect ind;  // coef null: a plain group (a launch's groups are all of one kind)
 };
 
 struct GemmArgs {
@@ -170,8 +171,10 @@ __device__ __forceinline__ void panel_coord(int s, bool kc, int &r, int &k) {
 // B value = B[k = l/16][j = l%16].  Result registers v = 0..3 of lane l hold C[row][l%16] with
 // row = 4*(l/16) + v for the FP32 form and row = l/16 + 4*v for the FP64 form.
 // ------------------------------------------------------------------------------------------------
-template <typename TIN, typename TC, int BM, int BN, int BK>
-__global__ void __launch_bounds__(256) k_gemm_fp(GemmArgs args) {
+// IND: groups with device-side operands and coefficients (GemmIndirect; FP64).  A variant of its own, held
+// to the plain kernel's 256 registers (two wavefronts per SIMD), which its epilogue would exceed by one.
+template <typename TIN, typename TC, int BM, int BN, int BK, bool IND = false>
+__global__ void __launch_bounds__(256, IND ? 2 : 1) k_gemm_fp(GemmArgs args) {
     int gi, b, tm, tn;
     if (!locate(args, gi, b, tm, tn)) return;
     const GemmGroup &g = args.g[gi];
@@ -182,6 +185,13 @@ __global__ void __launch_bounds__(256) k_gemm_fp(GemmArgs args) {
     const TIN *A = (const TIN *)g.A + b * g.sab + kb * g.sak;
     const TIN *B = (const TIN *)g.B + b * g.sbb + kb * g.sbk;
     TIN *C = (TIN *)g.C + b * g.scb + sp * g.scs;
+    if constexpr (IND) {
+        const int64_t t = b * g.ind.stride;
+        if (g.ind.coef[t + 3] != 0.0) return;
+        if (g.ind.a) A = g.ind.a[t] + kb * g.sak;
+        if (g.ind.b) B = g.ind.b[t] + kb * g.sbk;
+        if (g.ind.c && g.splits == 1) C = g.ind.c[t];
+    }
     constexpr int PAD = 1;  // rows of BM + 1: lanes storing one k-column of a row-major panel hit distinct banks
     // FP32 tiles double-buffer their panels (one barrier per panel: 4 % faster on the 2048^3 FP32
     // contraction); the FP64 kernel keeps one buffer, which leaves it the registers for two waves
@@ -304,7 +314,17 @@ __global__ void __launch_bounds__(256) k_gemm_fp(GemmArgs args) {
     else
         mainloop(CheckedPanels<TIN, BM, BK>{A, g.sam, g.sak, m0, g.M, K},
                  CheckedPanels<TIN, BN, BK>{B, g.sbn, g.sbk, n0, g.N, K});
-    const double alpha = g.alpha, beta = g.beta;
+    double alpha = g.alpha, beta = g.beta, gamma = 0.0;
+    const TIN *D = C;
+    if constexpr (IND) {
+        if (g.splits == 1) {  // (the partials of a split reduction are summed with these afterwards)
+            const int64_t t = b * g.ind.stride;
+            alpha = g.ind.coef[t];
+            gamma = g.ind.coef[t + 1];
+            beta = g.ind.coef[t + 2];
+            if (gamma != 0.0) D = g.ind.d[t];
+        }
+    }
 #pragma unroll
     for (int i = 0; i < TI; ++i)
 #pragma unroll
@@ -318,6 +338,8 @@ __global__ void __launch_bounds__(256) k_gemm_fp(GemmArgs args) {
                     int64_t o = r * g.scm + c * g.scn;
                     double val = alpha * (double)acc[i][j][v];
                     if (beta != 0.0) val += beta * (double)C[o];
+                    if constexpr (IND)
+                        if (gamma != 0.0) val += gamma * (double)D[o];
                     C[o] = (TIN)val;
                 }
             }
@@ -474,16 +496,30 @@ __global__ void __launch_bounds__(64) k_mfma_selftest(double *out) {
 }
 
 // C[b](r, c) = alpha * sum_sp W[b][sp](r, c) + beta * C[b](r, c) over the split partials W
-// (batch x splits consecutive M x N matrices), in a fixed order.
+// (batch x splits consecutive M x N matrices), in a fixed order; an indirect group's operands and
+// coefficients come from its tables.
 template <typename T>
 __global__ void k_split_sum(const T *__restrict__ W, int splits, int M, int N, int batch, T *C, int64_t scm,
-                            int64_t scn, int64_t scb, double alpha, double beta) {
+                            int64_t scn, int64_t scb, double alpha, double beta, GemmIndirect ind) {
     const int64_t MN = (int64_t)M * N, total = MN * batch;
     for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < total; i += (int64_t)gridDim.x * blockDim.x) {
         const int64_t b = i / MN, e = i - b * MN;
         const int64_t r = e / N, c = e - r * N;
         const T *w = W + b * splits * MN + e;
         double acc = 0.0;
+        if constexpr (sizeof(T) == 8) {
+            if (ind.coef) {
+                const int64_t t = b * ind.stride, o = r * scm + c * scn;
+                if (ind.coef[t + 3] != 0.0) continue;
+                for (int sp = 0; sp < splits; ++sp) acc += (double)w[sp * MN];
+                T *Cb = ind.c ? ind.c[t] : C + b * scb;
+                double v = ind.coef[t] * acc;
+                if (ind.coef[t + 2] != 0.0) v += ind.coef[t + 2] * Cb[o];
+                if (ind.coef[t + 1] != 0.0) v += ind.coef[t + 1] * ind.d[t][o];
+                Cb[o] = v;
+                continue;
+            }
+        }
         for (int sp = 0; sp < splits; ++sp) acc += (double)w[sp * MN];
         const int64_t o = b * scb + r * scm + c * scn;
         double v = alpha * acc;
@@ -535,6 +571,15 @@ static int launch_gemm(GemmArgs &a, int precision, int tile, hipStream_t s) {
     const bool big = tile == 128;
     switch (precision) {
         case GTN_PREC_F64:
+            if constexpr (sizeof(TIN) == 8) {
+                if (a.g[0].ind.coef) {
+                    if (big)
+                        hipLaunchKernelGGL((k_gemm_fp<TIN, double, 128, 128, 16, true>), dim3(grid), dim3(256), 0, s, a);
+                    else
+                        hipLaunchKernelGGL((k_gemm_fp<TIN, double, 64, 64, 16, true>), dim3(grid), dim3(256), 0, s, a);
+                    break;
+                }
+            }
             if (big)
                 hipLaunchKernelGGL((k_gemm_fp<TIN, double, 128, 128, 16>), dim3(grid), dim3(256), 0, s, a);
             else
@@ -647,7 +692,7 @@ static int scratch_ptr(void **out) {
 // tile <= 0 / target < 0: the heuristics (pick_tile, split_target)
 static int gemm_grouped_impl(const gtn_gemm_desc *groups, int n_groups, int dtype, int precision, void *stream,
                              void *fixed_ws, int64_t fixed_bytes, const char *name, int tile_cfg = 0,
-                             int target_cfg = -1) {
+                             int target_cfg = -1, const GemmIndirect *ind = nullptr) {
     GTN_REQUIRE(n_groups >= 0 && (n_groups == 0 || groups), "%s: bad groups", name);
     GTN_REQUIRE(dtype == GTN_F64 || dtype == GTN_F32, "gtn_gemm_grouped: dtype must be F64 or F32");
     const int tile = tile_cfg > 0 ? tile_cfg : pick_tile(groups, n_groups);
@@ -692,6 +737,7 @@ static int gemm_grouped_impl(const gtn_gemm_desc *groups, int n_groups, int dtyp
             g.scb = d.scb;
             g.alpha = d.alpha;
             g.beta = d.beta;
+            if (ind) g.ind = ind[base + i];
             g.splits = 1;
             g.kchunk = g.K;
             g.scs = 0;
@@ -793,10 +839,10 @@ static int gemm_grouped_impl(const gtn_gemm_desc *groups, int n_groups, int dtyp
                 const dim3 grid(grid_for((int64_t)g.M * g.N * g.batch, 256, 4096)), blk(256);
                 if (dtype == GTN_F64)
                     hipLaunchKernelGGL(k_split_sum<double>, grid, blk, 0, s, (const double *)g.C, g.splits, g.M, g.N,
-                                       g.batch, (double *)o.C, o.scm, o.scn, o.scb, o.alpha, o.beta);
+                                       g.batch, (double *)o.C, o.scm, o.scn, o.scb, o.alpha, o.beta, o.ind);
                 else
                     hipLaunchKernelGGL(k_split_sum<float>, grid, blk, 0, s, (const float *)g.C, g.splits, g.M, g.N,
-                                       g.batch, (float *)o.C, o.scm, o.scn, o.scb, o.alpha, o.beta);
+                                       g.batch, (float *)o.C, o.scm, o.scn, o.scb, o.alpha, o.beta, o.ind);
                 GTN_CHECK_LAUNCH();
             }
             if (ws) {
@@ -932,6 +978,21 @@ extern "C" int gtn_gemm_grouped(const gtn_gemm_desc *groups, int n_groups, int d
     int rc = tuned_config(groups, n_groups, dtype, precision, as_stream(stream), &tile, &target);
     if (rc) return rc;
     return gemm_grouped_impl(groups, n_groups, dtype, precision, stream, nullptr, 0, "gtn_gemm_grouped", tile, target);
+}
+
+int gtn::gemm_grouped_indirect(const gtn_gemm_desc *groups, const GemmIndirect *ind, int n_groups, void *const *tune_c,
+                               void *stream) {
+    int tile = 0, target = -1, rc;
+    if (tune_c) {
+        std::vector<gtn_gemm_desc> plain(groups, groups + n_groups);
+        for (int i = 0; i < n_groups; ++i) plain[i].C = tune_c[i];
+        rc = tuned_config(plain.data(), n_groups, GTN_F64, GTN_PREC_F64, as_stream(stream), &tile, &target);
+    } else {
+        bool found;
+        rc = tuned_lookup(groups, n_groups, GTN_F64, GTN_PREC_F64, &tile, &target, &found);
+    }
+    if (rc) return rc;
+    return gemm_grouped_impl(groups, n_groups, GTN_F64, GTN_PREC_F64, stream, nullptr, 0, "gtn_svd_blocks", tile, target, ind);
 }
 
 extern "C" int gtn_autotune_set(int on) {

@@ -137,11 +137,16 @@ struct SmallBatch {
     double shift_rel;
     int by_abs;
     int max_sweeps;
+    // k_chol_inv inside the filtered range finder: the blocks' state (else null), the values kept, the
+    // index of the product just done and the largest number of products
+    double *st[kMaxBatch];
+    int k[kMaxBatch];
+    int it, iters, cap;
 };
 struct SmallPtrs {
-    int p;
+    int p, k;
     const double *in;
-    double *out, *aux, *lam;
+    double *out, *aux, *lam, *st;
 };
 __device__ __forceinline__ SmallPtrs small_ptrs(const SmallBatch &B) {
     SmallPtrs r;
@@ -152,12 +157,16 @@ __device__ __forceinline__ SmallPtrs small_ptrs(const SmallBatch &B) {
         r.out = B.out[0] + bi * B.d_out;
         r.aux = B.aux[0] ? B.aux[0] + bi * B.d_aux : nullptr;
         r.lam = B.lam[0] ? B.lam[0] + bi * B.d_lam : nullptr;
+        r.st = B.st[0] ? B.st[0] + bi * B.d_in : nullptr;
+        r.k = B.k[0];
     } else {
         r.p = B.p[bi];
         r.in = B.in[bi];
         r.out = B.out[bi];
         r.aux = B.aux[bi];
         r.lam = B.lam[bi];
+        r.st = B.st[bi];
+        r.k = B.k[bi];
     }
     return r;
 }
@@ -306,6 +315,125 @@ __device__ __forceinline__ void chol_factor(double *A, int LD, double *Dv, int n
     }
 }
 
+// ---------------------------------------------------------------------------------------------
+// Filtered range finder (FP64 Gram iteration).  A block's basis is multiplied by a polynomial of its
+// Gram matrix G, one product per degree: kPre plain products G Y with CholeskyQR, whose R has
+// estimates of G's eigenvalues on its diagonal (R_jj -> lambda_j, decreasing; measured within 15 % of
+// lambda_k and 1.0 to 1.6 times lambda_{p+1} after two products), then Chebyshev polynomials of the
+// first kind on [0, b], b the largest of the last (at most 16) R_jj: T_{j+1} = 2 (2 G / b - 1) T_j -
+// T_{j-1}, the linear combination taken in the product's epilogue.  What lies in [0, b] stays within
+// one while lambda > b grows by exp(acosh(2 lambda / b - 1)) per degree: with lambda_k / lambda_{p+1} =
+// 2.6 (blocks of the leg-dim-64 workload) 13 products leave 1e-10 of the missing directions in the kept
+// ones where 20 plain products leave 4e-9.  A block stops when its kept values have grown by e^36
+// over the interval, at most at `cap` products (filter_cap).  Without a gap to speak of, or where a
+// degree's growth of the largest eigenvalue would put the kept ones under CholeskyQR's pivot floor, the
+// block goes on with plain products, and stops when (lambda_k / b)^products has reached e^36.
+// The basis is orthonormalised only after as many degrees as keep the growth of the largest
+// eigenvalue within 1e11 in the Gram matrix of the basis (at most three); T_{j-1} is multiplied by the
+// same R^{-1}.  All of this is per block and on the device (a recorded graph cannot branch): the state
+// holds the block's buffers and coefficients, the product, Gram and basis kernels of a finished or
+// resting block return at once.
+// ---------------------------------------------------------------------------------------------
+constexpr int kPre = 2;
+enum RfSlot {  // 8-byte slots of a block's state
+    kCur = 0,   // T_j (before the first degree: the basis)
+    kPrev,      // T_{j-1}, overwritten by T_{j+1}
+    kS1, kS2,   // two free buffers
+    kAq, kAp, kDq, kDp,  // sources and targets of the basis products with R^{-1} of this round
+    kProd = 8,  // coefficients (x, y, z, skip) of the product
+    kApplyQ = 12, kGram = 16, kApplyP = 20,  // of the basis product of T_j, of the Gram matrix, of T_{j-1}
+    kTotal = 24, kSince, kMaxSince, kCheb,
+    kRfSlots = 32
+};
+__device__ __forceinline__ double *rf_ptr(const double *st, int slot) { return __builtin_bit_cast(double *, st[slot]); }
+__device__ __forceinline__ double rf_bits(double *p) { return __builtin_bit_cast(double, p); }
+
+// first state of every block of a run: the orthonormalised start in Y; grid.x blocks of the run
+__global__ void k_rf_init(double *st, double *Y, double *Z, double *T, double *Bm, int iters, int64_t dws) {
+    const int64_t o = blockIdx.x * dws;
+    st += o;
+    if (threadIdx.x) return;
+    st[kCur] = rf_bits(Y + o);
+    st[kPrev] = rf_bits(Z + o);
+    st[kS1] = rf_bits(T + o);
+    st[kS2] = rf_bits(Bm + o);
+    for (int i = kProd; i < kRfSlots; ++i) st[i] = 0.0;
+    st[kProd] = st[kApplyQ] = st[kGram] = st[kApplyP] = 1.0;
+    st[kApplyQ + 3] = st[kApplyP + 3] = 1.0;
+    st[kGram + 3] = iters <= 1;
+    st[kTotal] = iters;
+    st[kMaxSince] = 1.0;
+}
+// the finished basis (rows x p) back to Y
+__global__ void k_rf_collect(const double *st, double *Y, int64_t n, int64_t dws) {
+    st += blockIdx.y * dws;
+    Y += blockIdx.y * dws;
+    const double *cur = rf_ptr(st, kCur);
+    if (cur == Y) return;
+    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) Y[i] = cur[i];
+}
+
+// One thread, after product `it`: the new basis has been written over T_{j-1}; diag (p values, or null
+// when this round does not orthonormalise) is the diagonal of R.
+__device__ void rf_advance(double *st, const double *diag, int p, int k, int it, int iters, int cap) {
+    double *cur = rf_ptr(st, kPrev), *prev = rf_ptr(st, kCur), *s1 = rf_ptr(st, kS1), *s2 = rf_ptr(st, kS2);
+    bool cheb = st[kCheb] != 0.0;
+    st[kApplyQ + 3] = st[kApplyP + 3] = 1.0;
+    if (diag && it == kPre) {
+        const int w = min(16, (p - k) / 2);
+        double b = 0.0, l0 = 0.0, lk = diag[k - 1];
+        for (int j = 0; j < p; ++j) l0 = fmax(l0, diag[j]);
+        for (int j = max(0, k - 4); j < k; ++j) lk = fmin(lk, diag[j]);
+        for (int j = p - w; j < p; ++j) b = fmax(b, diag[j]);
+        // directions under CholeskyQR's pivot floor (1e-14 in the Gram matrix) are dropped, R_jj = 0: for
+        // the convergence of the others they count as lying at the floor
+        const double rho = lk / fmax(b, 2e-7 * l0);
+        double total = iters;
+        if (w > 0 && rho > 1.05) {
+            const double x = 2.0 * (lk / b) - 1.0, grow = x + sqrt(x * x - 1.0);
+            // growth of lambda_k over that of the largest, squared in the basis' Gram matrix
+            const double under = grow * b / (4.0 * l0);
+            if (under * under > 1e-13) {  // (false for b = 0: NaN)
+                cheb = true;
+                total = fmin((double)cap, kPre + ceil((36.0 - kPre * log(rho)) / log(grow)));
+                st[kMaxSince] = fmin(3.0, fmax(1.0, floor(5.5 / log10(4.0 * l0 / b))));
+                st[kProd] = 2.0 / b, st[kProd + 1] = -1.0;
+            } else {
+                total = fmin((double)iters, ceil(36.0 / log(rho)));
+            }
+        }
+        st[kTotal] = fmax(total, kPre + 1.0);
+        st[kCheb] = cheb;
+    } else if (cheb) {
+        if (it == kPre + 1) {
+            st[kProd] *= 2.0, st[kProd + 1] = -2.0, st[kProd + 2] = -1.0;
+        }
+        if (diag) {
+            st[kAp] = rf_bits(prev), st[kDp] = rf_bits(s2), st[kApplyP + 3] = 0.0;
+        }
+    }
+    if (diag) {
+        st[kAq] = rf_bits(cur), st[kDq] = rf_bits(s1), st[kApplyQ + 3] = 0.0;
+        st[kCur] = rf_bits(s1);
+        st[kS1] = rf_bits(cur);
+        if (st[kApplyP + 3] == 0.0) {
+            st[kPrev] = rf_bits(s2);
+            st[kS2] = rf_bits(prev);
+        } else {
+            st[kPrev] = rf_bits(prev);
+        }
+        st[kSince] = 0.0;
+    } else {
+        st[kCur] = rf_bits(cur);
+        st[kPrev] = rf_bits(prev);
+        st[kSince] += 1.0;
+    }
+    if (it >= st[kTotal]) st[kProd + 3] = 1.0;  // finished
+    // the next round orthonormalises unless the block rests or the round is its last (the basis is
+    // orthonormalised twice after the loop)
+    st[kGram + 3] = it + 1 >= st[kTotal] || st[kSince] + 1.0 < st[kMaxSince];
+}
+
 __global__ void __launch_bounds__(1024) k_chol_inv(SmallBatch B) {
     HIP_DYNAMIC_SHARED(double, sm)
     const SmallPtrs P = small_ptrs(B);
@@ -318,6 +446,14 @@ __global__ void __launch_bounds__(1024) k_chol_inv(SmallBatch B) {
     const int tid = threadIdx.x, nt = blockDim.x;
     const int lane = tid & 63, wave = tid >> 6, nw = nt >> 6;
     const int li = lane & 15, lq = lane >> 4;  // MFMA operand coordinates of this lane
+    if (P.st) {
+        const bool done = P.st[kProd + 3] != 0.0, rest = P.st[kGram + 3] != 0.0;
+        __syncthreads();  // before thread 0 writes the state
+        if (rest) {
+            if (!done && tid == 0) rf_advance(P.st, nullptr, p, P.k, B.it, B.iters, B.cap);
+            return;
+        }
+    }
     // trace and largest diagonal entry, the same in every wavefront
     double tr = 0, dm = 0;
     for (int i = lane; i < p; i += 64) {
@@ -385,6 +521,12 @@ __global__ void __launch_bounds__(1024) k_chol_inv(SmallBatch B) {
     }
     for (int i = wave; i < p; i += nw)
         for (int j = lane; j < p; j += 64) Rinv[i * p + j] = (j >= i) ? ldexp(A[i * LD + j], e2) : 0.0;
+    if (P.st) {
+        __syncthreads();
+        for (int i = tid; i < p; i += nt) A[i] = ldexp(Dv[256 * (i >> 4) + 17 * (i & 15)], -e2);  // the diagonal of R
+        __syncthreads();
+        if (tid == 0) rf_advance(P.st, A, p, P.k, B.it, B.iters, B.cap);
+    }
 }
 
 // round-robin pairing of round `round` (p even): pair t is (a, b) with a != b, every index once
@@ -1368,6 +1510,7 @@ struct Blk {
     int32_t *eM, *eMT, *eYT, *eZT;
     int64_t omp, onp, opp;
     double *Gm;  // m x m Gram matrix M M^T of the Gram-iteration range finder (gram_of(opts))
+    double *St;  // its state (RfSlot)
     int64_t bytes;
 };
 
@@ -1436,7 +1579,7 @@ static void plan_block(const gtn_svd_block &b, const gtn_svd_opts &o, Blk &P, do
             oZs = oz ? take(dbl(kOzSlices * P.opp * P.onp)) : 0,
             oE = oz ? take(dbl(4 * (P.omp + P.onp + 2 * P.opp))) : 0;
     const bool gram = !P.small && gram_of(o, b);
-    int64_t oGm = gram ? take(b.m * b.m) : 0;
+    int64_t oGm = gram ? take(b.m * b.m) : 0, oSt = gram ? take(kRfSlots) : 0;
     P.bytes = (off * 8 + 255) / 256 * 256;
     P.ws = ws;
     if (ws) {
@@ -1468,6 +1611,7 @@ static void plan_block(const gtn_svd_block &b, const gtn_svd_opts &o, Blk &P, do
         P.eYT = oz ? P.eMT + P.onp : nullptr;
         P.eZT = oz ? P.eYT + P.opp : nullptr;
         P.Gm = gram ? ws + oGm : nullptr;
+        P.St = gram ? ws + oSt : nullptr;
     }
 }
 
@@ -1949,6 +2093,95 @@ static int gram_of_blocks(std::vector<Run> &rl, hipStream_t s) {
     return GTN_OK;
 }
 
+// products after which the Chebyshev filter is at least as converged, for every lambda_k / lambda_{p+1},
+// as `iters` plain products are (to e^32: the hardest ratio is the one where those just get there): 13
+// for 20, 20 for 45
+static int filter_cap(int iters) {
+    const double r = exp(32.0 / iters);
+    const int d = (int)ceil((32.0 - kPre * 32.0 / iters) / acosh(2.0 * r - 1.0));
+    return d + kPre < iters ? d + kPre : iters;
+}
+
+// The filtered range finder on the Gram matrices: Y (orthonormal) -> basis, left in Y.
+static int rf_filtered(std::vector<Run> &rl, int iters, hipStream_t s) {
+    for (Run &r : rl) {
+        Blk &f = *r.f;
+        R8N(f.St, kRfSlots, r.dws, r.n, "range-finder state");
+        for (double *b : {f.Y, f.Z, f.T, f.Bm}) R8N(b, f.b.m * f.p, r.dws, r.n, "range-finder basis");
+        LAUNCH(k_rf_init, dim3(r.n), dim3(64), 0, s, f.St, f.Y, f.Z, f.T, f.Bm, iters, r.dws);
+    }
+    auto table = [](double *st, int slot) { return (double *const *)(st + slot); };
+    for (int it = 1; it <= iters; ++it) {
+        std::vector<gtn_gemm_desc> g;
+        std::vector<GemmIndirect> ind;
+        std::vector<void *> out;
+        // `tune`: the buffers of `out` are free, so an untuned signature may be tried out on them
+        auto product = [&](bool tune) -> int {
+            int rc = gemm_grouped_indirect(g.data(), ind.data(), (int)g.size(), tune ? out.data() : nullptr, (void *)s);
+            g.clear();
+            ind.clear();
+            out.clear();
+            return rc;
+        };
+        for (Run &r : rl) {  // T_{j+1} = x G T_j + y T_j + z T_{j-1}, over T_{j-1}
+            Blk &f = *r.f;
+            const int64_t m = f.b.m, p = f.p;
+            g.push_back(gdr(f.Gm, m, 1, f.Y, p, 1, f.Z, p, m, p, m, r.n, r.dws, r.dws, r.dws));
+            ind.push_back(GemmIndirect{nullptr, table(f.St, kCur), table(f.St, kCur), table(f.St, kPrev), f.St + kProd, r.dws});
+            out.push_back(f.T);
+        }
+        int rc = product(it == 1);
+        if (rc) return rc;
+        for (Run &r : rl) {  // W = T_{j+1}^T T_{j+1}
+            Blk &f = *r.f;
+            const int64_t rows = f.b.m, p = f.p;
+            g.push_back(gdr(f.Z, 1, p, f.Z, p, 1, f.W, p, p, p, rows, r.n, r.dws, r.dws, r.dws));
+            ind.push_back(GemmIndirect{table(f.St, kPrev), table(f.St, kPrev), nullptr, nullptr, f.St + kGram, r.dws});
+            out.push_back(f.W);
+        }
+        rc = product(it == 1);
+        if (rc) return rc;
+        SmallBatch proto;
+        memset(&proto, 0, sizeof(proto));
+        proto.shift_rel = 1e-13;
+        proto.it = it;
+        proto.iters = iters;
+        proto.cap = filter_cap(iters);
+        rc = small_launch(
+            rl,
+            [](Blk &b, SmallBatch &sb, int i) {
+                sb.p[i] = (int)b.p;
+                sb.in[i] = b.W;
+                sb.out[i] = b.R;
+                sb.st[i] = b.St;
+                sb.k[i] = b.b.k;
+            },
+            k_chol_inv, sizeof(double), sizeof(double) * (kNB + 1), proto, s);
+        if (rc) return rc;
+        if (it == iters) break;
+        // T_j R^{-1}, and from the second degree on T_{j-1} R^{-1}; the rounds up to there orthonormalise in
+        // every block, so the free buffers are T, then Y and Bm
+        const bool both = it > kPre;
+        for (Run &r : rl) {
+            Blk &f = *r.f;
+            const int64_t m = f.b.m, p = f.p;
+            for (int side = 0; side <= both; ++side) {
+                g.push_back(gdr(f.Y, p, 1, f.R, p, 1, f.T, p, m, p, p, r.n, r.dws, r.dws, r.dws));
+                ind.push_back(GemmIndirect{table(f.St, side ? kAp : kAq), nullptr, nullptr, table(f.St, side ? kDp : kDq),
+                                           f.St + (side ? kApplyP : kApplyQ), r.dws});
+                out.push_back(side ? f.Bm : (both ? f.Y : f.T));
+            }
+        }
+        rc = product(it == 1 || it == kPre + 1);
+        if (rc) return rc;
+    }
+    for (Run &r : rl) {
+        Blk &f = *r.f;
+        LAUNCH(k_rf_collect, grid2(f.b.m * f.p, r.n), dim3(256), 0, s, (const double *)f.St, f.Y, f.b.m * f.p, r.dws);
+    }
+    return GTN_OK;
+}
+
 static int run_blocks(std::vector<Blk> &blocks, const gtn_svd_opts &o, hipStream_t s) {
     const int eig = o.mode == 1;
     std::vector<Blk *> small, large, all;
@@ -2038,25 +2271,14 @@ static int run_blocks(std::vector<Blk> &blocks, const gtn_svd_opts &o, hipStream
         if (rc) return rc;
         rc = orthonormalise(rl, o.iters > 0 ? 1 : 2, s);
         if (rc) return rc;
-        for (int it = 0; it < o.iters; ++it) {
+        if (gram && o.iters > 0) {
+            rc = rf_filtered(rl, o.iters, s);
+            if (rc) return rc;
+            rc = orthonormalise(rl, 2, s);
+            if (rc) return rc;
+        }
+        for (int it = 0; it < (gram ? 0 : o.iters); ++it) {
             const int prec = it >= o.iters - o.f64_tail ? GTN_PREC_F64 : (oz ? o.precision : gprec);
-            if (gram) {  // Y = G Y (into Z, which then becomes the basis)
-                g.clear();
-                for (Run &r : rl) {
-                    Blk &f = *r.f;
-                    R8N(f.Z, f.b.m * f.p, r.dws, r.n, "Gram iterate");
-                    g.push_back(gdr(f.Gm, f.b.m, 1, f.Y, f.p, 1, f.Z, f.p, f.b.m, f.p, f.b.m, r.n, r.dws, r.dws, r.dws));
-                }
-                rc = run(g, GTN_PREC_F64, s);
-                if (rc) return rc;
-                for (Run &r : rl)
-                    for (Blk *b : r.mem) std::swap(b->Y, b->Z);
-                const int every = o.orth_every > 1 ? o.orth_every : 1;
-                rc = (it + 1 == o.iters) ? orthonormalise(rl, 2, s)
-                                         : ((it + 1) % every == 0 ? orthonormalise(rl, 1, s) : GTN_OK);
-                if (rc) return rc;
-                continue;
-            }
             if (oz && prec != GTN_PREC_F64) {  // Z = M^T Y, Y = M Z on int8 slices
                 rc = oz_product(rl, true, &Blk::Y, &Blk::Z, s);
                 if (rc) return rc;

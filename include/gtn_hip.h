@@ -51,7 +51,10 @@ extern "C" {
 #define GTN_PREC_F64_GRAM 7 /* range finder of gtn_svd_blocks only: FP64 subspace iteration on the Gram
                              * matrix G = M M^T (formed once per call from its upper block triangle), one
                              * product G Y per iteration instead of M^T Y and M Z; blocks with m > n
-                             * use the alternating FP64 products */
+                             * use the alternating FP64 products.  After two products each block goes on
+                             * with Chebyshev polynomials of G and stops when its kept values have
+                             * converged, after at most `iters` products (13 for 20) that leave it no
+                             * further from converged than `iters` plain ones */
 
 int gtn_version(void);
 
@@ -333,7 +336,8 @@ typedef struct gtn_svd_opts {
     int32_t precision;  /* GTN_PREC_* for the range finder GEMMs */
     int32_t mode;       /* 0: SVD, 1: Hermitian eig */
     uint64_t seed;
-    int32_t orth_every; /* re-orthonormalise the basis every this many iterations (<= 1: every one) */
+    int32_t orth_every; /* re-orthonormalise the basis every this many iterations (<= 1: every one); the
+                         * Gram iteration (GTN_PREC_F64_GRAM) chooses this by itself */
     int32_t f64_tail;   /* the last f64_tail iterations run in FP64 whatever `precision` is (0: none) */
 } gtn_svd_opts;
 int64_t gtn_svd_workspace_bytes(const gtn_svd_block *blocks, int n_blocks, const gtn_svd_opts *opts);

@@ -121,3 +121,67 @@ def test_non_finite_blocks_raise():
             M[m // 2, n // 3] = bad
             with pytest.raises(L.GrassmannDeviceError):
                 _run([(M, 5)])
+
+def _decaying_blocks(rng, m, n, s, count):
+    blocks = []
+    for _ in range(count):
+        U, _r = np.linalg.qr(rng.standard_normal((m, m)))
+        V, _r = np.linalg.qr(rng.standard_normal((n, m)))
+        blocks.append((U * s) @ V.T)
+    return blocks
+
+
+@pytest.mark.parametrize("iters", [1, 2, 3, 4, 7, 20, 45])
+@pytest.mark.parametrize("rate", [0.9, 0.96, 0.985])
+def test_filtered_range_finder_is_no_further_off_than_plain_products(iters, rate):
+    """The Gram iteration's filter against the alternating products M^T Y, M Z of the same count: every
+    value within the bound that as many plain products give, (sigma_{p+1} / sigma_j)^(4 iters + 2) of it
+    (the error of a Ritz value is quadratic in the missing part of its vector; a Gaussian start of
+    p = 128 of 260 directions misses at most ~1e2 of it), plus rounding."""
+    rng = np.random.default_rng(iters)
+    k, p, m = 32, 128, 260
+    s = rate ** np.arange(m)
+    from grassmanntn_amd.core import settings
+    blocks = [(M, k) for M in _decaying_blocks(rng, m, 300, s, 2)]
+    old = settings.svd_iters
+    settings.svd_iters = iters
+    try:
+        with gtn.precision("f64", "f64_gram"):
+            outs, counts = _run(blocks)
+    finally:
+        settings.svd_iters = old
+    miss = 1e4 * (s[p] / s[:k]) ** (4 * iters + 2)
+    for (M, _k), o, c in zip(blocks, outs, counts):
+        ref = np.linalg.svd(M, compute_uv=False)[:k]
+        got = o[1].numpy()[:k]
+        assert c == k
+        assert np.all(got <= ref * (1 + 1e-13))
+        assert np.all(ref - got <= (miss + 1e-13) * ref[0]), (np.max((ref - got) / ref[0]), miss.max())
+
+
+@pytest.mark.parametrize("case", ["wide", "dropped", "low rank", "flat", "mixed"])
+def test_filtered_range_finder_special_spectra(case):
+    """Spectra at the rules' edges, several in one call: kept values near CholeskyQR's floor, directions
+    under it, rank below k, no gap at all, and blocks that stop at different products."""
+    rng = np.random.default_rng(11)
+    m, k = 260, 24
+    i = np.arange(m)
+    spectra = {"wide": 10.0 ** (-3.2 * np.minimum(i, 60) / 60.0) * np.where(i < 60, 1.0, 0.3),
+               "dropped": np.where(i < 40, 10.0 ** (-6.0 * i / 40), 0.0),
+               "low rank": np.where(i < 9, 0.7 ** i, 0.0),
+               "flat": np.ones(m)}
+    names = ["wide", "low rank", "dropped", "flat"] if case == "mixed" else [case, case]
+    blocks = [(_decaying_blocks(rng, m, 300, spectra[n], 1)[0], k) for n in names]
+    outs, counts = _run(blocks)
+    for name, (M, _k), o, c in zip(names, blocks, outs, counts):
+        ref = np.linalg.svd(M, compute_uv=False)
+        s = o[1].numpy()[:k]
+        u = o[0].numpy()[:, :c]
+        if name == "low rank":
+            assert c == 9
+        elif name == "dropped":
+            assert c >= np.count_nonzero(ref[:k] > 1e-3)
+        else:
+            assert c == k
+        np.testing.assert_allclose(s[:c], ref[:c], rtol=0, atol=(1e-12 if name == "flat" else 1e-13) * ref[0])
+        np.testing.assert_allclose(u.T @ u, np.eye(c), rtol=0, atol=1e-13)
