@@ -114,10 +114,70 @@ class Perm:
         return dst
 
 
+def compose(outer, inner):
+    """outer(inner(.)) as one gather, or None.  It is one when every axis between them carries a single
+    leg: each source axis of `outer` is one component, unsplit, laid out as `inner` writes it, and each
+    output axis of `inner` one component, read in the same encoder.  The legs of `outer` then feed what
+    those of `inner` fed, and both sign tables join into one over their legs' parities."""
+    shape = inner.out_shape()
+    if len(outer.ins) != len(shape):
+        return None
+    feed = {}
+    for cid, (dim, bit, sig, tg) in enumerate(outer.comps):
+        if len(tg) != 1 or tg[0][1] != 1 or tg[0][0] in feed:
+            return None
+        feed[tg[0][0]] = cid
+    through = {}
+    for b, ((dim, enc, sig, split, st, _lo), n, want) in enumerate(zip(outer.ins, shape, strides(shape))):
+        feeds = inner.outs[b][1]
+        if b not in feed or split or dim != n or (st != want and n > 1) or len(feeds) != 1 or feeds[0][1] != 1:
+            return None
+        v = feeds[0][0]
+        vdim, venc, vsig, vcomps = inner.virts[v]
+        if vdim != n or venc != enc or len(vcomps) != 1 or v in through:
+            return None
+        through[v] = b
+        cid = feed[b]
+        if outer.comps[cid][0] != n:
+            return None
+    if len(through) != len(inner.virts):
+        return None
+    G = Perm()
+    G.ins = [list(x) for x in inner.ins]
+    G.outs = list(outer.outs)
+    G.virts = [[d, e, sg, list(c)] for d, e, sg, c in outer.virts]
+    of_outer, of_inner, comps = [], [], []
+    for cid, (dim, bit, sig, tg) in enumerate(outer.comps):
+        b = tg[0][0]
+        icid = inner.virts[inner.outs[b][1][0][0]][3][0]
+        _d, ibit, isig, itg = inner.comps[icid]
+        k = -1
+        if bit >= 0 or ibit >= 0:
+            k = len(of_outer)
+            of_outer.append(bit)
+            of_inner.append(ibit)
+        flips = sig ^ isig ^ outer.ins[b][2] ^ inner.virts[inner.outs[b][1][0][0]][2]
+        comps.append([dim, k, bool(flips), list(itg)])
+    if len(of_outer) > L.MAX_BITS:
+        return None
+    G.comps = comps
+    codes = []
+    for m in range(1 << len(of_outer)):
+        x = outer.codes[sum(((m >> i) & 1) << o for i, o in enumerate(of_outer) if o >= 0)]
+        y = inner.codes[sum(((m >> i) & 1) << o for i, o in enumerate(of_inner) if o >= 0)]
+        codes.append(2 if 2 in (x, y) else x ^ y)
+    G.set_table(codes)
+    return G
+
+
 def run_composed(outer, inner, src, dst=None, alpha=1.0):
-    """outer(inner(src)) in one pass (gtn_permute2): `outer` is built against the contiguous tensor
-    that `inner` would write."""
+    """outer(inner(src)) in one pass: `outer` is built against the contiguous tensor that `inner` would
+    write.  One gather where the two compose (every contraction of a contraction), else gtn_permute2,
+    which maps each element through both."""
     lib = L.lib()
+    one = compose(outer, inner)
+    if one is not None:
+        return one.run(src, dst=dst, alpha=alpha)
     if dst is None:
         dst = DeviceArray.empty(outer.out_shape(), src.dtype)
     if dst.numel() == 0:

@@ -155,19 +155,25 @@ __device__ __forceinline__ int64_t perm_map(const PermArgs &a, uint64_t lin, uin
 // components feed a common input axis.  A group's contribution (source offset, parity bits, sign
 // flip) depends only on the values of its own virtual axes, so it is tabulated once per gather
 // shape, indexed by G = sum over the group's axes of V_v * radix_v, itself a linear function of the
-// output indices.  Per element the map is then an index decomposition, at most kTabGroups table
+// output indices.  Where every extent and stride is a power of two and no two indices share bits of the
+// offset, the map is linear over GF(2) (the encoder, the split and the parities are exclusive ors of the
+// index bits), so every virtual axis is a group of its own and the groups' offsets combine by exclusive
+// or, whatever input axes they share: the operand gather of a contraction's output, whose fused GEMM
+// indices mix the legs of both operand groups, has tables of a few thousand entries instead of none.  Per element the map is then an index decomposition, at most kTabGroups table
 // reads, a sum and an XOR, instead of the component walk of perm_map.
 // ---------------------------------------------------------------------------------------------
 constexpr int kTabGroups = 4;
-struct alignas(16) TabEntry {
-    int64_t off;
-    uint32_t code;  // parity bits | sign flip << 31
-    uint32_t pad;
-};
+// source offset in the low 53 bits, parity bits from bit 53, sign flip in bit 63
+typedef uint64_t TabEntry;
+constexpr int kTabOffBits = 53;
+constexpr uint32_t kTabNeg = 1u << (63 - kTabOffBits);
 struct TabArgs {
     int32_t ng;
     uint32_t gmul[AX][kTabGroups];  // G_g = sum_ax o_ax * gmul[ax][g]
     const TabEntry *tab[kTabGroups];
+    uint64_t signs;   // the sign table's first 32 entries, and whether it has no more
+    int32_t short_signs;
+    int32_t lin;      // offsets combine by exclusive or, else by addition
 };
 struct TabBuild {
     int32_t ng;
@@ -191,12 +197,22 @@ __global__ void k_perm_tables(PermArgs a, TabBuild t, TabEntry *out) {
         int64_t off;
         uint32_t bits, neg;
         perm_core(a, V, t.vmask[g], t.inmask[g], off, bits, neg);
-        TabEntry r;
-        r.off = off;
-        r.code = bits | (neg << 31);
-        r.pad = 0;
-        out[e] = r;
+        out[e] = (uint64_t)off | ((uint64_t)(bits | (neg ? kTabNeg : 0u)) << kTabOffBits);
     }
+}
+
+__device__ __forceinline__ int64_t tab_join(const TabArgs &t, int64_t x, int64_t y) { return t.lin ? x ^ y : x + y; }
+// adds a table entry to an offset and a code (parity bits and sign flip)
+__device__ __forceinline__ void tab_add(const TabArgs &t, TabEntry e, int64_t &off, uint32_t &c) {
+    off = tab_join(t, off, (int64_t)(e & (((uint64_t)1 << kTabOffBits) - 1)));
+    c ^= (uint32_t)(e >> kTabOffBits);
+}
+// sign table entry (0: +1, 1: -1, 2: zero) of a code; tables of up to five parity bits sit in a register
+__device__ __forceinline__ uint32_t tab_sign(const PermArgs &a, const TabArgs &t, uint32_t c) {
+    const uint32_t bits = c & (kTabNeg - 1);
+    if (!t.short_signs) return sign_code(a, bits, c / kTabNeg);
+    const uint32_t s = (uint32_t)(t.signs >> (2 * bits)) & 3u;
+    return s == 2u ? 2u : (s ^ (c / kTabNeg));
 }
 
 // Table indices of the output axes 0 .. hi for the row-major index `lin` over those axes.
@@ -223,53 +239,15 @@ __device__ __forceinline__ void tab_index(const PermArgs &a, const TabArgs &t, u
     }
 }
 
-// Source offset and sign code of the element with table indices G.
-__device__ __forceinline__ int64_t tab_lookup(const PermArgs &a, const TabArgs &t, const uint32_t (&G)[kTabGroups],
-                                              uint32_t &code) {
-    int64_t off = 0;
-    uint32_t c = 0;
-#pragma unroll
-    for (int g = 0; g < kTabGroups; ++g)
-        if (g < t.ng) {
-            const TabEntry e = t.tab[g][G[g]];
-            off += e.off;
-            c ^= e.code;
-        }
-    code = sign_code(a, c & 0x7fffffffu, c >> 31);
-    return off;
-}
-
 __device__ __forceinline__ int64_t tab_map(const PermArgs &a, const TabArgs &t, uint64_t lin, uint32_t &code) {
     uint32_t G[kTabGroups];
-#pragma unroll
-    for (int g = 0; g < kTabGroups; ++g) G[g] = 0;
-    uint64_t rest = lin;
-    for (int ax = a.n_out - 1; ax >= 0; --ax) {
-        uint32_t o;
-        if (a.out_shift[ax] >= 0) {
-            o = (uint32_t)(rest & (uint64_t)(a.out_dim[ax] - 1));
-            rest >>= a.out_shift[ax];
-        } else if ((rest >> 32) == 0) {
-            const uint32_t r32 = (uint32_t)rest, d = a.out_dim[ax];
-            o = r32 % d;
-            rest = r32 / d;
-        } else {
-            o = (uint32_t)(rest % a.out_dim[ax]);
-            rest /= a.out_dim[ax];
-        }
-#pragma unroll
-        for (int g = 0; g < kTabGroups; ++g) G[g] += o * t.gmul[ax][g];
-    }
+    tab_index(a, t, lin, a.n_out - 1, G);
     int64_t off = 0;
     uint32_t c = 0;
 #pragma unroll
     for (int g = 0; g < kTabGroups; ++g)
-        if (g < t.ng) {
-            const TabEntry e = t.tab[g][G[g]];
-            off += e.off;
-            c ^= e.code;
-        }
-    code = sign_code(a, c & 0x7fffffffu, c >> 31);
+        if (g < t.ng) tab_add(t, t.tab[g][G[g]], off, c);
+    code = tab_sign(a, t, c);
     return off;
 }
 
@@ -287,60 +265,11 @@ __device__ __forceinline__ int64_t map_elem(const PermArgs &a, const TabArgs &t,
 // kPermUnroll elements together, then their source reads, so kPermUnroll dependent load chains are in
 // flight per lane instead of one.
 constexpr int kPermUnroll = 4;
-// Output suffix for the chunk-uniform walk: the fewest trailing output axes (at most two) whose
-// extent is a multiple of the chunk and below 2^32 (the in-suffix index is 32-bit), so that every
-// chunk shares the indices of the axes before them; 0 when there is none.
-__device__ __forceinline__ int chunk_suffix(const PermArgs &a, int64_t chunk) {
-    if (a.n_out >= 1 && (int64_t)a.out_dim[a.n_out - 1] % chunk == 0) return 1;
-    if (a.n_out >= 2 && a.out_shift[a.n_out - 1] >= 0) {
-        const int64_t span = (int64_t)a.out_dim[a.n_out - 1] * a.out_dim[a.n_out - 2];
-        if (span % chunk == 0 && span < ((int64_t)1 << 32)) return 2;
-    }
-    return 0;
-}
 
 template <typename T, bool TAB>
 __global__ void __launch_bounds__(256) k_permute(PermArgs a, TabArgs tb, const T *__restrict__ src, T *__restrict__ dst) {
     const double al = a.alpha_re;
     const int64_t chunk = (int64_t)kPermUnroll * blockDim.x;
-    if constexpr (TAB) {
-        // chunk-uniform walk: the leading axes' table indices are formed once per chunk (the same in
-        // every lane), each element adds only its trailing one or two indices times their multipliers
-        const int ns = chunk_suffix(a, chunk);
-        if (ns > 0) {
-            const int last = a.n_out - 1;
-            const uint64_t span = ns == 1 ? a.out_dim[last] : (uint64_t)a.out_dim[last] * a.out_dim[last - 1];
-            for (int64_t i0 = blockIdx.x * chunk; i0 < a.total; i0 += (int64_t)gridDim.x * chunk) {
-                const uint64_t row = (uint64_t)i0 / span;
-                const uint32_t c0 = (uint32_t)((uint64_t)i0 - row * span);
-                uint32_t Gb[kTabGroups];
-                tab_index(a, tb, row, last - ns, Gb);
-                int64_t off[kPermUnroll];
-                uint32_t code[kPermUnroll];
-#pragma unroll
-                for (int u = 0; u < kPermUnroll; ++u) {
-                    const uint32_t c = c0 + threadIdx.x + u * blockDim.x;
-                    uint32_t o0 = c, o1 = 0;
-                    if (ns == 2) {
-                        o0 = c & (a.out_dim[last] - 1);
-                        o1 = c >> a.out_shift[last];
-                    }
-                    uint32_t G[kTabGroups];
-#pragma unroll
-                    for (int g = 0; g < kTabGroups; ++g)
-                        G[g] = Gb[g] + o0 * tb.gmul[last][g] + (ns == 2 ? o1 * tb.gmul[last - 1][g] : 0u);
-                    off[u] = tab_lookup(a, tb, G, code[u]);
-                }
-                double v[kPermUnroll];
-#pragma unroll
-                for (int u = 0; u < kPermUnroll; ++u) v[u] = (code[u] == 2u) ? 0.0 : (double)src[off[u]];
-#pragma unroll
-                for (int u = 0; u < kPermUnroll; ++u)
-                    dst[i0 + threadIdx.x + u * blockDim.x] = (T)(code[u] == 2u ? 0.0 : v[u] * (code[u] ? -al : al));
-            }
-            return;
-        }
-    }
     for (int64_t i0 = blockIdx.x * chunk + threadIdx.x; i0 < a.total; i0 += (int64_t)gridDim.x * chunk) {
         int64_t off[kPermUnroll];
         uint32_t code[kPermUnroll];
@@ -359,6 +288,86 @@ __global__ void __launch_bounds__(256) k_permute(PermArgs a, TabArgs tb, const T
             const int64_t i = i0 + u * (int64_t)blockDim.x;
             if (i < a.total) dst[i] = (T)(code[u] == 2u ? 0.0 : v[u] * (code[u] ? -al : al));
         }
+    }
+}
+
+// Row walk of a table-driven gather.  The output is rows of `width` consecutive elements, the trailing
+// ns axes; a workgroup takes one chunk of U * 256 columns of `rows_per` rows, one after another.  What
+// the leading axes add to the table indices is the same in every lane: groups that no trailing axis
+// feeds are looked up once per row, the others (usually one) per element, and not again while their
+// leading part stays the same.  An element then costs a source read and a few integer operations where
+// the walk above reads up to four entries for it.  MI355X, 64^4 doubles: encoder switch 71 -> 52 us
+// (5.2 TB/s), operand gathers of a contraction 55 -> 44 us (6.1 TB/s); tiles (below) with the same
+// economy 164 -> 82 us; 8^4 doubles 20 -> 5 us.
+struct RowArgs {
+    int64_t width, rows;
+    int32_t ns, chunks, rows_per;
+    uint32_t vary;  // groups that the trailing axes feed
+};
+template <typename T, int U>
+__global__ void __launch_bounds__(256) k_permute_rows(PermArgs a, TabArgs tb, RowArgs w, const T *__restrict__ src,
+                                                      T *__restrict__ dst) {
+    const double al = a.alpha_re;
+    const int last = a.n_out - 1, lead = last - w.ns;
+    const int64_t c0 = (int64_t)(blockIdx.x % w.chunks) * (U * 256);
+    const int64_t r0 = (int64_t)(blockIdx.x / w.chunks) * w.rows_per;
+    const int64_t r1 = r0 + w.rows_per < w.rows ? r0 + w.rows_per : w.rows;
+    // table indices of this lane's columns
+    uint32_t Gc[U][kTabGroups];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+#pragma unroll
+        for (int g = 0; g < kTabGroups; ++g) Gc[u][g] = 0;
+        uint32_t c = (uint32_t)c0 + threadIdx.x + u * 256;
+        for (int ax = last; ax > lead; --ax) {
+            const uint32_t o = ax > lead + 1 ? c & (a.out_dim[ax] - 1) : c;
+            if (ax > lead + 1) c >>= a.out_shift[ax];
+#pragma unroll
+            for (int g = 0; g < kTabGroups; ++g) Gc[u][g] += o * tb.gmul[ax][g];
+        }
+    }
+    int64_t offc[U];
+    uint32_t cc[U];
+    uint32_t Gv[kTabGroups];  // the leading part of the varying groups that offc and cc hold
+    for (int64_t row = r0; row < r1; ++row) {
+        uint32_t G[kTabGroups];
+        tab_index(a, tb, (uint64_t)row, lead, G);
+        int64_t offr = 0;
+        uint32_t cr = 0;
+        bool same = row > r0;
+#pragma unroll
+        for (int g = 0; g < kTabGroups; ++g)
+            if (g < tb.ng) {
+                if ((w.vary >> g) & 1u) {
+                    same = same && G[g] == Gv[g];
+                    Gv[g] = G[g];
+                } else {
+                    tab_add(tb, tb.tab[g][G[g]], offr, cr);
+                }
+            }
+        if (!same) {
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                offc[u] = 0;
+                cc[u] = 0;
+            }
+#pragma unroll
+            for (int g = 0; g < kTabGroups; ++g)
+                if (g < tb.ng && ((w.vary >> g) & 1u)) {
+#pragma unroll
+                    for (int u = 0; u < U; ++u) tab_add(tb, tb.tab[g][G[g] + Gc[u][g]], offc[u], cc[u]);
+                }
+        }
+        uint32_t code[U];
+        double v[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            code[u] = tab_sign(a, tb, cc[u] ^ cr);
+            v[u] = code[u] == 2u ? 0.0 : (double)src[tab_join(tb, offc[u], offr)];
+        }
+        T *d = dst + row * w.width + c0 + threadIdx.x;
+#pragma unroll
+        for (int u = 0; u < U; ++u) d[u * 256] = (T)(code[u] == 2u ? 0.0 : v[u] * (code[u] ? -al : al));
     }
 }
 
@@ -433,16 +442,44 @@ __global__ void __launch_bounds__(256) k_permute_tiled(PermArgs a, TabArgs tb, T
     const int64_t nblk = per * t.rest_total;
     const int d1 = (int)a.out_dim[t.t1], d0 = (int)a.out_dim[t.t0];
     const int64_t s1 = t.ostr[t.t1];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     for (int64_t blk = blockIdx.x; blk < nblk; blk += gridDim.x) {
         const int64_t r = blk / per;
         const int64_t q = blk - r * per;
         const int i1b = (int)(q / t.tiles0) * 64, i0b = (int)(q % t.tiles0) * 64;
         int64_t base = 0, rr = r;
+        uint32_t Gb[kTabGroups];
+        if constexpr (TAB) {
+#pragma unroll
+            for (int g = 0; g < kTabGroups; ++g)
+                Gb[g] = (uint32_t)i1b * tb.gmul[t.t1][g] + (uint32_t)i0b * tb.gmul[t.t0][g];
+        }
         for (int k = t.n_rest - 1; k >= 0; --k) {
             const int ax = t.rest_ax[k];
-            const int64_t d = a.out_dim[ax];
-            base += (rr % d) * t.ostr[ax];
-            rr /= d;
+            int64_t o;
+            if (a.out_shift[ax] >= 0) {
+                o = rr & (a.out_dim[ax] - 1);
+                rr >>= a.out_shift[ax];
+            } else {
+                o = rr % a.out_dim[ax];
+                rr /= a.out_dim[ax];
+            }
+            base += o * t.ostr[ax];
+            if constexpr (TAB) {
+#pragma unroll
+                for (int g = 0; g < kTabGroups; ++g) Gb[g] += (uint32_t)o * tb.gmul[ax][g];
+            }
+        }
+        // a lane's elements share i1 = i1b + lane, a wavefront's share i0: with tables, groups that i0
+        // does not feed are looked up once, groups that only i0 feeds at one address per wavefront
+        int64_t off1 = 0;
+        uint32_t c1 = 0;
+        const bool in1 = i1b + lane < d1;
+        if constexpr (TAB) {
+#pragma unroll
+            for (int g = 0; g < kTabGroups; ++g)
+                if (g < tb.ng && tb.gmul[t.t0][g] == 0)
+                    tab_add(tb, tb.tab[g][Gb[g] + (in1 ? (uint32_t)lane * tb.gmul[t.t1][g] : 0u)], off1, c1);
         }
         // 16 elements per lane in two batches of 8: index maps and table reads first, then the
         // source reads, so that 8 load chains are in flight per lane
@@ -452,20 +489,30 @@ __global__ void __launch_bounds__(256) k_permute_tiled(PermArgs a, TabArgs tb, T
             uint32_t code[8];
 #pragma unroll
             for (int u = 0; u < 8; ++u) {
-                const int e = threadIdx.x + 256 * (8 * h + u);
-                const int i1 = i1b + (e & 63), i0 = i0b + (e >> 6);
+                const int l0 = wave + 4 * (8 * h + u);
+                const int i1 = i1b + lane, i0 = i0b + l0;
                 code[u] = 2u;
                 off[u] = 0;
-                if (i1 < d1 && i0 < d0) off[u] = map_elem<TAB>(a, tb, (uint64_t)(base + i1 * s1 + i0), code[u]);
+                if (i1 < d1 && i0 < d0) {
+                    if constexpr (TAB) {
+                        uint32_t c = c1;
+                        off[u] = off1;
+#pragma unroll
+                        for (int g = 0; g < kTabGroups; ++g)
+                            if (g < tb.ng && tb.gmul[t.t0][g] != 0)
+                                tab_add(tb, tb.tab[g][Gb[g] + (uint32_t)l0 * tb.gmul[t.t0][g] + (uint32_t)lane * tb.gmul[t.t1][g]],
+                                        off[u], c);
+                        code[u] = tab_sign(a, tb, c);
+                    } else {
+                        off[u] = map_elem<TAB>(a, tb, (uint64_t)(base + i1 * s1 + i0), code[u]);
+                    }
+                }
             }
             double v[8];
 #pragma unroll
             for (int u = 0; u < 8; ++u) v[u] = (code[u] == 2u) ? 0.0 : (double)src[off[u]] * (code[u] ? -al : al);
 #pragma unroll
-            for (int u = 0; u < 8; ++u) {
-                const int e = threadIdx.x + 256 * (8 * h + u);
-                tile[e & 63][e >> 6] = v[u];
-            }
+            for (int u = 0; u < 8; ++u) tile[lane][wave + 4 * (8 * h + u)] = v[u];
         }
         __syncthreads();
         for (int e = threadIdx.x; e < 64 * 64; e += 256) {
@@ -905,9 +952,11 @@ static bool plan_tiles(const gtn_perm_desc *d, TileArgs &t) {
 }
 
 // Group the virtual axes for the table-driven map (k_perm_tables).  Returns false when the gather
-// is too small to repay a table or a group's table would be large.
+// is so small that one wavefront walks it, or a group's table would be large: the table is built once per
+// gather shape (about 20 us), and every gather without one walks the descriptor with its index vectors in
+// scratch memory, 12 to 20 us for the smallest (MI355X; 5 us with tables).
 static bool plan_groups(const gtn_perm_desc *d, int64_t total, TabBuild &tb, TabArgs &ta) {
-    if (total < (1 << 16) || d->n_virt == 0) return false;
+    if (total < 64 || d->n_virt == 0) return false;
     const int nv = d->n_virt;
     int64_t ext[AX];
     for (int v = 0; v < nv; ++v) ext[v] = 1;
@@ -915,7 +964,46 @@ static bool plan_groups(const gtn_perm_desc *d, int64_t total, TabBuild &tb, Tab
         for (int t = 0; t < 2; ++t)
             if (d->out_virt[ax][t] >= 0 && d->out_dim[ax] > 0)
                 ext[d->out_virt[ax][t]] += (d->out_dim[ax] - 1) * d->out_vmul[ax][t];
-    // union virtual axes whose components feed a common input axis
+    // the virtual axis that feeds each input axis (-1: none, -2: several), and whether the map is linear
+    // over GF(2)
+    bool lin = true;
+    {
+        int feeder[AX];
+        uint64_t fbits[AX] = {0}, used = 0;
+        for (int b = 0; b < d->n_in; ++b) feeder[b] = -1;
+        auto pow2 = [](int64_t x) { return x > 0 && (x & (x - 1)) == 0; };
+        int jj = 0;
+        for (int v = 0; v < nv; ++v)
+            for (int t = 0; t < d->virt_ncomp[v]; ++t, ++jj) {
+                lin = lin && pow2(d->comp_dim[jj]);
+                for (int u = 0; u < 2; ++u) {
+                    const int b = d->comp_in[jj][u];
+                    if (b < 0) continue;
+                    feeder[b] = feeder[b] == -1 || feeder[b] == v ? v : -2;
+                    if (d->comp_dim[jj] == 1) continue;
+                    lin = lin && pow2(d->comp_mult[jj][u]);
+                    const uint64_t bits = (uint64_t)(d->comp_dim[jj] - 1) * (uint64_t)d->comp_mult[jj][u];
+                    lin = lin && !(fbits[b] & bits);
+                    fbits[b] |= bits;
+                }
+            }
+        auto take = [&](int64_t n, int64_t stride) {  // offset bits of an index of n values
+            if (n <= 1 || stride == 0) return;
+            const uint64_t bits = (uint64_t)(n - 1) * (uint64_t)stride;
+            lin = lin && pow2(n) && pow2(stride) && !(used & bits);
+            used |= bits;
+        };
+        for (int b = 0; b < d->n_in && lin; ++b) {
+            lin = pow2(d->in_dim[b]) && !(d->in_sigma[b] && feeder[b] == -2);
+            if (d->in_split[b]) {
+                take(2 < d->in_dim[b] ? 2 : d->in_dim[b], d->in_stride_lo[b]);
+                take(d->in_dim[b] >> 1, d->in_stride[b]);
+            } else {
+                take(d->in_dim[b], d->in_stride[b]);
+            }
+        }
+    }
+    // union virtual axes whose components feed a common input axis (a linear map needs no union)
     int parent[AX];
     for (int v = 0; v < nv; ++v) parent[v] = v;
     auto root = [&](int v) {
@@ -934,7 +1022,7 @@ static bool plan_groups(const gtn_perm_desc *d, int64_t total, TabBuild &tb, Tab
                 feeds[v] |= 1u << b;
                 if (owner[b] < 0)
                     owner[b] = v;
-                else
+                else if (!lin)
                     parent[root(v)] = root(owner[b]);
             }
     // groups in order of their smallest virtual axis
@@ -980,10 +1068,13 @@ static bool plan_groups(const gtn_perm_desc *d, int64_t total, TabBuild &tb, Tab
     }
     int64_t entries = 0;
     for (int g = 0; g < ng; ++g) entries += gsize[g];
-    if (entries * 4 > total) return false;
+    if (entries > (total < (1 << 16) ? total : total / 4)) return false;
     memset(&tb, 0, sizeof(tb));
     memset(&ta, 0, sizeof(ta));
     tb.ng = ta.ng = ng;
+    ta.signs = (uint64_t)d->table[0] | (uint64_t)d->table[1] << 32;
+    ta.short_signs = d->n_bits <= 5;
+    ta.lin = lin;
     int64_t rad_of[AX];
     int grp_of[AX];
     for (int g = 0; g < ng; ++g) {
@@ -1021,6 +1112,14 @@ static std::mutex g_tab_mu;
 static std::map<std::string, TabCacheEntry> g_tab_cache;
 static int64_t g_tab_bytes = 0;
 constexpr int64_t kTabCacheBytes = 64ll << 20;
+constexpr int64_t kTabSlab = 1 << 20;
+struct TabStore {
+    char *next = nullptr;
+    int64_t left = 0;
+};
+static std::map<int, TabStore> g_tab_store;      // per device: the slab being cut
+static std::vector<void *> g_tab_slabs;
+static std::map<int, hipStream_t> g_tab_stream;  // per device: the stream tables are built on
 
 static int tab_tables(const PermArgs &a, const TabBuild &tb, hipStream_t s, TabArgs &ta) {
     int dev;
@@ -1040,25 +1139,36 @@ static int tab_tables(const PermArgs &a, const TabBuild &tb, hipStream_t s, TabA
         if (g_tab_bytes + n * (int64_t)sizeof(TabEntry) > kTabCacheBytes && !g_tab_cache.empty() &&
             !graphs_alive() && !capture_open()) {
             GTN_CHECK_HIP(hipDeviceSynchronize());
-            for (auto &e : g_tab_cache) GTN_CHECK_HIP(hipFree(e.second.dev));
+            for (void *slab : g_tab_slabs) GTN_CHECK_HIP(hipFree(slab));
+            g_tab_slabs.clear();
+            g_tab_store.clear();
             g_tab_cache.clear();
             g_tab_bytes = 0;
         }
-        TabEntry *p = nullptr;
-        GTN_CHECK_HIP(hipMalloc(&p, n * sizeof(TabEntry)));
+        // tables are cut from slabs, one at a time in use per device; the build stream is kept with it
+        TabStore &store = g_tab_store[dev];
+        const int64_t bytes = (n * (int64_t)sizeof(TabEntry) + 255) / 256 * 256;
+        if (store.left < bytes) {
+            const int64_t slab = bytes > kTabSlab ? bytes : kTabSlab;
+            void *p = nullptr;
+            GTN_CHECK_HIP(hipMalloc(&p, slab));
+            g_tab_slabs.push_back(p);
+            store.next = (char *)p;
+            store.left = slab;
+        }
+        hipStream_t &bs = g_tab_stream[dev];
+        if (!bs) GTN_CHECK_HIP(hipStreamCreateWithFlags(&bs, hipStreamNonBlocking));
         // built on a stream of their own and finished here: the tables are shared by later gathers
         // on any stream, and the caller's stream may be capturing a graph
-        hipStream_t bs = nullptr;
-        GTN_CHECK_HIP(hipStreamCreateWithFlags(&bs, hipStreamNonBlocking));
+        TabEntry *p = (TabEntry *)store.next;
         hipLaunchKernelGGL(k_perm_tables, dim3(grid_for(n, 256, 4096)), dim3(256), 0, bs, a, tb, p);
-        hipError_t le = hipGetLastError();
-        hipError_t se = hipStreamSynchronize(bs);
-        (void)hipStreamDestroy(bs);
-        GTN_CHECK_HIP(le);
-        GTN_CHECK_HIP(se);
+        GTN_CHECK_HIP(hipGetLastError());
+        GTN_CHECK_HIP(hipStreamSynchronize(bs));
         (void)s;
+        store.next += bytes;
+        store.left -= bytes;
         it = g_tab_cache.emplace(key, TabCacheEntry{p, n}).first;
-        g_tab_bytes += n * (int64_t)sizeof(TabEntry);
+        g_tab_bytes += bytes;
     }
     for (int g = 0; g < tb.ng; ++g) ta.tab[g] = it->second.dev + tb.start[g];
     return GTN_OK;
@@ -1072,6 +1182,38 @@ static bool tiles_enabled() {
         on = (e && atoi(e) == 0) ? 0 : 1;
     }
     return on == 1;
+}
+
+// Row walk (k_permute_rows) where some trailing axes -- all but the first of them powers of two, the
+// index within a row is decomposed by shifts -- make rows of whole chunks.  1024-column chunks for
+// gathers that still fill the device with them (four loads in flight per lane), 256 otherwise.  Each
+// workgroup takes up to 8 rows once there are more than 16 workgroups per compute unit without that.
+static bool plan_rows(const PermArgs &a, const TabArgs &tb, RowArgs &w, int &U) {
+    U = a.total >= (1 << 20) ? 4 : 1;
+    for (;; U = 1) {
+        const int64_t chunk = U * 256;
+        int64_t width = 1;
+        for (int ns = 1; ns <= a.n_out; ++ns) {
+            const int ax = a.n_out - ns;
+            if (ns > 1 && a.out_shift[ax + 1] < 0) break;
+            width *= a.out_dim[ax];
+            if (width >= ((int64_t)1 << 32)) break;
+            if (width % chunk) continue;
+            w.width = width;
+            w.rows = a.total / width;
+            w.ns = ns;
+            w.chunks = (int32_t)(width / chunk);
+            const int64_t per = w.rows * w.chunks / 4096;
+            w.rows_per = (int32_t)(per < 1 ? 1 : (per > 8 ? 8 : per));
+            if ((w.rows + w.rows_per - 1) / w.rows_per * w.chunks >= ((int64_t)1 << 31)) return false;
+            w.vary = 0;
+            for (int k = 0; k < ns; ++k)
+                for (int g = 0; g < tb.ng; ++g)
+                    if (tb.gmul[a.n_out - 1 - k][g]) w.vary |= 1u << g;
+            return true;
+        }
+        if (U == 1) return false;
+    }
 }
 
 int gtn_permute(const gtn_perm_desc *d, const void *src, void *dst, void *stream) {
@@ -1090,7 +1232,8 @@ int gtn_permute(const gtn_perm_desc *d, const void *src, void *dst, void *stream
     TabArgs tb;
     memset(&tb, 0, sizeof(tb));
     TabBuild build;
-    const bool tab = d->dtype != GTN_C128 && getenv("GTN_PERM_NO_TABLES") == nullptr && plan_groups(d, a.total, build, tb);
+    const bool tab = (d->dtype == GTN_F64 || d->dtype == GTN_F32) && getenv("GTN_PERM_NO_TABLES") == nullptr &&
+                     plan_groups(d, a.total, build, tb);
     if (tab) {
         rc = tab_tables(a, build, s, tb);
         if (rc) return rc;
@@ -1110,6 +1253,22 @@ int gtn_permute(const gtn_perm_desc *d, const void *src, void *dst, void *stream
             else
                 hipLaunchKernelGGL((k_permute_tiled<float, false>), gt, bt, 0, s, a, tb, t, (const float *)src, (float *)dst);
         }
+        GTN_CHECK_LAUNCH();
+        return GTN_OK;
+    }
+    RowArgs w;
+    int U;
+    if (tab && plan_rows(a, tb, w, U)) {
+        const dim3 gr((unsigned)((w.rows + w.rows_per - 1) / w.rows_per * w.chunks)), br(256);
+#define GTN_ROWS(T, N) hipLaunchKernelGGL((k_permute_rows<T, N>), gr, br, 0, s, a, tb, w, (const T *)src, (T *)dst)
+        if (d->dtype == GTN_F64) {
+            if (U == 4) GTN_ROWS(double, 4);
+            else GTN_ROWS(double, 1);
+        } else {
+            if (U == 4) GTN_ROWS(float, 4);
+            else GTN_ROWS(float, 1);
+        }
+#undef GTN_ROWS
         GTN_CHECK_LAUNCH();
         return GTN_OK;
     }

@@ -1,0 +1,39 @@
+"""gtn_permute bit for bit against its definition over random gathers: every table-driven path (row walk
+in 256- and 1024-column chunks, LDS tiles, element walk; groups joined by addition or exclusive or) and
+the descriptor walk, sizes from one element to beyond the largest chunk, F64 and F32."""
+import numpy as np
+import pytest
+
+from gather_reference import gather, offsets, random_gather
+
+pytestmark = pytest.mark.gpu
+
+gtn = pytest.importorskip("grassmanntn_amd")
+
+
+def _run(P, src, alpha):
+    from grassmanntn_amd._device import DeviceArray
+    return P.run(DeviceArray.from_numpy(src), alpha=alpha).numpy()
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("odd", [False, True])
+@pytest.mark.parametrize("sizes", [(1,), (2, 4), (4, 4, 4), (8, 8, 16), (16, 32, 16), (8, 8, 8, 8), (16, 16, 32, 16), (2, 64, 2, 128),
+                                   (32, 16, 64, 64), (256, 8, 1024)])
+def test_random_gathers(sizes, odd, dtype):
+    for seed in range(6):
+        rng = np.random.default_rng([seed, len(sizes), sizes[0], odd])
+        P, n = random_gather(rng, sizes, odd=odd, trace=seed == 5 and np.prod(sizes) <= 1 << 16)
+        src = rng.standard_normal(n).astype(dtype)
+        assert offsets(P)[0].max() < n
+        assert np.array_equal(_run(P, src, 1.0), gather(P, src, 1.0)), (sizes, seed)
+        assert np.array_equal(_run(P, src, -0.5), gather(P, src, -0.5)), (sizes, seed)
+
+
+def test_random_gathers_without_tables(monkeypatch):
+    monkeypatch.setenv("GTN_PERM_NO_TABLES", "1")
+    for seed in range(6):
+        rng = np.random.default_rng(seed)
+        P, n = random_gather(rng, (16, 32, 16), odd=seed % 2 == 1)
+        src = rng.standard_normal(n)
+        assert np.array_equal(_run(P, src, 1.0), gather(P, src, 1.0)), seed
