@@ -154,8 +154,8 @@ __device__ __forceinline__ int64_t perm_map(const PermArgs &a, uint64_t lin, uin
 // Table-driven map.  The virtual axes fall into groups: two virtual axes share a group when their
 // components feed a common input axis.  A group's contribution (source offset, parity bits, sign
 // flip) depends only on the values of its own virtual axes, so it is tabulated once per gather
-// shape, indexed by G = sum over the group's axes of V_v * radix_v, itself a linear function of the
-// output indices.  Where every extent and stride is a power of two and no two indices share bits of the
+// shape, indexed by G = the mixed-radix number of the output indices that feed those axes, in an order
+// that keeps the lanes of a wavefront on consecutive entries.  Where every extent and stride is a power of two and no two indices share bits of the
 // offset, the map is linear over GF(2) (the encoder, the split and the parities are exclusive ors of the
 // index bits), so every virtual axis is a group of its own and the groups' offsets combine by exclusive
 // or, whatever input axes they share: the operand gather of a contraction's output, whose fused GEMM
@@ -179,9 +179,9 @@ struct TabBuild {
     int32_t ng;
     int64_t start[kTabGroups + 1];  // first entry of each group's table
     uint32_t vmask[kTabGroups], inmask[kTabGroups];
-    int32_t nv[kTabGroups];
-    int8_t vid[kTabGroups][AX];
-    uint32_t vrad[kTabGroups][AX], vext[kTabGroups][AX];
+    int32_t nx[kTabGroups];  // the output axes that feed the group and their radices in its table
+    int8_t ax[kTabGroups][AX];
+    uint32_t rad[kTabGroups][AX];
 };
 
 __global__ void k_perm_tables(PermArgs a, TabBuild t, TabEntry *out) {
@@ -193,7 +193,12 @@ __global__ void k_perm_tables(PermArgs a, TabBuild t, TabEntry *out) {
         uint64_t V[AX];
 #pragma unroll
         for (int b = 0; b < AX; ++b) V[b] = 0;
-        for (int i = 0; i < t.nv[g]; ++i) V[t.vid[g][i]] = (G / t.vrad[g][i]) % t.vext[g][i];
+        for (int i = 0; i < t.nx[g]; ++i) {
+            const int ax = t.ax[g][i];
+            const uint64_t o = (G / t.rad[g][i]) % a.out_dim[ax];
+            if (a.out_virt[ax][0] >= 0) V[a.out_virt[ax][0]] += o * (uint64_t)a.out_vmul[ax][0];
+            if (a.out_virt[ax][1] >= 0) V[a.out_virt[ax][1]] += o * (uint64_t)a.out_vmul[ax][1];
+        }
         int64_t off;
         uint32_t bits, neg;
         perm_core(a, V, t.vmask[g], t.inmask[g], off, bits, neg);
@@ -423,11 +428,15 @@ __global__ void k_permute_c128(PermArgs a, const double2 *__restrict__ src, doub
 }
 
 // Tiled variant for gathers whose output's last axis is far apart in the source: output axis t1
-// (the one whose unit step moves the source the least) and the last output axis t0 form 64 x 64
-// tiles.  A tile is read with t1 fastest (consecutive source addresses), staged in LDS with its
-// signs applied, and written with t0 fastest (consecutive output addresses).
+// (the one whose consecutive indices share the most source lines) and the last output axis t0 form
+// n1 x n0 tiles.  A tile is read with t1 fastest (consecutive source addresses), staged in LDS with its
+// signs applied, and written with t0 fastest (consecutive output addresses).  Fused output axes are cut
+// into their legs first (split_axes): the leg that runs through consecutive addresses is often the upper
+// part of a fused index.  MI355X, eight 64^4 tensors: joins into parity blocks 738 -> 557 us, operand
+// gathers of the largest contraction 827 -> 478 us (the row walk before).
 struct TileArgs {
     int32_t t0, t1, n_rest, tiles0, tiles1;
+    int32_t sh0, sh1;  // n0 = 1 << sh0, n1 = 1 << sh1: 16, 32 or 64
     int32_t rest_ax[AX];
     int64_t ostr[AX];
     int64_t rest_total;
@@ -436,18 +445,23 @@ struct TileArgs {
 template <typename T, bool TAB>
 __global__ void __launch_bounds__(256) k_permute_tiled(PermArgs a, TabArgs tb, TileArgs t, const T *__restrict__ src,
                                                        T *__restrict__ dst) {
-    __shared__ double tile[64][65];
+    HIP_DYNAMIC_SHARED(double, tile)  // n1 x (n0 + 1)
     const double al = a.alpha_re;
-    const int64_t per = (int64_t)t.tiles0 * t.tiles1;
-    const int64_t nblk = per * t.rest_total;
+    const uint32_t per = (uint32_t)t.tiles0 * t.tiles1;
     const int d1 = (int)a.out_dim[t.t1], d0 = (int)a.out_dim[t.t0];
     const int64_t s1 = t.ostr[t.t1];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    for (int64_t blk = blockIdx.x; blk < nblk; blk += gridDim.x) {
-        const int64_t r = blk / per;
-        const int64_t q = blk - r * per;
-        const int i1b = (int)(q / t.tiles0) * 64, i0b = (int)(q % t.tiles0) * 64;
-        int64_t base = 0, rr = r;
+    const int n0 = 1 << t.sh0, n1 = 1 << t.sh1, ld = n0 + 1, count = n0 << t.sh1;
+    // element e = tid + 256 u of a tile: l1 = e % n1 (the same for every u), l0 = e / n1
+    const int l1 = threadIdx.x & (n1 - 1), l0s = threadIdx.x >> t.sh1, l0d = 256 >> t.sh1;
+    // one tile per workgroup, the tiles of an XCD consecutive (its L2 has the lines that neighbours share)
+    const uint32_t nblk = per * (uint32_t)t.rest_total, share = (nblk + 7) / 8;
+    const uint32_t blk = (blockIdx.x & 7) * share + (blockIdx.x >> 3);
+    if (blk < nblk && (blockIdx.x >> 3) < share) {
+        uint32_t rr = per == 1 ? blk : blk / per;
+        const uint32_t q = blk - rr * per;
+        const int i1b = (int)(per == 1 ? 0 : q / (uint32_t)t.tiles0) << t.sh1;
+        const int i0b = (int)(per == 1 ? 0 : q % (uint32_t)t.tiles0) << t.sh0;
+        int64_t base = 0;
         uint32_t Gb[kTabGroups];
         if constexpr (TAB) {
 #pragma unroll
@@ -456,7 +470,7 @@ __global__ void __launch_bounds__(256) k_permute_tiled(PermArgs a, TabArgs tb, T
         }
         for (int k = t.n_rest - 1; k >= 0; --k) {
             const int ax = t.rest_ax[k];
-            int64_t o;
+            uint32_t o;
             if (a.out_shift[ax] >= 0) {
                 o = rr & (a.out_dim[ax] - 1);
                 rr >>= a.out_shift[ax];
@@ -467,44 +481,42 @@ __global__ void __launch_bounds__(256) k_permute_tiled(PermArgs a, TabArgs tb, T
             base += o * t.ostr[ax];
             if constexpr (TAB) {
 #pragma unroll
-                for (int g = 0; g < kTabGroups; ++g) Gb[g] += (uint32_t)o * tb.gmul[ax][g];
+                for (int g = 0; g < kTabGroups; ++g) Gb[g] += o * tb.gmul[ax][g];
             }
         }
-        // a lane's elements share i1 = i1b + lane, a wavefront's share i0: with tables, groups that i0
-        // does not feed are looked up once, groups that only i0 feeds at one address per wavefront
+        // with tables, groups that t0 does not feed are looked up once per lane
+        const bool in1 = i1b + l1 < d1;
         int64_t off1 = 0;
         uint32_t c1 = 0;
-        const bool in1 = i1b + lane < d1;
         if constexpr (TAB) {
 #pragma unroll
             for (int g = 0; g < kTabGroups; ++g)
                 if (g < tb.ng && tb.gmul[t.t0][g] == 0)
-                    tab_add(tb, tb.tab[g][Gb[g] + (in1 ? (uint32_t)lane * tb.gmul[t.t1][g] : 0u)], off1, c1);
+                    tab_add(tb, tb.tab[g][Gb[g] + (in1 ? (uint32_t)l1 * tb.gmul[t.t1][g] : 0u)], off1, c1);
         }
-        // 16 elements per lane in two batches of 8: index maps and table reads first, then the
-        // source reads, so that 8 load chains are in flight per lane
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
+        // up to 16 elements per lane in batches of 8: index maps and table reads first, then the source
+        // reads, so that 8 load chains are in flight per lane
+        for (int e0 = 0; e0 < count; e0 += 8 * 256) {
             int64_t off[8];
             uint32_t code[8];
 #pragma unroll
             for (int u = 0; u < 8; ++u) {
-                const int l0 = wave + 4 * (8 * h + u);
-                const int i1 = i1b + lane, i0 = i0b + l0;
+                const int l0 = l0s + ((e0 >> 8) + u) * l0d;
+                const int i0 = i0b + l0;
                 code[u] = 2u;
                 off[u] = 0;
-                if (i1 < d1 && i0 < d0) {
+                if (in1 && l0 < n0 && i0 < d0) {
                     if constexpr (TAB) {
                         uint32_t c = c1;
                         off[u] = off1;
 #pragma unroll
                         for (int g = 0; g < kTabGroups; ++g)
                             if (g < tb.ng && tb.gmul[t.t0][g] != 0)
-                                tab_add(tb, tb.tab[g][Gb[g] + (uint32_t)l0 * tb.gmul[t.t0][g] + (uint32_t)lane * tb.gmul[t.t1][g]],
+                                tab_add(tb, tb.tab[g][Gb[g] + (uint32_t)l0 * tb.gmul[t.t0][g] + (uint32_t)l1 * tb.gmul[t.t1][g]],
                                         off[u], c);
                         code[u] = tab_sign(a, tb, c);
                     } else {
-                        off[u] = map_elem<TAB>(a, tb, (uint64_t)(base + i1 * s1 + i0), code[u]);
+                        off[u] = map_elem<TAB>(a, tb, (uint64_t)(base + (i1b + l1) * s1 + i0), code[u]);
                     }
                 }
             }
@@ -512,15 +524,17 @@ __global__ void __launch_bounds__(256) k_permute_tiled(PermArgs a, TabArgs tb, T
 #pragma unroll
             for (int u = 0; u < 8; ++u) v[u] = (code[u] == 2u) ? 0.0 : (double)src[off[u]] * (code[u] ? -al : al);
 #pragma unroll
-            for (int u = 0; u < 8; ++u) tile[lane][wave + 4 * (8 * h + u)] = v[u];
+            for (int u = 0; u < 8; ++u) {
+                const int l0 = l0s + ((e0 >> 8) + u) * l0d;
+                if (l0 < n0) tile[l1 * ld + l0] = v[u];
+            }
         }
         __syncthreads();
-        for (int e = threadIdx.x; e < 64 * 64; e += 256) {
-            const int l0 = e & 63, l1 = e >> 6;
-            const int i1 = i1b + l1, i0 = i0b + l0;
-            if (i1 < d1 && i0 < d0) dst[base + i1 * s1 + i0] = (T)tile[l1][l0];
+        for (int e = threadIdx.x; e < count; e += 256) {
+            const int w0 = e & (n0 - 1), w1 = e >> t.sh0;
+            const int i1 = i1b + w1, i0 = i0b + w0;
+            if (i1 < d1 && i0 < d0) dst[base + i1 * s1 + i0] = (T)tile[w1 * ld + w0];
         }
-        __syncthreads();
     }
 }
 
@@ -899,42 +913,130 @@ int gtn_index_tables(int64_t n, int32_t *popc, int8_t *sigma, int32_t *enc, void
     return GTN_OK;
 }
 
-// Source stride of a unit step of output axis `ax`: through its virtual axis, the least significant
-// component of that axis and the input axis it feeds (0 when it cannot be told: a trace, two virtual
-// axes, a split input).
-static int64_t unit_source_stride(const gtn_perm_desc *d, int ax) {
-    if (d->out_virt[ax][1] >= 0 || d->out_virt[ax][0] < 0) return 0;
-    const int v = d->out_virt[ax][0];
-    int j = 0;
-    for (int u = 0; u <= v; ++u) j += d->virt_ncomp[u];
-    j -= 1;  // the last (least significant) component of v
-    if (j < 0 || d->comp_in[j][1] >= 0) return 0;
-    const int b = d->comp_in[j][0];
-    if (d->in_split[b]) return 0;
-    return d->in_stride[b] * d->comp_mult[j][0] * d->out_vmul[ax][0];
+// The descriptor with every output axis that runs over several components of its virtual axis (a fused
+// index, or the half of one) cut at their boundaries, so that each leg is an axis of its own for the
+// tiles: an index c of stride m in V is (c / q, c % q) with strides m q and m.  Same elements, same order.
+static gtn_perm_desc split_axes(const gtn_perm_desc *d) {
+    gtn_perm_desc x = *d;
+    int n = 0;
+    int first[AX];
+    for (int v = 0, j = 0; v < d->n_virt; ++v) {
+        first[v] = j;
+        j += d->virt_ncomp[v];
+    }
+    int64_t dim[AX], mul[AX][2];
+    int32_t vid[AX][2];
+    for (int ax = 0; ax < d->n_out; ++ax) {
+        int64_t cuts[NC];
+        int nc = 0;
+        const int v = d->out_virt[ax][0];
+        const int64_t m = d->out_vmul[ax][0];
+        if (v >= 0 && d->out_virt[ax][1] < 0 && m > 0) {
+            int64_t pc = 1;
+            for (int j = d->virt_ncomp[v] - 1; j > 0; --j) {
+                pc *= d->comp_dim[first[v] + j];
+                if (pc > m && pc % m == 0 && d->out_dim[ax] % (pc / m) == 0 && pc / m < d->out_dim[ax]) cuts[nc++] = pc / m;
+            }
+        }
+        int64_t rest = d->out_dim[ax];
+        for (int c = nc - 1; c >= -1; --c) {
+            const int64_t below = c >= 0 ? cuts[c] : 1;
+            if (n == AX) return *d;
+            dim[n] = rest / below;
+            vid[n][0] = v;
+            vid[n][1] = d->out_virt[ax][1];
+            mul[n][0] = m * below;
+            mul[n][1] = d->out_vmul[ax][1];
+            rest = below;
+            ++n;
+        }
+    }
+    // every original axis may still follow: all fit
+    x.n_out = n;
+    for (int i = 0; i < n; ++i) {
+        x.out_dim[i] = dim[i];
+        for (int t = 0; t < 2; ++t) x.out_virt[i][t] = vid[i][t], x.out_vmul[i][t] = mul[i][t];
+    }
+    return x;
 }
 
-// The tiled kernel pays off when the output's last axis is strided in the source and another output
-// axis of at least 16 entries steps the source by one or two elements.
+// Source offset of an output element on the host (the index map of perm_map without its signs).
+static int64_t host_offset(const gtn_perm_desc *d, const int64_t *o) {
+    auto enc = [](uint64_t i) { return i ^ (uint64_t)(__builtin_popcountll(i >> 1) & 1); };
+    uint64_t V[AX] = {0}, F[AX] = {0};
+    for (int ax = 0; ax < d->n_out; ++ax)
+        for (int t = 0; t < 2; ++t)
+            if (d->out_virt[ax][t] >= 0) V[d->out_virt[ax][t]] += (uint64_t)(o[ax] * d->out_vmul[ax][t]);
+    int j = d->n_comp;
+    for (int v = d->n_virt - 1; v >= 0; --v) {
+        uint64_t c = d->virt_enc[v] ? enc(V[v]) : V[v];
+        for (int t = 0; t < d->virt_ncomp[v]; ++t) {
+            --j;
+            const uint64_t k = c % (uint64_t)d->comp_dim[j];
+            c /= (uint64_t)d->comp_dim[j];
+            for (int u = 0; u < 2; ++u)
+                if (d->comp_in[j][u] >= 0) F[d->comp_in[j][u]] += k * (uint64_t)d->comp_mult[j][u];
+        }
+    }
+    int64_t off = 0;
+    for (int b = 0; b < d->n_in; ++b) {
+        const uint64_t e = d->in_enc[b] ? enc(F[b]) : F[b];
+        off += d->in_split[b] ? (int64_t)(e & 1) * d->in_stride_lo[b] + (int64_t)(e >> 1) * d->in_stride[b]
+                              : (int64_t)e * d->in_stride[b];
+    }
+    return off;
+}
+
+// 128-byte source lines that 64 consecutive steps touch: along output axis `ax` alone, or (ax < 0) of the
+// output elements 0 .. 63; scaled to 64 steps.
+static int lines_of(const gtn_perm_desc *d, int ax, int es) {
+    int64_t o[AX] = {0}, seen[64];
+    int n = 0, steps = 0;
+    for (; steps < 64; ++steps) {
+        if (ax >= 0) {
+            if (steps >= d->out_dim[ax]) break;
+            o[ax] = steps;
+        } else {
+            int64_t rest = steps;
+            for (int x = d->n_out - 1; x >= 0; --x) {
+                o[x] = rest % d->out_dim[x];
+                rest /= d->out_dim[x];
+            }
+            if (rest) break;
+        }
+        const int64_t line = host_offset(d, o) * es / 128;
+        int k = 0;
+        while (k < n && seen[k] != line) ++k;
+        if (k == n) seen[n++] = line;
+    }
+    return steps ? n * 64 / steps : 64;
+}
+
+// Tiles pay where 64 consecutive output elements touch more than 16 source lines (a lane group's read
+// then takes a cycle per line, and lines are fetched again and again) and along some other axis of at
+// least 16 indices 64 steps touch at most a third of that.
 static bool plan_tiles(const gtn_perm_desc *d, TileArgs &t) {
-    const int n = d->n_out;
+    const int n = d->n_out, es = d->dtype == GTN_F32 ? 4 : 8;
     if (n < 2) return false;
     const int t0 = n - 1;
     if (d->out_dim[t0] < 16) return false;
-    const int64_t s0 = unit_source_stride(d, t0);
-    if (s0 >= 1 && s0 <= 2) return false;  // already coalesced
-    int t1 = -1;
+    const int flat = lines_of(d, -1, es);
+    if (flat <= 16) return false;
+    int t1 = -1, best = flat / 3 + 1;
     for (int ax = 0; ax < t0; ++ax) {
-        const int64_t sa = unit_source_stride(d, ax);
-        if (d->out_dim[ax] >= 16 && sa >= 1 && sa <= 2) {
+        if (d->out_dim[ax] < 16) continue;
+        const int la = lines_of(d, ax, es);
+        if (la < best) {
+            best = la;
             t1 = ax;
-            break;
         }
     }
     if (t1 < 0) return false;
     memset(&t, 0, sizeof(t));
     t.t0 = t0;
     t.t1 = t1;
+    t.sh0 = d->out_dim[t0] >= 64 ? 6 : (d->out_dim[t0] >= 32 ? 5 : 4);
+    t.sh1 = d->out_dim[t1] >= 64 ? 6 : (d->out_dim[t1] >= 32 ? 5 : 4);
     int64_t acc = 1;
     for (int ax = n - 1; ax >= 0; --ax) {
         t.ostr[ax] = acc;
@@ -946,24 +1048,19 @@ static bool plan_tiles(const gtn_perm_desc *d, TileArgs &t) {
             t.rest_ax[t.n_rest++] = ax;
             t.rest_total *= d->out_dim[ax];
         }
-    t.tiles0 = (int32_t)((d->out_dim[t0] + 63) / 64);
-    t.tiles1 = (int32_t)((d->out_dim[t1] + 63) / 64);
-    return true;
+    t.tiles0 = (int32_t)((d->out_dim[t0] + (1 << t.sh0) - 1) >> t.sh0);
+    t.tiles1 = (int32_t)((d->out_dim[t1] + (1 << t.sh1) - 1) >> t.sh1);
+    return (int64_t)t.tiles0 * t.tiles1 * t.rest_total < (1 << 30);
 }
 
 // Group the virtual axes for the table-driven map (k_perm_tables).  Returns false when the gather
 // is so small that one wavefront walks it, or a group's table would be large: the table is built once per
 // gather shape (about 20 us), and every gather without one walks the descriptor with its index vectors in
 // scratch memory, 12 to 20 us for the smallest (MI355X; 5 us with tables).
-static bool plan_groups(const gtn_perm_desc *d, int64_t total, TabBuild &tb, TabArgs &ta) {
+// `fast`: the output axis whose index runs fastest in the tables (-1: the last one that feeds the group).
+static bool plan_groups(const gtn_perm_desc *d, int64_t total, int fast, TabBuild &tb, TabArgs &ta) {
     if (total < 64 || d->n_virt == 0) return false;
     const int nv = d->n_virt;
-    int64_t ext[AX];
-    for (int v = 0; v < nv; ++v) ext[v] = 1;
-    for (int ax = 0; ax < d->n_out; ++ax)
-        for (int t = 0; t < 2; ++t)
-            if (d->out_virt[ax][t] >= 0 && d->out_dim[ax] > 0)
-                ext[d->out_virt[ax][t]] += (d->out_dim[ax] - 1) * d->out_vmul[ax][t];
     // the virtual axis that feeds each input axis (-1: none, -2: several), and whether the map is linear
     // over GF(2)
     bool lin = true;
@@ -1025,80 +1122,71 @@ static bool plan_groups(const gtn_perm_desc *d, int64_t total, TabBuild &tb, Tab
                 else if (!lin)
                     parent[root(v)] = root(owner[b]);
             }
-    // groups in order of their smallest virtual axis
+    // groups in order of their smallest virtual axis; a group's table has an entry for every value of the
+    // output axes that feed one of its virtual axes
     int gid[AX], ng = 0;
-    int64_t gsize[AX];
-    int members[AX][AX], nmem[AX];
+    uint32_t members[AX];
+    auto fed = [&](uint32_t mem, int ax) {
+        for (int t = 0; t < 2; ++t)
+            if (d->out_virt[ax][t] >= 0 && (mem >> d->out_virt[ax][t] & 1u)) return true;
+        return false;
+    };
+    auto size_of = [&](uint32_t mem) -> int64_t {
+        int64_t n = 1;
+        for (int ax = 0; ax < d->n_out; ++ax)
+            if (fed(mem, ax) && (n *= d->out_dim[ax]) > (1 << 22)) break;
+        return n;
+    };
     for (int v = 0; v < nv; ++v) gid[v] = -1;
     for (int v = 0; v < nv; ++v) {
         const int r = root(v);
         if (gid[r] < 0) {
             gid[r] = ng;
-            gsize[ng] = 1;
-            nmem[ng] = 0;
-            ++ng;
+            members[ng++] = 0;
         }
-        const int g = gid[r];
-        members[g][nmem[g]++] = v;
-        gsize[g] *= ext[v];
-        if (gsize[g] > (1 << 22)) return false;
+        members[gid[r]] |= 1u << v;
+        if (size_of(members[gid[r]]) > (1 << 22)) return false;
     }
     // merge the two smallest groups while there are too many
     while (ng > kTabGroups) {
         int a0 = 0, a1 = 1;
-        if (gsize[a1] < gsize[a0]) std::swap(a0, a1);
+        if (size_of(members[a1]) < size_of(members[a0])) std::swap(a0, a1);
         for (int g = 2; g < ng; ++g) {
-            if (gsize[g] < gsize[a0]) {
+            if (size_of(members[g]) < size_of(members[a0])) {
                 a1 = a0;
                 a0 = g;
-            } else if (gsize[g] < gsize[a1]) {
+            } else if (size_of(members[g]) < size_of(members[a1])) {
                 a1 = g;
             }
         }
         if (a1 < a0) std::swap(a0, a1);
-        gsize[a0] *= gsize[a1];
-        if (gsize[a0] > (1 << 22)) return false;
-        for (int i = 0; i < nmem[a1]; ++i) members[a0][nmem[a0]++] = members[a1][i];
-        for (int g = a1; g + 1 < ng; ++g) {
-            gsize[g] = gsize[g + 1];
-            nmem[g] = nmem[g + 1];
-            for (int i = 0; i < nmem[g]; ++i) members[g][i] = members[g + 1][i];
-        }
+        members[a0] |= members[a1];
+        if (size_of(members[a0]) > (1 << 22)) return false;
+        for (int g = a1; g + 1 < ng; ++g) members[g] = members[g + 1];
         --ng;
     }
     int64_t entries = 0;
-    for (int g = 0; g < ng; ++g) entries += gsize[g];
+    for (int g = 0; g < ng; ++g) entries += size_of(members[g]);
     if (entries > (total < (1 << 16) ? total : total / 4)) return false;
     memset(&tb, 0, sizeof(tb));
     memset(&ta, 0, sizeof(ta));
     tb.ng = ta.ng = ng;
-    ta.signs = (uint64_t)d->table[0] | (uint64_t)d->table[1] << 32;
-    ta.short_signs = d->n_bits <= 5;
     ta.lin = lin;
-    int64_t rad_of[AX];
-    int grp_of[AX];
     for (int g = 0; g < ng; ++g) {
-        tb.start[g + 1] = tb.start[g] + gsize[g];
-        tb.nv[g] = nmem[g];
+        tb.start[g + 1] = tb.start[g] + size_of(members[g]);
+        tb.vmask[g] = members[g];
+        for (int v = 0; v < nv; ++v)
+            if (members[g] >> v & 1u) tb.inmask[g] |= feeds[v];
         int64_t rad = 1;
-        for (int i = nmem[g] - 1; i >= 0; --i) {
-            const int v = members[g][i];
-            tb.vid[g][i] = (int8_t)v;
-            tb.vrad[g][i] = (uint32_t)rad;
-            tb.vext[g][i] = (uint32_t)ext[v];
-            rad_of[v] = rad;
-            grp_of[v] = g;
-            rad *= ext[v];
-            tb.vmask[g] |= 1u << v;
-            tb.inmask[g] |= feeds[v];
+        for (int i = d->n_out; i >= 0; --i) {  // axis `fast` first, then the output's from the last
+            const int ax = i == d->n_out ? fast : i;
+            if (ax < 0 || (i < d->n_out && ax == fast) || !fed(members[g], ax)) continue;
+            tb.ax[g][tb.nx[g]] = (int8_t)ax;
+            tb.rad[g][tb.nx[g]++] = (uint32_t)rad;
+            ta.gmul[ax][g] = (uint32_t)rad;
+            rad *= d->out_dim[ax];
         }
     }
-    for (int ax = 0; ax < d->n_out; ++ax)
-        for (int t = 0; t < 2; ++t) {
-            const int v = d->out_virt[ax][t];
-            if (v < 0) continue;
-            ta.gmul[ax][grp_of[v]] += (uint32_t)(d->out_vmul[ax][t] * rad_of[v]);
-        }
     return true;
 }
 
@@ -1216,6 +1304,37 @@ static bool plan_rows(const PermArgs &a, const TabArgs &tb, RowArgs &w, int &U) 
     }
 }
 
+// What gtn_permute does with a descriptor, planned once per gather shape (the sign table, alpha and the
+// size of the source aside) and device.
+struct PermPlan {
+    bool tab, tile, rows;
+    PermArgs a;  // of the descriptor the kernels walk; sign table and alpha filled in per call
+    TabBuild build;
+    TabArgs tb;
+    TileArgs t;
+    RowArgs w;
+    int U;
+};
+static std::mutex g_plan_mu;
+static std::map<std::string, PermPlan> g_plans;
+constexpr size_t kMaxPlans = 4096;
+
+static int plan_permute(const gtn_perm_desc *d, PermArgs &a, PermPlan &p) {
+    memset(&p, 0, sizeof(p));
+    const bool fp = d->dtype == GTN_F64 || d->dtype == GTN_F32;
+    p.a = a;
+    if (!fp) return GTN_OK;
+    const gtn_perm_desc x = split_axes(d);
+    PermArgs ax;
+    int rc = build_perm_args(&x, ax);
+    if (rc) return rc;
+    p.tile = tiles_enabled() && plan_tiles(&x, p.t);
+    p.tab = getenv("GTN_PERM_NO_TABLES") == nullptr && plan_groups(&x, ax.total, p.tile ? p.t.t1 : -1, p.build, p.tb);
+    p.a = ax;
+    p.rows = p.tab && !p.tile && plan_rows(p.a, p.tb, p.w, p.U);
+    return GTN_OK;
+}
+
 int gtn_permute(const gtn_perm_desc *d, const void *src, void *dst, void *stream) {
     GTN_REQUIRE(d && src && dst, "gtn_permute: null argument");
     PermArgs a;
@@ -1229,43 +1348,61 @@ int gtn_permute(const gtn_perm_desc *d, const void *src, void *dst, void *stream
         return GTN_OK;
     }
     hipStream_t s = as_stream(stream);
-    TabArgs tb;
-    memset(&tb, 0, sizeof(tb));
-    TabBuild build;
-    const bool tab = (d->dtype == GTN_F64 || d->dtype == GTN_F32) && getenv("GTN_PERM_NO_TABLES") == nullptr &&
-                     plan_groups(d, a.total, build, tb);
-    if (tab) {
-        rc = tab_tables(a, build, s, tb);
+    PermPlan p;
+    {
+        PermArgs k;
+        memcpy(&k, &a, sizeof(k));
+        memset(k.table, 0, sizeof(k.table));
+        k.alpha_re = k.alpha_im = 0.0;
+        const int32_t kind[2] = {d->dtype, getenv("GTN_PERM_NO_TABLES") != nullptr};
+        std::string key((const char *)kind, sizeof(kind));
+        key.append((const char *)&k, sizeof(k));
+        std::lock_guard<std::mutex> l(g_plan_mu);
+        auto it = g_plans.find(key);
+        if (it == g_plans.end()) {
+            rc = plan_permute(d, a, p);
+            if (rc) return rc;
+            if (g_plans.size() >= kMaxPlans) g_plans.clear();
+            it = g_plans.emplace(std::move(key), p).first;
+        }
+        p = it->second;
+    }
+    memcpy(p.a.table, a.table, sizeof(a.table));
+    p.a.alpha_re = a.alpha_re;
+    p.a.alpha_im = a.alpha_im;
+    p.tb.signs = (uint64_t)d->table[0] | (uint64_t)d->table[1] << 32;
+    p.tb.short_signs = d->n_bits <= 5;
+    if (p.tab) {
+        rc = tab_tables(p.a, p.build, s, p.tb);
         if (rc) return rc;
     }
-    TileArgs t;
-    if (d->dtype != GTN_C128 && tiles_enabled() && plan_tiles(d, t)) {
+    if (p.tile) {
+        const TileArgs &t = p.t;
         const int64_t nblk = (int64_t)t.tiles0 * t.tiles1 * t.rest_total;
-        dim3 gt((unsigned)(nblk < (1 << 20) ? nblk : (1 << 20))), bt(256);
+        dim3 gt((unsigned)((nblk + 7) / 8 * 8)), bt(256);
+        const size_t lds = sizeof(double) * ((size_t)1 << t.sh1) * ((1 << t.sh0) + 1);
+#define GTN_TILES(T, B) \
+    hipLaunchKernelGGL((k_permute_tiled<T, B>), gt, bt, lds, s, p.a, p.tb, t, (const T *)src, (T *)dst)
         if (d->dtype == GTN_F64) {
-            if (tab)
-                hipLaunchKernelGGL((k_permute_tiled<double, true>), gt, bt, 0, s, a, tb, t, (const double *)src, (double *)dst);
-            else
-                hipLaunchKernelGGL((k_permute_tiled<double, false>), gt, bt, 0, s, a, tb, t, (const double *)src, (double *)dst);
+            if (p.tab) GTN_TILES(double, true);
+            else GTN_TILES(double, false);
         } else {
-            if (tab)
-                hipLaunchKernelGGL((k_permute_tiled<float, true>), gt, bt, 0, s, a, tb, t, (const float *)src, (float *)dst);
-            else
-                hipLaunchKernelGGL((k_permute_tiled<float, false>), gt, bt, 0, s, a, tb, t, (const float *)src, (float *)dst);
+            if (p.tab) GTN_TILES(float, true);
+            else GTN_TILES(float, false);
         }
+#undef GTN_TILES
         GTN_CHECK_LAUNCH();
         return GTN_OK;
     }
-    RowArgs w;
-    int U;
-    if (tab && plan_rows(a, tb, w, U)) {
+    if (p.rows) {
+        const RowArgs &w = p.w;
         const dim3 gr((unsigned)((w.rows + w.rows_per - 1) / w.rows_per * w.chunks)), br(256);
-#define GTN_ROWS(T, N) hipLaunchKernelGGL((k_permute_rows<T, N>), gr, br, 0, s, a, tb, w, (const T *)src, (T *)dst)
+#define GTN_ROWS(T, N) hipLaunchKernelGGL((k_permute_rows<T, N>), gr, br, 0, s, p.a, p.tb, w, (const T *)src, (T *)dst)
         if (d->dtype == GTN_F64) {
-            if (U == 4) GTN_ROWS(double, 4);
+            if (p.U == 4) GTN_ROWS(double, 4);
             else GTN_ROWS(double, 1);
         } else {
-            if (U == 4) GTN_ROWS(float, 4);
+            if (p.U == 4) GTN_ROWS(float, 4);
             else GTN_ROWS(float, 1);
         }
 #undef GTN_ROWS
@@ -1273,22 +1410,20 @@ int gtn_permute(const gtn_perm_desc *d, const void *src, void *dst, void *stream
         return GTN_OK;
     }
     dim3 g(grid_for((a.total + kPermUnroll - 1) / kPermUnroll, 256, 1 << 20)), b(256);
+#define GTN_WALK(T, B) hipLaunchKernelGGL((k_permute<T, B>), g, b, 0, s, p.a, p.tb, (const T *)src, (T *)dst)
     switch (d->dtype) {
         case GTN_F64:
-            if (tab)
-                hipLaunchKernelGGL((k_permute<double, true>), g, b, 0, s, a, tb, (const double *)src, (double *)dst);
-            else
-                hipLaunchKernelGGL((k_permute<double, false>), g, b, 0, s, a, tb, (const double *)src, (double *)dst);
+            if (p.tab) GTN_WALK(double, true);
+            else GTN_WALK(double, false);
             break;
         case GTN_F32:
-            if (tab)
-                hipLaunchKernelGGL((k_permute<float, true>), g, b, 0, s, a, tb, (const float *)src, (float *)dst);
-            else
-                hipLaunchKernelGGL((k_permute<float, false>), g, b, 0, s, a, tb, (const float *)src, (float *)dst);
+            if (p.tab) GTN_WALK(float, true);
+            else GTN_WALK(float, false);
             break;
         case GTN_C128: hipLaunchKernelGGL(k_permute_c128, g, b, 0, s, a, (const double2 *)src, (double2 *)dst); break;
         default: set_error("gtn_permute: unsupported dtype %d", d->dtype); return GTN_ENOTSUP;
     }
+#undef GTN_WALK
     GTN_CHECK_LAUNCH();
     return GTN_OK;
 }
@@ -1317,8 +1452,12 @@ int gtn_permute2(const gtn_perm_desc *outer, const gtn_perm_desc *inner, const v
     memset(&tn, 0, sizeof(tn));
     TabBuild bo, bn;
     const bool tabs = getenv("GTN_PERM_NO_TABLES") == nullptr;
-    const bool tabo = tabs && plan_groups(outer, ao.total, bo, to);
-    const bool tabn = tabs && plan_groups(inner, an.total, bn, tn);
+    const bool tabo = tabs && plan_groups(outer, ao.total, -1, bo, to);
+    const bool tabn = tabs && plan_groups(inner, an.total, -1, bn, tn);
+    to.signs = (uint64_t)outer->table[0] | (uint64_t)outer->table[1] << 32;
+    tn.signs = (uint64_t)inner->table[0] | (uint64_t)inner->table[1] << 32;
+    to.short_signs = outer->n_bits <= 5;
+    tn.short_signs = inner->n_bits <= 5;
     if (tabo && (rc = tab_tables(ao, bo, s, to))) return rc;
     if (tabn && (rc = tab_tables(an, bn, s, tn))) return rc;
     dim3 g(grid_for((ao.total + kPermUnroll - 1) / kPermUnroll, 256, 1 << 20)), b(256);
