@@ -91,26 +91,6 @@ __global__ void k_transpose2d(const double *src, int64_t lds, double *dst, int64
         dst[c * ldd + r] = src[r * lds + c];
     }
 }
-// G[r][c] = G[c][r] for the entries whose row super-block (r / S) lies below their column's
-// (c / S): the part of a symmetric n x n matrix (ld) that a product over its upper block triangle
-// left out.  64 x 64 tiles through LDS; grid (n / 64 rounded up, same, blocks), blockIdx.z advancing
-// G by dG.
-__global__ void __launch_bounds__(256) k_mirror_lower(double *G, int64_t n, int64_t ld, int64_t S, int64_t dG) {
-    __shared__ double tile[64][65];
-    G += blockIdx.z * dG;
-    const int64_t r0 = (int64_t)blockIdx.y * 64, c0 = (int64_t)blockIdx.x * 64;
-    if (r0 / S <= (c0 + 63) / S) return;  // the tile is not wholly below the computed block triangle
-    const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;
-    for (int i = ty; i < 64; i += 4) {  // read the mirror tile (rows c0.., columns r0..) row by row
-        const int64_t rr = c0 + i, cc = r0 + tx;
-        tile[i][tx] = (rr < n && cc < n) ? G[rr * ld + cc] : 0.0;
-    }
-    __syncthreads();
-    for (int i = ty; i < 64; i += 4) {
-        const int64_t rr = r0 + i, cc = c0 + tx;
-        if (rr < n && cc < n) G[rr * ld + cc] = tile[tx][i];
-    }
-}
 __global__ void k_fill(double *x, int64_t rows, int64_t cols, int64_t ld, double v, int64_t dx) {
     x += blockIdx.y * dx;
     int64_t total = rows * cols;
@@ -2054,43 +2034,21 @@ static int oz_product(std::vector<Run> &rl, bool transposed_m, double *(Blk::*X)
     return GTN_OK;
 }
 
-// the Gram matrices G = M M^T of every block (m x m, FP64): products over the upper block triangle
-// in super-rows of S rows (grouped launches of at most 12 super-rows), then the lower part mirrored.
-// S = 128 (one 128-row tile) computes (1 + 128 / m) / 2 of the full product: 53 % at m = 2048.
-static int64_t gram_super_rows(int64_t m) {
-    int64_t S = 128;
-    while ((m + S - 1) / S > 16) S += 128;  // at most 16 super-rows per block
-    return S;
-}
+// The Gram matrices G = M M^T of every block (m x m, FP64).  One launch over the tiles of every block's
+// upper triangle: cut into a group per 128 rows, a call over four 2048 x 2048 blocks ran 504 tiles and
+// then, with a sixth of the device, the last 40 (1213 us on MI355X, 49 of it the copy to the lower half;
+// 645 us now).
 static int gram_of_blocks(std::vector<Run> &rl, hipStream_t s) {
     std::vector<gtn_gemm_desc> g;
     for (Run &r : rl) {
         Blk &f = *r.f;
         GTN_REQUIRE(f.Gm, "gtn_svd_blocks: no Gram matrix");
-        const int64_t m = f.b.m, S = gram_super_rows(m);
+        const int64_t m = f.b.m;
         R8N(f.Gm, m * m, r.dws, r.n, "Gram matrix");
         R8N(f.b.M, ext(f.b.m, f.b.n, f.b.lda), r.dM, r.n, "block");
-        if (!g.empty() && g.size() + (size_t)((m + S - 1) / S) > 12) {  // a launch takes at most 12 groups
-            int rc = run(g, GTN_PREC_F64, s);
-            if (rc) return rc;
-            g.clear();
-        }
-        for (int64_t r0 = 0; r0 < m; r0 += S) {
-            const int64_t rows = m - r0 < S ? m - r0 : S;
-            // G[r0.., r0..] = M[r0.., :] M[r0.., :]^T
-            g.push_back(gdr(f.b.M + r0 * f.b.lda, f.b.lda, 1, f.b.M + r0 * f.b.lda, 1, f.b.lda, f.Gm + r0 * m + r0, m, rows,
-                            m - r0, f.b.n, r.n, r.dM, r.dM, r.dws));
-        }
+        g.push_back(gdr(f.b.M, f.b.lda, 1, f.b.M, 1, f.b.lda, f.Gm, m, m, m, f.b.n, r.n, r.dM, r.dM, r.dws));
     }
-    int rc = run(g, GTN_PREC_F64, s);
-    if (rc) return rc;
-    for (Run &r : rl) {
-        Blk &f = *r.f;
-        const int64_t m = f.b.m, t = (m + 63) / 64;
-        GTN_REQUIRE(t <= 65535, "gtn_svd_blocks: Gram matrix too large");
-        LAUNCH(k_mirror_lower, dim3((unsigned)t, (unsigned)t, r.n), dim3(256), 0, s, f.Gm, m, m, gram_super_rows(m), r.dws);
-    }
-    return GTN_OK;
+    return gemm_symmetric(g.data(), (int)g.size(), (void *)s);
 }
 
 // products after which the Chebyshev filter is at least as converged, for every lambda_k / lambda_{p+1},

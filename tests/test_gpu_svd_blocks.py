@@ -185,3 +185,14 @@ def test_filtered_range_finder_special_spectra(case):
             assert c == k
         np.testing.assert_allclose(s[:c], ref[:c], rtol=0, atol=(1e-12 if name == "flat" else 1e-13) * ref[0])
         np.testing.assert_allclose(u.T @ u, np.eye(c), rtol=0, atol=1e-13)
+
+
+@pytest.mark.parametrize("m,n", [(129, 129), (191, 200), (192, 1000), (193, 193), (256, 257), (257, 2100), (383, 384)])
+def test_gram_matrix_tiles(m, n):
+    """Gram matrices whose size is around multiples of the 64 and 128 tiles, with short and long
+    reductions (split into chunks), through decompositions of a single block: the values to rounding."""
+    rng = np.random.default_rng(m)
+    s = np.maximum(0.6 ** np.arange(m), 1e-3 * 0.97 ** np.arange(m))
+    M = _decaying_blocks(rng, m, n, s, 1)[0]
+    outs, counts = _run([(M, 12)])
+    _check(M, 12, outs[0], counts[0])
