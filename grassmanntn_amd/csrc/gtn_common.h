@@ -63,6 +63,10 @@ struct GemmIndirect {
 int gemm_grouped_indirect(const gtn_gemm_desc *groups, const GemmIndirect *ind, int n_groups, void *const *tune_c,
                           void *stream);
 
+// gtn_gemm_grouped over FP64 products A B that are symmetric (B = A^T; M = N, beta = 0): only the tiles on
+// and above the diagonal are computed, (1 + 1 / tiles) / 2 of the product, and stored on both sides
+int gemm_symmetric(const gtn_gemm_desc *groups, int n_groups, void *stream);
+
 inline hipStream_t as_stream(void *s) { return reinterpret_cast<hipStream_t>(s); }
 
 // graph bookkeeping of the runtime (gtn_runtime.hip): instantiated graphs that may still be

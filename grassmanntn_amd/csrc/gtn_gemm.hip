@@ -40,6 +40,7 @@ struct GemmGroup {
     int64_t sam, sak, sbk, sbn, scm, scn, sab, sbb, scb, scs;
     double alpha, beta;
     GemmIndirect ind;  // coef null: a plain group (a launch's groups are all of one kind)
+    int32_t tri;       // symmetric product: only tiles on or above the diagonal, stored on both sides of it
 };
 
 struct GemmArgs {
@@ -62,9 +63,15 @@ __device__ __forceinline__ bool locate(const GemmArgs &a, int &gi, int &b, int &
     while (gi + 1 < a.n_groups && t >= a.tile_start[gi + 1]) ++gi;
     t -= a.tile_start[gi];
     const GemmGroup &g = a.g[gi];
-    int per_b = g.tiles_m * g.tiles_n;
+    int per_b = g.tri ? g.tiles_n * (g.tiles_n + 1) / 2 : g.tiles_m * g.tiles_n;
     b = t / per_b;
     t -= b * per_b;
+    if (g.tri) {  // rows of tiles_n, tiles_n - 1, ... tiles
+        tm = 0;
+        while (t >= g.tiles_n - tm) t -= g.tiles_n - tm++;
+        tn = tm + t;
+        return true;
+    }
     tm = t / g.tiles_n;
     tn = t - tm * g.tiles_n;
     return true;
@@ -173,8 +180,9 @@ __device__ __forceinline__ void panel_coord(int s, bool kc, int &r, int &k) {
 // ------------------------------------------------------------------------------------------------
 // IND: groups with device-side operands and coefficients (GemmIndirect; FP64).  A variant of its own, held
 // to the plain kernel's 256 registers (two wavefronts per SIMD), which its epilogue would exceed by one.
-template <typename TIN, typename TC, int BM, int BN, int BK, bool IND = false>
-__global__ void __launch_bounds__(256, IND ? 2 : 1) k_gemm_fp(GemmArgs args) {
+// TRI: symmetric products (GemmGroup::tri), likewise.
+template <typename TIN, typename TC, int BM, int BN, int BK, bool IND = false, bool TRI = false>
+__global__ void __launch_bounds__(256, IND || TRI ? 2 : 1) k_gemm_fp(GemmArgs args) {
     int gi, b, tm, tn;
     if (!locate(args, gi, b, tm, tn)) return;
     const GemmGroup &g = args.g[gi];
@@ -341,6 +349,8 @@ __global__ void __launch_bounds__(256, IND ? 2 : 1) k_gemm_fp(GemmArgs args) {
                     if constexpr (IND)
                         if (gamma != 0.0) val += gamma * (double)D[o];
                     C[o] = (TIN)val;
+                    if constexpr (TRI)
+                        if (tm != tn && g.splits == 1) C[c * g.scm + r * g.scn] = (TIN)val;
                 }
             }
 }
@@ -500,7 +510,7 @@ __global__ void __launch_bounds__(64) k_mfma_selftest(double *out) {
 // coefficients come from its tables.
 template <typename T>
 __global__ void k_split_sum(const T *__restrict__ W, int splits, int M, int N, int batch, T *C, int64_t scm,
-                            int64_t scn, int64_t scb, double alpha, double beta, GemmIndirect ind) {
+                            int64_t scn, int64_t scb, double alpha, double beta, GemmIndirect ind, int tri) {
     const int64_t MN = (int64_t)M * N, total = MN * batch;
     for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < total; i += (int64_t)gridDim.x * blockDim.x) {
         const int64_t b = i / MN, e = i - b * MN;
@@ -520,11 +530,13 @@ __global__ void k_split_sum(const T *__restrict__ W, int splits, int M, int N, i
                 continue;
             }
         }
+        if (tri && r / tri > c / tri) continue;  // a tile (of tri rows) that was not computed
         for (int sp = 0; sp < splits; ++sp) acc += (double)w[sp * MN];
         const int64_t o = b * scb + r * scm + c * scn;
         double v = alpha * acc;
         if (beta != 0.0) v += beta * (double)C[o];
         C[o] = (T)v;
+        if (tri && r / tri < c / tri) C[b * scb + c * scm + r * scn] = (T)v;
     }
 }
 
@@ -572,6 +584,13 @@ static int launch_gemm(GemmArgs &a, int precision, int tile, hipStream_t s) {
     switch (precision) {
         case GTN_PREC_F64:
             if constexpr (sizeof(TIN) == 8) {
+                if (a.g[0].tri) {
+                    if (big)
+                        hipLaunchKernelGGL((k_gemm_fp<TIN, double, 128, 128, 16, false, true>), dim3(grid), dim3(256), 0, s, a);
+                    else
+                        hipLaunchKernelGGL((k_gemm_fp<TIN, double, 64, 64, 16, false, true>), dim3(grid), dim3(256), 0, s, a);
+                    break;
+                }
                 if (a.g[0].ind.coef) {
                     if (big)
                         hipLaunchKernelGGL((k_gemm_fp<TIN, double, 128, 128, 16, true>), dim3(grid), dim3(256), 0, s, a);
@@ -624,7 +643,7 @@ static int launch_gemm(GemmArgs &a, int precision, int tile, hipStream_t s) {
 // 128 x 128 tiles when every group is at least 128 x 128 and the launch still has a tile for every
 // compute unit; 64 x 64 otherwise.  GTN_GEMM_TILE=64|128 in the environment forces a size (128 only
 // where every group is at least 128 x 128) for tuning and tests.
-static int pick_tile(const gtn_gemm_desc *groups, int n) {
+static int pick_tile(const gtn_gemm_desc *groups, int n, bool tri) {
     static int forced = -1;
     if (forced < 0) {
         const char *e = getenv("GTN_GEMM_TILE");
@@ -635,7 +654,8 @@ static int pick_tile(const gtn_gemm_desc *groups, int n) {
         const gtn_gemm_desc &d = groups[i];
         if (d.M == 0 || d.N == 0 || d.batch == 0) continue;
         if (d.M < 128 || d.N < 128) return 64;
-        t128 += ((d.M + 127) / 128) * ((d.N + 127) / 128) * d.batch;
+        const int64_t tn = (d.N + 127) / 128;
+        t128 += (tri ? tn * (tn + 1) / 2 : ((d.M + 127) / 128) * tn) * d.batch;
     }
     if (forced == 64 || forced == 128) return forced;
     return t128 >= 256 ? 128 : 64;
@@ -692,10 +712,10 @@ static int scratch_ptr(void **out) {
 // tile <= 0 / target < 0: the heuristics (pick_tile, split_target)
 static int gemm_grouped_impl(const gtn_gemm_desc *groups, int n_groups, int dtype, int precision, void *stream,
                              void *fixed_ws, int64_t fixed_bytes, const char *name, int tile_cfg = 0,
-                             int target_cfg = -1, const GemmIndirect *ind = nullptr) {
+                             int target_cfg = -1, const GemmIndirect *ind = nullptr, bool tri = false) {
     GTN_REQUIRE(n_groups >= 0 && (n_groups == 0 || groups), "%s: bad groups", name);
     GTN_REQUIRE(dtype == GTN_F64 || dtype == GTN_F32, "gtn_gemm_grouped: dtype must be F64 or F32");
-    const int tile = tile_cfg > 0 ? tile_cfg : pick_tile(groups, n_groups);
+    const int tile = tile_cfg > 0 ? tile_cfg : pick_tile(groups, n_groups, tri);
     const int BM = tile, BN = tile;
     hipStream_t s = as_stream(stream);
     for (int base = 0; base < n_groups; base += kMaxGroups) {
@@ -738,11 +758,12 @@ static int gemm_grouped_impl(const gtn_gemm_desc *groups, int n_groups, int dtyp
             g.alpha = d.alpha;
             g.beta = d.beta;
             if (ind) g.ind = ind[base + i];
+            g.tri = tri;
             g.splits = 1;
             g.kchunk = g.K;
             g.scs = 0;
             a.tile_start[used] = tiles;
-            int64_t t = (int64_t)g.tiles_m * g.tiles_n * g.batch;
+            int64_t t = (tri ? (int64_t)g.tiles_n * (g.tiles_n + 1) / 2 : (int64_t)g.tiles_m * g.tiles_n) * g.batch;
             GTN_REQUIRE(tiles + t < (1ll << 31), "gtn_gemm_grouped: too many tiles");
             tiles += (int)t;
             ++used;
@@ -825,7 +846,7 @@ static int gemm_grouped_impl(const gtn_gemm_desc *groups, int n_groups, int dtyp
                         g.beta = 0.0;
                         off += g.scb * g.batch;
                     }
-                    tiles += g.tiles_m * g.tiles_n * g.batch * g.splits;
+                    tiles += (tri ? g.tiles_n * (g.tiles_n + 1) / 2 : g.tiles_m * g.tiles_n) * g.batch * g.splits;
                 }
                 a.tile_start[used] = tiles;
             }
@@ -839,10 +860,12 @@ static int gemm_grouped_impl(const gtn_gemm_desc *groups, int n_groups, int dtyp
                 const dim3 grid(grid_for((int64_t)g.M * g.N * g.batch, 256, 4096)), blk(256);
                 if (dtype == GTN_F64)
                     hipLaunchKernelGGL(k_split_sum<double>, grid, blk, 0, s, (const double *)g.C, g.splits, g.M, g.N,
-                                       g.batch, (double *)o.C, o.scm, o.scn, o.scb, o.alpha, o.beta, o.ind);
+                                       g.batch, (double *)o.C, o.scm, o.scn, o.scb, o.alpha, o.beta, o.ind,
+                                       o.tri ? BM : 0);
                 else
                     hipLaunchKernelGGL(k_split_sum<float>, grid, blk, 0, s, (const float *)g.C, g.splits, g.M, g.N,
-                                       g.batch, (float *)o.C, o.scm, o.scn, o.scb, o.alpha, o.beta, o.ind);
+                                       g.batch, (float *)o.C, o.scm, o.scn, o.scb, o.alpha, o.beta, o.ind,
+                                       o.tri ? BM : 0);
                 GTN_CHECK_LAUNCH();
             }
             if (ws) {
@@ -879,7 +902,7 @@ static bool autotune_on() {
     return g_autotune == 1;
 }
 
-static std::string tune_key(const gtn_gemm_desc *g, int n, int dtype, int prec, int dev) {
+static std::string tune_key(const gtn_gemm_desc *g, int n, int dtype, int prec, int dev, bool tri) {
     std::string k;
     auto put = [&](int64_t v) { k.append((const char *)&v, sizeof(v)); };
     put(dev);
@@ -891,17 +914,17 @@ static std::string tune_key(const gtn_gemm_desc *g, int n, int dtype, int prec, 
         put(g[i].N);
         put(g[i].K);
         put(g[i].batch);
-        put((g[i].sak == 1) | ((g[i].sbk == 1) << 1) | ((g[i].scn == 1) << 2));
+        put((g[i].sak == 1) | ((g[i].sbk == 1) << 1) | ((g[i].scn == 1) << 2) | (tri << 3));
     }
     return k;
 }
 
 static int time_cfg(const gtn_gemm_desc *groups, int n, int dtype, int prec, hipStream_t s, int tile, int target,
-                    hipEvent_t e0, hipEvent_t e1, float *best) {
+                    hipEvent_t e0, hipEvent_t e1, float *best, bool tri) {
     *best = 1e30f;
     for (int r = 0; r < kTuneReps; ++r) {
         GTN_CHECK_HIP(hipEventRecord(e0, s));
-        int rc = gemm_grouped_impl(groups, n, dtype, prec, s, nullptr, 0, "gtn_gemm_grouped", tile, target);
+        int rc = gemm_grouped_impl(groups, n, dtype, prec, s, nullptr, 0, "gtn_gemm_grouped", tile, target, nullptr, tri);
         if (rc) return rc;
         GTN_CHECK_HIP(hipEventRecord(e1, s));
         GTN_CHECK_HIP(hipEventSynchronize(e1));
@@ -913,7 +936,8 @@ static int time_cfg(const gtn_gemm_desc *groups, int n, int dtype, int prec, hip
 }
 
 // the tuned configuration of this signature, if any (no timing)
-static int tuned_lookup(const gtn_gemm_desc *groups, int n, int dtype, int prec, int *tile, int *target, bool *found) {
+static int tuned_lookup(const gtn_gemm_desc *groups, int n, int dtype, int prec, int *tile, int *target, bool *found,
+                        bool tri = false) {
     *tile = 0;
     *target = -1;
     *found = false;
@@ -921,7 +945,7 @@ static int tuned_lookup(const gtn_gemm_desc *groups, int n, int dtype, int prec,
     int dev;
     GTN_CHECK_HIP(hipGetDevice(&dev));
     std::lock_guard<std::mutex> l(g_tune_mu);
-    auto it = g_tuned.find(tune_key(groups, n, dtype, prec, dev));
+    auto it = g_tuned.find(tune_key(groups, n, dtype, prec, dev, tri));
     if (it != g_tuned.end()) {
         *tile = it->second.tile;
         *target = it->second.target;
@@ -930,13 +954,14 @@ static int tuned_lookup(const gtn_gemm_desc *groups, int n, int dtype, int prec,
     return GTN_OK;
 }
 
-static int tuned_config(const gtn_gemm_desc *groups, int n, int dtype, int prec, hipStream_t s, int *tile, int *target) {
+static int tuned_config(const gtn_gemm_desc *groups, int n, int dtype, int prec, hipStream_t s, int *tile, int *target,
+                        bool tri = false) {
     bool found;
-    int rc0 = tuned_lookup(groups, n, dtype, prec, tile, target, &found);
+    int rc0 = tuned_lookup(groups, n, dtype, prec, tile, target, &found, tri);
     if (rc0 || found || !autotune_on() || dry_run() || n <= 0) return rc0;
     int dev;
     GTN_CHECK_HIP(hipGetDevice(&dev));
-    const std::string key = tune_key(groups, n, dtype, prec, dev);
+    const std::string key = tune_key(groups, n, dtype, prec, dev, tri);
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
     GTN_CHECK_HIP(hipStreamIsCapturing(s, &cs));
     if (cs != hipStreamCaptureStatusNone || capture_open()) return GTN_OK;
@@ -951,14 +976,14 @@ static int tuned_config(const gtn_gemm_desc *groups, int n, int dtype, int prec,
     GTN_CHECK_HIP(hipEventCreate(&e1));
     TuneCfg best{0, -1, 1e30f, 0};
     float ms_default = 0;
-    int rc = time_cfg(groups, n, dtype, prec, s, 0, -1, e0, e1, &ms_default);
+    int rc = time_cfg(groups, n, dtype, prec, s, 0, -1, e0, e1, &ms_default, tri);
     const int tiles[2] = {64, 128};
     const int targets[4] = {0, 512, 1024, 2048};
     for (int ti = 0; ti < 2 && !rc; ++ti) {
         if (tiles[ti] == 128 && !can128) continue;
         for (int gi = 0; gi < 4 && !rc; ++gi) {
             float ms;
-            rc = time_cfg(groups, n, dtype, prec, s, tiles[ti], targets[gi], e0, e1, &ms);
+            rc = time_cfg(groups, n, dtype, prec, s, tiles[ti], targets[gi], e0, e1, &ms, tri);
             if (!rc && ms < best.ms) best = TuneCfg{tiles[ti], targets[gi], ms, 0};
         }
     }
@@ -978,6 +1003,16 @@ extern "C" int gtn_gemm_grouped(const gtn_gemm_desc *groups, int n_groups, int d
     int rc = tuned_config(groups, n_groups, dtype, precision, as_stream(stream), &tile, &target);
     if (rc) return rc;
     return gemm_grouped_impl(groups, n_groups, dtype, precision, stream, nullptr, 0, "gtn_gemm_grouped", tile, target);
+}
+
+int gtn::gemm_symmetric(const gtn_gemm_desc *groups, int n_groups, void *stream) {
+    for (int i = 0; i < n_groups; ++i)
+        GTN_REQUIRE(groups[i].M == groups[i].N, "gtn_svd_blocks: a symmetric product is square");
+    int tile = 0, target = -1;
+    int rc = tuned_config(groups, n_groups, GTN_F64, GTN_PREC_F64, as_stream(stream), &tile, &target, true);
+    if (rc) return rc;
+    return gemm_grouped_impl(groups, n_groups, GTN_F64, GTN_PREC_F64, stream, nullptr, 0, "gtn_svd_blocks", tile, target,
+                             nullptr, true);
 }
 
 int gtn::gemm_grouped_indirect(const gtn_gemm_desc *groups, const GemmIndirect *ind, int n_groups, void *const *tune_c,
