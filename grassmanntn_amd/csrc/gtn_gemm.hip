@@ -160,18 +160,6 @@ struct InnerPanels {
     }
 };
 
-template <int ROWS, int BK>
-__device__ __forceinline__ void panel_coord(int s, bool kc, int &r, int &k) {
-    int e = threadIdx.x + 256 * s;
-    if (kc) {
-        r = e / BK;
-        k = e % BK;
-    } else {
-        k = e / ROWS;
-        r = e % ROWS;
-    }
-}
-
 // ------------------------------------------------------------------------------------------------
 // FP64 / FP32 kernels: 16x16x4 MFMA, LDS panels stored k-major [BK][ROWS + pad].
 // MFMA 16x16x4 operand layout (per lane l of the wave): A value = A[i = l%16][k = l/16],
@@ -356,16 +344,103 @@ __global__ void __launch_bounds__(256, IND || TRI ? 2 : 1) k_gemm_fp(GemmArgs ar
 }
 
 // ------------------------------------------------------------------------------------------------
-// BF16 split-product kernel: 16x16x32 MFMA.  LDS panels stored row-major [ROWS][BK + pad] so that a
+// BF16 split-product kernel: 16x16x32 MFMA.  LDS panels stored row-major [ROWS][32 + pad] so that a
 // lane's 8 consecutive k values are one 16-byte read.  Operand layout (lane l): A values
 // A[i = l%16][k = 8*(l/16) + t], t = 0..7; B values B[k = 8*(l/16) + t][j = l%16]; the result layout
 // is that of the 16x16x4 instructions.
 // ------------------------------------------------------------------------------------------------
 // SA / SB: BF16 terms each A / B element is split into (hi, mid, lo); the products of term t of A
 // and term u of B with t + u < max(SA, SB) are accumulated, smallest first.
-template <typename TIN, int SA, int SB, int BM, int BN, int BK>
-__global__ void __launch_bounds__(256) k_gemm_bf16(GemmArgs args) {
+constexpr int kBfK = 32;            // reduction per panel: one MFMA
+constexpr int kBfStride = kBfK + 8; // 80-byte rows: the 16 rows of an operand read start in distinct banks
+
+// One operand's ROWS x 32 panels.  A lane's slot is an octet, 8 consecutive k of one row, kept in the
+// operand's own type and written to LDS as one 16-byte store per term.  Reduction-contiguous operands
+// are read 16 bytes a lane (four lanes a row), row-contiguous ones one element a lane, 64 lanes on
+// consecutive rows; panels that leave the operand, and origins or strides that 16-byte loads cannot
+// take, are read element by element with a range check (out of range reads as zero).
+template <typename T, int ROWS>
+struct OctetPanels {
+    static constexpr int NS = ROWS / 64;  // octets per lane (256 lanes, 4 octets a row)
+    typedef T vec __attribute__((ext_vector_type(16 / sizeof(T))));
+    const T *p;
+    int64_t sr, sk;
+    int R0, R, K;
+    bool kc, wide, rows_in;
+    T reg[NS][8];
+    __device__ __forceinline__ OctetPanels(const T *p_, int64_t sr_, int64_t sk_, int R0_, int R_, int K_)
+        : p(p_), sr(sr_), sk(sk_), R0(R0_), R(R_), K(K_) {
+        kc = sk == 1;
+        wide = (((uint64_t)p) & 15) == 0 && (sr * (int64_t)sizeof(T)) % 16 == 0;
+        rows_in = R0 + ROWS <= R;
+    }
+    __device__ __forceinline__ void at(int s, int &r, int &q) const {
+        const int e = threadIdx.x + 256 * s;
+        r = kc ? e / 4 : e % ROWS;
+        q = kc ? e % 4 : e / ROWS;
+    }
+    __device__ __forceinline__ void load(int k0) {
+        const bool inside = rows_in && k0 + kBfK <= K;
+#pragma unroll
+        for (int s = 0; s < NS; ++s) {
+            int r, q;
+            at(s, r, q);
+            const int k = k0 + 8 * q;
+            if (inside && kc && wide) {
+                const vec *src = (const vec *)(p + (int64_t)(R0 + r) * sr + k);
+#pragma unroll
+                for (int t = 0; t < (int)sizeof(T) / 2; ++t) {
+                    const vec v = src[t];
+#pragma unroll
+                    for (int u = 0; u < 16 / (int)sizeof(T); ++u) reg[s][t * (16 / sizeof(T)) + u] = v[u];
+                }
+            } else if (inside) {
+                const T *src = p + (int64_t)(R0 + r) * sr + (int64_t)k * sk;
+#pragma unroll
+                for (int t = 0; t < 8; ++t) reg[s][t] = src[t * sk];
+            } else {
+#pragma unroll
+                for (int t = 0; t < 8; ++t) {
+                    // branch-free: out of range reads element (0, 0), valid for R, K >= 1, and drops it
+                    const bool ok = R0 + r < R && k + t < K;
+                    const T v = p[ok ? (int64_t)(R0 + r) * sr + (int64_t)(k + t) * sk : (int64_t)0];
+                    reg[s][t] = ok ? v : (T)0;
+                }
+            }
+        }
+    }
+    // split into S terms; each rest x - hi is exact in T
+    template <int S>
+    __device__ __forceinline__ void store(__bf16 (&X)[S][ROWS][kBfStride]) const {
+#pragma unroll
+        for (int s = 0; s < NS; ++s) {
+            int r, q;
+            at(s, r, q);
+            T x[8];
+#pragma unroll
+            for (int t = 0; t < 8; ++t) x[t] = reg[s][t];
+#pragma unroll
+            for (int u = 0; u < S; ++u) {
+                bf8 h;
+#pragma unroll
+                for (int t = 0; t < 8; ++t) {
+                    h[t] = (__bf16)(float)x[t];
+                    x[t] -= (T)(float)h[t];
+                }
+                *(bf8 *)&X[u][r][8 * q] = h;
+            }
+        }
+    }
+};
+
+// Bounded by what surrounds the matrix instructions: with one element, widened to FP64, a lane and slot, two
+// barriers a panel and 2-byte LDS stores, a 4096 x 256 x 256 product of five FP32 members (split A) took 45
+// to 55 us, 15 at the rate of a large copy; with octets and two panel buffers (three terms have room for
+// one) it takes 20 to 23.
+template <typename TIN, int SA, int SB, int BM, int BN>
+__global__ void __launch_bounds__(256, 2) k_gemm_bf16(GemmArgs args) {
     constexpr int NSPLIT = SA > SB ? SA : SB;
+    constexpr int NBUF = NSPLIT > 2 ? 1 : 2;
     int gi, b, tm, tn;
     if (!locate(args, gi, b, tm, tn)) return;
     const GemmGroup &g = args.g[gi];
@@ -376,10 +451,8 @@ __global__ void __launch_bounds__(256) k_gemm_bf16(GemmArgs args) {
     const TIN *A = (const TIN *)g.A + b * g.sab + kb * g.sak;
     const TIN *B = (const TIN *)g.B + b * g.sbb + kb * g.sbk;
     TIN *C = (TIN *)g.C + b * g.scb + sp * g.scs;
-    constexpr int PAD = 8;
-    __shared__ __attribute__((aligned(16))) __bf16 As[SA][BM][BK + PAD];
-    __shared__ __attribute__((aligned(16))) __bf16 Bs[SB][BN][BK + PAD];
-    constexpr int NA = BM * BK / 256, NB = BN * BK / 256;
+    __shared__ __attribute__((aligned(16))) __bf16 As[NBUF][SA][BM][kBfStride];
+    __shared__ __attribute__((aligned(16))) __bf16 Bs[NBUF][SB][BN][kBfStride];
     constexpr int WM = BM / 2, WN = BN / 2, TI = WM / 16, TJ = WN / 16;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int wm = (wave >> 1) * WM, wn = (wave & 1) * WN;
@@ -389,72 +462,51 @@ __global__ void __launch_bounds__(256) k_gemm_bf16(GemmArgs args) {
     for (int i = 0; i < TI; ++i)
 #pragma unroll
         for (int j = 0; j < TJ; ++j) acc[i][j] = f4{0, 0, 0, 0};
-    double ra[NA], rb[NB];
-    const bool akc = (g.sak == 1), bkc = (g.sbk == 1);
-    if (K > 0) {
-        load_panel<TIN, BM, BK>(A, g.sam, g.sak, m0, 0, g.M, K, ra);
-        load_panel<TIN, BN, BK>(B, g.sbn, g.sbk, n0, 0, g.N, K, rb);
-    }
-    for (int k0 = 0; k0 < K; k0 += BK) {
-        __syncthreads();
+    OctetPanels<TIN, BM> pa(A, g.sam, g.sak, m0, g.M, K);
+    OctetPanels<TIN, BN> pb(B, g.sbn, g.sbk, n0, g.N, K);
+    auto panel_mfma = [&](int buf) {
+        bf8 af[SA][TI], bfr[SB][TJ];
 #pragma unroll
-        for (int s = 0; s < NA; ++s) {
-            int r, k;
-            panel_coord<BM, BK>(s, akc, r, k);
-            double x = ra[s];
+        for (int t = 0; t < SA; ++t)
 #pragma unroll
-            for (int t = 0; t < SA; ++t) {
-                __bf16 h = (__bf16)(float)x;
-                As[t][r][k] = h;
-                x -= (double)(float)h;
-            }
-        }
+            for (int i = 0; i < TI; ++i) af[t][i] = *(const bf8 *)&As[buf][t][wm + 16 * i + lane % 16][8 * (lane / 16)];
 #pragma unroll
-        for (int s = 0; s < NB; ++s) {
-            int r, k;
-            panel_coord<BN, BK>(s, bkc, r, k);
-            double x = rb[s];
+        for (int t = 0; t < SB; ++t)
 #pragma unroll
-            for (int t = 0; t < SB; ++t) {
-                __bf16 h = (__bf16)(float)x;
-                Bs[t][r][k] = h;
-                x -= (double)(float)h;
-            }
-        }
-        __syncthreads();
-        if (k0 + BK < K) {
-            load_panel<TIN, BM, BK>(A, g.sam, g.sak, m0, k0 + BK, g.M, K, ra);
-            load_panel<TIN, BN, BK>(B, g.sbn, g.sbk, n0, k0 + BK, g.N, K, rb);
-        }
+            for (int j = 0; j < TJ; ++j) bfr[t][j] = *(const bf8 *)&Bs[buf][t][wn + 16 * j + lane % 16][8 * (lane / 16)];
 #pragma unroll
-        for (int kk = 0; kk < BK; kk += 32) {
-            bf8 af[SA][TI], bfr[SB][TJ];
+        for (int i = 0; i < TI; ++i)
 #pragma unroll
-            for (int t = 0; t < SA; ++t)
-#pragma unroll
-                for (int i = 0; i < TI; ++i)
-                    af[t][i] = *(const bf8 *)&As[t][wm + 16 * i + lane % 16][kk + 8 * (lane / 16)];
-#pragma unroll
-            for (int t = 0; t < SB; ++t)
-#pragma unroll
-                for (int j = 0; j < TJ; ++j)
-                    bfr[t][j] = *(const bf8 *)&Bs[t][wn + 16 * j + lane % 16][kk + 8 * (lane / 16)];
-#pragma unroll
-            for (int i = 0; i < TI; ++i)
-#pragma unroll
-                for (int j = 0; j < TJ; ++j) {
-                    // small cross terms first, the hi*hi product last
-                    if constexpr (NSPLIT == 3) {
-                        if constexpr (SA > 2) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[2][i], bfr[0][j], acc[i][j], 0, 0, 0);
-                        if constexpr (SA > 1 && SB > 1) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[1][i], bfr[1][j], acc[i][j], 0, 0, 0);
-                        if constexpr (SB > 2) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[0][i], bfr[2][j], acc[i][j], 0, 0, 0);
-                    }
-                    if constexpr (NSPLIT >= 2) {
-                        if constexpr (SA > 1) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[1][i], bfr[0][j], acc[i][j], 0, 0, 0);
-                        if constexpr (SB > 1) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[0][i], bfr[1][j], acc[i][j], 0, 0, 0);
-                    }
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[0][i], bfr[0][j], acc[i][j], 0, 0, 0);
+            for (int j = 0; j < TJ; ++j) {
+                // small cross terms first, the hi*hi product last
+                if constexpr (NSPLIT == 3) {
+                    if constexpr (SA > 2) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[2][i], bfr[0][j], acc[i][j], 0, 0, 0);
+                    if constexpr (SA > 1 && SB > 1) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[1][i], bfr[1][j], acc[i][j], 0, 0, 0);
+                    if constexpr (SB > 2) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[0][i], bfr[2][j], acc[i][j], 0, 0, 0);
                 }
+                if constexpr (NSPLIT >= 2) {
+                    if constexpr (SA > 1) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[1][i], bfr[0][j], acc[i][j], 0, 0, 0);
+                    if constexpr (SB > 1) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[0][i], bfr[1][j], acc[i][j], 0, 0, 0);
+                }
+                acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[0][i], bfr[0][j], acc[i][j], 0, 0, 0);
+            }
+    };
+    if (K > 0) {
+        pa.load(0);
+        pb.load(0);
+        int cur = 0;
+        for (int k0 = 0; k0 < K; k0 += kBfK) {
+            // two buffers: the one written here was last read before the barrier of the previous panel
+            if constexpr (NBUF == 1) __syncthreads();
+            pa.template store<SA>(As[cur]);
+            pb.template store<SB>(Bs[cur]);
+            if (k0 + kBfK < K) {  // the next panels are on their way while the matrix cores work
+                pa.load(k0 + kBfK);
+                pb.load(k0 + kBfK);
+            }
+            __syncthreads();
+            panel_mfma(cur);
+            if constexpr (NBUF == 2) cur ^= 1;
         }
     }
     const double alpha = g.alpha, beta = g.beta;
@@ -612,27 +664,27 @@ static int launch_gemm(GemmArgs &a, int precision, int tile, hipStream_t s) {
             break;
         case GTN_PREC_BF16X3:
             if (big)
-                hipLaunchKernelGGL((k_gemm_bf16<TIN, 2, 2, 128, 128, 32>), dim3(grid), dim3(256), 0, s, a);
+                hipLaunchKernelGGL((k_gemm_bf16<TIN, 2, 2, 128, 128>), dim3(grid), dim3(256), 0, s, a);
             else
-                hipLaunchKernelGGL((k_gemm_bf16<TIN, 2, 2, 64, 64, 32>), dim3(grid), dim3(256), 0, s, a);
+                hipLaunchKernelGGL((k_gemm_bf16<TIN, 2, 2, 64, 64>), dim3(grid), dim3(256), 0, s, a);
             break;
         case GTN_PREC_BF16X6:
             if (big)
-                hipLaunchKernelGGL((k_gemm_bf16<TIN, 3, 3, 128, 128, 32>), dim3(grid), dim3(256), 0, s, a);
+                hipLaunchKernelGGL((k_gemm_bf16<TIN, 3, 3, 128, 128>), dim3(grid), dim3(256), 0, s, a);
             else
-                hipLaunchKernelGGL((k_gemm_bf16<TIN, 3, 3, 64, 64, 32>), dim3(grid), dim3(256), 0, s, a);
+                hipLaunchKernelGGL((k_gemm_bf16<TIN, 3, 3, 64, 64>), dim3(grid), dim3(256), 0, s, a);
             break;
         case GTN_PREC_BF16:
             if (big)
-                hipLaunchKernelGGL((k_gemm_bf16<TIN, 1, 1, 128, 128, 32>), dim3(grid), dim3(256), 0, s, a);
+                hipLaunchKernelGGL((k_gemm_bf16<TIN, 1, 1, 128, 128>), dim3(grid), dim3(256), 0, s, a);
             else
-                hipLaunchKernelGGL((k_gemm_bf16<TIN, 1, 1, 64, 64, 32>), dim3(grid), dim3(256), 0, s, a);
+                hipLaunchKernelGGL((k_gemm_bf16<TIN, 1, 1, 64, 64>), dim3(grid), dim3(256), 0, s, a);
             break;
         case GTN_PREC_BF16_SPLIT_A:
             if (big)
-                hipLaunchKernelGGL((k_gemm_bf16<TIN, 2, 1, 128, 128, 32>), dim3(grid), dim3(256), 0, s, a);
+                hipLaunchKernelGGL((k_gemm_bf16<TIN, 2, 1, 128, 128>), dim3(grid), dim3(256), 0, s, a);
             else
-                hipLaunchKernelGGL((k_gemm_bf16<TIN, 2, 1, 64, 64, 32>), dim3(grid), dim3(256), 0, s, a);
+                hipLaunchKernelGGL((k_gemm_bf16<TIN, 2, 1, 64, 64>), dim3(grid), dim3(256), 0, s, a);
             break;
         default: set_error("gtn_gemm_grouped: unknown precision %d", precision); return GTN_ENOTSUP;
     }
