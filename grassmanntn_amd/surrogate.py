@@ -84,10 +84,12 @@ class MLPEnsemble:
         cmax = max(self.dims[1:])
         self.colpart = DeviceArray.empty(L.lib().gtn_mlp_colsum_workspace(self.E, cmax) // 8)
 
-    def _mm(self, A, sam, sak, sab, B, sbk, sbn, sbb, Cm, scm, M, N, K, scb):
-        d = _gemm_desc(A.data_ptr(), sam, sak, B.data_ptr(), sbk, sbn, Cm.data_ptr(), scm, 1, M, N, K,
-                       batch=self.E, sab=sab, sbb=sbb, scb=scb)
-        _gemm([d], L.GTN_F32, PREC)
+    def _desc(self, A, sam, sak, sab, B, sbk, sbn, sbb, Cm, scm, M, N, K, scb):
+        return _gemm_desc(A.data_ptr(), sam, sak, B.data_ptr(), sbk, sbn, Cm.data_ptr(), scm, 1, M, N, K,
+                          batch=self.E, sab=sab, sbb=sbb, scb=scb)
+
+    def _mm(self, *args):
+        _gemm([self._desc(*args)], L.GTN_F32, PREC)
 
     def forward(self, X):
         """X: device (n, d_0) FP32 shared by the members -> output (E, n, d_L) (a buffer of this
@@ -112,11 +114,13 @@ class MLPEnsemble:
         n = X.shape[0]
         lib = L.lib()
         dZ = dout
+        weights = []
         for l in range(self.L - 1, -1, -1):
             a, b = self.dims[l], self.dims[l + 1]
             Hin, shared = (X, True) if l == 0 else (self.A[l - 1], False)
             # dW = H^T dZ (E, a, b); db = column sums of dZ
-            self._mm(Hin, 1, a, 0 if shared else n * a, dZ, b, 1, n * b, self.W(l, self.grads), b, a, b, n, a * b)
+            weights.append(self._desc(Hin, 1, a, 0 if shared else n * a, dZ, b, 1, n * b, self.W(l, self.grads), b,
+                                      a, b, n, a * b))
             L.check(lib.gtn_mlp_colsum(L.ptr(dZ), self.E, n, b, L.ptr(self.b(l, self.grads)), L.ptr(self.colpart),
                                        L.stream_ptr()), "gtn_mlp_colsum")
             if l > 0:
@@ -126,6 +130,8 @@ class MLPEnsemble:
                 L.check(lib.gtn_mlp_act_backward(L.ptr(dH), L.ptr(self.P[l - 1]), self.E * n * a, L.GTN_ACT_GELU,
                                                  L.stream_ptr()), "gtn_mlp_act_backward")
                 dZ = dH
+        # every layer's dW in one launch: the 2- and 17-column products alone leave most of the device idle
+        _gemm(weights, L.GTN_F32, PREC)
 
     def loss_grad(self, out, T, w):
         """dL/dout into the last dZ buffer, per-member losses into self.loss; T (n, d_L) device FP32."""
