@@ -44,15 +44,16 @@ class DeviceArray:
     def __init__(self, storage, offset, shape, dtype):
         self.storage = storage
         self.offset = int(offset)
-        self.shape = tuple(int(s) for s in shape)
+        self.shape = tuple([int(s) for s in shape])
         self.dtype = np.dtype(dtype)
 
     # ---- construction -------------------------------------------------------------------------
     @staticmethod
     def empty(shape, dtype=np.float64):
-        shape = tuple(int(s) for s in (shape if isinstance(shape, (tuple, list)) else (shape,)))
         dt = np.dtype(dtype)
-        return DeviceArray(Storage(max(_numel(shape) * dt.itemsize, 1)), 0, shape, dt)
+        a = DeviceArray(None, 0, shape if isinstance(shape, (tuple, list)) else (shape,), dt)
+        a.storage = Storage(max(_numel(a.shape) * dt.itemsize, 1))
+        return a
 
     @staticmethod
     def zeros(shape, dtype=np.float64):

@@ -6,6 +6,7 @@ several raw axes such as (parity, half-index)); virtual axes split into componen
 add into the fused indices of the source's axes.
 """
 import ctypes as C
+import functools
 
 from . import _lib as L
 from ._device import DeviceArray
@@ -19,6 +20,7 @@ class Perm:
         self.ins = []     # [dim, enc, sigma, split, stride, stride_lo]
         self.codes = [0]
         self.n_bits = 0
+        self._descs = {}  # descriptors of the finished gather, by (dtype, source size, factor)
 
     def add_in(self, dim, stride, enc=False, sigma=False, split=False, stride_lo=0):
         self.ins.append([int(dim), bool(enc), bool(sigma), bool(split), int(stride), int(stride_lo)])
@@ -47,6 +49,17 @@ class Perm:
         self.n_bits = n
 
     def desc(self, dtype, src_elems, alpha=1.0):
+        """The descriptor for one source; a gather that has been run is not built any further."""
+        key = (dtype, src_elems, alpha)
+        d = self._descs.get(key)
+        if d is None:
+            d = self._desc(dtype, src_elems, alpha)
+            if len(self._descs) >= 8:
+                self._descs = {}
+            self._descs[key] = d
+        return d
+
+    def _desc(self, dtype, src_elems, alpha):
         d = L.PermDesc()
         if len(self.outs) > L.MAX_AX or len(self.virts) > L.MAX_AX or len(self.ins) > L.MAX_AX:
             raise NotImplementedError("gather with more than %d axes" % L.MAX_AX)
@@ -114,6 +127,7 @@ class Perm:
         return dst
 
 
+@functools.lru_cache(maxsize=256)
 def compose(outer, inner):
     """outer(inner(.)) as one gather, or None.  It is one when every axis between them carries a single
     leg: each source axis of `outer` is one component, unsplit, laid out as `inner` writes it, and each

@@ -12,6 +12,7 @@ characters.  Every monomial of q involves characters that live together on one o
 output, so q splits into q_A + q_B + q_out; each part becomes a sign table that the device applies
 while it gathers that tensor (the kernel computes the parities by popcount).
 """
+import functools
 import itertools
 
 HYBRID = "*"
@@ -38,6 +39,7 @@ def fresh_char(used):
     fail("Error[get_char]: Running out of index character!")
 
 
+@functools.lru_cache(maxsize=1024)
 def denumerate(string):
     """Multi-character numbered indices ('i12') become single fresh characters (__init__.py:1610-1631)."""
     toks = []

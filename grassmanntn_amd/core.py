@@ -5,8 +5,10 @@ join_legs / split_legs, svd / eig with '(ij)(kl)' grouping, hconjugate, sqrt / p
 lives in HBM as DeviceArrays owned by libgtn_hip.so; every numeric step runs in its HIP kernels.
 """
 import ctypes as C
+import functools
 import math
 import sys
+from typing import NamedTuple
 
 import numpy as np
 
@@ -133,6 +135,28 @@ def _to_device(x):
 
 def _is_pp(T, axis):
     return T.encoder == "parity-preserving" and T.statistics[axis] in FERMI
+
+
+class _Legs(NamedTuple):
+    """What a gather plan needs to know of a tensor: no data, no identity."""
+    shape: tuple
+    statistics: tuple
+    encoder: str
+    format: str
+
+    @property
+    def ndim(self):
+        return len(self.shape)
+
+
+def _legs(T):
+    return _Legs(tuple(T.shape), tuple(T.statistics), T.encoder, T.format)
+
+
+# Plans (the gathers and sizes of one operation) depend on subscripts, shapes, statistics, encoders and
+# formats alone and are kept by these values, the last 512 of each kind; building one anew cost most of a
+# small call: einsum of two 8^4 tensors took 137 us, with its plan at hand 38.
+_planned = functools.lru_cache(maxsize=512)
 
 
 # --------------------------------------------------------------------------------------------------
@@ -566,6 +590,13 @@ def is_grassmann_even(T):
 def _relayout(T, order, out_encoder, sigma=None, parity_lin=None, table_chars=None, codes=None, alpha=1.0):
     """out axis a = T axis order[a], in `out_encoder`; sigma[a]: multiply sigma(canonical index) of
     source axis a; parity_lin[a]: multiply (-1)^p of source axis a."""
+    P = _relayout_plan(_legs(T), tuple(order), out_encoder, tuple(sigma) if sigma else None,
+                       tuple(parity_lin) if parity_lin else None)
+    return P.run(T.data, alpha=alpha)
+
+
+@_planned
+def _relayout_plan(T, order, out_encoder, sigma, parity_lin):
     P = Perm()
     ins = []
     st = strides(T.shape)
@@ -584,7 +615,7 @@ def _relayout(T, order, out_encoder, sigma=None, parity_lin=None, table_chars=No
     if lin_axes:
         n = len(lin_axes)
         P.set_table([bin(m).count("1") & 1 for m in range(1 << n)])
-    return P.run(T.data, alpha=alpha)
+    return P
 
 
 # --------------------------------------------------------------------------------------------------
@@ -609,12 +640,9 @@ def einsum(*args, ignore_anticommutation=False):
     first = ops[0]
     if nobj >= 3:
         return _einsum_pairwise(subscripts, ops, ignore_anticommutation)
-    plan = contraction(subscripts, [(o.statistics, o.shape) for o in ops])
     if nobj == 1:
-        res = _einsum1(plan, ops[0], first, ignore_anticommutation)
-    else:
-        res = _einsum2(plan, ops[0], ops[1], first, ignore_anticommutation)
-    return res
+        return _einsum1(subscripts, first, bool(ignore_anticommutation))
+    return _einsum2(subscripts, first, ops[1], bool(ignore_anticommutation))
 
 
 def _einsum_pairwise(subscripts, ops, ignore):
@@ -730,6 +758,11 @@ def _source_dtype(T):
 def _gather_permuted(src, order, codes, fbits):
     """out[x] = code(parities of x) * src[x permuted]: out axis a is source axis order[a]; bit k of the
     table index is the parity of out axis fbits[k]."""
+    return _permuted_plan(_legs(src), tuple(order), tuple(codes), tuple(fbits)).run(src.data)
+
+
+@_planned
+def _permuted_plan(src, order, codes, fbits):
     P = Perm()
     st = strides(src.shape)
     ins = [P.add_in(src.shape[b], st[b], enc=_is_pp(src, b), sigma=(src.format == "matrix" and src.statistics[b] == -1))
@@ -741,7 +774,7 @@ def _gather_permuted(src, order, codes, fbits):
         P.add_comp(v, src.shape[b], [(ins[b], 1)], bit=fbits.index(a) if a in fbits else -1)
         P.add_out(src.shape[b], [(v, 1)])
     P.set_table(codes)
-    return P.run(src.data)
+    return P
 
 
 def permuted_view(T, subscripts):
@@ -764,7 +797,18 @@ def permuted_view(T, subscripts):
     return _PermutedView(T, order, codes, fbits, plan.out_stats)
 
 
-def _einsum1(plan, A, first, ignore):
+class _Plan1(NamedTuple):
+    gather: Perm
+    reduced: int  # values that each output sums; 0: nothing is summed
+    shape: tuple
+    stats: tuple
+    has_output: bool
+
+
+@_planned
+def _einsum1_plan(subscripts, A, ignore):
+    plan = contraction(subscripts, [(A.statistics, A.shape)])
+    first = A
     s = plan.inputs[0]
     out = plan.output
     dims = plan.dims
@@ -790,19 +834,24 @@ def _einsum1(plan, A, first, ignore):
         P.add_comp(v, dims[c], tg, bit=fa.index(c) if c in fa else -1, sigma=c in pairs)
         P.add_out(dims[c], [(v, 1)])
     P.set_table(codes)
-    g = P.run(A.data)
-    red = _prod(dims[c] for c in summed)
-    if summed:
-        rows = g.numel() // red
+    return _Plan1(P, _prod(dims[c] for c in summed) if summed else 0, tuple(dims[c] for c in out), plan.out_stats,
+                  plan.has_output)
+
+
+def _einsum1(subscripts, A, ignore):
+    plan = _einsum1_plan(subscripts, _legs(A), ignore)
+    g = plan.gather.run(A.data)
+    if plan.reduced:
+        rows = g.numel() // plan.reduced
         r = DeviceArray.empty(rows, g.dtype)
-        L.check(L.lib().gtn_reduce_last(L.ptr(g), L.ptr(r), rows, red, L.dtype_code(g), L.stream_ptr()), "reduce")
-        g = r.reshape(tuple(dims[c] for c in out))
+        L.check(L.lib().gtn_reduce_last(L.ptr(g), L.ptr(r), rows, plan.reduced, L.dtype_code(g), L.stream_ptr()), "reduce")
+        g = r
     if not plan.has_output:
         return g.numpy().reshape(-1)[0].item()
     res = dense.__new__(dense)
-    res.data = g.reshape(tuple(dims[c] for c in out))
-    res.statistics = plan.out_stats
-    res.encoder, res.format = first.encoder, first.format
+    res.data = g.reshape(plan.shape)
+    res.statistics = plan.stats
+    res.encoder, res.format = A.encoder, A.format
     res._even = True if A._even else None
     return res
 
@@ -847,17 +896,11 @@ def _gemm(groups, dtype_code, prec):
 
 
 def _gemm_desc(A, sam, sak, B, sbk, sbn, Cp, scm, scn, M, N, K, batch=1, sab=0, sbb=0, scb=0, alpha=1.0, beta=0.0):
-    d = L.GemmDesc()
-    d.A, d.B, d.C = A, B, Cp
-    d.M, d.N, d.K, d.batch = M, N, K, batch
-    d.sam, d.sak, d.sbk, d.sbn, d.scm, d.scn = sam, sak, sbk, sbn, scm, scn
-    d.sab, d.sbb, d.scb = sab, sbb, scb
-    d.alpha, d.beta = alpha, beta
-    return d
+    return L.GemmDesc(A, B, Cp, M, N, K, batch, sam, sak, sbk, sbn, scm, scn, sab, sbb, scb, alpha, beta)
 
 
-def _operand_gather(T, s, plan, layout, fchars, codes, sig_chars):
-    """Gather operand T (index string s) into the GEMM layout.
+def _operand_plan(T, s, plan, layout, fchars, codes, sig_chars):
+    """The gather of operand T (index string s) into the GEMM layout.
 
     layout: list of raw axes, each ('b', char) bosonic/batch leg, ('P',) parity, ('F', group) the
     half (blocked) or full fused fermionic index of a group; groups: dict name -> list of chars."""
@@ -899,20 +942,33 @@ def _operand_gather(T, s, plan, layout, fchars, codes, sig_chars):
             else:
                 P.add_out(full, [(virt_of[("F", item[1])], 1)])
     P.set_table(codes)
+    return P
+
+
+def _run_gather(P, T):
     if isinstance(T, _PendingOutput) and T._data is None:
         return run_composed(P, T._perm, T._src)
     return P.run(T.data)
 
 
-def _einsum2(plan, A, B, first, ignore):
+class _Plan2(NamedTuple):
+    gather_a: Perm
+    gather_b: Perm
+    gather_out: Perm   # None: a number
+    sizes: tuple       # batch, parity blocks, M, N, K
+    reduced: tuple     # values of A and B summed before the product
+    stats: tuple
+
+
+@_planned
+def _einsum2_plan(subscripts, A, B, blocked, ignore):
+    plan = contraction(subscripts, [(A.statistics, A.shape), (B.statistics, B.shape)])
+    first = A
     sA, sB = plan.inputs
     out = plan.output
     dims = plan.dims
     setA, setB, setO = set(sA), set(sB), set(out)
     uA, uB = list(dict.fromkeys(sA)), list(dict.fromkeys(sB))
-    dA, dB = np.dtype(_source_dtype(A)), np.dtype(_source_dtype(B))
-    if not all(d in (np.dtype(np.float64), np.dtype(np.complex128)) for d in (dA, dB)) and dA != dB:
-        raise NotImplementedError("operands of different dtypes")
     isF = lambda c: _fermionic(plan, c)
     batch = [c for c in uA if c in setB and c in setO]
     contr = [c for c in uA if c in setB and c not in setO]
@@ -930,7 +986,6 @@ def _einsum2(plan, A, B, first, ignore):
     hasR = _prod(dims[c] for c in RF) >= 2
     hasK = _prod(dims[c] for c in KF) >= 2
     hasN = _prod(dims[c] for c in NF) >= 2
-    blocked = A.is_even() and B.is_even()
     split = blocked and hasR and hasK and hasN
     fa = [c for c in uA if isF(c)]
     fb = [c for c in uB if isF(c)]
@@ -975,8 +1030,8 @@ def _einsum2(plan, A, B, first, ignore):
     NFb, NFf = plainify(NF, hasN)
     layA = layout_for(RB + RFb, RFf, hasR, KB + KFb, KFf, hasK, redA, ("R", "K"))
     layB = layout_for(KB + KFb, KFf, hasK, NB + NFb, NFf, hasN, redB, ("K", "N"))
-    Ag = _operand_gather(A, sA, plan, layA, fa, codesA, sigA)
-    Bg = _operand_gather(B, sB, plan, layB, fb, codesB, sigB)
+    PA = _operand_plan(A, sA, plan, layA, fa, codesA, sigA)
+    PB = _operand_plan(B, sB, plan, layB, fb, codesB, sigB)
     half = 2 if blocked else 1
     nb = _prod(dims[c] for c in batch)
     nP = 2 if split else 1
@@ -984,18 +1039,9 @@ def _einsum2(plan, A, B, first, ignore):
     K = _prod(dims[c] for c in KB + KFb) * (_prod(dims[c] for c in KFf) // half if hasK else 1)
     N = _prod(dims[c] for c in NB + NFb) * (_prod(dims[c] for c in NFf) // half if hasN else 1)
     ra, rb = _prod(dims[c] for c in redA), _prod(dims[c] for c in redB)
-    lib = L.lib()
-    if ra > 1:
-        t = DeviceArray.empty(Ag.numel() // ra, Ag.dtype)
-        L.check(lib.gtn_reduce_last(L.ptr(Ag), L.ptr(t), t.numel(), ra, L.dtype_code(Ag), L.stream_ptr()), "reduce")
-        Ag = t
-    if rb > 1:
-        t = DeviceArray.empty(Bg.numel() // rb, Bg.dtype)
-        L.check(lib.gtn_reduce_last(L.ptr(Bg), L.ptr(t), t.numel(), rb, L.dtype_code(Bg), L.stream_ptr()), "reduce")
-        Bg = t
-    Cg = _contract_blocks(Ag, Bg, nb, nP, M, N, K)
+    sizes, reduced = (nb, nP, M, N, K), (ra, rb)
     if not plan.has_output:
-        return Cg.numpy().reshape(-1)[0].item()
+        return _Plan2(PA, PB, None, sizes, reduced, ())
     # output gather from the GEMM layout [batch][P][RB][RFh][NB][NFw]
     shapeC = [dims[c] for c in batch] + ([2] if split else []) + [dims[c] for c in RB + RFb]
     if hasR:
@@ -1043,13 +1089,39 @@ def _einsum2(plan, A, B, first, ignore):
         P.add_comp(v, dims[c], [(i, m)], bit=fo.index(c) if c in fo else -1)
         P.add_out(dims[c], [(v, 1)])
     P.set_table(codesO)
+    return _Plan2(PA, PB, P, sizes, reduced, plan.out_stats)
+
+
+def _reduce_last(X, n):
+    t = DeviceArray.empty(X.numel() // n, X.dtype)
+    L.check(L.lib().gtn_reduce_last(L.ptr(X), L.ptr(t), t.numel(), n, L.dtype_code(X), L.stream_ptr()), "reduce")
+    return t
+
+
+def _einsum2(subscripts, A, B, ignore):
+    blocked = bool(A.is_even() and B.is_even())
+    plan = _einsum2_plan(subscripts, _legs(A), _legs(B), blocked, ignore)
+    dA, dB = _source_dtype(A), _source_dtype(B)
+    if dA != dB and not all(d in (np.dtype(np.float64), np.dtype(np.complex128)) for d in (dA, dB)):
+        raise NotImplementedError("operands of different dtypes")
+    Ag = _run_gather(plan.gather_a, A)
+    Bg = _run_gather(plan.gather_b, B)
+    if plan.reduced[0] > 1:
+        Ag = _reduce_last(Ag, plan.reduced[0])
+    if plan.reduced[1] > 1:
+        Bg = _reduce_last(Bg, plan.reduced[1])
+    nb, nP, M, N, K = plan.sizes
+    Cg = _contract_blocks(Ag, Bg, nb, nP, M, N, K)
+    if plan.gather_out is None:
+        return Cg.numpy().reshape(-1)[0].item()
+    even = True if blocked else None
     if _defer[0]:
-        return _PendingOutput(P, Cg, plan.out_stats, first.encoder, first.format, True if blocked else None)
+        return _PendingOutput(plan.gather_out, Cg, plan.stats, A.encoder, A.format, even)
     res = dense.__new__(dense)
-    res.data = P.run(Cg)
-    res.statistics = plan.out_stats
-    res.encoder, res.format = first.encoder, first.format
-    res._even = True if blocked else None
+    res.data = plan.gather_out.run(Cg)
+    res.statistics = plan.stats
+    res.encoder, res.format = A.encoder, A.format
+    res._even = even
     return res
 
 
@@ -1198,27 +1270,36 @@ def _join_gather(T, string_inp, make_format="standard", intermediate_stat=None, 
     decomposition) the gather writes the two parity blocks M[b][p::2, p::2] instead, as a
     (B, 2, m/2, n/2) array (BlockSVD's ME / MO, __init__.py:3990-3996): the parity p is an output axis
     of its own feeding both fused legs."""
-    string_inp = denumerate(string_inp.replace(" ", ""))
     inter = tuple(intermediate_stat) if not np.isscalar(intermediate_stat) else (intermediate_stat,)
+    through = None
+    if isinstance(T, _PermutedView) and T._data is None:
+        through = (tuple(T._src.shape), tuple(T._order), tuple(T._codes), tuple(T._fbits))
+    P, view, fin_shape, fin_stats = _join_plan(string_inp, _legs(T), make_format, inter, blocks, through)
+    return P, (T._src.data if view else T.data), fin_shape, fin_stats
+
+
+@_planned
+def _join_plan(string_inp, T, make_format, inter, blocks, through):
+    """through: (source shape, order, codes, fbits) of a permuted view that has not been materialised."""
+    string_inp = denumerate(string_inp.replace(" ", ""))
     groups, srt = group_info(string_inp, T.statistics, T.shape)
     sgn_pos = _grouping_sign_axes(srt, inter)
     info = _intermediate(srt, inter)
     P = Perm()
-    view = (isinstance(T, _PermutedView) and T._data is None and T.format == "standard"
-            and len(set(sgn_pos) | set(T._fbits)) <= 10)
+    if through:
+        src_shape, order, codes, fbits = through
+    view = bool(through and T.format == "standard" and len(set(sgn_pos) | set(fbits)) <= 10)
     std = T.format == "matrix"  # input must first go to standard: sigma on its -1 legs
     if view:
         # read the permuted view's source directly: T axis a is source axis order[a]; the view's
         # sign table joins the grouping sign in this gather's table
-        st_src = strides(T._src.shape)
-        ins = [P.add_in(T.shape[a], st_src[T._order[a]], enc=_is_pp(T, a)) for a in range(T.ndim)]
-        src_data = T._src.data
+        st_src = strides(src_shape)
+        ins = [P.add_in(T.shape[a], st_src[order[a]], enc=_is_pp(T, a)) for a in range(T.ndim)]
     else:
         st = strides(T.shape)
         ins = [P.add_in(T.shape[a], st[a], enc=_is_pp(T, a), sigma=(std and T.statistics[a] == -1))
                for a in range(T.ndim)]
-        src_data = T.data
-    bit_axes = sorted(set(sgn_pos) | (set(T._fbits) if view else set()))
+    bit_axes = sorted(set(sgn_pos) | (set(fbits) if view else set()))
     nb = len(bit_axes)
     bitpos = {p: k for k, p in enumerate(bit_axes)}
     fin_shape, fin_stats = [], []
@@ -1271,21 +1352,27 @@ def _join_gather(T, string_inp, make_format="standard", intermediate_stat=None, 
         for m in range(1 << nb):
             code = sum((m >> bitpos[p]) & 1 for p in sgn_pos) & 1
             if view:
-                t = T._codes[sum(((m >> bitpos[a]) & 1) << k for k, a in enumerate(T._fbits))]
+                t = codes[sum(((m >> bitpos[a]) & 1) << k for k, a in enumerate(fbits))]
                 code = 2 if t == 2 else code ^ t
             table.append(code)
         P.set_table(table)
-    return P, src_data, fin_shape, fin_stats
+    return P, view, tuple(fin_shape), tuple(fin_stats)
 
 
 @_sparse_in
 def split_legs(T, string_inp, final_stat, final_shape, intermediate_stat=None, save_memory=False):
     """Inverse of join_legs (__init__.py:3070-3170), including its early return for matrix-format
     input: such input comes back canonical and in matrix format."""
-    string_inp = denumerate(string_inp.replace(" ", ""))
     inter = tuple(intermediate_stat) if not np.isscalar(intermediate_stat) else (intermediate_stat,)
     final_stat = tuple(final_stat)
-    final_shape = tuple(final_shape)
+    data = _split_plan(string_inp, _legs(T), final_stat, tuple(final_shape), inter).run(T.data)
+    return T._like(data, statistics=final_stat, encoder=("canonical" if T.format == "matrix" else T.encoder),
+                   format=T.format, even=T._even)
+
+
+@_planned
+def _split_plan(string_inp, T, final_stat, final_shape, inter):
+    string_inp = denumerate(string_inp.replace(" ", ""))
     groups, srt = group_info(string_inp, final_stat, final_shape)
     sgn_pos = _grouping_sign_axes(srt, inter)
     info = _intermediate(srt, inter)
@@ -1327,9 +1414,7 @@ def split_legs(T, string_inp, final_stat, final_shape, intermediate_stat=None, s
         P.add_out(d, [(v, 1)])
     if sgn_pos:
         P.set_table([bin(m).count("1") & 1 for m in range(1 << len(sgn_pos))])
-    data = P.run(T.data)
-    res = T._like(data, statistics=final_stat, encoder=("canonical" if matrix else enc), format=fmt, even=T._even)
-    return res
+    return P
 
 
 # --------------------------------------------------------------------------------------------------
@@ -1386,6 +1471,11 @@ def _block_assemble(outs, kk, m, n, dt, kept=None):
 def _interleave(stack, rows, cols, row_stride, par_stride):
     """full[r][c] = stack[r % 2][r // 2][c // 2] when r and c have equal parity, else 0 (both dims
     even): the interleaving of get_full_matrix (__init__.py:4017-4028)."""
+    return _interleave_plan(rows, cols, row_stride, par_stride).run(stack)
+
+
+@_planned
+def _interleave_plan(rows, cols, row_stride, par_stride):
     P = Perm()
     ir = P.add_in(rows, row_stride, enc=True, split=True, stride_lo=par_stride)
     ic = P.add_in(cols, 1, enc=True, split=True, stride_lo=0)
@@ -1396,7 +1486,7 @@ def _interleave(stack, rows, cols, row_stride, par_stride):
     P.add_out(rows, [(vr, 1)])
     P.add_out(cols, [(vc, 1)])
     P.set_table([0, 2, 2, 0])  # zero unless both indices have the same parity
-    return P.run(stack)
+    return P
 
 
 def _parity_leak_dev(M):
@@ -1421,6 +1511,12 @@ def _strided_block(M, par, out=None):
     """Contiguous copy of M[par::2, par::2] (the ME / MO extraction of __init__.py:3990-3996), into
     `out` when given."""
     m, n = M.shape
+    off = par * n + par
+    return _strided_plan(m, n).run(M.flat(off, M.numel() - off), dst=out)
+
+
+@_planned
+def _strided_plan(m, n):
     P = Perm()
     i0 = P.add_in(max(m - 1, 1), n)
     i1 = P.add_in(max(n - 1, 1), 1)
@@ -1430,8 +1526,7 @@ def _strided_block(M, par, out=None):
     P.add_comp(v1, n // 2, [(i1, 2)])
     P.add_out(m // 2, [(v0, 1)])
     P.add_out(n // 2, [(v1, 1)])
-    off = par * n + par
-    return P.run(M.flat(off, M.numel() - off), dst=out)
+    return P
 
 
 def _runs(keys):
