@@ -529,7 +529,10 @@ __device__ __forceinline__ void rr_pair(int t, int round, int p, int &i, int &j)
 //     factor L (G = L L^T), factored here; normalised, the rotated columns are G's eigenvectors.  The
 //     basis comes out of an orthogonal iteration, so G is close to diagonal and L to converged.
 //   - a small block with both sides at most 128: its own columns (m <= n) or rows (m > n); no Gram
-//     matrix squares its condition.
+//     matrix squares its condition.  Its rows (the vectors' components) go by decreasing norm through a
+//     modified Gram-Schmidt process, X = L Q, and the rotations start from L's columns: the same left
+//     singular vectors (L L^T = X X^T, and L is as accurate as from reflections, whatever becomes of
+//     Q), but graded, which takes 9 sweeps where the block's own columns took 14.
 // One workgroup of W = ceil(nvec / 16) wavefronts per problem.  The vectors live in LDS (vector j at
 // stride N + 1) in 2 W groups of eight; in each of the 2 W - 1 turns of a sweep a wavefront takes two
 // groups into registers (two components of sixteen vectors per lane), does the 64 rotations between
@@ -540,7 +543,7 @@ __device__ __forceinline__ void rr_pair(int t, int round, int p, int &i, int &j)
 // block and the eigenvectors replayed from a log afterwards) the matrix is touched in LDS once per
 // eight rounds and there is no replay.  It is bound by instruction issue: about 240 instructions of
 // 4 cycles (a lane swap 12) per eight rotations, 8 wavefronts on 4 SIMDs.  MI355X, four 128 x 128
-// problems: blocks of a leg-dim-16 step 3.5 ms -> 1.7 ms, Rayleigh-Ritz matrices of a leg-dim-64 step
+// problems: blocks of a leg-dim-16 step 3.5 ms -> 1.4 ms (1.9 ms from their own columns), Rayleigh-Ritz matrices of a leg-dim-64 step
 // 1.8 ms -> 0.6 ms.
 // A pair is left alone when |x.y| <= 1e-15 |x| |y| or one of the two is below 1e-15 of the largest
 // vector (the rank rule drops values at 1e-14).  A sweep whose rotations all have |x.y| <= 1e-9 |x| |y|
@@ -624,10 +627,93 @@ __device__ __forceinline__ void os_rotate(double (&x)[2], double (&y)[2], double
     }
 }
 
+// X (component r of vector j at X[j * LD + r], len components, N x N with zeros around) <- the lower
+// triangular L of X = L Q, component i of it the one that was `rowof[i]`, by decreasing norm.  Row i
+// stays in the registers of wavefront i % W (its elements over the lanes); a step takes the pivot row
+// from LDS (`work`, 3 N values), projects it out of the rows after it and stores L's column, one barrier
+// a step.
+__device__ __forceinline__ void os_lower(double *X, int LD, int N, int W, int len, double *work, int *rowof, int tid, int nt) {
+    const int lane = tid & 63, wave = tid >> 6, nw = nt >> 6;
+    const bool two = N > 64, in0 = lane < N, in1 = two && lane + 64 < N;
+    for (int r = wave; r < N; r += nw) {
+        double a = in0 ? X[lane * LD + r] : 0.0, b = in1 ? X[(lane + 64) * LD + r] : 0.0;
+        a = fma(a, a, b * b);
+        for (int o = 32; o > 0; o >>= 1) a += __shfl_xor(a, o, 64);
+        if (lane == 0) work[r] = a;
+    }
+    __syncthreads();
+    for (int e = tid; e < N; e += nt) {  // ties, and the zero rows from len on, by index
+        const double ke = work[e];
+        int rank = 0;
+        for (int f = 0; f < N; ++f) {
+            const double kf = work[f];
+            if (kf > ke || (kf == ke && f < e)) ++rank;
+        }
+        rowof[rank] = e;
+    }
+    __syncthreads();
+    double a[16][2];
+    if (wave < W) {
+#pragma unroll
+        for (int q = 0; q < 16; ++q) {
+            const int r = rowof[W * q + wave];
+            a[q][0] = in0 ? X[lane * LD + r] : 0.0;
+            a[q][1] = in1 ? X[(lane + 64) * LD + r] : 0.0;
+        }
+    }
+    double *pivot = work + N;
+    auto publish = [&](int k, const double (&x)[2]) {
+        if (in0) pivot[(k & 1) * N + lane] = x[0];
+        if (in1) pivot[(k & 1) * N + lane + 64] = x[1];
+    };
+    if (wave == 0) publish(0, a[0]);
+    __syncthreads();  // every row is in registers
+    for (int e = tid; e < N * LD; e += nt) X[e] = 0.0;
+#pragma unroll
+    for (int q0 = 0; q0 < 16; ++q0) {
+        for (int w0 = 0; w0 < W && W * q0 + w0 < len; ++w0) {
+            const int k = W * q0 + w0;
+            __syncthreads();  // pivot k is there; the other buffer's readers are done
+            if (wave < W) {
+                const double *pk = pivot + (k & 1) * N;
+                const double p0 = in0 ? pk[lane] : 0.0, p1 = in1 ? pk[lane + 64] : 0.0;
+                double v[8];
+#pragma unroll
+                for (int q = 1; q < 8; ++q) v[q] = 0.0;
+                v[0] = fma(p0, p0, p1 * p1);
+                const double pp = lane_read(reduce8(v, lane), 0);
+                // a row that is zero, or whose square underflows, has nothing to project out
+                const double rs = pp > 1e-290 ? rsqrt_nr(pp) : 0.0, inv = rs * rs;
+#pragma unroll
+                for (int h = q0 / 8; h < 2; ++h) {
+#pragma unroll
+                    for (int q = 0; q < 8; ++q) v[q] = fma(a[8 * h + q][0], p0, a[8 * h + q][1] * p1);
+                    const double d = reduce8(v, lane), c = d * inv;
+                    const int i = W * (8 * h + (lane >> 3)) + wave;
+                    if ((lane & 7) == 0 && i >= k) X[k * LD + i] = d * rs;
+#pragma unroll
+                    for (int q = 0; q < 8; ++q) {
+                        if (8 * h + q < q0) continue;
+                        const double cq = lane_read(c, 8 * q);
+                        a[8 * h + q][0] = fma(-cq, p0, a[8 * h + q][0]);
+                        a[8 * h + q][1] = fma(-cq, p1, a[8 * h + q][1]);
+                    }
+                }
+                if (w0 + 1 < W) {
+                    if (wave == w0 + 1) publish(k + 1, a[q0]);
+                } else if (q0 < 15) {
+                    if (wave == 0) publish(k + 1, a[q0 < 15 ? q0 + 1 : 15]);
+                }
+            }
+        }
+    }
+    __syncthreads();
+}
+
 __global__ void __launch_bounds__(512) k_jacobi_onesided(OsArgs A) {
     HIP_DYNAMIC_SHARED(double, sm)
     __shared__ double red[16];
-    __shared__ int order[kOsMax];
+    __shared__ int order[kOsMax], rowof[kOsMax];
     __shared__ int active;
     int gi = 0;
     while (gi + 1 < A.n && (int)blockIdx.x >= A.start[gi + 1]) ++gi;
@@ -637,6 +723,7 @@ __global__ void __launch_bounds__(512) k_jacobi_onesided(OsArgs A) {
     double *out = E.out + bi * E.dout;
     const int nvec = E.nvec, len = E.len, p = E.p;
     const int W = (nvec + 15) / 16, N = 16 * W, LD = N + 1;  // len <= N
+    const int Wv = E.direct ? (len + 15) / 16 : W;           // 16 Wv vectors are left to rotate
     double *X = sm;              // vector j at X + j * LD
     double *nrm = sm + N * LD;   // squared norms (the Cholesky's diagonal tiles before)
     const int tid = threadIdx.x, nt = blockDim.x, lane = tid & 63, wave = tid >> 6, nw = nt >> 6;
@@ -684,7 +771,10 @@ __global__ void __launch_bounds__(512) k_jacobi_onesided(OsArgs A) {
         }
         for (int i = 16 + wave; i < N; i += nw)
             for (int j = lane; j < i / 16 * 16; j += 64) X[i * LD + j] = 0.0;
+        for (int i = tid; i < N; i += nt) rowof[i] = i;
         __syncthreads();
+    } else {
+        os_lower(X, LD, N, W, len, nrm, rowof, tid, nt);
     }
     // squared norms into nrm, the vectors by decreasing norm (ties by index) into order
     const bool two = len > 64;
@@ -710,10 +800,10 @@ __global__ void __launch_bounds__(512) k_jacobi_onesided(OsArgs A) {
     rank_vectors();
     double zero = 1e-30 * nrm[order[0]];
     // ---- sweeps
-    const int nblk = 2 * W, g = lane >> 3;
+    const int nblk = 2 * Wv;
     for (int sweep = 0; sweep < kMaxSweeps; ++sweep) {
         for (int turn = 0; turn < nblk - 1; ++turn) {
-            if (wave < W) {
+            if (wave < Wv) {
                 int bi0, bj0;
                 rr_pair(wave, turn, nblk, bi0, bj0);
                 double xa[8][2], xb[8][2];
@@ -816,7 +906,7 @@ __global__ void __launch_bounds__(512) k_jacobi_onesided(OsArgs A) {
         const int j = order[c];
         // vectors that no rotation made orthogonal (below the zero rule) are not directions
         const double f = nrm[j] > 1e-29 * nrm[order[0]] ? 1.0 / sqrt(nrm[j]) : 0.0;
-        for (int r = wave; r < len; r += nw) out[r * p + c] = X[j * LD + r] * f;
+        for (int r = wave; r < len; r += nw) out[rowof[r] * p + c] = X[j * LD + r] * f;
     }
 }
 

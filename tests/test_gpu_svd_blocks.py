@@ -60,6 +60,23 @@ def test_small_blocks_of_low_rank(m, n, r):
     assert np.all(outs[0][1].numpy()[r:] == 0.0)
 
 
+@pytest.mark.parametrize("m,n", [(3, 128), (16, 100), (17, 128), (100, 17), (64, 65), (128, 128)])
+def test_small_blocks_with_zero_repeated_and_graded_rows(m, n):
+    """Shorter sides well below the longer one, rows graded over ten decades in no order, rows of zeros and
+    rows that repeat: what the triangular factor of a small block is built from."""
+    rng = np.random.default_rng(100 * m + n)
+    M = rng.standard_normal((m, n)) * 10.0 ** rng.uniform(-10, 0, m)[:, None]
+    M[m // 2] = 0.0
+    M[m - 1] = M[0]
+    r = m - 2 if m <= n else n
+    outs, counts = _run([(M, min(m, n))])
+    assert counts[0] == r
+    u, s, v = (x.numpy() for x in outs[0][:3])
+    ref = np.linalg.svd(M, compute_uv=False)
+    np.testing.assert_allclose(s, ref, rtol=0, atol=1e-13 * ref[0])
+    np.testing.assert_allclose((u * s) @ v, M, rtol=0, atol=1e-13 * ref[0])
+
+
 def test_small_blocks_scaled_and_repeated():
     """Entries far from one in magnitude, and values that coincide (a scaled orthogonal block)."""
     rng = np.random.default_rng(5)
