@@ -593,21 +593,55 @@ __global__ void k_split_sum(const T *__restrict__ W, int splits, int M, int N, i
 }
 
 // Split-K workspace: one grow-only buffer per device.  Launches on one stream are ordered; a launch
-// on another stream first waits for the event recorded after the buffer's last use.
+// on another stream first waits for the event recorded after the buffer's last use (or, inside a
+// SplitScope, after the scope's last use).
 struct SplitWs {
     void *p = nullptr;
     size_t bytes = 0;
     hipStream_t last = nullptr;
     hipEvent_t done = nullptr;
     bool used = false;
+    bool pending = false;  // used since the event was recorded (only while a SplitScope holds the lock)
 };
 static std::mutex g_ws_mu;
 static std::map<int, SplitWs> g_ws;
+static thread_local bool t_scope = false;          // this thread holds g_ws_mu through a SplitScope
+static thread_local SplitWs *t_scope_ws = nullptr;  // with uses that wait for their event
+
+static int split_done(SplitWs &w) {
+    w.pending = false;
+    GTN_CHECK_HIP(hipEventRecord(w.done, w.last));
+    return GTN_OK;
+}
+
+SplitScope::SplitScope() : outer_(t_scope) {
+    if (outer_) return;
+    g_ws_mu.lock();
+    t_scope = true;
+}
+
+int SplitScope::finish() {
+    if (!open_) return GTN_OK;
+    open_ = false;
+    if (outer_) return GTN_OK;
+    int rc = GTN_OK;
+    if (t_scope_ws && t_scope_ws->pending) rc = split_done(*t_scope_ws);
+    t_scope_ws = nullptr;
+    t_scope = false;
+    g_ws_mu.unlock();
+    return rc;
+}
 
 static std::vector<void *> g_ws_retired;  // outgrown workspaces a graph may still hold
 
 static int split_workspace(SplitWs &w, size_t bytes, hipStream_t s) {
-    if (w.used && w.last != s) GTN_CHECK_HIP(hipStreamWaitEvent(s, w.done, 0));
+    if (w.used && w.last != s) {
+        if (w.pending) {
+            int rc = split_done(w);
+            if (rc) return rc;
+        }
+        GTN_CHECK_HIP(hipStreamWaitEvent(s, w.done, 0));
+    }
     if (w.bytes < bytes) {
         if (w.p) {
             if (graphs_alive() || capture_open()) {
@@ -876,9 +910,11 @@ static int gemm_grouped_impl(const gtn_gemm_desc *groups, int n_groups, int dtyp
                 } else {
                     int dev;
                     GTN_CHECK_HIP(hipGetDevice(&dev));
-                    lk.lock();
+                    if (!t_scope) lk.lock();
                     ws = &g_ws[dev];
-                    int rc = split_workspace(*ws, (size_t)need * es, s);
+                    int rc = GTN_OK;
+                    if (t_scope_ws && t_scope_ws != ws && t_scope_ws->pending) rc = split_done(*t_scope_ws);  // another device
+                    if (!rc) rc = split_workspace(*ws, (size_t)need * es, s);
                     if (rc) return rc;
                     base_ws = (char *)ws->p;
                 }
@@ -921,9 +957,15 @@ static int gemm_grouped_impl(const gtn_gemm_desc *groups, int n_groups, int dtyp
                 GTN_CHECK_LAUNCH();
             }
             if (ws) {
-                GTN_CHECK_HIP(hipEventRecord(ws->done, s));
                 ws->last = s;
                 ws->used = true;
+                if (t_scope) {
+                    ws->pending = true;
+                    t_scope_ws = ws;
+                } else {
+                    int rcd = split_done(*ws);
+                    if (rcd) return rcd;
+                }
             }
         }
     }

@@ -2560,5 +2560,8 @@ extern "C" int gtn_svd_blocks(const gtn_svd_block *blocks, int n_blocks, const g
         plan_block(b, *opts, bs[i], (double *)base);
         base += bs[i].bytes;
     }
-    return run_blocks(bs, *opts, as_stream(stream));
+    SplitScope scope;
+    const int rc = run_blocks(bs, *opts, as_stream(stream));
+    const int rc2 = scope.finish();
+    return rc ? rc : rc2;
 }
