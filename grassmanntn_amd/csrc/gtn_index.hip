@@ -818,20 +818,40 @@ struct OddArgs {
     int32_t ndim;
     uint32_t dims[GTN_PERM_MAX_AX];
     int32_t ferm_mask, pp_mask;
+    uint64_t parity;  // MASK: the parity of an entry is that of these bits of its flat index
 };
-template <typename T>
+template <typename I>
+__device__ __forceinline__ uint32_t odd_entry(const OddArgs &a, I r) {
+    uint32_t par = 0;
+    for (int ax = a.ndim - 1; ax >= 0; --ax) {
+        const I d = (I)a.dims[ax], k = r % d;
+        r /= d;
+        if ((a.ferm_mask >> ax) & 1) par ^= ((a.pp_mask >> ax) & 1) ? (uint32_t)(k & 1) : (popc64(k) & 1u);
+    }
+    return par;
+}
+// Sum of squares of the odd entries, V of them per 16-byte load.  A read of the whole tensor, and bound by
+// that where every axis up to the last fermionic one is a power of two (MASK: fermionic legs always are, so
+// only a bosonic leg behind one is not): a 64 x 64 x 64 x 64 tensor takes 27 us, with an index
+// division an axis and 8-byte loads 54 for two axes.
+template <typename T, int V, bool MASK>
 __global__ void k_odd_partial(OddArgs a, const T *__restrict__ x, int64_t n, double *part) {
     __shared__ double sh[16];
+    struct alignas(V * sizeof(T)) Vec {
+        T v[V];
+    };
     double acc = 0;
-    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
-        uint64_t r = (uint64_t)i;
-        uint32_t par = 0;
-        for (int ax = a.ndim - 1; ax >= 0; --ax) {
-            uint64_t k = r % a.dims[ax];
-            r /= a.dims[ax];
-            if ((a.ferm_mask >> ax) & 1) par ^= ((a.pp_mask >> ax) & 1) ? (uint32_t)(k & 1) : (popc64(k) & 1u);
+    const bool narrow = n < ((int64_t)1 << 32);
+#pragma unroll 4
+    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n / V; i += (int64_t)gridDim.x * blockDim.x) {
+        const Vec w = ((const Vec *)x)[i];
+#pragma unroll
+        for (int u = 0; u < V; ++u) {
+            const uint64_t e = (uint64_t)i * V + u;
+            const uint32_t par = MASK ? popc64(e & a.parity) & 1u
+                                      : (narrow ? odd_entry<uint32_t>(a, (uint32_t)e) : odd_entry<uint64_t>(a, e));
+            acc += par ? sq(w.v[u]) : 0.0;
         }
-        if (par) acc += sq(x[i]);
     }
     double t = block_sum(acc, sh);
     if (threadIdx.x == 0) part[blockIdx.x] = t;
@@ -1655,11 +1675,42 @@ int gtn_odd_norm(const void *x, int ndim, const int64_t *dims, const int32_t *fe
     double *part;
     int rc = partial_buffer(s, &part);
     if (rc) return rc;
-    int g = grid_for(n, 256, 1024);
+    bool mask = true;
+    int64_t below = 1;  // entries of the axes behind
+    for (int i = ndim - 1; i >= 0; --i) {
+        const int64_t d = dims[i];
+        const bool pow2 = d > 0 && (d & (d - 1)) == 0;
+        if (!pow2 && (a.ferm_mask & ((2 << i) - 1))) mask = false;
+        if (!mask || !pow2) break;  // (no fermionic axis is left where the last axis read was none)
+        if (ferm[i] && d > 1) a.parity |= pp[i] ? (uint64_t)below : (uint64_t)below * (uint64_t)(d - 1);
+        below *= d;
+    }
+    const int g = grid_for(n, 256, 1024);
+    const dim3 grid(g), blk(256);
+    auto launch = [&](auto *p, auto wide) {
+        using T = std::remove_const_t<std::remove_pointer_t<decltype(p)>>;
+        constexpr int V = decltype(wide)::value;
+        if (mask)
+            hipLaunchKernelGGL((k_odd_partial<T, V, true>), grid, blk, 0, s, a, p, n, part);
+        else
+            hipLaunchKernelGGL((k_odd_partial<T, V, false>), grid, blk, 0, s, a, p, n, part);
+    };
+    const bool al = ((uintptr_t)x & 15) == 0;
+    using one = std::integral_constant<int, 1>;
     switch (dtype) {
-        case GTN_F64: hipLaunchKernelGGL(k_odd_partial<double>, dim3(g), dim3(256), 0, s, a, (const double *)x, n, part); break;
-        case GTN_F32: hipLaunchKernelGGL(k_odd_partial<float>, dim3(g), dim3(256), 0, s, a, (const float *)x, n, part); break;
-        case GTN_C128: hipLaunchKernelGGL(k_odd_partial<double2>, dim3(g), dim3(256), 0, s, a, (const double2 *)x, n, part); break;
+        case GTN_F64:
+            if (al && n % 2 == 0)
+                launch((const double *)x, std::integral_constant<int, 2>{});
+            else
+                launch((const double *)x, one{});
+            break;
+        case GTN_F32:
+            if (al && n % 4 == 0)
+                launch((const float *)x, std::integral_constant<int, 4>{});
+            else
+                launch((const float *)x, one{});
+            break;
+        case GTN_C128: launch((const double2 *)x, one{}); break;
         default: set_error("gtn_odd_norm: unsupported dtype"); return GTN_ENOTSUP;
     }
     GTN_CHECK_LAUNCH();

@@ -1152,34 +1152,25 @@ __global__ void k_sigma(const double *lam, int k, int eig_mode, double *S, doubl
 // elements, element j of vector i at X[i * sv + j * se]) is sigma_i times a unit vector, so
 // sigma_i = ||x_i|| carries FP64 relative accuracy down to ~1e-16 sigma_0 (sqrt of a Gram eigenvalue
 // cannot resolve sigma below ~1e-8 sigma_0).  Then the rank rule of __init__.py:3939-3941 as in
-// k_sigma.  One workgroup of 256 threads (four wavefronts) per block; wavefront w reduces vectors
-// i = w, w + 4, ...
-__global__ void __launch_bounds__(256) k_sigma_norms(const double *X, int k, int64_t len, int64_t sv, int64_t se,
-                                                     double *S, double *inv, double *keep, int64_t dX, int64_t dS,
-                                                     int64_t dw) {
+// k_sigma.  grid (k, blocks): a workgroup reduces its vector and the first one, whose norm the rule
+// needs (one workgroup for all k vectors of a block: 69 us at 32 x 2048, now 5).
+__device__ double wg_norm2(const double *x, int64_t len, int64_t se, double *sh) {
+    double acc = 0.0;
+    for (int64_t j = threadIdx.x; j < len; j += blockDim.x) acc = fma(x[j * se], x[j * se], acc);
+    return wg_sum(acc, sh);
+}
+__global__ void __launch_bounds__(256) k_sigma_norms(const double *X, int64_t len, int64_t sv, int64_t se, double *S, double *inv,
+                                                     double *keep, int64_t dX, int64_t dS, int64_t dw) {
+    __shared__ double sh[4];
     X += blockIdx.y * dX;
-    S += blockIdx.y * dS;
-    inv += blockIdx.y * dw;
-    keep += blockIdx.y * dw;
-    __shared__ double sh[256];  // k <= 256 (checked on the host)
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    for (int i = w; i < k; i += 4) {
-        double acc = 0.0;
-        for (int64_t j = lane; j < len; j += 64) {
-            double x = X[i * sv + j * se];
-            acc = fma(x, x, acc);
-        }
-        for (int o = 32; o > 0; o >>= 1) acc += __shfl_xor(acc, o, 64);
-        if (lane == 0) sh[i] = sqrt(acc);
-    }
-    __syncthreads();
-    const double s0 = sh[0];
-    for (int i = threadIdx.x; i < k; i += blockDim.x) {
-        double s = sh[i];
-        bool kp = fabs(s / (s0 + 1e-14)) > 1e-14;
-        S[i] = (s != s) ? s : (kp ? s : 0.0);
-        inv[i] = kp ? 1.0 / s : 0.0;
-        keep[i] = kp ? 1.0 : 0.0;
+    const int i = blockIdx.x;
+    const double first = wg_norm2(X, len, se, sh);
+    const double s = sqrt(i ? wg_norm2(X + i * sv, len, se, sh) : first), s0 = sqrt(first);
+    if (threadIdx.x == 0) {
+        const bool kp = fabs(s / (s0 + 1e-14)) > 1e-14;
+        S[blockIdx.y * dS + i] = (s != s) ? s : (kp ? s : 0.0);
+        inv[blockIdx.y * dw + i] = kp ? 1.0 / s : 0.0;
+        keep[blockIdx.y * dw + i] = kp ? 1.0 : 0.0;
     }
 }
 __global__ void k_scale_rows(double *X, int k, int64_t n, int64_t ld, const double *f, int64_t dX, int64_t df) {
@@ -2471,11 +2462,11 @@ static int run_blocks(std::vector<Blk> &blocks, const gtn_svd_opts &o, hipStream
             R8N(f.keep, k, r.dws, r.n, "keep");
             if (f.small && !f.left) {
                 R8N(B.U, ext(B.m, k, B.ldu), r.dU, r.n, "U");
-                LAUNCH(k_sigma_norms, dim3(1, r.n), dim3(256), 0, s, (const double *)B.U, (int)k, B.m, (int64_t)1, B.ldu,
+                LAUNCH(k_sigma_norms, dim3((unsigned)k, r.n), dim3(256), 0, s, (const double *)B.U, B.m, (int64_t)1, B.ldu,
                        B.S, f.inv, f.keep, r.dU, r.dS, r.dws);
             } else {
                 R8N(B.Vt, ext(k, B.n, B.ldv), r.dV, r.n, "Vt");
-                LAUNCH(k_sigma_norms, dim3(1, r.n), dim3(256), 0, s, (const double *)B.Vt, (int)k, B.n, B.ldv, (int64_t)1,
+                LAUNCH(k_sigma_norms, dim3((unsigned)k, r.n), dim3(256), 0, s, (const double *)B.Vt, B.n, B.ldv, (int64_t)1,
                        B.S, f.inv, f.keep, r.dV, r.dS, r.dws);
             }
         }
