@@ -24,7 +24,7 @@ from . import _lib as L
 from . import core
 from ._device import DeviceArray
 from ._perm import Perm
-from ._plan import fresh_char, parse_partition
+from ._plan import HYBRID, fresh_char, parse_partition
 from .core import dense, einsum, join_legs, split_legs, precision, settings
 
 
@@ -151,16 +151,27 @@ def svd_batch(calls, cutoff):
     for j in jobs:
         P, m, n, mh, nh, d = j["P"], j["m"], j["n"], j["mh"], j["nh"], j["d"]
         T, left, right, z = j["T"], j["left"], j["right"], j["z"]
-        U = _interleave_batch(j["SU"], P, m, 2 * d, row_stride=d, par_stride=mh * d, batch_stride=2 * mh * d)
-        V = _interleave_batch(j["SV"], P, 2 * d, n, row_stride=nh, par_stride=d * nh, batch_stride=2 * d * nh)
         S = DeviceArray.empty((P, 2 * d, 2 * d))
         L.check(lib.gtn_diag_interleave(L.ptr(S), P, d, L.ptr(j["sv"]), L.GTN_F64, L.stream_ptr()),
                 "gtn_diag_interleave")
-        s0, s1 = j["mstats"][1], j["mstats"][2]
-        U, S, V = _mk(U, (0, s0, 1)), _mk(S, (0, -1, 1)), _mk(V, (0, -1, s1))
         nl = len(left)
         xstats, xshape = T.statistics[1:], T.shape[1:]
         nc = fresh_char(left + right + z)
+        ustats, vstats = (0,) + tuple(xstats[:nl]) + (1,), (0, -1) + tuple(xstats[nl:])
+        if j["G"] is not None and HYBRID not in T.statistics:
+            GU = core._factor_plan("(%s)(%s)%s" % (z, left, nc), ustats, (P,) + tuple(xshape[:nl]) + (2 * d,), (0, -1, 1),
+                                   T.encoder, T.format)
+            GV = core._factor_plan("(%s)%s(%s)" % (z, nc, right), vstats, (P, 2 * d) + tuple(xshape[nl:]), (0, -1, 1),
+                                   T.encoder, T.format)
+            if GU is not None and GV is not None:
+                out.append((core._factor(T, GU.run(j["SU"]), ustats),
+                            core._factor(T, core._switched_diagonal(T, S, (0, -1, 1)), (0, -1, 1)),
+                            core._factor(T, GV.run(j["SV"]), vstats)))
+                continue
+        U = _interleave_batch(j["SU"], P, m, 2 * d, row_stride=d, par_stride=mh * d, batch_stride=2 * mh * d)
+        V = _interleave_batch(j["SV"], P, 2 * d, n, row_stride=nh, par_stride=d * nh, batch_stride=2 * d * nh)
+        s0, s1 = j["mstats"][1], j["mstats"][2]
+        U, S, V = _mk(U, (0, s0, 1)), _mk(S, (0, -1, 1)), _mk(V, (0, -1, s1))
         U = split_legs(U, "(%s)(%s)%s" % (z, left, nc), (0,) + tuple(xstats[:nl]) + (1,),
                        (P,) + tuple(xshape[:nl]) + (2 * d,), intermediate_stat=(0, -1, 1))
         S = S.switch_encoder()

@@ -576,15 +576,19 @@ def is_grassmann_even(T):
     from .block import block
     if isinstance(T, block):
         return T.is_even()
-    lib = L.lib()
+    return float(_odd_norm_dev(T).item()) == 0.0
+
+
+def _odd_norm_dev(T):
+    """Squared norm of T's entries of odd total fermionic parity, left on the device."""
     nd = T.ndim
     dims = (C.c_int64 * max(nd, 1))(*T.shape)
     fer = (C.c_int32 * max(nd, 1))(*[1 if s in FERMI else 0 for s in T.statistics])
     pp = (C.c_int32 * max(nd, 1))(*[1 if T.encoder == "parity-preserving" else 0] * nd)
     out = DeviceArray.empty(1, np.float64)
-    L.check(lib.gtn_odd_norm(L.ptr(T.data), nd, dims, fer, pp, L.dtype_code(T.data), L.ptr(out), L.stream_ptr()),
+    L.check(L.lib().gtn_odd_norm(L.ptr(T.data), nd, dims, fer, pp, L.dtype_code(T.data), L.ptr(out), L.stream_ptr()),
             "gtn_odd_norm")
-    return float(out.item()) == 0.0
+    return out
 
 
 def _relayout(T, order, out_encoder, sigma=None, parity_lin=None, table_chars=None, codes=None, alpha=1.0):
@@ -1266,10 +1270,10 @@ def join_legs(T, string_inp, make_format="standard", intermediate_stat=None, sav
 
 def _join_gather(T, string_inp, make_format="standard", intermediate_stat=None, blocks=False):
     """The gather of join_legs: (Perm, source data, fused shape, fused statistics).  With blocks=True
-    (a bosonic first group, then two purely fermionic groups: the batched matrices M[b] of a
-    decomposition) the gather writes the two parity blocks M[b][p::2, p::2] instead, as a
-    (B, 2, m/2, n/2) array (BlockSVD's ME / MO, __init__.py:3990-3996): the parity p is an output axis
-    of its own feeding both fused legs."""
+    (two groups with fermionic legs, the matrix of a decomposition, after a bosonic first group where
+    there are three, a batch of them) the gather writes the two parity blocks M[b][p::2, p::2] instead,
+    as a (B, 2, m/2, n/2) array (BlockSVD's ME / MO, __init__.py:3990-3996): the parity p is an output
+    axis of its own feeding both fused legs."""
     inter = tuple(intermediate_stat) if not np.isscalar(intermediate_stat) else (intermediate_stat,)
     through = None
     if isinstance(T, _PermutedView) and T._data is None:
@@ -1304,11 +1308,11 @@ def _join_plan(string_inp, T, make_format, inter, blocks, through):
     bitpos = {p: k for k, p in enumerate(bit_axes)}
     fin_shape, fin_stats = [], []
     if blocks:
-        ok = (len(srt) == 3 and info[0][3] == 0 and all(info[g][2] == 0 and info[g][3] and info[g][1] % 2 == 0
-                                                          for g in (1, 2)))
+        ok = (len(srt) in (2, 3) and (len(srt) == 2 or info[0][3] == 0)
+              and all(info[g][3] and info[g][1] % 2 == 0 and inter[g] in FERMI for g in (-2, -1)))
         if not ok:
-            raise ValueError("_join_gather: blocks=True needs a bosonic group and two fermionic groups")
-        fvirt = []
+            raise ValueError("_join_gather: blocks=True needs two groups with fermionic legs")
+        halves = []  # (virtual axes of the bosons and the fermions, their sizes) of the two groups
     for g, (chars, stg, dm, pos) in enumerate(srt):
         bd, fd, bn, fn, final = info[g]
         # the fused leg: bosons (high) then fermions; the fermionic part is switched to the
@@ -1323,19 +1327,17 @@ def _join_plan(string_inp, T, make_format, inter, blocks, through):
                 if t in FERMI:
                     P.add_comp(vf, d, [(ins[p], 1)], bit=bitpos.get(p, -1))
             # two raw axes (boson high, fermion low) whose C-order product is the fused leg
-            P.add_out(bd, [(vb, 1)])
-            P.add_out(fd, [(vf, 1)])
+            if blocks:
+                halves.append((vb, bd, vf, fd))
+            else:
+                P.add_out(bd, [(vb, 1)])
+                P.add_out(fd, [(vf, 1)])
         elif fn:
             vf = P.add_virt(fd, enc=inter[g] in FERMI, sigma=(make_format == "matrix" and inter[g] == -1))
             for t, d, p in zip(stg, dm, pos):
                 P.add_comp(vf, d, [(ins[p], 1)], bit=bitpos.get(p, -1))
             if blocks:
-                fvirt.append((vf, fd))
-                if len(fvirt) == 2:  # (parity, row / 2, column / 2): index = 2 half + parity
-                    (vr, mr), (vc, nc) = fvirt
-                    P.add_out(2, [(vr, 1), (vc, 1)])
-                    P.add_out(mr // 2, [(vr, 2)])
-                    P.add_out(nc // 2, [(vc, 2)])
+                halves.append((-1, 1, vf, fd))
             else:
                 P.add_out(fd, [(vf, 1)])
         else:
@@ -1347,6 +1349,12 @@ def _join_plan(string_inp, T, make_format, inter, blocks, through):
             P.add_out(bd, [(vb, 1)])
         fin_shape.append(bd * fd)
         fin_stats.append(final)
+    if blocks:  # (parity, row / 2, column / 2): fermionic index = 2 half + parity
+        P.add_out(2, [(halves[0][2], 1), (halves[1][2], 1)])
+        for vb, bd, vf, fd in halves:
+            if vb >= 0:
+                P.add_out(bd, [(vb, 1)])
+            P.add_out(fd // 2, [(vf, 2)])
     if nb:
         table = []
         for m in range(1 << nb):
@@ -1420,8 +1428,16 @@ def _split_plan(string_inp, T, final_stat, final_shape, inter):
 # --------------------------------------------------------------------------------------------------
 # svd / eig (__init__.py:3931-4698)
 # --------------------------------------------------------------------------------------------------
+class _Joined(NamedTuple):
+    """The matrix of a decomposition, not written as such: `gather` writes its two parity blocks from `src`."""
+    gather: Perm
+    src: DeviceArray
+    shape: tuple
+    dtype: object
+
+
 def _block_prepare(Mdata, cutoff, rule="dense"):
-    """Parity blocks ME, MO of a parity-preserving (-1,+1) matrix and the number of values to compute
+    """Parity blocks ME, MO of a parity-preserving (-1,+1) matrix (an array or a _Joined) and the number of values to compute
     in each: int(cutoff/2) per block (BlockSVD / BlockEig, __init__.py:3953-4029, 4347-4422), or
     ceil(cutoff/2) even and floor(cutoff/2) odd with rule="block" (decompose_block,
     __init__.py:5076-5085)."""
@@ -1442,30 +1458,111 @@ def _block_prepare(Mdata, cutoff, rule="dense"):
 
 
 def _block_assemble(outs, kk, m, n, dt, kept=None):
-    """Full interleaved (U, S, Vt) from the two blocks' results, both padded to the next power of two
-    of the larger kept count kk (the rank rule of SortedSVD: the nonzero values read back);
-    `kept` (a list) receives that count."""
+    """(U of both blocks, (2, m / 2, d); V of both, (2, d, n / 2); the interleaved diagonal S (2 d, 2 d); d)
+    from the two blocks' results, both padded to the next power of two d of the larger kept count kk
+    (the rank rule of SortedSVD: the nonzero values read back); `kept` (a list) receives that count.
+    Where nothing is padded and the two results follow each other, they are the stacks already."""
     d = max(kk)
     if kept is not None:
         kept.append(d)
     d = int(2 ** math.ceil(math.log2(d))) if d > 0 else 1
     mh, nh = m // 2, n // 2
-    # stack the kept columns / rows of both blocks, zero-padded to d, then interleave by parity
+    S = DeviceArray.zeros((2 * d, 2 * d), dt)
+    for par, (U_b, S_b, V_b, k) in enumerate(outs):
+        if kk[par]:  # S[2j + par, 2j + par] = s_par[j]
+            copy2d(S, 2 * (2 * d + 1), S_b, 1, kk[par], 1, dst_off=par * (2 * d + 1))
+    (U0, _, V0, k0), (U1, _, V1, k1) = outs
+    if kk[0] == kk[1] == k0 == k1 == d and _follows(U0, U1) and _follows(V0, V1):
+        return (DeviceArray(U0.storage, U0.offset, (2, mh, d), dt), DeviceArray(V0.storage, V0.offset, (2, d, nh), dt), S, d)
     SU = DeviceArray.zeros((2, mh, d), dt)
     SV = DeviceArray.zeros((2, d, nh), dt)
-    sv = DeviceArray.zeros((2 * d,), dt)
     for par, (U_b, S_b, V_b, k) in enumerate(outs):
         kp = kk[par]
         if kp == 0:
             continue
         copy2d(SU, d, U_b, k, mh, kp, dst_off=par * mh * d)
         copy2d(SV, nh, V_b, n // 2, kp, nh, dst_off=par * d * nh)
-        copy2d(sv, 2, S_b, 1, kp, 1, dst_off=par)  # sv[2j + par] = s_par[j]
-    U = _interleave(SU, m, 2 * d, row_stride=d, par_stride=mh * d)
-    Vt = _interleave(SV, 2 * d, n, row_stride=nh, par_stride=d * nh)
-    S = DeviceArray.zeros((2 * d, 2 * d), dt)
-    copy2d(S, 2 * d + 1, sv, 1, 2 * d, 1)  # the diagonal
-    return U, S, Vt
+    return SU, SV, S, d
+
+
+def _follows(a, b):
+    return a.storage is b.storage and b.offset == a.offset + a.nbytes
+
+
+@_planned
+def _factor_plan(string, stats, shape, inter, encoder, fmt):
+    """The gather from stacked parity blocks (..., 2, rows / 2, columns / 2) of a matrix (fermionic legs in
+    the parity-preserving encoder, matrix format) to its legs `string` of `stats` and `shape` in the given
+    encoder and format, odd entries zero: interleaving, split_legs and both switches in one pass.  Groups
+    before the last two are bosonic (a batch).  None where its sign table would be too large."""
+    _, srt = group_info(string, stats, shape)
+    info = _intermediate(srt, inter)
+    fermions = [p for chars, stg, dm, pos in srt[-2:] for t, p in zip(stg, pos) if t in FERMI]
+    if len(fermions) > L.MAX_BITS:
+        return None
+    signed = set(_grouping_sign_axes(srt, inter))
+    P = Perm()
+    hr, hc = (info[g][0] * info[g][1] // 2 for g in (-2, -1))
+    src_of = {}
+    for g, (chars, stg, dm, pos) in enumerate(srt):
+        bd, fd = info[g][0], info[g][1]
+        at = g - len(srt)
+        stride = {-1: 1, -2: hc}.get(at, 2 * hr * hc)  # of the group's half index (a batch: whole index)
+        if at < -2:
+            m = bd
+            i_b = P.add_in(bd, stride)
+        else:
+            m, mf = bd, fd
+            i_b = P.add_in(bd, stride * (fd // 2)) if bd > 1 or info[g][2] else -1
+            i_f = P.add_in(fd, stride, enc=True, sigma=inter[g] == -1, split=True, stride_lo=hr * hc if at == -2 else 0)
+        for t, d, p in zip(stg, dm, pos):
+            if t in BOSE:
+                m //= d
+                src_of[p] = (i_b, m)
+            else:
+                mf //= d
+                src_of[p] = (i_f, mf)
+    bit = {p: k for k, p in enumerate(fermions)}
+    for p, (t, d) in enumerate(zip(stats, shape)):
+        v = P.add_virt(d, enc=encoder == "parity-preserving" and t in FERMI, sigma=fmt == "matrix" and t == -1)
+        P.add_comp(v, d, [src_of[p]], bit=bit.get(p, -1))
+        P.add_out(d, [(v, 1)])
+    flips = sum(1 << bit[p] for p in signed if p in bit)
+    P.set_table([2 if bin(m).count("1") & 1 else bin(m & flips).count("1") & 1 for m in range(1 << len(fermions))])
+    return P
+
+
+def _factors_of_blocks(job, SU, SV, S, d):
+    """(U, S, V) of a blocked decomposition from its stacked parity blocks, or None where the general
+    path has to take it (hybrid legs, whose format cannot be switched, or too many legs for one gather)."""
+    T, left, right = job.T, job.left, job.right
+    nl = len(left)
+    ustats, vstats = tuple(T.statistics[:nl]) + (1,), (-1,) + tuple(T.statistics[nl:])
+    if HYBRID in ustats or HYBRID in vstats or any(h % 2 for h in (job.shape[0], job.shape[1])):
+        return None
+    ushape, vshape = tuple(T.shape[:nl]) + (2 * d,), (2 * d,) + tuple(T.shape[nl:])
+    nc = fresh_char(left + right)
+    GU = _factor_plan("(" + left + ")" + nc, ustats, ushape, (-1, 1), T.encoder, T.format)
+    GV = _factor_plan(nc + "(" + right + ")", vstats, vshape, (-1, 1), T.encoder, T.format)
+    if GU is None or GV is None:
+        return None
+    U, V = GU.run(SU), GV.run(SV)
+    return (_factor(T, U, ustats), _factor(T, _switched_diagonal(T, S, (-1, 1)), (-1, 1)), _factor(T, V, vstats))
+
+
+def _factor(T, data, stats):
+    r = dense.__new__(dense)
+    r.data, r.statistics, r.encoder, r.format, r._even = data, stats, T.encoder, T.format, True
+    return r
+
+
+def _switched_diagonal(T, S, stats):
+    """S (parity-preserving, matrix format) in T's encoder and format."""
+    if T.encoder == "parity-preserving" and T.format == "matrix":
+        return S
+    M = _Legs(tuple(S.shape), stats, "parity-preserving", "matrix")
+    sigma = tuple(t == -1 for t in stats) if T.format == "standard" else None
+    return _relayout_plan(M, tuple(range(len(stats))), T.encoder, sigma, None).run(S)
 
 
 def _interleave(stack, rows, cols, row_stride, par_stride):
@@ -1557,7 +1654,10 @@ def _materialize(specs):
         for j in range(cnt):
             M, par, k = specs[st + j]
             view = buf.flat(j * mh * nh, mh * nh, (mh, nh))
-            _strided_block(M, par, out=view)
+            if not isinstance(M, _Joined):
+                _strided_block(M, par, out=view)
+            elif par == 0:  # the odd block is the next one
+                M.gather.run(M.src, dst=buf.flat(j * mh * nh, 2 * mh * nh, M.gather.out_shape()))
             res.append((view, k))
     return res
 
@@ -1644,7 +1744,7 @@ class _Pending:
 
 class _Job:
     """One svd / eig call in flight: the joined matrix, its blocks and what the split needs."""
-    __slots__ = ("T", "left", "right", "cutoff", "M", "blocks", "blocked", "kept", "done", "leak")
+    __slots__ = ("T", "left", "right", "cutoff", "shape", "mstats", "blocks", "blocked", "kept", "done", "leak")
 
 
 def _decompose_prepare(T, string, cutoff, mode, rule):
@@ -1691,10 +1791,24 @@ def _decompose_prepare(T, string, cutoff, mode, rule):
         job.blocks = []
         return job
     inter = (0 if all(s == 0 for s in sl) else -1, 0 if all(s == 0 for s in sr) else 1)
-    M = join_legs(T, "(" + left + ")(" + right + ")", "matrix", intermediate_stat=inter)
-    M = M.force_encoder("parity-preserving")
-    job.M = M
+    string = "(" + left + ")(" + right + ")"
+    check = not _pkg_flag("skip_parity_blocking_check", False)
+    if 0 not in inter:
+        try:
+            G, src, shape, job.mstats = _join_gather(T, string, "matrix", inter, blocks=True)
+        except ValueError:  # a group without fermionic legs, or of odd fermionic size
+            pass
+        else:
+            # the blocks straight from the tensor; what the parity check sums is the tensor's odd part
+            job.shape, job.blocked = shape, True
+            job.blocks = _block_prepare(_Joined(G, src, shape, src.dtype), cutoff, rule)
+            if check:
+                unread = isinstance(T, _PermutedView) and T._data is None
+                job.leak = (_odd_norm_dev(T._src if unread else T), shape[0], shape[1])
+            return job
+    M = join_legs(T, string, "matrix", intermediate_stat=inter)
     Md = M.data
+    job.shape, job.mstats = Md.shape, M.statistics
     if M.statistics[0] == 0 or M.statistics[1] == 0:
         mm, nn = Md.shape
         k = min(mm, nn) if cutoff is None else min(mm, nn, cutoff)
@@ -1703,20 +1817,19 @@ def _decompose_prepare(T, string, cutoff, mode, rule):
     else:
         job.blocked = True
         job.blocks = _block_prepare(Md, cutoff, rule)
-        if not _pkg_flag("skip_parity_blocking_check", False):
+        if check:
             job.leak = (_parity_leak_dev(Md), Md.shape[0], Md.shape[1])
     return job
 
 
 def _decompose_finish(job, outs, counts):
-    T, M = job.T, job.M
-    Md = M.data
+    T = job.T
     fmt, enc = T.format, T.encoder
     xstats, xshape = T.statistics, T.shape
     left, right = job.left, job.right
     nl = len(left)
     if not job.blocked:
-        mm, nn = Md.shape
+        mm, nn = job.shape
         U_b, S_b, V_b, k = outs[0]
         nz = counts[0]
         U = DeviceArray.zeros((mm, max(nz, 1)), np.float64)
@@ -1727,9 +1840,15 @@ def _decompose_finish(job, outs, counts):
             copy2d(Vt, nn, V_b, nn, nz, nn)
             copy2d(S, nz + 1, S_b, 1, nz, 1)
     else:
-        U, S, Vt = _block_assemble(outs, counts, Md.shape[0], Md.shape[1], Md.dtype, job.kept)
+        SU, SV, S, d = _block_assemble(outs, counts, job.shape[0], job.shape[1], np.float64, job.kept)
+        direct = _factors_of_blocks(job, SU, SV, S, d)
+        if direct is not None:
+            return direct
+        m, n = job.shape
+        U = _interleave(SU, m, 2 * d, row_stride=d, par_stride=m // 2 * d)
+        Vt = _interleave(SV, 2 * d, n, row_stride=n // 2, par_stride=d * (n // 2))
     ls, rs = -1, 1
-    s0, s1 = M.statistics
+    s0, s1 = job.mstats
 
     def mk(data, stats):
         r = dense.__new__(dense)
@@ -1861,11 +1980,21 @@ def power(T, p, rcond=1e-10):
     if isinstance(T, block):
         return power_block(T, p)
     fmt, enc = T.format, T.encoder
-    M = T.force_format("matrix").force_encoder("canonical")
+    M = _converted(T, "canonical", "matrix")
     lib = L.lib()
     L.check(lib.gtn_power_diag(L.ptr(M.data), M.data.numel(), 1, L.dtype_code(M.data), float(p), float(rcond),
                                L.stream_ptr()), "gtn_power_diag")
-    return M.force_format(fmt).force_encoder(enc)
+    return _converted(M, enc, fmt)
+
+
+def _converted(T, encoder, fmt):
+    """T.force_format(fmt).force_encoder(encoder) in one pass."""
+    if T.format == fmt or T.encoder == encoder:
+        return T.force_format(fmt) if T.encoder == encoder else T.force_encoder(encoder)
+    if HYBRID in T.statistics:
+        return T.switch_format()  # raises
+    out = _relayout(T, range(T.ndim), out_encoder=encoder, sigma=[s == -1 for s in T.statistics])
+    return T._like(out, encoder=encoder, format=fmt, even=T._even)
 
 
 def sqrt(T, rcond=1e-10):

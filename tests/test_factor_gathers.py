@@ -1,0 +1,49 @@
+"""The gathers around a decomposition that skip its matrix: parity blocks straight from the tensor, factors
+straight from the stacked blocks, and the odd part of the tensor, against the general path (join_legs and
+strided blocks; interleaving, split_legs and the switches) over legs, orders, encoders and formats."""
+import itertools
+
+import numpy as np
+import pytest
+
+from conftest import random_even
+from kernel_emulator import emulate
+
+# statistics, shape, partition: one and several legs a side, bosons first, last and between, odd bosons
+FORMS = [((1, 1, -1, -1), (4, 2, 4, 2), "ab|cd"), ((1, -1, -1, 1), (2, 4, 4, 4), "a|bcd"),
+         ((0, 1, -1, 0, 1), (3, 4, 4, 2, 4), "abc|de"), ((1, 0, -1, -1, 0, 0, 1), (4, 3, 2, 2, 2, 3, 4), "abcd|efg"),
+         ((-1, 1), (8, 8), "a|b"), ((1, 0, 0, -1), (2, 5, 3, 4), "ab|cd")]
+
+
+@pytest.mark.parametrize("form", range(len(FORMS)))
+def test_factors_and_blocks_match_the_general_path(form, monkeypatch):
+    stats, shape, part = FORMS[form]
+    rng = np.random.default_rng(form)
+    with emulate():
+        import grassmanntn_amd as gtn
+        from grassmanntn_amd import core
+        for enc, fmt, cutoff in itertools.product(("canonical", "parity-preserving"), ("standard", "matrix"), (None, 3, 4)):
+            T = gtn.dense(random_even(rng, shape, stats).data, statistics=stats).force_encoder(enc).force_format(fmt)
+            got = T.svd(part, cutoff)
+            with monkeypatch.context() as m:
+                def refuse(*a, blocks=False, **k):
+                    if blocks:
+                        raise ValueError
+                    return whole(*a, **k)
+                whole = core._join_gather
+                m.setattr(core, "_join_gather", refuse)
+                m.setattr(core, "_factors_of_blocks", lambda *a: None)
+                want = T.svd(part, cutoff)
+            for g, w in zip(got, want):
+                assert (g.statistics, g.encoder, g.format, tuple(g.shape)) == (w.statistics, w.encoder, w.format, tuple(w.shape))
+                assert np.array_equal(g.numpy(), w.numpy()), (stats, enc, fmt, cutoff)
+
+
+@pytest.mark.parametrize("form", range(len(FORMS)))
+def test_odd_tensors_are_refused(form):
+    stats, shape, part = FORMS[form]
+    with emulate():
+        import grassmanntn_amd as gtn
+        T = gtn.dense(np.random.default_rng(1).standard_normal(shape), statistics=stats)
+        with pytest.raises(NameError):
+            T.svd(part, 4)
