@@ -549,6 +549,15 @@ __device__ __forceinline__ void rr_pair(int t, int round, int p, int &i, int &j)
 // vector (the rank rule drops values at 1e-14).  A sweep whose rotations all have |x.y| <= 1e-9 |x| |y|
 // and angles of at most 1e-8 is the last: what they undo in other pairs is their product.  The vectors
 // are taken by decreasing norm, which saves sweeps.
+// Only `keep` vectors are wanted.  Once a sweep's rotations in the first T = ceil(keep / 8) groups have all
+// had tangents of at most 0.1, the sweeps leave out the pairs without one of these groups: T wavefronts
+// work in a turn, which takes 5.5 us and not 8.7 where they are at most a quarter of the workgroup's (with
+// half of them, 5.5 + the bound below saved nothing: 985 us and 1014 at keep = 32 of 128).  Convergence is
+// linear then, by the cosines left among the others, and the last sweep is one whose rotations all have
+// |x.y| <= 1e-12 |x| |y|.  What is left out must not hide a larger value: the row sums of |x_i.x_j| over
+// the others bound their largest squared value (Gershgorin; 128 x 128 dot products on the matrix cores,
+// 15 us), and where that is above the last wanted one all pairs are rotated again.  keep = 8 of 128, blocks of
+// a leg-dim-16 step: 1.38 ms -> 1.2 ms.
 // ---------------------------------------------------------------------------------------------
 constexpr int kOsMax = 128;    // vectors, and components per vector
 constexpr int kOsEntries = 8;  // geometries per launch
@@ -558,6 +567,7 @@ struct OsEntry {
     int64_t din, dout;     // per-problem strides
     int64_t sv, sc;        // direct: component r of vector j at in[j * sv + r * sc]
     int32_t nvec, len, p;
+    int32_t keep;          // leading vectors wanted; the columns behind them need not be orthogonal
     int32_t direct;        // 0: in is G (p x p), its Cholesky columns are the vectors
 };
 struct OsArgs {
@@ -603,9 +613,10 @@ __device__ __forceinline__ double reduce8(const double (&v)[8], int lane) {
 
 // Sine s, half-angle tangent h and tangent t of the rotation that makes two vectors with squared norms
 // al, be and dot product g orthogonal: all 0 when they count as orthogonal.  coarse: the rotation may
-// leave other pairs further from orthogonal than the next sweep's threshold.
+// leave other pairs further from orthogonal than the next sweep's threshold (cosine squared above fine_g or
+// tangent above fine_t); steep: its tangent is above 0.1.
 __device__ __forceinline__ void os_angle(double al, double be, double g, double zero, double &s, double &h, double &t,
-                                         bool &coarse) {
+                                         double fine_g, double fine_t, bool &coarse, bool &steep) {
     const double gg = g * g, ab = al * be;
     const bool rot = gg > 1e-30 * ab && al > zero && be > zero;
     const double d = be - al, g2 = rot ? 2.0 * g : 1.0;
@@ -615,7 +626,8 @@ __device__ __forceinline__ void os_angle(double al, double be, double g, double 
     t = rot ? tt : 0.0;
     s = rot ? c * tt : 0.0;
     h = s * rcp_nr(1.0 + c);
-    coarse = coarse || (rot && (gg > 1e-18 * ab || fabs(tt) > 1e-8));
+    coarse = coarse || (rot && (gg > fine_g * ab || fabs(tt) > fine_t));
+    steep = steep || (rot && fabs(tt) > 0.1);
 }
 // (x, y) <- (c x - s y, s x + c y) as three shears, h = s / (1 + c): in place, three multiply-adds
 __device__ __forceinline__ void os_rotate(double (&x)[2], double (&y)[2], double s, double h) {
@@ -714,7 +726,7 @@ __global__ void __launch_bounds__(512) k_jacobi_onesided(OsArgs A) {
     HIP_DYNAMIC_SHARED(double, sm)
     __shared__ double red[16];
     __shared__ int order[kOsMax], rowof[kOsMax];
-    __shared__ int active;
+    __shared__ int active, steep_any;  // a sweep's coarse rotations; its steep ones in the leading groups
     int gi = 0;
     while (gi + 1 < A.n && (int)blockIdx.x >= A.start[gi + 1]) ++gi;
     const OsEntry &E = A.e[gi];
@@ -751,7 +763,7 @@ __global__ void __launch_bounds__(512) k_jacobi_onesided(OsArgs A) {
     bad = wg_sum(bad, red);
     for (int o = 32; o > 0; o >>= 1) mx = fmax(mx, __shfl_xor(mx, o, 64));
     if (lane == 0) red[wave] = mx;
-    if (tid == 0) active = 0;
+    if (tid == 0) active = steep_any = 0;
     __syncthreads();
     mx = 0.0;
     for (int i = 0; i < nw; ++i) mx = fmax(mx, red[i]);
@@ -801,11 +813,52 @@ __global__ void __launch_bounds__(512) k_jacobi_onesided(OsArgs A) {
     double zero = 1e-30 * nrm[order[0]];
     // ---- sweeps
     const int nblk = 2 * Wv;
+    const int T = (E.keep + 7) / 8;
+    bool can_part = 4 * T <= Wv, part = false;
+    int nparts = 0;
+    // bound of the largest squared value among the vectors behind the leading groups
+    auto others_bound = [&]() {
+        double worst = 0.0;
+        if (wave < Wv) {
+            const int ri = order[16 * wave + (lane & 15)] * LD + (lane >> 4);
+            double sum[4] = {0.0, 0.0, 0.0, 0.0};
+            for (int J = T / 2; J < Wv; ++J) {
+                const int rj = order[16 * J + (lane & 15)] * LD + (lane >> 4);
+                d4 c = {0.0, 0.0, 0.0, 0.0};
+                for (int k = 0; k < N; k += 4) c = __builtin_amdgcn_mfma_f64_16x16x4f64(X[ri + k], X[rj + k], c, 0, 0, 0);
+                const bool in = 16 * J + (lane & 15) >= 8 * T;
+#pragma unroll
+                for (int v = 0; v < 4; ++v) sum[v] += in ? fabs(c[v]) : 0.0;
+            }
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                for (int o = 8; o > 0; o >>= 1) sum[v] += __shfl_xor(sum[v], o, 64);
+                if (16 * wave + (lane >> 4) + 4 * v >= 8 * T) worst = fmax(worst, sum[v]);
+            }
+        }
+        for (int o = 32; o > 0; o >>= 1) worst = fmax(worst, __shfl_xor(worst, o, 64));
+        if (lane == 0) red[wave] = worst;
+        __syncthreads();
+        for (int i = 0; i < nw; ++i) worst = fmax(worst, red[i]);
+        __syncthreads();
+        return worst;
+    };
     for (int sweep = 0; sweep < kMaxSweeps; ++sweep) {
         for (int turn = 0; turn < nblk - 1; ++turn) {
-            if (wave < Wv) {
+            int mine = wave < Wv ? wave : -1;
+            if (part) {  // the wave-th of the turn's pairs with a leading group
+                mine = -1;
+                for (int j = 0, c = 0; j < Wv; ++j) {
+                    int x, y;
+                    rr_pair(j, turn, nblk, x, y);
+                    if (min(x, y) < T && c++ == wave) mine = j;
+                }
+            }
+            if (mine >= 0) {
                 int bi0, bj0;
-                rr_pair(wave, turn, nblk, bi0, bj0);
+                rr_pair(mine, turn, nblk, bi0, bj0);
+                const double fine_g = part ? 1e-24 : 1e-18, fine_t = part ? 1e-11 : 1e-8;
+                bool steep = false, inner = false;
                 double xa[8][2], xb[8][2];
                 int ra[8], rb[8];
 #pragma unroll
@@ -845,7 +898,7 @@ __global__ void __launch_bounds__(512) k_jacobi_onesided(OsArgs A) {
                             y[q + 4] = fma(xb[j][0], xb[j][0], xb[j][1] * xb[j][1]);
                         }
                         double s, h, t;
-                        os_angle(reduce8(w, lane), reduce8(y, lane), reduce8(v, lane), zero, s, h, t, coarse);
+                        os_angle(reduce8(w, lane), reduce8(y, lane), reduce8(v, lane), zero, s, h, t, fine_g, fine_t, coarse, inner);
                         if (!__any(s != 0.0)) continue;
                         any = true;
 #pragma unroll
@@ -856,6 +909,8 @@ __global__ void __launch_bounds__(512) k_jacobi_onesided(OsArgs A) {
                             os_rotate(xb[i], xb[j], lane_read(s, 8 * q + 32), lane_read(h, 8 * q + 32));
                         }
                     }
+                    steep = inner && (lane < 32 ? bi0 : bj0) < T;  // (lanes 0..31 had the first group's pairs)
+                    inner = false;
                     dots(xa, xa, v, 0);
                     na = reduce8(v, lane);
                     dots(xb, xb, v, 0);
@@ -868,7 +923,7 @@ __global__ void __launch_bounds__(512) k_jacobi_onesided(OsArgs A) {
                     dots(xa, xb, v, r);
                     const double gam = reduce8(v, lane);
                     double s, h, t;
-                    os_angle(na, nb, gam, zero, s, h, t, coarse);
+                    os_angle(na, nb, gam, zero, s, h, t, fine_g, fine_t, coarse, inner);
                     na = fma(-t, gam, na);
                     nb = fma(t, gam, nb);
                     nb = __shfl(nb, (lane + 8) & 63, 64);  // the next round's partner sits one lane group on
@@ -890,16 +945,24 @@ __global__ void __launch_bounds__(512) k_jacobi_onesided(OsArgs A) {
                         }
                     }
                     if (__any(coarse) && lane == 0) active = 1;  // every writer stores the same value
+                    if (__any(steep || (inner && min(bi0, bj0) < T)) && lane == 0) steep_any = 1;
                 }
             }
             __syncthreads();
         }
-        const int go = active;
-        rank_vectors();  // (its barriers come before the next write of `active`)
+        const int go = active, steep_left = steep_any;
+        rank_vectors();  // (its barriers come before the next write of the flags)
         zero = 1e-30 * nrm[order[0]];
-        if (tid == 0) active = 0;
+        if (tid == 0) active = steep_any = 0;
         __syncthreads();
-        if (!go) break;
+        if (!go) {
+            if (!part || others_bound() <= nrm[order[E.keep - 1]]) break;
+            part = can_part = false;
+        } else if (part) {
+            if (++nparts == 8) part = can_part = false;
+        } else {
+            part = can_part && !steep_left;
+        }
     }
     // ---- the vectors by decreasing norm, normalised
     for (int c = lane; c < p; c += 64) {
@@ -1153,7 +1216,7 @@ __global__ void k_sigma(const double *lam, int k, int eig_mode, double *S, doubl
 // sigma_i = ||x_i|| carries FP64 relative accuracy down to ~1e-16 sigma_0 (sqrt of a Gram eigenvalue
 // cannot resolve sigma below ~1e-8 sigma_0).  Then the rank rule of __init__.py:3939-3941 as in
 // k_sigma.  grid (k, blocks): a workgroup reduces its vector and the first one, whose norm the rule
-// needs (one workgroup for all k vectors of a block: 69 us at 32 x 2048, now 5).
+// needs (one workgroup for all k vectors of a block: 69 us at 32 x 2048, now 7).
 __device__ double wg_norm2(const double *x, int64_t len, int64_t se, double *sh) {
     double acc = 0.0;
     for (int64_t j = threadIdx.x; j < len; j += blockDim.x) acc = fma(x[j * se], x[j * se], acc);
@@ -1983,6 +2046,7 @@ static int jacobi_onesided(std::vector<Run> &runs, hipStream_t s) {
             const gtn_svd_block &B = f.b;
             OsEntry &e = a.e[a.n];
             e.p = (int)f.p;
+            e.keep = (int)B.k;
             e.out = f.Vs;
             e.dout = r.dws;
             e.direct = f.small;

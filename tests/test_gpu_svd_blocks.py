@@ -77,6 +77,24 @@ def test_small_blocks_with_zero_repeated_and_graded_rows(m, n):
     np.testing.assert_allclose((u * s) @ v, M, rtol=0, atol=1e-13 * ref[0])
 
 
+@pytest.mark.parametrize("k", [1, 8, 9, 16, 24, 32, 33])
+@pytest.mark.parametrize("spectrum", ["flat", "equal", "pairs", "edge", "cluster", "steep", "random"])
+def test_few_values_of_small_blocks(k, spectrum):
+    """Fewer values than half a block has, where the pairs behind them are left out towards the end: spectra
+    without a gap behind the last value wanted, with equal values around it and with large ones hidden
+    in vectors that all have smaller norms."""
+    rng = np.random.default_rng(k)
+    n = 128 if k > 16 else 96
+    s = {"flat": 1.0 - 1e-3 * np.arange(n), "equal": np.ones(n), "pairs": 0.97 ** (np.arange(n) // 2 * 2.0),
+         "edge": np.where(np.arange(n) < k, 1.0, 1.0 - 1e-9), "cluster": np.where(np.arange(n) < k // 2, 1.0, 0.5),
+         "steep": 0.7 ** np.arange(n), "random": np.sort(rng.uniform(0, 1, n))[::-1]}[spectrum]
+    Q, _ = np.linalg.qr(rng.standard_normal((n, n)))
+    R, _ = np.linalg.qr(rng.standard_normal((n, n)))
+    outs, counts = _run([((Q * s) @ R, k), (Q * s, k)])
+    for M, o, c in zip(((Q * s) @ R, Q * s), outs, counts):
+        _check(M, k, o, c)
+
+
 def test_small_blocks_scaled_and_repeated():
     """Entries far from one in magnitude, and values that coincide (a scaled orthogonal block)."""
     rng = np.random.default_rng(5)
