@@ -325,8 +325,14 @@ __global__ void __launch_bounds__(256) k_permute_rows(PermArgs a, TabArgs tb, Ro
         for (int g = 0; g < kTabGroups; ++g) Gc[u][g] = 0;
         uint32_t c = (uint32_t)c0 + threadIdx.x + u * 256;
         for (int ax = last; ax > lead; --ax) {
-            const uint32_t o = ax > lead + 1 ? c & (a.out_dim[ax] - 1) : c;
-            if (ax > lead + 1) c >>= a.out_shift[ax];
+            uint32_t o = c;
+            if (ax > lead + 1 && a.out_shift[ax] >= 0) {
+                o = c & (a.out_dim[ax] - 1);
+                c >>= a.out_shift[ax];
+            } else if (ax > lead + 1) {  // once a lane and column, for all rows
+                o = c % a.out_dim[ax];
+                c /= a.out_dim[ax];
+            }
 #pragma unroll
             for (int g = 0; g < kTabGroups; ++g) Gc[u][g] += o * tb.gmul[ax][g];
         }
@@ -1292,8 +1298,9 @@ static bool tiles_enabled() {
     return on == 1;
 }
 
-// Row walk (k_permute_rows) where some trailing axes -- all but the first of them powers of two, the
-// index within a row is decomposed by shifts -- make rows of whole chunks.  1024-column chunks for
+// Row walk (k_permute_rows) where some trailing axes make rows of whole chunks; a last axis that is no power
+// of two needs three axes and more for that, and a division a column (32^4 x 9 doubles: 64 us by
+// k_permute's walk, 35 by rows).  1024-column chunks for
 // gathers that still fill the device with them (four loads in flight per lane), 256 otherwise.  Each
 // workgroup takes up to 8 rows once there are more than 16 workgroups per compute unit without that.
 static bool plan_rows(const PermArgs &a, const TabArgs &tb, RowArgs &w, int &U) {
@@ -1303,7 +1310,6 @@ static bool plan_rows(const PermArgs &a, const TabArgs &tb, RowArgs &w, int &U) 
         int64_t width = 1;
         for (int ns = 1; ns <= a.n_out; ++ns) {
             const int ax = a.n_out - ns;
-            if (ns > 1 && a.out_shift[ax + 1] < 0) break;
             width *= a.out_dim[ax];
             if (width >= ((int64_t)1 << 32)) break;
             if (width % chunk) continue;
