@@ -21,6 +21,7 @@
 
 namespace gtn {
 
+typedef double d2 __attribute__((ext_vector_type(2)));
 typedef double d4 __attribute__((ext_vector_type(4)));
 typedef float f4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf8 __attribute__((ext_vector_type(8)));
@@ -351,24 +352,27 @@ __global__ void __launch_bounds__(256, IND || TRI ? 2 : 1) k_gemm_fp(GemmArgs ar
 // ------------------------------------------------------------------------------------------------
 // SA / SB: BF16 terms each A / B element is split into (hi, mid, lo); the products of term t of A
 // and term u of B with t + u < max(SA, SB) are accumulated, smallest first.
-constexpr int kBfK = 32;            // reduction per panel: one MFMA
-constexpr int kBfStride = kBfK + 8; // 80-byte rows: the 16 rows of an operand read start in distinct banks
+constexpr int kBfK = 32;             // reduction per panel: one MFMA
+constexpr int kBfStride = kBfK + 8;  // 80-byte rows: the 16 rows of an operand read start in distinct banks
+constexpr int kF64K = 8;  // FP64: reduction per panel, two MFMAs; rows of 80 bytes, likewise
+constexpr int kF64Stride = kF64K + 2;
 
-// One operand's ROWS x 32 panels.  A lane's slot is an octet, 8 consecutive k of one row, kept in the
-// operand's own type and written to LDS as one 16-byte store per term.  Reduction-contiguous operands
+// One operand's ROWS x BK panels in rows.  A lane's slot is V = BK / 4 consecutive k of one row, 16 bytes in
+// LDS, kept in the operand's own type until it is stored.  Reduction-contiguous operands
 // are read 16 bytes a lane (four lanes a row), row-contiguous ones one element a lane, 64 lanes on
 // consecutive rows; panels that leave the operand, and origins or strides that 16-byte loads cannot
 // take, are read element by element with a range check (out of range reads as zero).
-template <typename T, int ROWS>
-struct OctetPanels {
-    static constexpr int NS = ROWS / 64;  // octets per lane (256 lanes, 4 octets a row)
+template <typename T, int ROWS, int BK>
+struct RowPanels {
+    static constexpr int NS = ROWS / 64;  // slots per lane (256 lanes, 4 slots a row)
+    static constexpr int V = BK / 4;
     typedef T vec __attribute__((ext_vector_type(16 / sizeof(T))));
     const T *p;
     int64_t sr, sk;
     int R0, R, K;
     bool kc, wide, rows_in;
-    T reg[NS][8];
-    __device__ __forceinline__ OctetPanels(const T *p_, int64_t sr_, int64_t sk_, int R0_, int R_, int K_)
+    T reg[NS][V];
+    __device__ __forceinline__ RowPanels(const T *p_, int64_t sr_, int64_t sk_, int R0_, int R_, int K_)
         : p(p_), sr(sr_), sk(sk_), R0(R0_), R(R_), K(K_) {
         kc = sk == 1;
         wide = (((uint64_t)p) & 15) == 0 && (sr * (int64_t)sizeof(T)) % 16 == 0;
@@ -380,16 +384,16 @@ struct OctetPanels {
         q = kc ? e % 4 : e / ROWS;
     }
     __device__ __forceinline__ void load(int k0) {
-        const bool inside = rows_in && k0 + kBfK <= K;
+        const bool inside = rows_in && k0 + BK <= K;
 #pragma unroll
         for (int s = 0; s < NS; ++s) {
             int r, q;
             at(s, r, q);
-            const int k = k0 + 8 * q;
-            if (inside && kc && wide) {
+            const int k = k0 + V * q;
+            if (V * sizeof(T) >= 16 && inside && kc && wide) {
                 const vec *src = (const vec *)(p + (int64_t)(R0 + r) * sr + k);
 #pragma unroll
-                for (int t = 0; t < (int)sizeof(T) / 2; ++t) {
+                for (int t = 0; t < V * (int)sizeof(T) / 16; ++t) {
                     const vec v = src[t];
 #pragma unroll
                     for (int u = 0; u < 16 / (int)sizeof(T); ++u) reg[s][t * (16 / sizeof(T)) + u] = v[u];
@@ -397,10 +401,10 @@ struct OctetPanels {
             } else if (inside) {
                 const T *src = p + (int64_t)(R0 + r) * sr + (int64_t)k * sk;
 #pragma unroll
-                for (int t = 0; t < 8; ++t) reg[s][t] = src[t * sk];
+                for (int t = 0; t < V; ++t) reg[s][t] = src[t * sk];
             } else {
 #pragma unroll
-                for (int t = 0; t < 8; ++t) {
+                for (int t = 0; t < V; ++t) {
                     // branch-free: out of range reads element (0, 0), valid for R, K >= 1, and drops it
                     const bool ok = R0 + r < R && k + t < K;
                     const T v = p[ok ? (int64_t)(R0 + r) * sr + (int64_t)(k + t) * sk : (int64_t)0];
@@ -429,6 +433,15 @@ struct OctetPanels {
                 }
                 *(bf8 *)&X[u][r][8 * q] = h;
             }
+        }
+    }
+    __device__ __forceinline__ void store(double (&X)[ROWS][kF64Stride]) const {
+        static_assert(V == 2, "a slot is 16 bytes in LDS");
+#pragma unroll
+        for (int s = 0; s < NS; ++s) {
+            int r, q;
+            at(s, r, q);
+            *(d2 *)&X[r][2 * q] = d2{(double)reg[s][0], (double)reg[s][1]};
         }
     }
 };
@@ -462,8 +475,8 @@ __global__ void __launch_bounds__(256, 2) k_gemm_bf16(GemmArgs args) {
     for (int i = 0; i < TI; ++i)
 #pragma unroll
         for (int j = 0; j < TJ; ++j) acc[i][j] = f4{0, 0, 0, 0};
-    OctetPanels<TIN, BM> pa(A, g.sam, g.sak, m0, g.M, K);
-    OctetPanels<TIN, BN> pb(B, g.sbn, g.sbk, n0, g.N, K);
+    RowPanels<TIN, BM, kBfK> pa(A, g.sam, g.sak, m0, g.M, K);
+    RowPanels<TIN, BN, kBfK> pb(B, g.sbn, g.sbk, n0, g.N, K);
     auto panel_mfma = [&](int buf) {
         bf8 af[SA][TI], bfr[SB][TJ];
 #pragma unroll
@@ -523,6 +536,210 @@ __global__ void __launch_bounds__(256, 2) k_gemm_bf16(GemmArgs args) {
                     double val = alpha * (double)acc[i][j][v];
                     if (beta != 0.0) val += beta * (double)C[o];
                     C[o] = (TIN)val;
+                }
+            }
+}
+
+// RowPanels<T, ROWS, kF64K> where every panel lies inside the operand, within 2^31 bytes of the slab's first
+// element: buffer loads from a scalar resource at the slab's origin, one 32-bit offset a lane and uniform
+// offsets for the slots.  KC: reduction-contiguous on 16-byte boundaries; else row-contiguous (sr == 1).
+template <typename T, int ROWS, bool KC>
+struct InnerRows {
+    static constexpr int NS = ROWS / 64, V = 2;
+    __amdgpu_buffer_rsrc_t rsrc;
+    uint32_t voff, kbytes, slot;
+    int lds;
+    T reg[NS][V];
+    __device__ __forceinline__ InnerRows(const T *p, int64_t sr, int64_t sk, int R0) {
+        const int t = threadIdx.x, r = KC ? t / 4 : t % ROWS, q = KC ? t % 4 : t / ROWS;
+        const uint64_t o = (uint64_t)(p + (int64_t)R0 * sr);
+        const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)o), hi = __builtin_amdgcn_readfirstlane((uint32_t)(o >> 32));
+        rsrc = __builtin_amdgcn_make_buffer_rsrc((void *)(((uint64_t)hi << 32) | lo), (short)0, 0x7fffffff, 0x00020000);
+        voff = (uint32_t)(((int64_t)r * sr + (int64_t)(V * q) * sk) * (int64_t)sizeof(T));
+        kbytes = __builtin_amdgcn_readfirstlane((uint32_t)(sk * (int64_t)sizeof(T)));
+        slot = __builtin_amdgcn_readfirstlane((uint32_t)((KC ? 64 * sr : V * (256 / ROWS) * sk) * (int64_t)sizeof(T)));
+        lds = r * kF64Stride + V * q;
+    }
+    static __device__ __forceinline__ bool fits(const T *p, int64_t sr, int64_t sk, int R0, int R, int K) {
+        return (KC ? sk == 1 && (((uint64_t)p) & 15) == 0 && (sr * (int64_t)sizeof(T)) % 16 == 0 : sr == 1) && R0 + ROWS <= R &&
+               sr >= 0 && sk >= 0 && ((int64_t)(ROWS - 1) * sr + (int64_t)(K - 1) * sk) * (int64_t)sizeof(T) < ((int64_t)1 << 31);
+    }
+    __device__ __forceinline__ void load(int k0) {
+        const uint32_t vo = voff + (uint32_t)k0 * kbytes;
+#pragma unroll
+        for (int s = 0; s < NS; ++s) {
+            if constexpr (KC && V * sizeof(T) >= 16) {
+                typedef unsigned u4v __attribute__((ext_vector_type(4)));
+#pragma unroll
+                for (int h = 0; h < V * (int)sizeof(T) / 16; ++h) {
+                    const u4v x = __builtin_amdgcn_raw_buffer_load_b128(rsrc, (int)(vo + 16 * h), (int)(s * slot), 0);
+                    __builtin_memcpy(&reg[s][h * (16 / sizeof(T))], &x, 16);
+                }
+            } else {
+#pragma unroll
+                for (int t = 0; t < V; ++t) {
+                    if constexpr (sizeof(T) == 8)
+                        reg[s][t] = __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(rsrc, (int)vo, (int)(s * slot + t * kbytes), 0));
+                    else
+                        reg[s][t] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rsrc, (int)vo, (int)(s * slot + t * kbytes), 0));
+                }
+            }
+        }
+    }
+    __device__ __forceinline__ void store(double (&X)[ROWS][kF64Stride]) const {
+#pragma unroll
+        for (int s = 0; s < NS; ++s)
+            *(d2 *)(&X[0][0] + lds + s * (KC ? 64 * kF64Stride : V * (256 / ROWS))) = d2{(double)reg[s][0], (double)reg[s][1]};
+    }
+};
+
+// FP64 products with unbroken matrix work: 16x16x4 MFMA on panels in rows, two LDS buffers, one barrier a
+// panel of eight.  Lane l holds the slot of k = 2 (l / 16), 2 (l / 16) + 1 of its row, one 16-byte read, and the
+// s-th of a panel's two instructions per tile multiplies the s-th of them: the same k in both operands, which
+// is all that the sum asks for.  What fills LDS and registers for the next panels is placed between the matrix
+// instructions (`panel`).  Against k_gemm_fp (panels of 16 stored k by k in one buffer, two barriers and an LDS
+// wait in the open a panel), TFLOP/s on N(0,1) entries: 8192^3 67.5 -> 75.3, two products of 2048^3 61 to 65 ->
+// 71, 32 of 2048 x 128 x 2048 58 to 61 -> 65, nominal peak 78.6 (torch's products beside it 69 to 73 on the
+// square sizes).  Launches that leave most of a compute unit idle wait for memory more often with panels of
+// eight (59 products of 640 x 128 x 640 took 835 us and not 780), and the range finder's epilogue would spill:
+// those stay with k_gemm_fp, and the autotuner times both for the others.  TRI: symmetric products.
+template <typename TIN, int BM, int BN, bool TRI = false>
+__global__ void __launch_bounds__(256, 2) k_gemm_f64_pipe(GemmArgs args) {
+    int gi, b, tm, tn;
+    if (!locate(args, gi, b, tm, tn)) return;
+    const GemmGroup &g = args.g[gi];
+    const int sp = b % g.splits;
+    b /= g.splits;
+    const int kb = sp * g.kchunk;
+    const int K = min(g.K - kb, g.kchunk);
+    const TIN *A = (const TIN *)g.A + b * g.sab + kb * g.sak;
+    const TIN *B = (const TIN *)g.B + b * g.sbb + kb * g.sbk;
+    TIN *C = (TIN *)g.C + b * g.scb + sp * g.scs;
+    __shared__ __attribute__((aligned(16))) double As[2][BM][kF64Stride];
+    __shared__ __attribute__((aligned(16))) double Bs[2][BN][kF64Stride];
+    constexpr int WM = BM / 2, WN = BN / 2, TI = WM / 16, TJ = WN / 16;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int wm = (wave >> 1) * WM, wn = (wave & 1) * WN;
+    const int m0 = tm * BM, n0 = tn * BN;
+    d4 acc[TI][TJ];
+#pragma unroll
+    for (int i = 0; i < TI; ++i)
+#pragma unroll
+        for (int j = 0; j < TJ; ++j) acc[i][j] = d4{0, 0, 0, 0};
+    struct Frag {
+        d2 a[TI], b[TJ];
+    };
+    auto fetch = [&](int buf, Frag &f) {
+#pragma unroll
+        for (int i = 0; i < TI; ++i) f.a[i] = *(const d2 *)&As[buf][wm + 16 * i + lane % 16][2 * (lane / 16)];
+#pragma unroll
+        for (int j = 0; j < TJ; ++j) f.b[j] = *(const d2 *)&Bs[buf][wn + 16 * j + lane % 16][2 * (lane / 16)];
+    };
+    auto multiply = [&](const Frag &f, int s) {  // one of a panel's two instructions per tile
+#pragma unroll
+        for (int i = 0; i < TI; ++i)
+#pragma unroll
+            for (int j = 0; j < TJ; ++j)
+                acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(f.a[i][s], f.b[j][s], acc[i][j], 0, 0, 0);
+    };
+    // One panel, its operands in `f`: the next panel's go to LDS and the one after that is loaded while the
+    // first half of the instructions runs, and after the barrier the next panel's operands are read into
+    // `next` under the second half; the groups put this order between the instructions.  (Buffer `to` was last
+    // read before the barrier of the panel before.)
+    auto panel = [&](auto &pa, auto &pb, const Frag &f, Frag &next, int to, int k2, auto has1, auto has2) {
+        if constexpr (decltype(has1)::value) {
+            pa.store(As[to]);
+            pb.store(Bs[to]);
+        }
+        if constexpr (decltype(has2)::value) {
+            pa.load(k2);
+            pb.load(k2);
+        }
+        multiply(f, 0);
+        if constexpr (decltype(has2)::value) {
+#pragma unroll
+            for (int t = 0; t < TI * TJ; ++t) {
+                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // matrix
+                __builtin_amdgcn_sched_group_barrier(0x200, 1, 0);  // LDS write
+                __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);  // load
+                __builtin_amdgcn_sched_group_barrier(0x002, 3, 0);  // vector
+            }
+        }
+        if constexpr (decltype(has1)::value) {
+            __syncthreads();
+            fetch(to, next);
+        }
+        multiply(f, 1);
+        if constexpr (decltype(has1)::value) {
+#pragma unroll
+            for (int t = 0; t < TI + TJ; ++t) {
+                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // LDS read
+            }
+        }
+    };
+    auto mainloop = [&](auto &&pa, auto &&pb) {
+        constexpr std::true_type yes{};
+        constexpr std::false_type no{};
+        if (K <= 0) return;
+        pa.load(0);
+        pb.load(0);
+        pa.store(As[0]);
+        pb.store(Bs[0]);
+        if (K > kF64K) {
+            pa.load(kF64K);
+            pb.load(kF64K);
+        }
+        __syncthreads();
+        Frag f0, f1;
+        fetch(0, f0);
+        int k0 = 0;
+        for (; k0 + 3 * kF64K < K; k0 += 2 * kF64K) {  // two panels a turn: neither set of operands is copied
+            panel(pa, pb, f0, f1, 1, k0 + 2 * kF64K, yes, yes);
+            panel(pa, pb, f1, f0, 0, k0 + 3 * kF64K, yes, yes);
+        }
+        // one to three panels are left, the first of them in f0
+        if (k0 + 2 * kF64K < K) {
+            panel(pa, pb, f0, f1, 1, k0 + 2 * kF64K, yes, yes);
+            panel(pa, pb, f1, f0, 0, 0, yes, no);
+            panel(pa, pb, f0, f1, 1, 0, no, no);
+        } else if (k0 + kF64K < K) {
+            panel(pa, pb, f0, f1, 1, 0, yes, no);
+            panel(pa, pb, f1, f0, 0, 0, no, no);
+        } else {
+            panel(pa, pb, f0, f1, 1, 0, no, no);
+        }
+    };
+    const bool whole = K % kF64K == 0;
+    const bool akc = g.sak == 1, bkc = g.sbk == 1;
+    const bool fast_a = whole && (akc ? InnerRows<TIN, BM, true>::fits(A, g.sam, g.sak, m0, g.M, K)
+                                      : InnerRows<TIN, BM, false>::fits(A, g.sam, g.sak, m0, g.M, K));
+    const bool fast_b = whole && (bkc ? InnerRows<TIN, BN, true>::fits(B, g.sbn, g.sbk, n0, g.N, K)
+                                      : InnerRows<TIN, BN, false>::fits(B, g.sbn, g.sbk, n0, g.N, K));
+    if (fast_a && fast_b && akc && !bkc)
+        mainloop(InnerRows<TIN, BM, true>(A, g.sam, g.sak, m0), InnerRows<TIN, BN, false>(B, g.sbn, g.sbk, n0));
+    else if (fast_a && fast_b && !akc && !bkc)
+        mainloop(InnerRows<TIN, BM, false>(A, g.sam, g.sak, m0), InnerRows<TIN, BN, false>(B, g.sbn, g.sbk, n0));
+    else if (fast_a && fast_b && bkc && akc)
+        mainloop(InnerRows<TIN, BM, true>(A, g.sam, g.sak, m0), InnerRows<TIN, BN, true>(B, g.sbn, g.sbk, n0));
+    else
+        mainloop(RowPanels<TIN, BM, kF64K>(A, g.sam, g.sak, m0, g.M, K), RowPanels<TIN, BN, kF64K>(B, g.sbn, g.sbk, n0, g.N, K));
+    const double alpha = g.alpha, beta = g.beta;
+#pragma unroll
+    for (int i = 0; i < TI; ++i)
+#pragma unroll
+        for (int j = 0; j < TJ; ++j)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                int r = m0 + wm + 16 * i + (lane / 16) + 4 * v;
+                int c = n0 + wn + 16 * j + lane % 16;
+                if (r < g.M && c < g.N) {
+                    int64_t o = r * g.scm + c * g.scn;
+                    double val = alpha * acc[i][j][v];
+                    if (beta != 0.0) val += beta * (double)C[o];
+                    C[o] = (TIN)val;
+                    if constexpr (TRI)
+                        if (tm != tn && g.splits == 1) C[c * g.scm + r * g.scn] = (TIN)val;
                 }
             }
 }
@@ -662,13 +879,29 @@ static int split_workspace(SplitWs &w, size_t bytes, hipStream_t s) {
 
 // tile: 64 (64 x 64 tiles) or 128 (128 x 128 tiles; each of the 4 wavefronts owns 64 x 64)
 template <typename TIN>
-static int launch_gemm(GemmArgs &a, int precision, int tile, hipStream_t s) {
+static int launch_gemm(GemmArgs &a, int precision, int tile, bool pipe, hipStream_t s) {
     int total = a.tile_start[a.n_groups];
     if (total == 0) return GTN_OK;
     int grid = (total + 7) / 8 * 8;
     const bool big = tile == 128;
     switch (precision) {
         case GTN_PREC_F64:
+            if (pipe && !a.g[0].ind.coef) {
+                if constexpr (sizeof(TIN) == 8) {
+                    if (a.g[0].tri) {
+                        if (big)
+                            hipLaunchKernelGGL((k_gemm_f64_pipe<TIN, 128, 128, true>), dim3(grid), dim3(256), 0, s, a);
+                        else
+                            hipLaunchKernelGGL((k_gemm_f64_pipe<TIN, 64, 64, true>), dim3(grid), dim3(256), 0, s, a);
+                        break;
+                    }
+                }
+                if (big)
+                    hipLaunchKernelGGL((k_gemm_f64_pipe<TIN, 128, 128>), dim3(grid), dim3(256), 0, s, a);
+                else
+                    hipLaunchKernelGGL((k_gemm_f64_pipe<TIN, 64, 64>), dim3(grid), dim3(256), 0, s, a);
+                break;
+            }
             if constexpr (sizeof(TIN) == 8) {
                 if (a.g[0].tri) {
                     if (big)
@@ -798,11 +1031,12 @@ static int scratch_ptr(void **out) {
 // tile <= 0 / target < 0: the heuristics (pick_tile, split_target)
 static int gemm_grouped_impl(const gtn_gemm_desc *groups, int n_groups, int dtype, int precision, void *stream,
                              void *fixed_ws, int64_t fixed_bytes, const char *name, int tile_cfg = 0,
-                             int target_cfg = -1, const GemmIndirect *ind = nullptr, bool tri = false) {
+                             int target_cfg = -1, const GemmIndirect *ind = nullptr, bool tri = false, int pipe_cfg = -1) {
     GTN_REQUIRE(n_groups >= 0 && (n_groups == 0 || groups), "%s: bad groups", name);
     GTN_REQUIRE(dtype == GTN_F64 || dtype == GTN_F32, "gtn_gemm_grouped: dtype must be F64 or F32");
     const int tile = tile_cfg > 0 ? tile_cfg : pick_tile(groups, n_groups, tri);
     const int BM = tile, BN = tile;
+    const bool pipe = pipe_cfg >= 0 ? pipe_cfg : tile == 128;  // untuned: launches that fill the device (pick_tile)
     hipStream_t s = as_stream(stream);
     for (int base = 0; base < n_groups; base += kMaxGroups) {
         GemmArgs a;
@@ -939,7 +1173,7 @@ static int gemm_grouped_impl(const gtn_gemm_desc *groups, int n_groups, int dtyp
                 a.tile_start[used] = tiles;
             }
         }
-        int rc = dtype == GTN_F64 ? launch_gemm<double>(a, precision, tile, s) : launch_gemm<float>(a, precision, tile, s);
+        int rc = dtype == GTN_F64 ? launch_gemm<double>(a, precision, tile, pipe, s) : launch_gemm<float>(a, precision, tile, pipe, s);
         if (rc) return rc;
         if (!orig.empty()) {
             for (int i = 0; i < used; ++i) {
@@ -974,7 +1208,8 @@ static int gemm_grouped_impl(const gtn_gemm_desc *groups, int n_groups, int dtyp
 
 // ---- autotuner: launch configuration per call signature -------------------------------------
 // Candidates: tile 64 or 128 (128 only where every group is at least 128 x 128) times split-K
-// target 0 (no split), 512, 1024 or 2048 workgroups.  The first eager call of a signature (element
+// target 0 (no split), 512, 1024 or 2048 workgroups, for FP64 products on k_gemm_fp, and then
+// k_gemm_f64_pipe in both tiles at the split found best and the usual one.  The first eager call of a signature (element
 // type, precision, and per group M, N, K, batch and operand layouts) times every candidate with HIP
 // events (best of kTuneReps launches each) on its own operands and keeps the fastest; calls made while
 // the stream is capturing a graph, and calls with beta != 0 (whose output a trial would change), use
@@ -982,6 +1217,7 @@ static int gemm_grouped_impl(const gtn_gemm_desc *groups, int n_groups, int dtyp
 struct TuneCfg {
     int tile, target;
     float ms, ms_default;
+    int pipe;
 };
 static std::mutex g_tune_mu;
 static std::map<std::string, TuneCfg> g_tuned;
@@ -996,7 +1232,8 @@ static bool autotune_on() {
     return g_autotune == 1;
 }
 
-static std::string tune_key(const gtn_gemm_desc *g, int n, int dtype, int prec, int dev, bool tri) {
+enum { kPlain = 0, kTri = 1, kIndirect = 2 };  // kinds of launches, tuned apart
+static std::string tune_key(const gtn_gemm_desc *g, int n, int dtype, int prec, int dev, int kind) {
     std::string k;
     auto put = [&](int64_t v) { k.append((const char *)&v, sizeof(v)); };
     put(dev);
@@ -1008,17 +1245,17 @@ static std::string tune_key(const gtn_gemm_desc *g, int n, int dtype, int prec, 
         put(g[i].N);
         put(g[i].K);
         put(g[i].batch);
-        put((g[i].sak == 1) | ((g[i].sbk == 1) << 1) | ((g[i].scn == 1) << 2) | (tri << 3));
+        put((g[i].sak == 1) | ((g[i].sbk == 1) << 1) | ((g[i].scn == 1) << 2) | (kind << 3));
     }
     return k;
 }
 
 static int time_cfg(const gtn_gemm_desc *groups, int n, int dtype, int prec, hipStream_t s, int tile, int target,
-                    hipEvent_t e0, hipEvent_t e1, float *best, bool tri) {
+                    hipEvent_t e0, hipEvent_t e1, float *best, bool tri, int pipe) {
     *best = 1e30f;
     for (int r = 0; r < kTuneReps; ++r) {
         GTN_CHECK_HIP(hipEventRecord(e0, s));
-        int rc = gemm_grouped_impl(groups, n, dtype, prec, s, nullptr, 0, "gtn_gemm_grouped", tile, target, nullptr, tri);
+        int rc = gemm_grouped_impl(groups, n, dtype, prec, s, nullptr, 0, "gtn_gemm_grouped", tile, target, nullptr, tri, pipe);
         if (rc) return rc;
         GTN_CHECK_HIP(hipEventRecord(e1, s));
         GTN_CHECK_HIP(hipEventSynchronize(e1));
@@ -1030,32 +1267,35 @@ static int time_cfg(const gtn_gemm_desc *groups, int n, int dtype, int prec, hip
 }
 
 // the tuned configuration of this signature, if any (no timing)
-static int tuned_lookup(const gtn_gemm_desc *groups, int n, int dtype, int prec, int *tile, int *target, bool *found,
-                        bool tri = false) {
+static int tuned_lookup(const gtn_gemm_desc *groups, int n, int dtype, int prec, int *tile, int *target, int *pipe, bool *found,
+                        int kind = kPlain) {
     *tile = 0;
     *target = -1;
+    *pipe = kind == kIndirect ? 0 : -1;
     *found = false;
     if (!autotune_on() || dry_run() || n <= 0) return GTN_OK;
     int dev;
     GTN_CHECK_HIP(hipGetDevice(&dev));
     std::lock_guard<std::mutex> l(g_tune_mu);
-    auto it = g_tuned.find(tune_key(groups, n, dtype, prec, dev, tri));
+    auto it = g_tuned.find(tune_key(groups, n, dtype, prec, dev, kind));
     if (it != g_tuned.end()) {
         *tile = it->second.tile;
         *target = it->second.target;
+        *pipe = it->second.pipe;
         *found = true;
     }
     return GTN_OK;
 }
 
 static int tuned_config(const gtn_gemm_desc *groups, int n, int dtype, int prec, hipStream_t s, int *tile, int *target,
-                        bool tri = false) {
+                        int *pipe, int kind = kPlain) {
+    const bool tri = kind == kTri;
     bool found;
-    int rc0 = tuned_lookup(groups, n, dtype, prec, tile, target, &found, tri);
+    int rc0 = tuned_lookup(groups, n, dtype, prec, tile, target, pipe, &found, kind);
     if (rc0 || found || !autotune_on() || dry_run() || n <= 0) return rc0;
     int dev;
     GTN_CHECK_HIP(hipGetDevice(&dev));
-    const std::string key = tune_key(groups, n, dtype, prec, dev, tri);
+    const std::string key = tune_key(groups, n, dtype, prec, dev, kind);
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
     GTN_CHECK_HIP(hipStreamIsCapturing(s, &cs));
     if (cs != hipStreamCaptureStatusNone || capture_open()) return GTN_OK;
@@ -1068,18 +1308,28 @@ static int tuned_config(const gtn_gemm_desc *groups, int n, int dtype, int prec,
     hipEvent_t e0, e1;
     GTN_CHECK_HIP(hipEventCreate(&e0));
     GTN_CHECK_HIP(hipEventCreate(&e1));
-    TuneCfg best{0, -1, 1e30f, 0};
+    TuneCfg best{0, -1, 1e30f, 0, 0};
     float ms_default = 0;
-    int rc = time_cfg(groups, n, dtype, prec, s, 0, -1, e0, e1, &ms_default, tri);
+    int rc = time_cfg(groups, n, dtype, prec, s, 0, -1, e0, e1, &ms_default, tri, kind == kIndirect ? 0 : -1);
     const int tiles[2] = {64, 128};
     const int targets[4] = {0, 512, 1024, 2048};
     for (int ti = 0; ti < 2 && !rc; ++ti) {
         if (tiles[ti] == 128 && !can128) continue;
         for (int gi = 0; gi < 4 && !rc; ++gi) {
             float ms;
-            rc = time_cfg(groups, n, dtype, prec, s, tiles[ti], targets[gi], e0, e1, &ms, tri);
-            if (!rc && ms < best.ms) best = TuneCfg{tiles[ti], targets[gi], ms, 0};
+            rc = time_cfg(groups, n, dtype, prec, s, tiles[ti], targets[gi], e0, e1, &ms, tri, 0);
+            if (!rc && ms < best.ms) best = TuneCfg{tiles[ti], targets[gi], ms, 0, 0};
         }
+    }
+    if (prec == GTN_PREC_F64 && kind != kIndirect) {
+        const int tried[2] = {best.target, split_target()};
+        for (int t = 0; t < (tried[0] == tried[1] ? 1 : 2); ++t)
+            for (int ti = 0; ti < 2 && !rc; ++ti) {
+                if (tiles[ti] == 128 && !can128) continue;
+                float ms;
+                rc = time_cfg(groups, n, dtype, prec, s, tiles[ti], tried[t], e0, e1, &ms, tri, 1);
+                if (!rc && ms < best.ms) best = TuneCfg{tiles[ti], tried[t], ms, 0, 1};
+            }
     }
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
@@ -1089,39 +1339,41 @@ static int tuned_config(const gtn_gemm_desc *groups, int n, int dtype, int prec,
     g_tuned[key] = best;
     *tile = best.tile;
     *target = best.target;
+    *pipe = best.pipe;
     return GTN_OK;
 }
 
 extern "C" int gtn_gemm_grouped(const gtn_gemm_desc *groups, int n_groups, int dtype, int precision, void *stream) {
-    int tile = 0, target = -1;
-    int rc = tuned_config(groups, n_groups, dtype, precision, as_stream(stream), &tile, &target);
+    int tile = 0, target = -1, pipe = -1;
+    int rc = tuned_config(groups, n_groups, dtype, precision, as_stream(stream), &tile, &target, &pipe);
     if (rc) return rc;
-    return gemm_grouped_impl(groups, n_groups, dtype, precision, stream, nullptr, 0, "gtn_gemm_grouped", tile, target);
+    return gemm_grouped_impl(groups, n_groups, dtype, precision, stream, nullptr, 0, "gtn_gemm_grouped", tile, target,
+                             nullptr, false, pipe);
 }
 
 int gtn::gemm_symmetric(const gtn_gemm_desc *groups, int n_groups, void *stream) {
     for (int i = 0; i < n_groups; ++i)
         GTN_REQUIRE(groups[i].M == groups[i].N, "gtn_svd_blocks: a symmetric product is square");
-    int tile = 0, target = -1;
-    int rc = tuned_config(groups, n_groups, GTN_F64, GTN_PREC_F64, as_stream(stream), &tile, &target, true);
+    int tile = 0, target = -1, pipe = -1;
+    int rc = tuned_config(groups, n_groups, GTN_F64, GTN_PREC_F64, as_stream(stream), &tile, &target, &pipe, kTri);
     if (rc) return rc;
     return gemm_grouped_impl(groups, n_groups, GTN_F64, GTN_PREC_F64, stream, nullptr, 0, "gtn_svd_blocks", tile, target,
-                             nullptr, true);
+                             nullptr, true, pipe);
 }
 
 int gtn::gemm_grouped_indirect(const gtn_gemm_desc *groups, const GemmIndirect *ind, int n_groups, void *const *tune_c,
                                void *stream) {
-    int tile = 0, target = -1, rc;
+    int tile = 0, target = -1, pipe = 0, rc;
     if (tune_c) {
         std::vector<gtn_gemm_desc> plain(groups, groups + n_groups);
         for (int i = 0; i < n_groups; ++i) plain[i].C = tune_c[i];
-        rc = tuned_config(plain.data(), n_groups, GTN_F64, GTN_PREC_F64, as_stream(stream), &tile, &target);
+        rc = tuned_config(plain.data(), n_groups, GTN_F64, GTN_PREC_F64, as_stream(stream), &tile, &target, &pipe, kIndirect);
     } else {
         bool found;
-        rc = tuned_lookup(groups, n_groups, GTN_F64, GTN_PREC_F64, &tile, &target, &found);
+        rc = tuned_lookup(groups, n_groups, GTN_F64, GTN_PREC_F64, &tile, &target, &pipe, &found, kIndirect);
     }
     if (rc) return rc;
-    return gemm_grouped_impl(groups, n_groups, GTN_F64, GTN_PREC_F64, stream, nullptr, 0, "gtn_svd_blocks", tile, target, ind);
+    return gemm_grouped_impl(groups, n_groups, GTN_F64, GTN_PREC_F64, stream, nullptr, 0, "gtn_svd_blocks", tile, target, ind, false, 0);
 }
 
 extern "C" int gtn_autotune_set(int on) {
@@ -1168,20 +1420,20 @@ extern "C" int gtn_gemm_grouped_noalloc(const gtn_gemm_desc *groups, int n_group
     void *p = nullptr;
     int rc = scratch_ptr(&p);
     if (rc) return rc;
-    int tile = 0, target = -1;
+    int tile = 0, target = -1, pipe = -1;
     bool found = false;
-    rc = tuned_lookup(groups, n_groups, dtype, precision, &tile, &target, &found);
+    rc = tuned_lookup(groups, n_groups, dtype, precision, &tile, &target, &pipe, &found);
     if (rc) return rc;
     if (found && target > 1024) {
         // a larger split target than the heuristics' may need more scratch than there is
         rc = gemm_grouped_impl(groups, n_groups, dtype, precision, stream, p, kNoAllocScratchBytes,
-                               "gtn_gemm_grouped_noalloc", tile, target);
+                               "gtn_gemm_grouped_noalloc", tile, target, nullptr, false, pipe);
         if (rc != GTN_ENOMEM) return rc;
         tile = 0;
-        target = -1;
+        target = pipe = -1;
     }
     return gemm_grouped_impl(groups, n_groups, dtype, precision, stream, p, kNoAllocScratchBytes,
-                             "gtn_gemm_grouped_noalloc", tile, target);
+                             "gtn_gemm_grouped_noalloc", tile, target, nullptr, false, pipe);
 }
 
 // int8 16x16x64 lane-layout self-test (the operands are deterministic small integers; one wavefront)

@@ -197,6 +197,13 @@ inline T emu_buffer_load(emu_buffer_rsrc r, int voffset, int soffset) {
 inline unsigned long long __builtin_amdgcn_raw_buffer_load_b64(emu_buffer_rsrc r, int vo, int so, int) {
     return emu_buffer_load<unsigned long long>(r, vo, so);
 }
+typedef unsigned emu_u4 __attribute__((ext_vector_type(4)));
+inline emu_u4 __builtin_amdgcn_raw_buffer_load_b128(emu_buffer_rsrc r, int vo, int so, int) {
+    const unsigned long long lo = emu_buffer_load<unsigned long long>(r, vo, so);
+    const unsigned long long hi = emu_buffer_load<unsigned long long>(r, vo + 8, so);
+    return emu_u4{(unsigned)lo, (unsigned)(lo >> 32), (unsigned)hi, (unsigned)(hi >> 32)};
+}
+inline void __builtin_amdgcn_sched_group_barrier(int, int, int) {}
 inline unsigned __builtin_amdgcn_raw_buffer_load_b32(emu_buffer_rsrc r, int vo, int so, int) {
     return emu_buffer_load<unsigned>(r, vo, so);
 }
