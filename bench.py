@@ -275,7 +275,7 @@ def rf_gemm_roofline(P, reps=20):
             tile = e.tile
     return {"bound": "mfma", "achieved": ach, "peak": MFMA_PEAK_TF["f64"], "unit": "TFLOP/s",
             "frac": ach / MFMA_PEAK_TF["f64"], "traffic": measured_traffic("rf_gemm_f64"),
-            "kernel": "range-finder GEMM k_gemm_fp<double,double,%d,%d,16>: %d parity blocks of 2048 x 2048 "
+            "kernel": "range-finder GEMM (gtn_gemm_grouped, autotuned, %d x %d tiles): %d parity blocks of 2048 x 2048 "
                       "times 2048 x 128 (N(0,1) entries) per launch, FP64" % (tile, tile, nb),
             "flop_per_launch": flop, "avg_launch_ms": ms, "launches": reps}
 
