@@ -544,7 +544,7 @@ __device__ __forceinline__ void rr_pair(int t, int round, int p, int &i, int &j)
 // eight rounds and there is no replay.  It is bound by instruction issue: about 240 instructions of
 // 4 cycles (a lane swap 12) per eight rotations, 8 wavefronts on 4 SIMDs.  MI355X, four 128 x 128
 // problems: blocks of a leg-dim-16 step 3.5 ms -> 1.4 ms (1.9 ms from their own columns), Rayleigh-Ritz matrices of a leg-dim-64 step
-// 1.8 ms -> 0.6 ms.
+// 1.8 ms -> 1.0 ms.
 // A pair is left alone when |x.y| <= 1e-15 |x| |y| or one of the two is below 1e-15 of the largest
 // vector (the rank rule drops values at 1e-14).  A sweep whose rotations all have |x.y| <= 1e-9 |x| |y|
 // and angles of at most 1e-8 is the last: what they undo in other pairs is their product.  The vectors
