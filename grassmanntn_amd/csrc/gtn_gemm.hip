@@ -21,7 +21,6 @@
 
 namespace gtn {
 
-typedef double d2 __attribute__((ext_vector_type(2)));
 typedef double d4 __attribute__((ext_vector_type(4)));
 typedef float f4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf8 __attribute__((ext_vector_type(8)));
@@ -354,8 +353,13 @@ __global__ void __launch_bounds__(256, IND || TRI ? 2 : 1) k_gemm_fp(GemmArgs ar
 // and term u of B with t + u < max(SA, SB) are accumulated, smallest first.
 constexpr int kBfK = 32;             // reduction per panel: one MFMA
 constexpr int kBfStride = kBfK + 8;  // 80-byte rows: the 16 rows of an operand read start in distinct banks
-constexpr int kF64K = 8;  // FP64: reduction per panel, two MFMAs; rows of 80 bytes, likewise
-constexpr int kF64Stride = kF64K + 2;
+// k_gemm_pipe: a panel is four 16-byte slots a row, 2 FP64 or 4 FP32 k each; rows of 80 bytes, likewise
+template <typename TC>
+constexpr int kSlot = 16 / (int)sizeof(TC);
+template <typename TC>
+constexpr int kDepth = 4 * kSlot<TC>;
+template <typename TC>
+constexpr int kStride = 5 * kSlot<TC>;
 
 // One operand's ROWS x BK panels in rows.  A lane's slot is V = BK / 4 consecutive k of one row, 16 bytes in
 // LDS, kept in the operand's own type until it is stored.  Reduction-contiguous operands
@@ -435,13 +439,18 @@ struct RowPanels {
             }
         }
     }
-    __device__ __forceinline__ void store(double (&X)[ROWS][kF64Stride]) const {
-        static_assert(V == 2, "a slot is 16 bytes in LDS");
+    template <typename TC>
+    __device__ __forceinline__ void store(TC (&X)[ROWS][kStride<TC>]) const {
+        static_assert(V == kSlot<TC>, "a slot is 16 bytes in LDS");
+        typedef TC slot_t __attribute__((ext_vector_type(V)));
 #pragma unroll
         for (int s = 0; s < NS; ++s) {
             int r, q;
             at(s, r, q);
-            *(d2 *)&X[r][2 * q] = d2{(double)reg[s][0], (double)reg[s][1]};
+            slot_t h;
+#pragma unroll
+            for (int t = 0; t < V; ++t) h[t] = (TC)reg[s][t];
+            *(slot_t *)&X[r][V * q] = h;
         }
     }
 };
@@ -540,12 +549,12 @@ __global__ void __launch_bounds__(256, 2) k_gemm_bf16(GemmArgs args) {
             }
 }
 
-// RowPanels<T, ROWS, kF64K> where every panel lies inside the operand, within 2^31 bytes of the slab's first
+// RowPanels<T, ROWS, kDepth<TC>> where every panel lies inside the operand, within 2^31 bytes of the slab's first
 // element: buffer loads from a scalar resource at the slab's origin, one 32-bit offset a lane and uniform
 // offsets for the slots.  KC: reduction-contiguous on 16-byte boundaries; else row-contiguous (sr == 1).
-template <typename T, int ROWS, bool KC>
+template <typename T, typename TC, int ROWS, bool KC>
 struct InnerRows {
-    static constexpr int NS = ROWS / 64, V = 2;
+    static constexpr int NS = ROWS / 64, V = kSlot<TC>;
     __amdgpu_buffer_rsrc_t rsrc;
     uint32_t voff, kbytes, slot;
     int lds;
@@ -558,7 +567,7 @@ struct InnerRows {
         voff = (uint32_t)(((int64_t)r * sr + (int64_t)(V * q) * sk) * (int64_t)sizeof(T));
         kbytes = __builtin_amdgcn_readfirstlane((uint32_t)(sk * (int64_t)sizeof(T)));
         slot = __builtin_amdgcn_readfirstlane((uint32_t)((KC ? 64 * sr : V * (256 / ROWS) * sk) * (int64_t)sizeof(T)));
-        lds = r * kF64Stride + V * q;
+        lds = r * kStride<TC> + V * q;
     }
     static __device__ __forceinline__ bool fits(const T *p, int64_t sr, int64_t sk, int R0, int R, int K) {
         return (KC ? sk == 1 && (((uint64_t)p) & 15) == 0 && (sr * (int64_t)sizeof(T)) % 16 == 0 : sr == 1) && R0 + ROWS <= R &&
@@ -586,25 +595,32 @@ struct InnerRows {
             }
         }
     }
-    __device__ __forceinline__ void store(double (&X)[ROWS][kF64Stride]) const {
+    __device__ __forceinline__ void store(TC (&X)[ROWS][kStride<TC>]) const {
+        typedef TC slot_t __attribute__((ext_vector_type(V)));
 #pragma unroll
-        for (int s = 0; s < NS; ++s)
-            *(d2 *)(&X[0][0] + lds + s * (KC ? 64 * kF64Stride : V * (256 / ROWS))) = d2{(double)reg[s][0], (double)reg[s][1]};
+        for (int s = 0; s < NS; ++s) {
+            slot_t h;
+#pragma unroll
+            for (int t = 0; t < V; ++t) h[t] = (TC)reg[s][t];
+            *(slot_t *)(&X[0][0] + lds + s * (KC ? 64 * kStride<TC> : V * (256 / ROWS))) = h;
+        }
     }
 };
 
-// FP64 products with unbroken matrix work: 16x16x4 MFMA on panels in rows, two LDS buffers, one barrier a
-// panel of eight.  Lane l holds the slot of k = 2 (l / 16), 2 (l / 16) + 1 of its row, one 16-byte read, and the
-// s-th of a panel's two instructions per tile multiplies the s-th of them: the same k in both operands, which
-// is all that the sum asks for.  What fills LDS and registers for the next panels is placed between the matrix
-// instructions (`panel`).  Against k_gemm_fp (panels of 16 stored k by k in one buffer, two barriers and an LDS
-// wait in the open a panel), TFLOP/s on N(0,1) entries: 8192^3 67.5 -> 75.3, two products of 2048^3 61 to 65 ->
-// 71, 32 of 2048 x 128 x 2048 58 to 61 -> 65, nominal peak 78.6 (torch's products beside it 69 to 73 on the
-// square sizes).  Launches that leave most of a compute unit idle wait for memory more often with panels of
-// eight (59 products of 640 x 128 x 640 took 835 us and not 780), and the range finder's epilogue would spill:
-// those stay with k_gemm_fp, and the autotuner times both for the others.  TRI: symmetric products.
-template <typename TIN, int BM, int BN, bool TRI = false>
-__global__ void __launch_bounds__(256, 2) k_gemm_f64_pipe(GemmArgs args) {
+// Products with unbroken matrix work, in FP64, and in FP32 on FP32 operands: 16x16x4 MFMA on panels in rows, two
+// LDS buffers, one barrier a panel of eight (FP32: sixteen).  Lane l holds the slot of k = V (l / 16) .. + V - 1
+// of its row, one 16-byte read, and the s-th of a panel's V instructions per tile multiplies the s-th of them:
+// the same k in both operands, which is all that the sum asks for.  What fills LDS and registers for the next
+// panels is placed between the matrix instructions (`panel`).  Against k_gemm_fp (panels of 16 stored k by k,
+// LDS waits in the open and, in FP64, two barriers around one buffer a panel), TFLOP/s on N(0,1) entries, FP64:
+// 8192^3 67.5 -> 75.3, two products of 2048^3 61 to 65 -> 71, 32 of 2048 x 128 x 2048 58 to 61 -> 65, nominal
+// peak 78.6 (torch's products beside it 69 to 73 on the square sizes); FP32: 8192^3 109 -> 149, two of 2048^3
+// 110 -> 140, peak 157.  Launches that leave most of a compute unit idle wait for memory more often with the
+// shorter panels (59 products of 640 x 128 x 640 took 835 us and not 780), and the range finder's epilogue would
+// spill: those stay with k_gemm_fp, and the autotuner times both for the others.  So does FP32 arithmetic on FP64
+// operands, bound by their conversion (105 to 112 against 110 to 113).  TRI: symmetric products.
+template <typename TIN, typename TC, int BM, int BN, bool TRI = false>
+__global__ void __launch_bounds__(256, 2) k_gemm_pipe(GemmArgs args) {
     int gi, b, tm, tn;
     if (!locate(args, gi, b, tm, tn)) return;
     const GemmGroup &g = args.g[gi];
@@ -615,32 +631,41 @@ __global__ void __launch_bounds__(256, 2) k_gemm_f64_pipe(GemmArgs args) {
     const TIN *A = (const TIN *)g.A + b * g.sab + kb * g.sak;
     const TIN *B = (const TIN *)g.B + b * g.sbb + kb * g.sbk;
     TIN *C = (TIN *)g.C + b * g.scb + sp * g.scs;
-    __shared__ __attribute__((aligned(16))) double As[2][BM][kF64Stride];
-    __shared__ __attribute__((aligned(16))) double Bs[2][BN][kF64Stride];
+    constexpr int V = kSlot<TC>, DEPTH = kDepth<TC>;
+    __shared__ __attribute__((aligned(16))) TC As[2][BM][kStride<TC>];
+    __shared__ __attribute__((aligned(16))) TC Bs[2][BN][kStride<TC>];
     constexpr int WM = BM / 2, WN = BN / 2, TI = WM / 16, TJ = WN / 16;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int wm = (wave >> 1) * WM, wn = (wave & 1) * WN;
     const int m0 = tm * BM, n0 = tn * BN;
-    d4 acc[TI][TJ];
+    using acc_t = typename std::conditional<sizeof(TC) == 8, d4, f4>::type;
+    acc_t acc[TI][TJ];
 #pragma unroll
     for (int i = 0; i < TI; ++i)
 #pragma unroll
-        for (int j = 0; j < TJ; ++j) acc[i][j] = d4{0, 0, 0, 0};
+        for (int j = 0; j < TJ; ++j) acc[i][j] = acc_t{0, 0, 0, 0};
+    typedef TC slot_t __attribute__((ext_vector_type(V)));
     struct Frag {
-        d2 a[TI], b[TJ];
+        slot_t a[TI], b[TJ];
     };
     auto fetch = [&](int buf, Frag &f) {
 #pragma unroll
-        for (int i = 0; i < TI; ++i) f.a[i] = *(const d2 *)&As[buf][wm + 16 * i + lane % 16][2 * (lane / 16)];
+        for (int i = 0; i < TI; ++i) f.a[i] = *(const slot_t *)&As[buf][wm + 16 * i + lane % 16][V * (lane / 16)];
 #pragma unroll
-        for (int j = 0; j < TJ; ++j) f.b[j] = *(const d2 *)&Bs[buf][wn + 16 * j + lane % 16][2 * (lane / 16)];
+        for (int j = 0; j < TJ; ++j) f.b[j] = *(const slot_t *)&Bs[buf][wn + 16 * j + lane % 16][V * (lane / 16)];
     };
-    auto multiply = [&](const Frag &f, int s) {  // one of a panel's two instructions per tile
+    auto multiply = [&](const Frag &f, int half) {  // V / 2 of a panel's V instructions per tile
 #pragma unroll
-        for (int i = 0; i < TI; ++i)
+        for (int s = half * (V / 2); s < (half + 1) * (V / 2); ++s)
 #pragma unroll
-            for (int j = 0; j < TJ; ++j)
-                acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(f.a[i][s], f.b[j][s], acc[i][j], 0, 0, 0);
+            for (int i = 0; i < TI; ++i)
+#pragma unroll
+                for (int j = 0; j < TJ; ++j) {
+                    if constexpr (sizeof(TC) == 8)
+                        acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(f.a[i][s], f.b[j][s], acc[i][j], 0, 0, 0);
+                    else
+                        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(f.a[i][s], f.b[j][s], acc[i][j], 0, 0, 0);
+                }
     };
     // One panel, its operands in `f`: the next panel's go to LDS and the one after that is loaded while the
     // first half of the instructions runs, and after the barrier the next panel's operands are read into
@@ -659,7 +684,7 @@ __global__ void __launch_bounds__(256, 2) k_gemm_f64_pipe(GemmArgs args) {
         if constexpr (decltype(has2)::value) {
 #pragma unroll
             for (int t = 0; t < TI * TJ; ++t) {
-                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // matrix
+                __builtin_amdgcn_sched_group_barrier(0x008, V / 2, 0);  // matrix
                 __builtin_amdgcn_sched_group_barrier(0x200, 1, 0);  // LDS write
                 __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);  // load
                 __builtin_amdgcn_sched_group_barrier(0x002, 3, 0);  // vector
@@ -673,7 +698,7 @@ __global__ void __launch_bounds__(256, 2) k_gemm_f64_pipe(GemmArgs args) {
         if constexpr (decltype(has1)::value) {
 #pragma unroll
             for (int t = 0; t < TI + TJ; ++t) {
-                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                __builtin_amdgcn_sched_group_barrier(0x008, V / 2, 0);
                 __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // LDS read
             }
         }
@@ -686,44 +711,44 @@ __global__ void __launch_bounds__(256, 2) k_gemm_f64_pipe(GemmArgs args) {
         pb.load(0);
         pa.store(As[0]);
         pb.store(Bs[0]);
-        if (K > kF64K) {
-            pa.load(kF64K);
-            pb.load(kF64K);
+        if (K > DEPTH) {
+            pa.load(DEPTH);
+            pb.load(DEPTH);
         }
         __syncthreads();
         Frag f0, f1;
         fetch(0, f0);
         int k0 = 0;
-        for (; k0 + 3 * kF64K < K; k0 += 2 * kF64K) {  // two panels a turn: neither set of operands is copied
-            panel(pa, pb, f0, f1, 1, k0 + 2 * kF64K, yes, yes);
-            panel(pa, pb, f1, f0, 0, k0 + 3 * kF64K, yes, yes);
+        for (; k0 + 3 * DEPTH < K; k0 += 2 * DEPTH) {  // two panels a turn: neither set of operands is copied
+            panel(pa, pb, f0, f1, 1, k0 + 2 * DEPTH, yes, yes);
+            panel(pa, pb, f1, f0, 0, k0 + 3 * DEPTH, yes, yes);
         }
         // one to three panels are left, the first of them in f0
-        if (k0 + 2 * kF64K < K) {
-            panel(pa, pb, f0, f1, 1, k0 + 2 * kF64K, yes, yes);
+        if (k0 + 2 * DEPTH < K) {
+            panel(pa, pb, f0, f1, 1, k0 + 2 * DEPTH, yes, yes);
             panel(pa, pb, f1, f0, 0, 0, yes, no);
             panel(pa, pb, f0, f1, 1, 0, no, no);
-        } else if (k0 + kF64K < K) {
+        } else if (k0 + DEPTH < K) {
             panel(pa, pb, f0, f1, 1, 0, yes, no);
             panel(pa, pb, f1, f0, 0, 0, no, no);
         } else {
             panel(pa, pb, f0, f1, 1, 0, no, no);
         }
     };
-    const bool whole = K % kF64K == 0;
+    const bool whole = K % DEPTH == 0;
     const bool akc = g.sak == 1, bkc = g.sbk == 1;
-    const bool fast_a = whole && (akc ? InnerRows<TIN, BM, true>::fits(A, g.sam, g.sak, m0, g.M, K)
-                                      : InnerRows<TIN, BM, false>::fits(A, g.sam, g.sak, m0, g.M, K));
-    const bool fast_b = whole && (bkc ? InnerRows<TIN, BN, true>::fits(B, g.sbn, g.sbk, n0, g.N, K)
-                                      : InnerRows<TIN, BN, false>::fits(B, g.sbn, g.sbk, n0, g.N, K));
+    const bool fast_a = whole && (akc ? InnerRows<TIN, TC, BM, true>::fits(A, g.sam, g.sak, m0, g.M, K)
+                                      : InnerRows<TIN, TC, BM, false>::fits(A, g.sam, g.sak, m0, g.M, K));
+    const bool fast_b = whole && (bkc ? InnerRows<TIN, TC, BN, true>::fits(B, g.sbn, g.sbk, n0, g.N, K)
+                                      : InnerRows<TIN, TC, BN, false>::fits(B, g.sbn, g.sbk, n0, g.N, K));
     if (fast_a && fast_b && akc && !bkc)
-        mainloop(InnerRows<TIN, BM, true>(A, g.sam, g.sak, m0), InnerRows<TIN, BN, false>(B, g.sbn, g.sbk, n0));
+        mainloop(InnerRows<TIN, TC, BM, true>(A, g.sam, g.sak, m0), InnerRows<TIN, TC, BN, false>(B, g.sbn, g.sbk, n0));
     else if (fast_a && fast_b && !akc && !bkc)
-        mainloop(InnerRows<TIN, BM, false>(A, g.sam, g.sak, m0), InnerRows<TIN, BN, false>(B, g.sbn, g.sbk, n0));
+        mainloop(InnerRows<TIN, TC, BM, false>(A, g.sam, g.sak, m0), InnerRows<TIN, TC, BN, false>(B, g.sbn, g.sbk, n0));
     else if (fast_a && fast_b && bkc && akc)
-        mainloop(InnerRows<TIN, BM, true>(A, g.sam, g.sak, m0), InnerRows<TIN, BN, true>(B, g.sbn, g.sbk, n0));
+        mainloop(InnerRows<TIN, TC, BM, true>(A, g.sam, g.sak, m0), InnerRows<TIN, TC, BN, true>(B, g.sbn, g.sbk, n0));
     else
-        mainloop(RowPanels<TIN, BM, kF64K>(A, g.sam, g.sak, m0, g.M, K), RowPanels<TIN, BN, kF64K>(B, g.sbn, g.sbk, n0, g.N, K));
+        mainloop(RowPanels<TIN, BM, DEPTH>(A, g.sam, g.sak, m0, g.M, K), RowPanels<TIN, BN, DEPTH>(B, g.sbn, g.sbk, n0, g.N, K));
     const double alpha = g.alpha, beta = g.beta;
 #pragma unroll
     for (int i = 0; i < TI; ++i)
@@ -731,11 +756,12 @@ __global__ void __launch_bounds__(256, 2) k_gemm_f64_pipe(GemmArgs args) {
         for (int j = 0; j < TJ; ++j)
 #pragma unroll
             for (int v = 0; v < 4; ++v) {
-                int r = m0 + wm + 16 * i + (lane / 16) + 4 * v;
+                const int row = sizeof(TC) == 8 ? (lane / 16) + 4 * v : 4 * (lane / 16) + v;
+                int r = m0 + wm + 16 * i + row;
                 int c = n0 + wn + 16 * j + lane % 16;
                 if (r < g.M && c < g.N) {
                     int64_t o = r * g.scm + c * g.scn;
-                    double val = alpha * acc[i][j][v];
+                    double val = alpha * (double)acc[i][j][v];
                     if (beta != 0.0) val += beta * (double)C[o];
                     C[o] = (TIN)val;
                     if constexpr (TRI)
@@ -890,16 +916,16 @@ static int launch_gemm(GemmArgs &a, int precision, int tile, bool pipe, hipStrea
                 if constexpr (sizeof(TIN) == 8) {
                     if (a.g[0].tri) {
                         if (big)
-                            hipLaunchKernelGGL((k_gemm_f64_pipe<TIN, 128, 128, true>), dim3(grid), dim3(256), 0, s, a);
+                            hipLaunchKernelGGL((k_gemm_pipe<TIN, double, 128, 128, true>), dim3(grid), dim3(256), 0, s, a);
                         else
-                            hipLaunchKernelGGL((k_gemm_f64_pipe<TIN, 64, 64, true>), dim3(grid), dim3(256), 0, s, a);
+                            hipLaunchKernelGGL((k_gemm_pipe<TIN, double, 64, 64, true>), dim3(grid), dim3(256), 0, s, a);
                         break;
                     }
                 }
                 if (big)
-                    hipLaunchKernelGGL((k_gemm_f64_pipe<TIN, 128, 128>), dim3(grid), dim3(256), 0, s, a);
+                    hipLaunchKernelGGL((k_gemm_pipe<TIN, double, 128, 128>), dim3(grid), dim3(256), 0, s, a);
                 else
-                    hipLaunchKernelGGL((k_gemm_f64_pipe<TIN, 64, 64>), dim3(grid), dim3(256), 0, s, a);
+                    hipLaunchKernelGGL((k_gemm_pipe<TIN, double, 64, 64>), dim3(grid), dim3(256), 0, s, a);
                 break;
             }
             if constexpr (sizeof(TIN) == 8) {
@@ -924,6 +950,15 @@ static int launch_gemm(GemmArgs &a, int precision, int tile, bool pipe, hipStrea
                 hipLaunchKernelGGL((k_gemm_fp<TIN, double, 64, 64, 16>), dim3(grid), dim3(256), 0, s, a);
             break;
         case GTN_PREC_F32:
+            if constexpr (sizeof(TIN) == 4) {
+                if (pipe) {
+                    if (big)
+                        hipLaunchKernelGGL((k_gemm_pipe<TIN, float, 128, 128>), dim3(grid), dim3(256), 0, s, a);
+                    else
+                        hipLaunchKernelGGL((k_gemm_pipe<TIN, float, 64, 64>), dim3(grid), dim3(256), 0, s, a);
+                    break;
+                }
+            }
             if (big)
                 hipLaunchKernelGGL((k_gemm_fp<TIN, float, 128, 128, 16>), dim3(grid), dim3(256), 0, s, a);
             else
@@ -1208,8 +1243,8 @@ static int gemm_grouped_impl(const gtn_gemm_desc *groups, int n_groups, int dtyp
 
 // ---- autotuner: launch configuration per call signature -------------------------------------
 // Candidates: tile 64 or 128 (128 only where every group is at least 128 x 128) times split-K
-// target 0 (no split), 512, 1024 or 2048 workgroups, for FP64 products on k_gemm_fp, and then
-// k_gemm_f64_pipe in both tiles at the split found best and the usual one.  The first eager call of a signature (element
+// target 0 (no split), 512, 1024 or 2048 workgroups, on k_gemm_fp, and then, where there is one,
+// k_gemm_pipe in both tiles at the split found best and the usual one.  The first eager call of a signature (element
 // type, precision, and per group M, N, K, batch and operand layouts) times every candidate with HIP
 // events (best of kTuneReps launches each) on its own operands and keeps the fastest; calls made while
 // the stream is capturing a graph, and calls with beta != 0 (whose output a trial would change), use
@@ -1321,7 +1356,7 @@ static int tuned_config(const gtn_gemm_desc *groups, int n, int dtype, int prec,
             if (!rc && ms < best.ms) best = TuneCfg{tiles[ti], targets[gi], ms, 0, 0};
         }
     }
-    if (prec == GTN_PREC_F64 && kind != kIndirect) {
+    if ((prec == GTN_PREC_F64 && kind != kIndirect) || (prec == GTN_PREC_F32 && dtype == GTN_F32)) {
         const int tried[2] = {best.target, split_target()};
         for (int t = 0; t < (tried[0] == tried[1] ? 1 : 2); ++t)
             for (int ti = 0; ti < 2 && !rc; ++ti) {
