@@ -40,7 +40,7 @@ class _Settings:
     svd_precision = "f64_gram"
     svd_oversample = 96
     # subspace iterations: error ~ (sigma_{p+1} / sigma_k)^(2 iters); "f64_gram" reaches the same with fewer
-    # products (13 for 20) and stops a block earlier where it has converged
+    # products where the spectrum allows it (6 to 15 for 20 on the blocks of a TRG step)
     svd_iters = 20
     # CholeskyQR of the basis every this many iterations.  Every iteration: between two
     # orthonormalisations a direction grows by (sigma_i / sigma_0)^(2 every), and one whose squared

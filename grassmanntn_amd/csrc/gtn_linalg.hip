@@ -121,7 +121,7 @@ struct SmallBatch {
     // index of the product just done and the largest number of products
     double *st[kMaxBatch];
     int k[kMaxBatch];
-    int it, iters, cap;
+    int it, iters;
 };
 struct SmallPtrs {
     int p, k;
@@ -297,24 +297,42 @@ __device__ __forceinline__ void chol_factor(double *A, int LD, double *Dv, int n
 
 // ---------------------------------------------------------------------------------------------
 // Filtered range finder (FP64 Gram iteration).  A block's basis is multiplied by a polynomial of its
-// Gram matrix G, one product per degree: kPre plain products G Y with CholeskyQR, whose R has
-// estimates of G's eigenvalues on its diagonal (R_jj -> lambda_j, decreasing; measured within 15 % of
-// lambda_k and 1.0 to 1.6 times lambda_{p+1} after two products), then Chebyshev polynomials of the
-// first kind on [0, b], b the largest of the last (at most 16) R_jj: T_{j+1} = 2 (2 G / b - 1) T_j -
-// T_{j-1}, the linear combination taken in the product's epilogue.  What lies in [0, b] stays within
-// one while lambda > b grows by exp(acosh(2 lambda / b - 1)) per degree: with lambda_k / lambda_{p+1} =
-// 2.6 (blocks of the leg-dim-64 workload) 13 products leave 1e-10 of the missing directions in the kept
-// ones where 20 plain products leave 4e-9.  A block stops when its kept values have grown by e^36
-// over the interval, at most at `cap` products (filter_cap).  Without a gap to speak of, or where a
-// degree's growth of the largest eigenvalue would put the kept ones under CholeskyQR's pivot floor, the
-// block goes on with plain products, and stops when (lambda_k / b)^products has reached e^36.
+// Gram matrix G, one product per degree: plain products G Y with CholeskyQR, whose R has estimates of G's
+// eigenvalues on its diagonal (R_jj -> lambda_j, decreasing), then Chebyshev polynomials of the first kind
+// on [0, b], b the largest of the last (at most 16) R_jj: T_{j+1} = 2 (2 G / b - 1) T_j - T_{j-1}, the
+// linear combination taken in the product's epilogue.  What lies in [0, b] stays within one while
+// lambda > b grows by exp(acosh(2 lambda / b - 1)) per degree.  Above b a degree separates any two
+// eigenvalues at least as well as a plain product does, for every b below them.
+// What the rules guard against is a wrong b, and a tail far below b that plain products would remove:
+//   - The filter waits for b: after two products b is 0.46 (a plateau wider than the basis) to 4 times
+//     lambda_{p+1}.  It starts after kPlain products at the earliest, and only once b has grown by at most
+//     kSettled in the last of them, and lambda_k is at least kMinGap times b.  Blocks that never get
+//     there do `iters` plain products.
+//   - It is to reach `need`, the logarithm of the separation that `iters` plain products would give: between
+//     R_kk and the smallest of the last R_jj, times kMargin; at most e^34 (rounding).
+//   - Each later R has the growth of its directions since the last on its diagonal.  The logarithm of the
+//     ratio of R_kk to the last R_jj is the separation reached (`kConv`); where the last ones grow, b was
+//     too small: need and the products left are estimated anew from both rates.  A block never does
+//     more than `iters` products.
+// Replayed in numpy for 584 geometric, plateau, stepped and random piecewise spectra (m 260 to 2048, k 4 to
+// 112), values and residuals are nowhere further off than those of `iters` plain products.  (With b and the
+// count fixed after two products 93 of them were: residuals of up to 7e-6 of sigma_0^2 and values of 3e-11
+// of sigma_0 on plateaus that plain products resolve to rounding.)  20 plain products become 6 to 15 on the
+// workloads' blocks (6 to 13 with that count), 15 on those of leg dim 64.  A margin of 1.1 saves one of the
+// 15 and leaves one of the random spectra ten times further off than plain products do.
+// Where a degree's growth of the largest eigenvalue would put the kept ones under CholeskyQR's pivot floor,
+// the block goes on with plain products, and stops when (lambda_k / b)^products has reached e^34.
 // The basis is orthonormalised only after as many degrees as keep the growth of the largest
 // eigenvalue within 1e11 in the Gram matrix of the basis (at most three); T_{j-1} is multiplied by the
 // same R^{-1}.  All of this is per block and on the device (a recorded graph cannot branch): the state
 // holds the block's buffers and coefficients, the product, Gram and basis kernels of a finished or
 // resting block return at once.
 // ---------------------------------------------------------------------------------------------
-constexpr int kPre = 2;
+constexpr int kPlain = 3;           // products before the filter, at least
+constexpr double kSettled = 1.05;   // growth of b in a product that counts as settled
+constexpr double kMinGap = 1.1;     // lambda_k / b from which the filter is worth its start
+constexpr double kMargin = 1.2;     // of the ratio that plain products are credited with
+constexpr double kRounding = 34.0;  // e^-34 = 2e-15, an order below the rounding of m-term sums
 enum RfSlot {  // 8-byte slots of a block's state
     kCur = 0,   // T_j (before the first degree: the basis)
     kPrev,      // T_{j-1}, overwritten by T_{j+1}
@@ -322,7 +340,10 @@ enum RfSlot {  // 8-byte slots of a block's state
     kAq, kAp, kDq, kDp,  // sources and targets of the basis products with R^{-1} of this round
     kProd = 8,  // coefficients (x, y, z, skip) of the product
     kApplyQ = 12, kGram = 16, kApplyP = 20,  // of the basis product of T_j, of the Gram matrix, of T_{j-1}
-    kTotal = 24, kSince, kMaxSince, kCheb,
+    kTotal = 24, kSince, kMaxSince,
+    kStart,  // the product after which the filter started, 0: not yet
+    kEdge,   // b of the last round
+    kConv,   // logarithm of the separation reached
     kRfSlots = 32
 };
 __device__ __forceinline__ double *rf_ptr(const double *st, int slot) { return __builtin_bit_cast(double *, st[slot]); }
@@ -355,37 +376,52 @@ __global__ void k_rf_collect(const double *st, double *Y, int64_t n, int64_t dws
 
 // One thread, after product `it`: the new basis has been written over T_{j-1}; diag (p values, or null
 // when this round does not orthonormalise) is the diagonal of R.
-__device__ void rf_advance(double *st, const double *diag, int p, int k, int it, int iters, int cap) {
+__device__ void rf_advance(double *st, const double *diag, int p, int k, int it, int iters) {
     double *cur = rf_ptr(st, kPrev), *prev = rf_ptr(st, kCur), *s1 = rf_ptr(st, kS1), *s2 = rf_ptr(st, kS2);
-    bool cheb = st[kCheb] != 0.0;
     st[kApplyQ + 3] = st[kApplyP + 3] = 1.0;
-    if (diag && it == kPre) {
+    if (diag) {
         const int w = min(16, (p - k) / 2);
-        double b = 0.0, l0 = 0.0, lk = diag[k - 1];
-        for (int j = 0; j < p; ++j) l0 = fmax(l0, diag[j]);
+        double lk = diag[k - 1], b = 0.0, lo = INFINITY;
         for (int j = max(0, k - 4); j < k; ++j) lk = fmin(lk, diag[j]);
-        for (int j = p - w; j < p; ++j) b = fmax(b, diag[j]);
-        // directions under CholeskyQR's pivot floor (1e-14 in the Gram matrix) are dropped, R_jj = 0: for
-        // the convergence of the others they count as lying at the floor
-        const double rho = lk / fmax(b, 2e-7 * l0);
-        double total = iters;
-        if (w > 0 && rho > 1.05) {
-            const double x = 2.0 * (lk / b) - 1.0, grow = x + sqrt(x * x - 1.0);
-            // growth of lambda_k over that of the largest, squared in the basis' Gram matrix
-            const double under = grow * b / (4.0 * l0);
-            if (under * under > 1e-13) {  // (false for b = 0: NaN)
-                cheb = true;
-                total = fmin((double)cap, kPre + ceil((36.0 - kPre * log(rho)) / log(grow)));
-                st[kMaxSince] = fmin(3.0, fmax(1.0, floor(5.5 / log10(4.0 * l0 / b))));
-                st[kProd] = 2.0 / b, st[kProd + 1] = -1.0;
-            } else {
-                total = fmin((double)iters, ceil(36.0 / log(rho)));
+        for (int j = p - w; j < p; ++j) b = fmax(b, diag[j]), lo = fmin(lo, diag[j]);
+        if (st[kStart] == 0.0) {
+            double l0 = 0.0, total = iters;
+            for (int j = 0; j < p; ++j) l0 = fmax(l0, diag[j]);
+            // directions under CholeskyQR's pivot floor (1e-14 in the Gram matrix) are dropped, R_jj = 0: for
+            // the convergence of the others they count as lying at the floor
+            const double floor_ = 2e-7 * l0, gap = lk / fmax(b, floor_);
+            if (w > 0 && it >= kPlain && b <= kSettled * st[kEdge] && gap > kMinGap) {  // (NaN: false)
+                const double x = 2.0 * (lk / b) - 1.0, grow = x + sqrt(x * x - 1.0);
+                // growth of lambda_k over that of the largest, squared in the basis' Gram matrix
+                const double under = grow * b / (4.0 * l0);
+                if (under * under > 1e-13) {  // (false for b = 0: NaN)
+                    const double need = fmin(kRounding, iters * log(kMargin * lk / fmax(lo, floor_)));
+                    st[kStart] = it;
+                    st[kConv] = it * log(gap);
+                    total = it + ceil((need - st[kConv] + log(2.0)) / log(grow));
+                    st[kMaxSince] = fmin(3.0, fmax(1.0, floor(5.5 / log10(4.0 * l0 / b))));
+                    st[kProd] = 2.0 / b, st[kProd + 1] = -1.0;
+                } else {
+                    total = ceil(kRounding / log(gap));
+                }
             }
+            st[kTotal] = fmin((double)iters, fmax(total, it + 1.0));
+            st[kEdge] = b;
+        } else {
+            const double s = st[kSince] + 1.0, gk = fmax(lk, 1.0), gb = fmax(b, 1.0);
+            const bool first = it == st[kStart] + s;  // T_s itself; later on growth per degree is exp
+            const double tk = (first ? acosh(gk) : log(gk)) / s, tb = (first ? acosh(gb) : log(gb)) / s;
+            st[kConv] += log(gk / gb);
+            double total = iters;
+            if (tk > tb + 1e-3) {
+                const double need = fmin(kRounding, iters * log(kMargin * (1.0 + cosh(tk)) / (1.0 + cosh(tb))));
+                total = it + ceil((need - st[kConv]) / (tk - tb));
+            }
+            st[kTotal] = fmin((double)iters, fmax(fmax(st[kTotal], total), it + 1.0));
         }
-        st[kTotal] = fmax(total, kPre + 1.0);
-        st[kCheb] = cheb;
-    } else if (cheb) {
-        if (it == kPre + 1) {
+    }
+    if (st[kStart] != 0.0 && it > st[kStart]) {
+        if (it == st[kStart] + 1.0) {
             st[kProd] *= 2.0, st[kProd + 1] = -2.0, st[kProd + 2] = -1.0;
         }
         if (diag) {
@@ -430,7 +466,7 @@ __global__ void __launch_bounds__(1024) k_chol_inv(SmallBatch B) {
         const bool done = P.st[kProd + 3] != 0.0, rest = P.st[kGram + 3] != 0.0;
         __syncthreads();  // before thread 0 writes the state
         if (rest) {
-            if (!done && tid == 0) rf_advance(P.st, nullptr, p, P.k, B.it, B.iters, B.cap);
+            if (!done && tid == 0) rf_advance(P.st, nullptr, p, P.k, B.it, B.iters);
             return;
         }
     }
@@ -505,7 +541,7 @@ __global__ void __launch_bounds__(1024) k_chol_inv(SmallBatch B) {
         __syncthreads();
         for (int i = tid; i < p; i += nt) A[i] = ldexp(Dv[256 * (i >> 4) + 17 * (i & 15)], -e2);  // the diagonal of R
         __syncthreads();
-        if (tid == 0) rf_advance(P.st, A, p, P.k, B.it, B.iters, B.cap);
+        if (tid == 0) rf_advance(P.st, A, p, P.k, B.it, B.iters);
     }
 }
 
@@ -2196,15 +2232,6 @@ static int gram_of_blocks(std::vector<Run> &rl, hipStream_t s) {
     return gemm_symmetric(g.data(), (int)g.size(), (void *)s);
 }
 
-// products after which the Chebyshev filter is at least as converged, for every lambda_k / lambda_{p+1},
-// as `iters` plain products are (to e^32: the hardest ratio is the one where those just get there): 13
-// for 20, 20 for 45
-static int filter_cap(int iters) {
-    const double r = exp(32.0 / iters);
-    const int d = (int)ceil((32.0 - kPre * 32.0 / iters) / acosh(2.0 * r - 1.0));
-    return d + kPre < iters ? d + kPre : iters;
-}
-
 // The filtered range finder on the Gram matrices: Y (orthonormal) -> basis, left in Y.
 static int rf_filtered(std::vector<Run> &rl, int iters, hipStream_t s) {
     for (Run &r : rl) {
@@ -2249,7 +2276,6 @@ static int rf_filtered(std::vector<Run> &rl, int iters, hipStream_t s) {
         proto.shift_rel = 1e-13;
         proto.it = it;
         proto.iters = iters;
-        proto.cap = filter_cap(iters);
         rc = small_launch(
             rl,
             [](Blk &b, SmallBatch &sb, int i) {
@@ -2262,9 +2288,9 @@ static int rf_filtered(std::vector<Run> &rl, int iters, hipStream_t s) {
             k_chol_inv, sizeof(double), sizeof(double) * (kNB + 1), proto, s);
         if (rc) return rc;
         if (it == iters) break;
-        // T_j R^{-1}, and from the second degree on T_{j-1} R^{-1}; the rounds up to there orthonormalise in
-        // every block, so the free buffers are T, then Y and Bm
-        const bool both = it > kPre;
+        // T_j R^{-1}, and from the first degree on T_{j-1} R^{-1}; the rounds up to there orthonormalise in
+        // every block, so the free buffers are T, and T and Bm at the first degree
+        const bool both = it > kPlain;
         for (Run &r : rl) {
             Blk &f = *r.f;
             const int64_t m = f.b.m, p = f.p;
@@ -2272,10 +2298,10 @@ static int rf_filtered(std::vector<Run> &rl, int iters, hipStream_t s) {
                 g.push_back(gdr(f.Y, p, 1, f.R, p, 1, f.T, p, m, p, p, r.n, r.dws, r.dws, r.dws));
                 ind.push_back(GemmIndirect{table(f.St, side ? kAp : kAq), nullptr, nullptr, table(f.St, side ? kDp : kDq),
                                            f.St + (side ? kApplyP : kApplyQ), r.dws});
-                out.push_back(side ? f.Bm : (both ? f.Y : f.T));
+                out.push_back(side ? f.Bm : f.T);
             }
         }
-        rc = product(it == 1 || it == kPre + 1);
+        rc = product(it == 1 || it == kPlain + 1);
         if (rc) return rc;
     }
     for (Run &r : rl) {

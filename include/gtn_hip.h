@@ -51,10 +51,11 @@ extern "C" {
 #define GTN_PREC_F64_GRAM 7 /* range finder of gtn_svd_blocks only: FP64 subspace iteration on the Gram
                              * matrix G = M M^T (formed once per call from its upper block triangle), one
                              * product G Y per iteration instead of M^T Y and M Z; blocks with m > n
-                             * use the alternating FP64 products.  After two products each block goes on
-                             * with Chebyshev polynomials of G and stops when its kept values have
-                             * converged, after at most `iters` products (13 for 20) that leave it no
-                             * further from converged than `iters` plain ones */
+                             * use the alternating FP64 products.  Once the edge of a block's basis has
+                             * settled (after three products at the earliest) it goes on with Chebyshev
+                             * polynomials of G, and stops where its kept space is as far from the rest as
+                             * `iters` plain products would bring it, by estimates from each CholeskyQR
+                             * that err towards more products; never more than `iters` */
 
 int gtn_version(void);
 
