@@ -4,6 +4,7 @@
 #include <stdlib.h>
 #include <string.h>
 #include <math.h>
+#include <algorithm>
 #include <vector>
 #include <utility>
 #include <map>
@@ -433,6 +434,9 @@ __global__ void k_permute_c128(PermArgs a, const double2 *__restrict__ src, doub
     }
 }
 
+// Workgroups of a gather at most (about: HIP refuses 2^32 work items in a dimension, 2^24 workgroups of 256)
+constexpr int64_t kMaxGrid = 1 << 23;
+
 // Tiled variant for gathers whose output's last axis is far apart in the source: output axis t1
 // (the one whose consecutive indices share the most source lines) and the last output axis t0 form
 // n1 x n0 tiles.  A tile is read with t1 fastest (consecutive source addresses), staged in LDS with its
@@ -443,6 +447,7 @@ __global__ void k_permute_c128(PermArgs a, const double2 *__restrict__ src, doub
 struct TileArgs {
     int32_t t0, t1, n_rest, tiles0, tiles1;
     int32_t sh0, sh1;  // n0 = 1 << sh0, n1 = 1 << sh1: 16, 32 or 64
+    uint32_t slot0;    // first tile of each XCD's share that this launch does
     int32_t rest_ax[AX];
     int64_t ostr[AX];
     int64_t rest_total;
@@ -460,9 +465,9 @@ __global__ void __launch_bounds__(256) k_permute_tiled(PermArgs a, TabArgs tb, T
     // element e = tid + 256 u of a tile: l1 = e % n1 (the same for every u), l0 = e / n1
     const int l1 = threadIdx.x & (n1 - 1), l0s = threadIdx.x >> t.sh1, l0d = 256 >> t.sh1;
     // one tile per workgroup, the tiles of an XCD consecutive (its L2 has the lines that neighbours share)
-    const uint32_t nblk = per * (uint32_t)t.rest_total, share = (nblk + 7) / 8;
-    const uint32_t blk = (blockIdx.x & 7) * share + (blockIdx.x >> 3);
-    if (blk < nblk && (blockIdx.x >> 3) < share) {
+    const uint32_t nblk = per * (uint32_t)t.rest_total, share = (nblk + 7) / 8, slot = t.slot0 + (blockIdx.x >> 3);
+    const uint32_t blk = (blockIdx.x & 7) * share + slot;
+    if (blk < nblk && slot < share) {
         uint32_t rr = per == 1 ? blk : blk / per;
         const uint32_t q = blk - rr * per;
         const int i1b = (int)(per == 1 ? 0 : q / (uint32_t)t.tiles0) << t.sh1;
@@ -1302,7 +1307,8 @@ static bool tiles_enabled() {
 // of two needs three axes and more for that, and a division a column (32^4 x 9 doubles: 64 us by
 // k_permute's walk, 35 by rows).  1024-column chunks for
 // gathers that still fill the device with them (four loads in flight per lane), 256 otherwise.  Each
-// workgroup takes up to 8 rows once there are more than 16 workgroups per compute unit without that.
+// workgroup takes up to 8 rows once there are more than 16 workgroups per compute unit without that, and more
+// where the grid would exceed kMaxGrid.
 static bool plan_rows(const PermArgs &a, const TabArgs &tb, RowArgs &w, int &U) {
     U = a.total >= (1 << 20) ? 4 : 1;
     for (;; U = 1) {
@@ -1317,9 +1323,9 @@ static bool plan_rows(const PermArgs &a, const TabArgs &tb, RowArgs &w, int &U) 
             w.rows = a.total / width;
             w.ns = ns;
             w.chunks = (int32_t)(width / chunk);
-            const int64_t per = w.rows * w.chunks / 4096;
-            w.rows_per = (int32_t)(per < 1 ? 1 : (per > 8 ? 8 : per));
-            if ((w.rows + w.rows_per - 1) / w.rows_per * w.chunks >= ((int64_t)1 << 31)) return false;
+            const int64_t per = w.rows * w.chunks / 4096, least = (w.rows * w.chunks + kMaxGrid - 1) / kMaxGrid;
+            w.rows_per = (int32_t)std::max<int64_t>(per < 1 ? 1 : (per > 8 ? 8 : per), least);
+            if ((w.rows + w.rows_per - 1) / w.rows_per * w.chunks >= 2 * kMaxGrid) return false;
             w.vary = 0;
             for (int k = 0; k < ns; ++k)
                 for (int g = 0; g < tb.ng; ++g)
@@ -1403,21 +1409,25 @@ int gtn_permute(const gtn_perm_desc *d, const void *src, void *dst, void *stream
         if (rc) return rc;
     }
     if (p.tile) {
-        const TileArgs &t = p.t;
+        TileArgs &t = p.t;
         const int64_t nblk = (int64_t)t.tiles0 * t.tiles1 * t.rest_total;
-        dim3 gt((unsigned)((nblk + 7) / 8 * 8)), bt(256);
         const size_t lds = sizeof(double) * ((size_t)1 << t.sh1) * ((1 << t.sh0) + 1);
+        // kMaxGrid tiles a launch, an eighth of them of each XCD's share
+        for (int64_t done = 0; done < (nblk + 7) / 8; done += kMaxGrid / 8) {
+            t.slot0 = (uint32_t)done;
+            const dim3 gt((unsigned)(8 * std::min((nblk + 7) / 8 - done, kMaxGrid / 8))), bt(256);
 #define GTN_TILES(T, B) \
     hipLaunchKernelGGL((k_permute_tiled<T, B>), gt, bt, lds, s, p.a, p.tb, t, (const T *)src, (T *)dst)
-        if (d->dtype == GTN_F64) {
-            if (p.tab) GTN_TILES(double, true);
-            else GTN_TILES(double, false);
-        } else {
-            if (p.tab) GTN_TILES(float, true);
-            else GTN_TILES(float, false);
-        }
+            if (d->dtype == GTN_F64) {
+                if (p.tab) GTN_TILES(double, true);
+                else GTN_TILES(double, false);
+            } else {
+                if (p.tab) GTN_TILES(float, true);
+                else GTN_TILES(float, false);
+            }
 #undef GTN_TILES
-        GTN_CHECK_LAUNCH();
+            GTN_CHECK_LAUNCH();
+        }
         return GTN_OK;
     }
     if (p.rows) {
