@@ -20,8 +20,8 @@ __device__ __forceinline__ float gelu_grad(float x) {
 }
 
 // The two elementwise passes run over 16-byte vectors where rows and buffers allow it (V = 4; V = 1
-// otherwise), the column index in 32 bits: at 5 x 4096 x 256 values 14 us became 11 (bias) and 14
-// 10.5 (derivative), against 10 at the rate of a large copy.
+// otherwise), without a division an element for the column: at 5 x 4096 x 256 values 14 us became 11
+// (bias) and 14 10.5 (derivative), against 10 at the rate of a large copy.
 template <int V>
 struct alignas(4 * V) Floats {
     float x[V];
@@ -96,19 +96,20 @@ __global__ void k_colsum_final(const double *part, int64_t E, int64_t c, float *
 }
 
 // dout = 2 w_j (out - target) / n; loss[e] = sum_{r,j} w_j (out - target)^2 / n; the target (n x c) is
-// shared by the members.  grid (E, 1 + blocks): the first workgroup of a member sums its loss (in a fixed
-// order, four loads in flight a lane), the others write dout.  One workgroup of 256 a member that did both,
+// shared by the members.  Of a member's workgroups (grid.y, counted from `first`) number 0 sums its loss (in a
+// fixed order, four loads in flight a lane), the others, `writers` of them, write dout.  One workgroup of 256 a member that did both,
 // an index division and a round trip to memory an element, took 138 us at 4096 x 17 values; this takes 13.5.
 constexpr int kMseBlock = 1024;
 __global__ void __launch_bounds__(kMseBlock) k_mse(const float *out, const float *target, const float *w, int64_t n, int64_t c,
-                                                   float *dout, double *loss) {
+                                                   float *dout, double *loss, int first, int writers) {
     __shared__ double sh[kMseBlock / 64];
     const int64_t e = blockIdx.x, total = n * c;
     const float *oe = out + e * total;
-    if (blockIdx.y > 0) {
+    const int number = first + (int)blockIdx.y;
+    if (number > 0) {
         float *de = dout + e * total;
-        const int64_t step = (int64_t)(gridDim.y - 1) * kMseBlock;
-        for (int64_t i = (int64_t)(blockIdx.y - 1) * kMseBlock + threadIdx.x; i < total; i += step) {
+        const int64_t step = (int64_t)writers * kMseBlock;
+        for (int64_t i = (int64_t)(number - 1) * kMseBlock + threadIdx.x; i < total; i += step) {
             const double d = (double)oe[i] - (double)target[i];
             de[i] = (float)(2.0 * w[i % c] * d / (double)n);
         }
@@ -226,8 +227,21 @@ int gtn_mlp_colsum(const float *x, int64_t E, int64_t n, int64_t c, float *out, 
 int gtn_mlp_mse(const float *out, const float *target, const float *weight, int64_t E, int64_t n, int64_t c, float *dout,
                 double *loss, void *stream) {
     GTN_REQUIRE(E >= 1 && n >= 1 && c >= 1 && out && target && weight && dout, "gtn_mlp_mse: bad argument");
-    hipLaunchKernelGGL(k_mse, dim3((unsigned)E, 1 + grid_for(n * c, kMseBlock, 256)), dim3(kMseBlock), 0, as_stream(stream),
-                       out, target, weight, n, c, dout, loss);
+    const int writers = grid_for(n * c, kMseBlock, 256);
+    hipStream_t s = as_stream(stream);
+    auto overlaps = [](const float *a, int64_t na, const float *b, int64_t nb) {
+        return (uintptr_t)a < (uintptr_t)(b + nb) && (uintptr_t)b < (uintptr_t)(a + na);
+    };
+    if (overlaps(dout, E * n * c, out, E * n * c) || overlaps(dout, E * n * c, target, n * c)) {
+        // in place: the loss is summed before anything is written
+        hipLaunchKernelGGL(k_mse, dim3((unsigned)E, 1), dim3(kMseBlock), 0, s, out, target, weight, n, c, dout, loss, 0, writers);
+        GTN_CHECK_LAUNCH();
+        hipLaunchKernelGGL(k_mse, dim3((unsigned)E, writers), dim3(kMseBlock), 0, s, out, target, weight, n, c, dout, loss, 1,
+                           writers);
+    } else {
+        hipLaunchKernelGGL(k_mse, dim3((unsigned)E, 1 + writers), dim3(kMseBlock), 0, s, out, target, weight, n, c, dout, loss,
+                           0, writers);
+    }
     GTN_CHECK_LAUNCH();
     return GTN_OK;
 }

@@ -356,7 +356,7 @@ int gtn_svd_blocks(const gtn_svd_block *blocks, int n_blocks, const gtn_svd_opts
  * gtn_mlp_colsum: out[e][j] = sum_r x[e][r][j] (bias gradients; FP64 accumulation in a fixed order:
  *   partial sums of row chunks in part_dev, gtn_mlp_colsum_workspace(E, c) bytes, then their sum).
  * gtn_mlp_mse: with target (n x c) shared by the members and weight (c): dout = 2 w_j (out - t) / n,
- *   loss[e] = sum w_j (out - t)^2 / n (loss may be NULL).
+ *   loss[e] = sum w_j (out - t)^2 / n (loss may be NULL); dout may take out's place.
  * gtn_adamw: AdamW (decoupled weight decay) on count parameters at step t = step[0] + 1, learning
  *   rate lr_min + (lr_max - lr_min) (1 + cos(pi (t - 1) / (total_steps - 1))) / 2; then step[0] += 1.
  * gtn_ensemble_stats: mean and population standard deviation over the E members (sd may be NULL).
