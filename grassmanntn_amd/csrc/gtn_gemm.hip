@@ -143,10 +143,10 @@ struct InnerPanels {
         kbytes = __builtin_amdgcn_readfirstlane((uint32_t)(sk * (int64_t)sizeof(T)));
         sbytes = __builtin_amdgcn_readfirstlane((uint32_t)((kc ? (256 / BK) * sr : (256 / ROWS) * sk) * (int64_t)sizeof(T)));
     }
-    // the slab fits the resource: rows R0 .. R0 + ROWS - 1 exist and all offsets stay below 2^31
+    // the slab fits the resource: rows R0 .. R0 + ROWS - 1 exist and the last element ends within 2^31 - 1 bytes
     static __device__ __forceinline__ bool fits(int64_t sr, int64_t sk, int R0, int R, int K) {
         return R0 + ROWS <= R && sr >= 0 && sk >= 0 &&
-               ((int64_t)(ROWS - 1) * sr + (int64_t)(K - 1) * sk) * (int64_t)sizeof(T) < ((int64_t)1 << 31);
+               ((int64_t)(ROWS - 1) * sr + (int64_t)(K - 1) * sk + 1) * (int64_t)sizeof(T) < ((int64_t)1 << 31);
     }
     __device__ __forceinline__ void load(int k0, double (&reg)[ROWS * BK / 256]) const {
         const uint32_t vo = voff0 + (uint32_t)k0 * kbytes;
@@ -571,7 +571,7 @@ struct InnerRows {
     }
     static __device__ __forceinline__ bool fits(const T *p, int64_t sr, int64_t sk, int R0, int R, int K) {
         return (KC ? sk == 1 && (((uint64_t)p) & 15) == 0 && (sr * (int64_t)sizeof(T)) % 16 == 0 : sr == 1) && R0 + ROWS <= R &&
-               sr >= 0 && sk >= 0 && ((int64_t)(ROWS - 1) * sr + (int64_t)(K - 1) * sk) * (int64_t)sizeof(T) < ((int64_t)1 << 31);
+               sr >= 0 && sk >= 0 && ((int64_t)(ROWS - 1) * sr + (int64_t)(K - 1) * sk + 1) * (int64_t)sizeof(T) < ((int64_t)1 << 31);
     }
     __device__ __forceinline__ void load(int k0) {
         const uint32_t vo = voff + (uint32_t)k0 * kbytes;
