@@ -67,10 +67,10 @@ int gemm_grouped_indirect(const gtn_gemm_desc *groups, const GemmIndirect *ind, 
 // and above the diagonal are computed, (1 + 1 / tiles) / 2 of the product, and stored on both sides
 int gemm_symmetric(const gtn_gemm_desc *groups, int n_groups, void *stream);
 
-// While one of these lives, this thread's grouped GEMMs hold the split reductions' workspace and
-// its lock throughout, and the event that orders other streams behind them is recorded once, by finish() (or
-// the destructor): a record between two launches leaves the device idle for 5.6 us, and a decomposition has
-// 50 split reductions.
+// While one of these lives, the event that orders other streams behind this thread's split reductions is
+// recorded once, by finish() (or the destructor), or by whoever uses their workspace on another stream before
+// that: a record between two launches leaves the device idle for 5.6 us, and a decomposition has
+// 50 split reductions.  The streams used live at least as long.  No lock is held between the reductions.
 class SplitScope {
 public:
     SplitScope();

@@ -835,43 +835,44 @@ __global__ void k_split_sum(const T *__restrict__ W, int splits, int M, int N, i
     }
 }
 
-// Split-K workspace: one grow-only buffer per device.  Launches on one stream are ordered; a launch
-// on another stream first waits for the event recorded after the buffer's last use (or, inside a
-// SplitScope, after the scope's last use).
+// Split-K workspace: one grow-only buffer per device, under g_ws_mu from a launch's look-up to its last use.
+// Launches on one stream are ordered; a launch on another stream first waits for the event recorded after
+// the buffer's last use.  Inside a SplitScope the record is left to the scope's end or to the first other
+// stream, whose thread records it behind all that the last stream has been given by then.
 struct SplitWs {
     void *p = nullptr;
     size_t bytes = 0;
     hipStream_t last = nullptr;
     hipEvent_t done = nullptr;
     bool used = false;
-    bool pending = false;  // used since the event was recorded (only while a SplitScope holds the lock)
+    const SplitScope *pending = nullptr;  // the scope whose use the event does not cover yet
 };
 static std::mutex g_ws_mu;
 static std::map<int, SplitWs> g_ws;
-static thread_local bool t_scope = false;          // this thread holds g_ws_mu through a SplitScope
-static thread_local SplitWs *t_scope_ws = nullptr;  // with uses that wait for their event
+static thread_local const SplitScope *t_scope = nullptr;  // this thread's open scope
 
 static int split_done(SplitWs &w) {
-    w.pending = false;
+    w.pending = nullptr;
     GTN_CHECK_HIP(hipEventRecord(w.done, w.last));
     return GTN_OK;
 }
 
-SplitScope::SplitScope() : outer_(t_scope) {
-    if (outer_) return;
-    g_ws_mu.lock();
-    t_scope = true;
+SplitScope::SplitScope() : outer_(t_scope != nullptr) {
+    if (!outer_) t_scope = this;
 }
 
 int SplitScope::finish() {
     if (!open_) return GTN_OK;
     open_ = false;
     if (outer_) return GTN_OK;
+    t_scope = nullptr;
     int rc = GTN_OK;
-    if (t_scope_ws && t_scope_ws->pending) rc = split_done(*t_scope_ws);
-    t_scope_ws = nullptr;
-    t_scope = false;
-    g_ws_mu.unlock();
+    std::lock_guard<std::mutex> l(g_ws_mu);
+    for (auto &kv : g_ws)
+        if (kv.second.pending == this) {
+            const int r = split_done(kv.second);
+            if (r) rc = r;
+        }
     return rc;
 }
 
@@ -1179,11 +1180,9 @@ static int gemm_grouped_impl(const gtn_gemm_desc *groups, int n_groups, int dtyp
                 } else {
                     int dev;
                     GTN_CHECK_HIP(hipGetDevice(&dev));
-                    if (!t_scope) lk.lock();
+                    lk.lock();
                     ws = &g_ws[dev];
-                    int rc = GTN_OK;
-                    if (t_scope_ws && t_scope_ws != ws && t_scope_ws->pending) rc = split_done(*t_scope_ws);  // another device
-                    if (!rc) rc = split_workspace(*ws, (size_t)need * es, s);
+                    int rc = split_workspace(*ws, (size_t)need * es, s);
                     if (rc) return rc;
                     base_ws = (char *)ws->p;
                 }
@@ -1229,8 +1228,7 @@ static int gemm_grouped_impl(const gtn_gemm_desc *groups, int n_groups, int dtyp
                 ws->last = s;
                 ws->used = true;
                 if (t_scope) {
-                    ws->pending = true;
-                    t_scope_ws = ws;
+                    ws->pending = t_scope;
                 } else {
                     int rcd = split_done(*ws);
                     if (rcd) return rcd;

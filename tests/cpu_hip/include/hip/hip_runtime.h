@@ -58,6 +58,7 @@ struct Idx {
 extern thread_local Idx tid, bid;
 extern Idx bdim, gdim;
 extern thread_local hipStream_t launch_stream;  // of the launch under way
+extern thread_local void *launch_kernel;
 void *dyn_lds();
 void sync_block();
 void sync_wave();
@@ -356,6 +357,7 @@ void run_grid(dim3 grid, dim3 block, size_t shm, void (*body)(void *), void *ctx
 template <typename... KArgs, typename... Args>
 inline void hipLaunchKernelGGL(void (*k)(KArgs...), dim3 grid, dim3 block, size_t shm, hipStream_t stream, Args... args) {
     emu::launch_stream = stream;
+    emu::launch_kernel = (void *)k;
     struct Ctx {
         void (*k)(KArgs...);
         std::tuple<KArgs...> a;

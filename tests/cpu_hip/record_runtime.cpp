@@ -5,6 +5,7 @@
 // tracked.
 #include <hip/hip_runtime.h>
 
+#include <dlfcn.h>
 #include <map>
 #include <set>
 #include <string>
@@ -13,6 +14,7 @@ namespace emu {
 thread_local Idx tid, bid;
 Idx bdim, gdim;
 thread_local hipStream_t launch_stream = nullptr;
+thread_local void *launch_kernel = nullptr;
 void *dyn_lds() { return nullptr; }
 void sync_block() {}
 void sync_wave() {}
@@ -24,11 +26,15 @@ namespace {
 struct Op {
     char kind;  // 'L' launch, 'R' event record, 'W' wait for an event, 'F' free, 'S' wait of the host
     hipStream_t stream;
-    void *what;
+    void *what;               // event, address or kernel
     unsigned long long grid;  // workgroups of a launch
     unsigned block;
 };
 std::mutex mu;
+std::condition_variable cv;
+hipStream_t held = nullptr;  // launches on this stream ...
+std::string held_kernel;     // ... of kernels with this in their name wait ...
+int launches_left = 0;       // ... after so many more of them
 std::vector<Op> ops;
 std::map<void *, size_t> live;
 int errors = 0;            // launches that HIP refuses
@@ -40,18 +46,28 @@ void log(Op o) {
 }
 }  // namespace
 
+extern "C" const char *rec_kernel(void *k) {
+    Dl_info i;
+    return dladdr(k, &i) && i.dli_sname ? i.dli_sname : "";
+}
+
 // HIP takes at most 2^32 - 1 work items in a dimension and 1024 in a workgroup
 void emu::run_grid(dim3 g, dim3 b, size_t shm, void (*)(void *), void *) {
     const bool bad = (unsigned long long)g.x * b.x >= (1ull << 32) || (unsigned long long)g.y * b.y >= (1ull << 32) ||
                      (unsigned long long)g.z * b.z >= (1ull << 32) || g.y > 65535 || g.z > 65535 || g.x == 0 || g.y == 0 ||
                      g.z == 0 || b.x * b.y * b.z > 1024 || shm > 160 * 1024;
-    std::lock_guard<std::mutex> l(mu);
+    std::unique_lock<std::mutex> l(mu);
+    auto mine = [] {
+        return held && held == emu::launch_stream && strstr(rec_kernel(emu::launch_kernel), held_kernel.c_str());
+    };
+    cv.wait(l, [&] { return !mine() || launches_left > 0; });
+    if (mine()) --launches_left;
     if (bad) {
         ++errors;
         last = 9;  // invalid configuration
         return;
     }
-    ops.push_back(Op{'L', emu::launch_stream, nullptr, (unsigned long long)g.x * g.y * g.z, b.x});
+    ops.push_back(Op{'L', emu::launch_stream, emu::launch_kernel, (unsigned long long)g.x * g.y * g.z, b.x});
 }
 
 extern "C" {
@@ -59,6 +75,15 @@ void rec_reset() {
     std::lock_guard<std::mutex> l(mu);
     ops.clear();
     errors = 0;
+}
+// launches of kernels named *kernel* on `stream` (null: none) wait once `after` more of them have been made, until
+// the next call
+void rec_hold(void *stream, const char *kernel, int after) {
+    std::lock_guard<std::mutex> l(mu);
+    held = stream;
+    held_kernel = kernel;
+    launches_left = after;
+    cv.notify_all();
 }
 int rec_errors() { return errors; }
 int rec_count() {

@@ -32,7 +32,7 @@ def build():
     with cf.ThreadPoolExecutor(4) as ex:
         objs = list(ex.map(compile_, srcs))
     tmp = "%s.%d" % (OUT, os.getpid())
-    subprocess.run([CXX, "-shared", "-Wl,-Bsymbolic", "-o", tmp] + objs + ["-lpthread"], check=True)
+    subprocess.run([CXX, "-shared", "-Wl,-Bsymbolic", "-o", tmp] + objs + ["-lpthread", "-ldl"], check=True)
     os.replace(tmp, OUT)
     for o in objs:
         os.remove(o)
@@ -41,11 +41,16 @@ def build():
 
 @functools.lru_cache(maxsize=1)
 def recorder():
-    return C.CDLL(build())
+    lib = C.CDLL(build())
+    lib.rec_kernel.restype = C.c_char_p
+    lib.rec_kernel.argtypes = [C.c_void_p]
+    lib.rec_hold.argtypes = [C.c_void_p, C.c_char_p, C.c_int]
+    lib.gtn_svd_workspace_bytes.restype = C.c_int64
+    return lib
 
 
 def ops(lib):
-    """[(kind, stream, event or address, workgroups, lanes a workgroup)] since the last rec_reset."""
+    """[(kind, stream, event, address or kernel, workgroups, lanes a workgroup)] since the last rec_reset."""
     out = []
     for i in range(lib.rec_count()):
         k, s, w, g, b = C.c_char(), C.c_void_p(), C.c_void_p(), C.c_ulonglong(), C.c_uint()
