@@ -9,6 +9,7 @@
 #include <utility>
 #include <map>
 #include <mutex>
+#include <shared_mutex>
 #include <string>
 
 namespace gtn {
@@ -1227,7 +1228,10 @@ struct TabCacheEntry {
     TabEntry *dev;
     int64_t entries;
 };
-static std::mutex g_tab_mu;
+// shared from a gather's look-up to its launch, exclusive while tables are built and dropped: a table that a
+// launch has been given is not released before that launch is on its stream
+static std::shared_mutex g_tab_mu;
+static std::mutex g_tab_turn;  // passed on the way in, and kept by who builds: launches do not keep it waiting forever
 static std::map<std::string, TabCacheEntry> g_tab_cache;
 static int64_t g_tab_bytes = 0;
 constexpr int64_t kTabCacheBytes = 64ll << 20;
@@ -1240,56 +1244,96 @@ static std::map<int, TabStore> g_tab_store;      // per device: the slab being c
 static std::vector<void *> g_tab_slabs;
 static std::map<int, hipStream_t> g_tab_stream;  // per device: the stream tables are built on
 
-static int tab_tables(const PermArgs &a, const TabBuild &tb, hipStream_t s, TabArgs &ta) {
+// one gather's tables: what they are made from, and where their addresses go
+struct TabWant {
+    const PermArgs *a;
+    const TabBuild *build;
+    TabArgs *out;
+    std::string key;
+};
+// held until the launch
+struct TabHold {
+    std::unique_lock<std::mutex> turn;
+    std::shared_lock<std::shared_mutex> shared;
+    std::unique_lock<std::shared_mutex> exclusive;
+};
+
+static int64_t tab_bytes(const TabBuild &b) { return (b.start[b.ng] * (int64_t)sizeof(TabEntry) + 255) / 256 * 256; }
+
+static int build_table(const TabWant &w, int dev) {
+    // tables are cut from slabs, one at a time in use per device; the build stream is kept with it
+    TabStore &store = g_tab_store[dev];
+    const int64_t n = w.build->start[w.build->ng], bytes = tab_bytes(*w.build);
+    if (store.left < bytes) {
+        const int64_t slab = bytes > kTabSlab ? bytes : kTabSlab;
+        void *p = nullptr;
+        GTN_CHECK_HIP(hipMalloc(&p, slab));
+        g_tab_slabs.push_back(p);
+        store.next = (char *)p;
+        store.left = slab;
+    }
+    hipStream_t &bs = g_tab_stream[dev];
+    if (!bs) GTN_CHECK_HIP(hipStreamCreateWithFlags(&bs, hipStreamNonBlocking));
+    // built on a stream of their own and finished here: the tables are shared by later gathers
+    // on any stream, and the caller's stream may be capturing a graph
+    TabEntry *p = (TabEntry *)store.next;
+    hipLaunchKernelGGL(k_perm_tables, dim3(grid_for(n, 256, 4096)), dim3(256), 0, bs, *w.a, *w.build, p);
+    GTN_CHECK_HIP(hipGetLastError());
+    GTN_CHECK_HIP(hipStreamSynchronize(bs));
+    store.next += bytes;
+    store.left -= bytes;
+    g_tab_cache.emplace(w.key, TabCacheEntry{p, n});
+    g_tab_bytes += bytes;
+    return GTN_OK;
+}
+
+static bool tab_find(const TabWant &w) {
+    auto it = g_tab_cache.find(w.key);
+    if (it == g_tab_cache.end()) return false;
+    for (int g = 0; g < w.build->ng; ++g) w.out->tab[g] = it->second.dev + w.build->start[g];
+    return true;
+}
+
+// The tables of `count` gathers (of one launch), built where they are not there yet; `hold` has to outlive the launch.
+static int tab_tables(TabWant *want, int count, TabHold &hold) {
     int dev;
     GTN_CHECK_HIP(hipGetDevice(&dev));
-    PermArgs k;
-    memcpy(&k, &a, sizeof(k));
-    memset(k.table, 0, sizeof(k.table));
-    k.alpha_re = k.alpha_im = 0.0;
-    std::string key((const char *)&dev, sizeof(dev));
-    key.append((const char *)&k, sizeof(k));
-    key.append((const char *)&tb, sizeof(tb));
-    std::lock_guard<std::mutex> l(g_tab_mu);
-    auto it = g_tab_cache.find(key);
-    if (it == g_tab_cache.end()) {
-        const int64_t n = tb.start[tb.ng];
-        // over budget: drop the cache, unless a graph may hold some of its tables
-        if (g_tab_bytes + n * (int64_t)sizeof(TabEntry) > kTabCacheBytes && !g_tab_cache.empty() &&
-            !graphs_alive() && !capture_open()) {
-            GTN_CHECK_HIP(hipDeviceSynchronize());
-            for (void *slab : g_tab_slabs) GTN_CHECK_HIP(hipFree(slab));
-            g_tab_slabs.clear();
-            g_tab_store.clear();
-            g_tab_cache.clear();
-            g_tab_bytes = 0;
-        }
-        // tables are cut from slabs, one at a time in use per device; the build stream is kept with it
-        TabStore &store = g_tab_store[dev];
-        const int64_t bytes = (n * (int64_t)sizeof(TabEntry) + 255) / 256 * 256;
-        if (store.left < bytes) {
-            const int64_t slab = bytes > kTabSlab ? bytes : kTabSlab;
-            void *p = nullptr;
-            GTN_CHECK_HIP(hipMalloc(&p, slab));
-            g_tab_slabs.push_back(p);
-            store.next = (char *)p;
-            store.left = slab;
-        }
-        hipStream_t &bs = g_tab_stream[dev];
-        if (!bs) GTN_CHECK_HIP(hipStreamCreateWithFlags(&bs, hipStreamNonBlocking));
-        // built on a stream of their own and finished here: the tables are shared by later gathers
-        // on any stream, and the caller's stream may be capturing a graph
-        TabEntry *p = (TabEntry *)store.next;
-        hipLaunchKernelGGL(k_perm_tables, dim3(grid_for(n, 256, 4096)), dim3(256), 0, bs, a, tb, p);
-        GTN_CHECK_HIP(hipGetLastError());
-        GTN_CHECK_HIP(hipStreamSynchronize(bs));
-        (void)s;
-        store.next += bytes;
-        store.left -= bytes;
-        it = g_tab_cache.emplace(key, TabCacheEntry{p, n}).first;
-        g_tab_bytes += bytes;
+    for (int i = 0; i < count; ++i) {
+        PermArgs k;
+        memcpy(&k, want[i].a, sizeof(k));
+        memset(k.table, 0, sizeof(k.table));
+        k.alpha_re = k.alpha_im = 0.0;
+        want[i].key.assign((const char *)&dev, sizeof(dev));
+        want[i].key.append((const char *)&k, sizeof(k));
+        want[i].key.append((const char *)want[i].build, sizeof(TabBuild));
     }
-    for (int g = 0; g < tb.ng; ++g) ta.tab[g] = it->second.dev + tb.start[g];
+    hold.turn = std::unique_lock<std::mutex>(g_tab_turn);
+    hold.shared = std::shared_lock<std::shared_mutex>(g_tab_mu);
+    hold.turn.unlock();
+    bool there = true;
+    for (int i = 0; i < count; ++i) there = tab_find(want[i]) && there;
+    if (there) return GTN_OK;
+    hold.shared.unlock();
+    hold.turn.lock();
+    hold.exclusive = std::unique_lock<std::shared_mutex>(g_tab_mu);
+    int64_t more = 0;
+    for (int i = 0; i < count; ++i) more += tab_find(want[i]) ? 0 : tab_bytes(*want[i].build);
+    // over budget: drop the cache, unless a graph may hold some of its tables
+    if (more && g_tab_bytes + more > kTabCacheBytes && !g_tab_cache.empty() && !graphs_alive() && !capture_open()) {
+        GTN_CHECK_HIP(hipDeviceSynchronize());
+        g_tab_store.clear();
+        g_tab_cache.clear();
+        g_tab_bytes = 0;
+        std::vector<void *> slabs;
+        slabs.swap(g_tab_slabs);
+        for (void *slab : slabs) GTN_CHECK_HIP(hipFree(slab));
+    }
+    for (int i = 0; i < count; ++i) {
+        if (tab_find(want[i])) continue;
+        int rc = build_table(want[i], dev);
+        if (rc) return rc;
+        (void)tab_find(want[i]);
+    }
     return GTN_OK;
 }
 
@@ -1404,8 +1448,10 @@ int gtn_permute(const gtn_perm_desc *d, const void *src, void *dst, void *stream
     p.a.alpha_im = a.alpha_im;
     p.tb.signs = (uint64_t)d->table[0] | (uint64_t)d->table[1] << 32;
     p.tb.short_signs = d->n_bits <= 5;
+    TabHold hold;
     if (p.tab) {
-        rc = tab_tables(p.a, p.build, s, p.tb);
+        TabWant want{&p.a, &p.build, &p.tb, {}};
+        rc = tab_tables(&want, 1, hold);
         if (rc) return rc;
     }
     if (p.tile) {
@@ -1494,8 +1540,12 @@ int gtn_permute2(const gtn_perm_desc *outer, const gtn_perm_desc *inner, const v
     tn.signs = (uint64_t)inner->table[0] | (uint64_t)inner->table[1] << 32;
     to.short_signs = outer->n_bits <= 5;
     tn.short_signs = inner->n_bits <= 5;
-    if (tabo && (rc = tab_tables(ao, bo, s, to))) return rc;
-    if (tabn && (rc = tab_tables(an, bn, s, tn))) return rc;
+    TabWant want[2];
+    int wants = 0;
+    if (tabo) want[wants++] = TabWant{&ao, &bo, &to, {}};
+    if (tabn) want[wants++] = TabWant{&an, &bn, &tn, {}};
+    TabHold hold;
+    if (wants && (rc = tab_tables(want, wants, hold))) return rc;
     dim3 g(grid_for((ao.total + kPermUnroll - 1) / kPermUnroll, 256, 1 << 20)), b(256);
 #define GTN_P2(T, A, B) hipLaunchKernelGGL((k_permute2<T, A, B>), g, b, 0, s, ao, to, an, tn, (const T *)src, (T *)dst)
     if (outer->dtype == GTN_F64) {

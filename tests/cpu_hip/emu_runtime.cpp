@@ -8,6 +8,7 @@ thread_local Idx tid, bid;
 Idx bdim, gdim;
 thread_local hipStream_t launch_stream = nullptr;
 thread_local void *launch_kernel = nullptr;
+thread_local size_t launch_bytes = 0;
 static thread_local int t_lane = 0, t_wave = 0;
 
 // barrier over the live threads of a group; a thread that leaves the kernel drops out

@@ -59,6 +59,7 @@ extern thread_local Idx tid, bid;
 extern Idx bdim, gdim;
 extern thread_local hipStream_t launch_stream;  // of the launch under way
 extern thread_local void *launch_kernel;
+extern thread_local size_t launch_bytes;  // of its arguments, ctx of run_grid
 void *dyn_lds();
 void sync_block();
 void sync_wave();
@@ -362,6 +363,7 @@ inline void hipLaunchKernelGGL(void (*k)(KArgs...), dim3 grid, dim3 block, size_
         void (*k)(KArgs...);
         std::tuple<KArgs...> a;
     } ctx{k, std::tuple<KArgs...>((KArgs)args...)};
+    emu::launch_bytes = sizeof(Ctx);
     emu::run_grid(grid, block, shm, [](void *p) {
         Ctx *c = (Ctx *)p;
         std::apply(c->k, c->a);

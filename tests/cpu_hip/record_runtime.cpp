@@ -15,6 +15,7 @@ thread_local Idx tid, bid;
 Idx bdim, gdim;
 thread_local hipStream_t launch_stream = nullptr;
 thread_local void *launch_kernel = nullptr;
+thread_local size_t launch_bytes = 0;
 void *dyn_lds() { return nullptr; }
 void sync_block() {}
 void sync_wave() {}
@@ -36,8 +37,10 @@ hipStream_t held = nullptr;  // launches on this stream ...
 std::string held_kernel;     // ... of kernels with this in their name wait ...
 int launches_left = 0;       // ... after so many more of them
 std::vector<Op> ops;
-std::map<void *, size_t> live;
+std::map<void *, size_t> live, freed;  // freed blocks are kept, so that no address is used twice
 int errors = 0;            // launches that HIP refuses
+int stale = 0;             // launches with an address in a freed block among their arguments
+void (*on_instantiate)() = nullptr;
 thread_local int last = 0;
 long next_handle = 16;
 void log(Op o) {
@@ -52,7 +55,7 @@ extern "C" const char *rec_kernel(void *k) {
 }
 
 // HIP takes at most 2^32 - 1 work items in a dimension and 1024 in a workgroup
-void emu::run_grid(dim3 g, dim3 b, size_t shm, void (*)(void *), void *) {
+void emu::run_grid(dim3 g, dim3 b, size_t shm, void (*)(void *), void *args) {
     const bool bad = (unsigned long long)g.x * b.x >= (1ull << 32) || (unsigned long long)g.y * b.y >= (1ull << 32) ||
                      (unsigned long long)g.z * b.z >= (1ull << 32) || g.y > 65535 || g.z > 65535 || g.x == 0 || g.y == 0 ||
                      g.z == 0 || b.x * b.y * b.z > 1024 || shm > 160 * 1024;
@@ -67,6 +70,14 @@ void emu::run_grid(dim3 g, dim3 b, size_t shm, void (*)(void *), void *) {
         last = 9;  // invalid configuration
         return;
     }
+    for (size_t i = 0; i + 8 <= emu::launch_bytes; i += 8) {
+        char *p = *(char **)((char *)args + i);
+        auto it = freed.upper_bound(p);
+        if (it != freed.begin() && p < (char *)std::prev(it)->first + std::prev(it)->second) {
+            ++stale;
+            break;
+        }
+    }
     ops.push_back(Op{'L', emu::launch_stream, emu::launch_kernel, (unsigned long long)g.x * g.y * g.z, b.x});
 }
 
@@ -74,8 +85,10 @@ extern "C" {
 void rec_reset() {
     std::lock_guard<std::mutex> l(mu);
     ops.clear();
-    errors = 0;
+    errors = stale = 0;
 }
+int rec_stale() { return stale; }
+void rec_on_instantiate(void (*f)()) { on_instantiate = f; }
 // launches of kernels named *kernel* on `stream` (null: none) wait once `after` more of them have been made, until
 // the next call
 void rec_hold(void *stream, const char *kernel, int after) {
@@ -118,9 +131,9 @@ hipError_t hipFree(void *p) {
     std::lock_guard<std::mutex> l(mu);
     auto it = live.find(p);
     if (it == live.end()) return 1;
+    freed[p] = it->second;
     live.erase(it);
     ops.push_back(Op{'F', nullptr, p, 0, 0});
-    free(p);
     return hipSuccess;
 }
 hipError_t hipMemGetInfo(size_t *f, size_t *t) {
@@ -179,12 +192,12 @@ hipError_t hipEventElapsedTime(float *ms, hipEvent_t, hipEvent_t) {
 hipError_t hipEventDestroy(hipEvent_t) { return hipSuccess; }
 hipError_t hipStreamCreateWithFlags(hipStream_t *s, unsigned) { return handle(s); }
 hipError_t hipStreamDestroy(hipStream_t) { return hipSuccess; }
-hipError_t hipStreamBeginCapture(hipStream_t, hipStreamCaptureMode) { return hipErrorNotSupported; }
-hipError_t hipStreamEndCapture(hipStream_t, hipGraph_t *g) {
-    *g = nullptr;
-    return hipErrorNotSupported;
+hipError_t hipStreamBeginCapture(hipStream_t, hipStreamCaptureMode) { return hipSuccess; }
+hipError_t hipStreamEndCapture(hipStream_t, hipGraph_t *g) { return handle(g); }
+hipError_t hipGraphInstantiate(hipGraphExec_t *x, hipGraph_t, hipGraphNode_t *, char *, size_t) {
+    if (on_instantiate) on_instantiate();
+    return handle(x);
 }
-hipError_t hipGraphInstantiate(hipGraphExec_t *, hipGraph_t, hipGraphNode_t *, char *, size_t) { return hipErrorNotSupported; }
 hipError_t hipGraphDestroy(hipGraph_t) { return hipSuccess; }
-hipError_t hipGraphLaunch(hipGraphExec_t, hipStream_t) { return hipErrorNotSupported; }
+hipError_t hipGraphLaunch(hipGraphExec_t, hipStream_t) { return hipSuccess; }
 hipError_t hipGraphExecDestroy(hipGraphExec_t) { return hipSuccess; }
