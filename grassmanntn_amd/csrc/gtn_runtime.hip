@@ -261,10 +261,13 @@ int gtn_graph_begin(void *stream, int pool) {
 
 int gtn_graph_end(void *stream, void **graph_exec) {
     GTN_REQUIRE(stream, "gtn_graph_end: null stream");
-    {
-        std::lock_guard<std::mutex> l(g_mu);
-        g_cur_pool = 0;
-    }
+    // the capture counts as open until its graph counts as alive: what the graph may hold is kept throughout
+    struct Close {
+        ~Close() {
+            std::lock_guard<std::mutex> l(g_mu);
+            g_cur_pool = 0;
+        }
+    } close;
     hipGraph_t g = nullptr;
     hipError_t e = hipStreamEndCapture(as_stream(stream), &g);
     if (e != hipSuccess || !g) {

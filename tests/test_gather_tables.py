@@ -82,3 +82,26 @@ def test_a_thread_about_to_launch_keeps_its_tables(lib):
     b.join(30)
     assert not a.is_alive() and not b.is_alive()
     assert lib.rec_stale() == 0
+
+
+def test_tables_of_a_capture_are_kept(lib):
+    """From the first capture to the last graph's end nothing that a graph may hold is dropped; that holds
+    for the moments between the capture's end and the graph's making too."""
+    alive, open_ = lib["_ZN3gtn12graphs_aliveEv"], lib["_ZN3gtn12capture_openEv"]
+    seen = []
+    hook = C.CFUNCTYPE(None)(lambda: seen.append(alive() or open_()))
+    lib.rec_on_instantiate(hook)
+    try:
+        s, x = C.c_void_p(STREAM), C.c_void_p()
+        assert lib.gtn_graph_begin(s, 1) == 0
+        d = _gather(144)
+        _permute(lib, d, STREAM)
+        assert lib.gtn_graph_end(s, C.byref(x)) == 0
+        for n in (152, 160, 168):
+            _permute(lib, _gather(n))
+        _permute(lib, d, STREAM)
+        assert lib.rec_stale() == 0 and seen and all(seen)
+        assert lib.gtn_graph_destroy(x) == 0
+        assert not alive() and not open_()
+    finally:
+        lib.rec_on_instantiate(None)
