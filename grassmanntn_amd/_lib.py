@@ -84,7 +84,7 @@ class AdamwOpts(C.Structure):
 class TuneEntry(C.Structure):
     _fields_ = [
         ("dtype", C.c_int32), ("precision", C.c_int32), ("n_groups", C.c_int32), ("tile", C.c_int32),
-        ("split_target", C.c_int32), ("pad_", C.c_int32), ("M", C.c_int64), ("N", C.c_int64), ("K", C.c_int64),
+        ("split_target", C.c_int32), ("kernel", C.c_int32), ("M", C.c_int64), ("N", C.c_int64), ("K", C.c_int64),
         ("batch", C.c_int64), ("ms_best", C.c_float), ("ms_default", C.c_float),
     ]
 
@@ -116,6 +116,7 @@ def _bind(lib):
         "gtn_permute2": (C.c_int, [C.POINTER(PermDesc), C.POINTER(PermDesc), vp, vp, vp]),
         "gtn_sign_tensor": (C.c_int, [i32, C.POINTER(C.c_int64), C.POINTER(C.c_uint32), vp, vp]),
         "gtn_gemm_grouped": (C.c_int, [C.POINTER(GemmDesc), i32, i32, i32, vp]),
+        "gtn_gemm_grouped_as": (C.c_int, [C.POINTER(GemmDesc), i32, i32, i32, i32, i32, i32, i32, vp]),
         "gtn_gemm_grouped_noalloc": (C.c_int, [C.POINTER(GemmDesc), i32, i32, i32, vp]),
         "gtn_gemm_noalloc_max_scratch": (C.c_int64, []),
         "gtn_mfma_selftest": (C.c_int, [vp, vp]),

@@ -1384,6 +1384,24 @@ extern "C" int gtn_gemm_grouped(const gtn_gemm_desc *groups, int n_groups, int d
                              nullptr, false, pipe);
 }
 
+extern "C" int gtn_gemm_grouped_as(const gtn_gemm_desc *groups, int n_groups, int dtype, int precision, int tile,
+                                   int split_target, int kernel, int symmetric, void *stream) {
+    GTN_REQUIRE(n_groups >= 0 && (n_groups == 0 || groups), "gtn_gemm_grouped_as: bad groups");
+    GTN_REQUIRE((tile == 64 || tile == 128) && split_target >= 0 && split_target <= 4096 && (kernel == 0 || kernel == 1),
+                "gtn_gemm_grouped_as: bad configuration");
+    GTN_REQUIRE(kernel == 0 || precision == GTN_PREC_F64 || (precision == GTN_PREC_F32 && dtype == GTN_F32),
+                "gtn_gemm_grouped_as: this precision has one kernel");
+    GTN_REQUIRE(!symmetric || (dtype == GTN_F64 && precision == GTN_PREC_F64), "gtn_gemm_grouped_as: symmetric products are FP64");
+    for (int i = 0; i < n_groups; ++i) {
+        const gtn_gemm_desc &d = groups[i];
+        if (d.M == 0 || d.N == 0 || d.batch == 0) continue;
+        GTN_REQUIRE(tile == 64 || (d.M >= 128 && d.N >= 128), "gtn_gemm_grouped_as: a group below the tile's size");
+        GTN_REQUIRE(!symmetric || (d.M == d.N && d.beta == 0.0), "gtn_gemm_grouped_as: not a symmetric product");
+    }
+    return gemm_grouped_impl(groups, n_groups, dtype, precision, stream, nullptr, 0, "gtn_gemm_grouped_as", tile, split_target,
+                             nullptr, symmetric != 0, kernel);
+}
+
 int gtn::gemm_symmetric(const gtn_gemm_desc *groups, int n_groups, void *stream) {
     for (int i = 0; i < n_groups; ++i)
         GTN_REQUIRE(groups[i].M == groups[i].N, "gtn_svd_blocks: a symmetric product is square");
@@ -1437,6 +1455,7 @@ extern "C" int gtn_autotune_report(gtn_tune_entry *out, int max_entries) {
         e.batch = k[7];
         e.tile = kv.second.tile;
         e.split_target = kv.second.target;
+        e.kernel = kv.second.pipe;
         e.ms_best = kv.second.ms;
         e.ms_default = kv.second.ms_default;
     }

@@ -218,20 +218,28 @@ int gtn_gemm_grouped(const gtn_gemm_desc *groups, int n_groups, int dtype, int p
  * layouts -- runs every candidate configuration (tile 64 or 128, the latter only where every group
  * is at least 128 x 128; split-K target off, 512, 1024 or 2048 workgroups) on its own operands, times
  * each with HIP events (best of 3), and keeps the fastest for every later call of that signature in
- * the process.  Calls issued while their stream is capturing a graph, and calls with beta != 0, are
+ * the process.  FP64 products, and FP32 ones of FP32 tensors, have a second kernel whose loads run under
+ * its matrix instructions (`kernel` 1); it is tried in both tiles at the split found best and at the
+ * usual one.  Calls issued while their stream is capturing a graph, and calls with beta != 0, are
  * never timed: they use the tuned configuration if there is one, else the heuristics (128 x 128 tiles
- * when every group is at least 128 x 128 and the launch has >= 256 of them; split-K towards 1024
- * workgroups when it has < 512 tiles).  Results are identical up to the summation order of split-K
- * partials.  gtn_autotune_report copies up to max_entries tuned signatures (first group's sizes) and
- * returns how many there are. */
+ * and the second kernel when every group is at least 128 x 128 and the launch has >= 256 tiles of that
+ * size; split-K towards 1024 workgroups when it has < 512 tiles).  Results are identical up to the order
+ * of summation.  gtn_autotune_report copies up to max_entries tuned signatures (first group's sizes) and
+ * returns how many there are.
+ * gtn_gemm_grouped_as: gtn_gemm_grouped with the configuration given by the caller (tests, tuning): tile 64 or
+ * 128, split target >= 0 (0: no split), kernel 0 or 1.  symmetric: products whose result is symmetric
+ * (FP64 throughout, M = N, beta = 0), of which the tiles on and above the diagonal are computed and stored
+ * on both sides. */
 typedef struct gtn_tune_entry {
-    int32_t dtype, precision, n_groups, tile, split_target, pad_;
+    int32_t dtype, precision, n_groups, tile, split_target, kernel;
     int64_t M, N, K, batch;
     float ms_best, ms_default;
 } gtn_tune_entry;
 int gtn_autotune_set(int on);
 int gtn_autotune_clear(void);
 int gtn_autotune_report(gtn_tune_entry *out, int max_entries);
+int gtn_gemm_grouped_as(const gtn_gemm_desc *groups, int n_groups, int dtype, int precision, int tile, int split_target,
+                        int kernel, int symmetric, void *stream);
 
 /* Allocation-free variant of gtn_gemm_grouped.  It has no counterpart in the reference: it is for
  * callers that cannot allocate device memory (code under HIP graph capture, tight serving loops,
