@@ -1278,13 +1278,23 @@ def _join_gather(T, string_inp, make_format="standard", intermediate_stat=None, 
     through = None
     if isinstance(T, _PermutedView) and T._data is None:
         through = (tuple(T._src.shape), tuple(T._order), tuple(T._codes), tuple(T._fbits))
-    P, view, fin_shape, fin_stats = _join_plan(string_inp, _legs(T), make_format, inter, blocks, through)
+    try:
+        plan = _join_plan(string_inp, _legs(T), make_format, inter, blocks, through)
+    except ValueError as e:
+        if not blocks:
+            raise
+        # (callers take a ValueError to mean that the groups have no parity blocks)
+        raise RuntimeError("the gather of %r could not be planned" % string_inp) from e
+    if plan is None:
+        raise ValueError("_join_gather: blocks=True needs two groups with fermionic legs")
+    P, view, fin_shape, fin_stats = plan
     return P, (T._src.data if view else T.data), fin_shape, fin_stats
 
 
 @_planned
 def _join_plan(string_inp, T, make_format, inter, blocks, through):
-    """through: (source shape, order, codes, fbits) of a permuted view that has not been materialised."""
+    """through: (source shape, order, codes, fbits) of a permuted view that has not been materialised.  None
+    where the groups have no parity blocks to write."""
     string_inp = denumerate(string_inp.replace(" ", ""))
     groups, srt = group_info(string_inp, T.statistics, T.shape)
     sgn_pos = _grouping_sign_axes(srt, inter)
@@ -1311,7 +1321,7 @@ def _join_plan(string_inp, T, make_format, inter, blocks, through):
         ok = (len(srt) in (2, 3) and (len(srt) == 2 or info[0][3] == 0)
               and all(info[g][3] and info[g][1] % 2 == 0 and inter[g] in FERMI for g in (-2, -1)))
         if not ok:
-            raise ValueError("_join_gather: blocks=True needs two groups with fermionic legs")
+            return None
         halves = []  # (virtual axes of the bosons and the fermions, their sizes) of the two groups
     for g, (chars, stg, dm, pos) in enumerate(srt):
         bd, fd, bn, fn, final = info[g]

@@ -47,3 +47,25 @@ def test_odd_tensors_are_refused(form):
         T = gtn.dense(np.random.default_rng(1).standard_normal(shape), statistics=stats)
         with pytest.raises(NameError):
             T.svd(part, 4)
+
+
+@pytest.mark.parametrize("batched", [False, True])
+def test_a_mistake_in_the_block_gather_is_not_taken_for_groups_without_blocks(batched, monkeypatch):
+    """A ValueError from planning the gather reaches the caller; it does not select the general path."""
+    with emulate():
+        import grassmanntn_amd as gtn
+        from grassmanntn_amd import batch, core
+        whole = core._join_plan
+
+        def planted(string, legs, fmt, inter, blocks, through):
+            if blocks:
+                raise ValueError("planted")
+            return whole(string, legs, fmt, inter, blocks, through)
+
+        monkeypatch.setattr(core, "_join_plan", planted)
+        X = random_even(np.random.default_rng(2), (4, 4, 4, 4), (1, 1, -1, -1)).data
+        with pytest.raises(Exception, match="could not be planned|planted"):
+            if batched:
+                batch.svd_batch([(gtn.dense(np.stack([X, X]), statistics=(0, 1, 1, -1, -1)), "ab|cd")], 4)
+            else:
+                gtn.dense(X, statistics=(1, 1, -1, -1)).svd("ab|cd", 4)
