@@ -234,7 +234,9 @@ def batched_path(gtn, P, steps, warmup, schedule, T0s):
 def rf_gemm_roofline(P, reps=20):
     """The batched step's dominant kernel: the range finder's FP64 GEMM of its parity blocks (4P blocks
     of 2048 x 2048 times 2048 x 128, one launch), run `reps` times on the same shape and timed with
-    HIP events on the library's stream.  Algorithmic work 2 M N K per block."""
+    HIP events on the library's stream.  The kernel is the step's k_gemm_fp in the faster of its tiles, with
+    the operands of plain products; the step's variant takes them from device memory and adds the
+    recurrence's two terms as it stores.  Algorithmic work 2 M N K per block."""
     import ctypes as C
     from grassmanntn_amd import _lib as L
     from grassmanntn_amd._device import DeviceArray, Event, synchronize
@@ -255,27 +257,28 @@ def rf_gemm_roofline(P, reps=20):
                    sab=m * k, sbb=k * p, scb=m * p)
     arr = (L.GemmDesc * 1)(d)
     lib = L.lib()
-    for _ in range(2):
-        L.check(lib.gtn_gemm_grouped(arr, 1, L.GTN_F64, L.PREC["f64"], L.stream_ptr()), "gemm")
-    synchronize()
-    e0, e1 = Event(), Event()
-    e0.record()
-    for _ in range(reps):
-        L.check(lib.gtn_gemm_grouped(arr, 1, L.GTN_F64, L.PREC["f64"], L.stream_ptr()), "gemm")
-    e1.record()
-    synchronize()
-    ms = e0.elapsed_ms(e1) / reps
+
+    def launch(tile):
+        L.check(lib.gtn_gemm_grouped_as(arr, 1, L.GTN_F64, L.PREC["f64"], tile, 0, 0, 0, L.stream_ptr()), "gemm")
+
+    def timed(tile, reps):
+        e0, e1 = Event(), Event()
+        e0.record()
+        for _ in range(reps):
+            launch(tile)
+        e1.record()
+        synchronize()
+        return e0.elapsed_ms(e1) / reps
+
+    for t in (64, 128):
+        timed(t, 2)
+    tile = min((64, 128), key=lambda t: timed(t, 3))
+    ms = timed(tile, reps)
     flop = 2.0 * m * p * k * nb
     ach = flop / (ms / 1000.0) / 1e12
-    # the launch configuration the autotuner settled on for this signature (first calls above)
-    tile = 128 if nb * (m // 128) >= 256 else 64
-    rep = (L.TuneEntry * 256)()
-    for e in rep[:min(lib.gtn_autotune_report(rep, 256), 256)]:
-        if (e.M, e.N, e.K, e.batch, e.n_groups, e.precision) == (m, p, k, nb, 1, L.PREC["f64"]):
-            tile = e.tile
     return {"bound": "mfma", "achieved": ach, "peak": MFMA_PEAK_TF["f64"], "unit": "TFLOP/s",
             "frac": ach / MFMA_PEAK_TF["f64"], "traffic": measured_traffic("rf_gemm_f64"),
-            "kernel": "range-finder GEMM (gtn_gemm_grouped, autotuned, %d x %d tiles): %d parity blocks of 2048 x 2048 "
+            "kernel": "range-finder GEMM (k_gemm_fp, %d x %d tiles, plain operands): %d parity blocks of 2048 x 2048 "
                       "times 2048 x 128 (N(0,1) entries) per launch, FP64" % (tile, tile, nb),
             "flop_per_launch": flop, "avg_launch_ms": ms, "launches": reps}
 
@@ -388,10 +391,11 @@ def main():
     ap.add_argument("--no-einsum", action="store_true", help="skip the standalone 'ijkl,klmn->ijmn' "
                     "contraction of two 64^4 tensors")
     ap.add_argument("--verbose", action="store_true", help="per-step progress and norms on stderr")
-    ap.add_argument("--svd-iters", type=int, default=0, help="subspace iterations of the block SVD "
-                    "(0: the library default)")
+    ap.add_argument("--svd-iters", type=int, default=0, help="subspace iterations of the block SVD, for the "
+                    "f64_gram range finder the most a block does (0: the library default)")
     ap.add_argument("--svd-orth-every", type=int, default=0, help="re-orthonormalise the range-finder "
-                    "basis every this many iterations (0: the library default)")
+                    "basis every this many iterations (0: the library default; the f64_gram range finder "
+                    "chooses this per block and takes no notice)")
     ap.add_argument("--svd-oversample", type=int, default=-1, help="range-finder columns beyond the kept "
                     "rank (-1: the library default)")
     args = ap.parse_args()
@@ -445,7 +449,8 @@ def main():
         "config": {"workload": "TRG at leg dim 64, chi 64: %d seeded site tensors (seeds %d..%d) coarse-grained "
                                "together for %d steps, one HIP-graph replay per step" % (P, SEED, SEED + P - 1, K),
                    "leg_dim": D, "chi": CHI, "points": P, "steps": K, "svd_iters": gtn.settings.svd_iters,
-                   "svd_oversample": gtn.settings.svd_oversample, "svd_orth_every": gtn.settings.svd_orth_every},
+                   "svd_oversample": gtn.settings.svd_oversample,
+                   "svd_orth_every": "per block" if mixed_sched(0)[1] == "f64_gram" else gtn.settings.svd_orth_every},
         "ms_per_point_step_mixed": mixed["gpu_ms"] / (P * K),
         "graph_prepare_s": mixed["prepare_s"],
     }
