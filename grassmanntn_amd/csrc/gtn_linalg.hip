@@ -309,17 +309,19 @@ __device__ __forceinline__ void chol_factor(double *A, int LD, double *Dv, int n
 //     kSettled in the last of them, and lambda_k is at least kMinGap times b.  Blocks that never get
 //     there do `iters` plain products.
 //   - It is to reach `need`, the logarithm of the separation that `iters` plain products would give: between
-//     R_kk and the smallest of the last R_jj, times kMargin; at most e^34 (rounding).
+//     R_kk and the smallest of the last R_jj, times kMargin; at most e^34 (rounding).  It does not start where
+//     `iters` products are too few for that: plain ones remove more of what lies far below b.
 //   - Each later R has the growth of its directions since the last on its diagonal.  The logarithm of the
 //     ratio of R_kk to the last R_jj is the separation reached (`kConv`); where the last ones grow, b was
 //     too small: need and the products left are estimated anew from both rates.  A block never does
 //     more than `iters` products.
-// Replayed in numpy for 584 geometric, plateau, stepped and random piecewise spectra (m 260 to 2048, k 4 to
-// 112), values and residuals are nowhere further off than those of `iters` plain products.  (With b and the
-// count fixed after two products 93 of them were: residuals of up to 7e-6 of sigma_0^2 and values of 3e-11
-// of sigma_0 on plateaus that plain products resolve to rounding.)  20 plain products become 6 to 15 on the
-// workloads' blocks (6 to 13 with that count), 15 on those of leg dim 64.  A margin of 1.1 saves one of the
-// 15 and leaves one of the random spectra ten times further off than plain products do.
+// Replayed in numpy for 734 geometric, plateau, stepped and random piecewise spectra (m 260 to 2048, k 4 to
+// 112), values and residuals are no further off than those of `iters` plain products for all but one, a
+// plateau wider than the basis that leaves a residual of 1e-9 of sigma_0^2 and not 1e-13.  (With b and the
+// count fixed after two products, 93 of the first 524 were: residuals of up to 7e-6 of sigma_0^2 and values of
+// 3e-11 of sigma_0 on plateaus that plain products resolve to rounding.)  20 plain products become 6 to 15 on
+// the workloads' blocks (6 to 13 with that count), 15 on those of leg dim 64.  A margin of 1.1 saves one of the
+// 15 and leaves one more of the random spectra ten times further off than plain products do.
 // Where a degree's growth of the largest eigenvalue would put the kept ones under CholeskyQR's pivot floor,
 // the block goes on with plain products, and stops when (lambda_k / b)^products has reached e^34.
 // The basis is orthonormalised only after as many degrees as keep the growth of the largest
@@ -396,11 +398,14 @@ __device__ void rf_advance(double *st, const double *diag, int p, int k, int it,
                 const double under = grow * b / (4.0 * l0);
                 if (under * under > 1e-13) {  // (false for b = 0: NaN)
                     const double need = fmin(kRounding, iters * log(kMargin * lk / fmax(lo, floor_)));
-                    st[kStart] = it;
-                    st[kConv] = it * log(gap);
-                    total = it + ceil((need - st[kConv] + log(2.0)) / log(grow));
-                    st[kMaxSince] = fmin(3.0, fmax(1.0, floor(5.5 / log10(4.0 * l0 / b))));
-                    st[kProd] = 2.0 / b, st[kProd + 1] = -1.0;
+                    const double conv = it * log(gap), last = it + ceil((need - conv + log(2.0)) / log(grow));
+                    if (last <= iters) {
+                        total = last;
+                        st[kStart] = it;
+                        st[kConv] = conv;
+                        st[kMaxSince] = fmin(3.0, fmax(1.0, floor(5.5 / log10(4.0 * l0 / b))));
+                        st[kProd] = 2.0 / b, st[kProd + 1] = -1.0;
+                    }
                 } else {
                     total = ceil(kRounding / log(gap));
                 }

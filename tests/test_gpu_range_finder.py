@@ -71,3 +71,12 @@ def test_blocks_that_start_and_stop_apart():
     i = np.arange(700)
     _compare([0.97 ** i, 0.999 ** i, np.where(i < 126, 1.0, 0.44), np.where(i < 9, 0.7 ** i, 0.0), np.maximum(0.8 ** i, 1e-7),
               np.where(i < 16, 1.0, np.where(i < 113, 0.5, 0.2))], 16)
+
+
+@pytest.mark.parametrize("edges,levels", [((100, 131, 246, 294, 295), (1.0, 0.32, 0.17, 0.067, 0.026, 0.013)),
+                                          ((100, 130, 222), (1.0, 0.393, 0.225, 0.177))])
+def test_small_gaps_over_a_deep_tail(edges, levels):
+    """A slow fall across the basis' width and steps behind it: the gap is small and the rest lies far below,
+    so plain products bring it to rounding in a count that the filter's growth does not suffice in."""
+    i = np.arange(700)
+    _compare([np.asarray(levels)[np.searchsorted(edges, i, side="right")] * np.exp(-0.002 * i)], 8)
