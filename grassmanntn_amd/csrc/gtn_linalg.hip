@@ -344,7 +344,7 @@ enum RfSlot {  // 8-byte slots of a block's state
     kApplyQ = 12, kGram = 16, kApplyP = 20,  // of the basis product of T_j, of the Gram matrix, of T_{j-1}
     kTotal = 24, kSince, kMaxSince,
     kStart,  // the product after which the filter started, 0: not yet
-    kEdge,   // b of the last round
+    kEdge,   // b of the last R
     kConv,   // logarithm of the separation reached
     kRfSlots = 32
 };
