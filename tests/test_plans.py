@@ -62,3 +62,25 @@ def test_kept_plans_give_what_new_ones_give(stats):
             new = outcome(c)
             assert type(new) is type(x) is type(y)
             assert np.array_equal(new, x) and np.array_equal(new, y) if not isinstance(new, str) else new == x == y
+
+
+@pytest.mark.parametrize("order", list(itertools.permutations(range(4)))[::5])
+def test_pairs_of_even_and_odd_operands(order):
+    """Contractions of fresh operands whose evenness is not known, the same shapes with both, one and none of
+    them even in any order: each as the oracle gives it, whatever plan an earlier pair has left."""
+    from oracle import gtn_oracle as O
+    stats, shape = (1, 1, -1, -1), (4, 2, 4, 2)
+    other, oshape = (1, 1, -1, -1), (4, 2, 2, 4)
+    with emulate():
+        import grassmanntn_amd as gtn
+        pairs = list(itertools.product((True, False), repeat=2))
+        for rep in range(2):
+            for i in order:
+                ea, eb = pairs[i]
+                rng = np.random.default_rng([rep, i])
+                X = random_even(rng, shape, stats).data if ea else rng.standard_normal(shape)
+                Y = random_even(rng, oshape, other).data if eb else rng.standard_normal(oshape)
+                got = gtn.einsum("ijkl,klmn->ijmn", gtn.dense(X, statistics=stats), gtn.dense(Y, statistics=other))
+                want = O.einsum("ijkl,klmn->ijmn", O.dense(X, statistics=stats), O.dense(Y, statistics=other))
+                np.testing.assert_allclose(got.numpy(), want.data, rtol=0, atol=1e-13)
+                assert got.is_even() == (ea and eb) or not np.any(want.data)
